@@ -52,7 +52,9 @@ def listed():
         {"name": "decode_ragged", "kind": "decode_seqs", "heads": 32, "d": 128, "ffn": 16384, "causal": True, "fused": True, "geglu": True,
          "cache_len": 1088, "batch": 11, "past": 1000},
         # The scheduler draining a mixed queue: prompts of different lengths, each followed by decode steps that requests share.
-        {"name": "queue_mixed", "kind": "queue", **fast, "cache_len": 576, "requests": 6, "seq": 500, "steps": 6},
+        # With residual connections, as every layer has that is meant to be iterated: without them one step's rounding grows
+        # two and a half times with every step that follows (random weights), and no two summation orders can be compared.
+        {"name": "queue_mixed", "kind": "queue", **fast, "pre_ln": True, "cache_len": 576, "requests": 6, "seq": 500, "steps": 6},
     ]
 
 
@@ -83,7 +85,7 @@ def _draw_once(rng):
     elif kind == "decode_seqs":
         c.update(kind="decode_seqs", fused=True, layers=1, cache_len=1088, batch=_log_int(rng, 2, 24), past=_log_int(rng, 64, 1087))
     else:
-        c.update(kind="queue", fused=True, layers=1, cache_len=576, requests=rng.randint(3, 8), seq=rng.randint(100, 512), steps=rng.randint(2, 8))
+        c.update(kind="queue", fused=True, pre_ln=True, layers=1, cache_len=576, requests=rng.randint(3, 8), seq=rng.randint(100, 512), steps=rng.randint(2, 8))
     return c
 
 
@@ -268,10 +270,7 @@ def work(case):
 def tolerance(case):
     """About four times what one implementation showed against the same layers computed by torch with fp64 sums and the same
     roundings between the kernels: fp32 1.6e-6 (largest element 8.4e-6 after two layers), fp16 6e-4 (one layer, fused) to 2.2e-3
-    (four layers), largest element 1.2e-2.  The decode steps of a queue start from one another's roundings."""
-    c = _full(case)
-    if c["dtype"] == "f32":
+    (four layers), largest element 1.2e-2."""
+    if _full(case)["dtype"] == "f32":
         return {"rel": 6e-6, "max": 4e-5}
-    if c["kind"] == "queue":
-        return {"rel": 1.6e-2, "max": 1e-1}
     return {"rel": 8e-3, "max": 5e-2}
