@@ -24,10 +24,12 @@ int check_launch(const char* what);
 // What is known about a stream (runtime.hip): the compute units its kernels may run on (fewer than the device for a CU-masked
 // stream) and its split-K workspace (nullptr for a stream the library neither created nor was told about with lg_stream_attach).
 constexpr size_t LG_SPLITK_WORKSPACE_BYTES = (size_t)64 << 20;
+constexpr int LG_ARRIVAL_COUNTERS = 4096;
 struct StreamInfo {
     int cus;
     float* ws;
     size_t ws_bytes;
+    unsigned* arrivals;  // LG_ARRIVAL_COUNTERS counters behind the workspace, zero between launches
 };
 StreamInfo stream_info(hipStream_t stream);
 int device_cu_count();

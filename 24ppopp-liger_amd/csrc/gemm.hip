@@ -12,10 +12,9 @@
 
 namespace lg {
 
-int launch_gemm_fast_f16(const GemmArgs& g, const GemmGroup& grp, int wlayout, int batch, hipStream_t stream, bool* handled);
 int launch_gemm_skinny_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled);
 int launch_gemv_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled);
-int launch_gemm_skinny_kn_f16(const GemmArgs& g, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled);
+int launch_gemm_skinny_sliced_f16(const GemmArgs& g, int wlayout, int batch, hipStream_t stream, bool* handled);
 
 // ---------------------------------------------------------------------------------------------------
 // fp16 generic kernel
@@ -165,18 +164,24 @@ static void launch_generic_epi(const GemmArgs& g, dim3 grid, hipStream_t stream)
     }
 }
 
+// The kernels that run a problem, or a group as one launch: the matrix-vector kernel (1-4 rows), the unsliced weight-streaming
+// kernel (few rows and features enough to give every compute unit two waves) and the tiles fitted to the token count.
+static int launch_one_problem(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled) {
+    int rc = launch_gemv_f16(g, grp, rows, wlayout, batch, stream, handled);
+    if (*handled) return rc;
+    rc = launch_gemm_skinny_f16(g, grp, rows, wlayout, batch, stream, handled);
+    if (*handled) return rc;
+    return launch_gemm_tiles_f16(g, grp, rows, wlayout, batch, stream, handled);
+}
+
 static int gemm_f16_dispatch(GemmArgs g, int wlayout, int batch, hipStream_t stream) {
     if (g.M == 0 || g.N == 0 || batch == 0) return LG_OK;
     if (g.K == 0) { set_error("gemm: k == 0 is not supported"); return LG_ERR_INVALID; }
     bool handled = false;
     const GemmGroup one = single_group(g);
-    int rc = launch_gemm_fast_f16(g, one, wlayout, batch, stream, &handled);
+    int rc = launch_one_problem(g, one, nullptr, wlayout, batch, stream, &handled);
     if (handled) return rc;
-    rc = launch_gemv_f16(g, one, nullptr, wlayout, batch, stream, &handled);
-    if (handled) return rc;
-    rc = launch_gemm_skinny_f16(g, one, nullptr, wlayout, batch, stream, &handled);
-    if (handled) return rc;
-    rc = launch_gemm_skinny_kn_f16(g, nullptr, wlayout, batch, stream, &handled);
+    rc = launch_gemm_skinny_sliced_f16(g, wlayout, batch, stream, &handled);
     if (handled) return rc;
     const bool aligned = aligned16(g.X) && aligned16(g.W) && aligned16(g.Y) && (g.ldx % 8 == 0) && (g.ldw % 8 == 0) &&
                          (g.strideX % 8 == 0) && (g.strideW % 8 == 0) && (g.strideY % 4 == 0) &&
@@ -472,7 +477,7 @@ int lg_gemm_fused_f16(int transa, int m, int n, int k, const void* A, int lda, c
     return gemm_f16_dispatch(g, transa == LG_OP_TILED ? W_TILED : (transa ? W_NK : W_KN), 1, (hipStream_t)stream);
 }
 
-// mode: -1 = choose the plan, 1 = one launch if the kernels allow it (a sub-group of a plan), 0 = member by member
+// mode: -1 = choose the plan, 1 = one launch if the kernels allow it (a sub-group of a plan)
 static int gemm_fused_grouped_f16_impl(int mode, int transa, int m, int n, int k, int count, const void* const* A, int lda, const void* B, int ldb,
                                        void* const* C, const int* ldc, int epilogue, const void* const* bias, int epi_arg0, int epi_arg1,
                                        int epi_arg2, void* stream) {
@@ -480,8 +485,8 @@ static int gemm_fused_grouped_f16_impl(int mode, int transa, int m, int n, int k
         set_error("gemm_fused_grouped_f16: count must be 1..%d and the pointer arrays non-null", LG_MAX_GROUP);
         return LG_ERR_INVALID;
     }
-    // the pipelined kernel (many token rows, either weight layout) and the weight-streaming kernels (few token rows, weights
-    // [out, in]) run the whole group as one launch; every other case is `count` plain calls
+    // One launch for the group, member by member, or in pieces: whichever the kernels' own estimate says is the fastest.  All
+    // ways give the same bits (the number of K-slices does not depend on it).
     GemmGroup grp{};
     grp.count = count;
     bool one_launch = m > 0 && n > 0 && k > 0 && count > 1 && B != nullptr;
@@ -492,45 +497,45 @@ static int gemm_fused_grouped_f16_impl(int mode, int transa, int m, int n, int k
         grp.ldy[i] = ldc[i];
         if (!A[i] || !C[i] || (epilogue != LG_EPI_NONE && !bias[i])) one_launch = false;  // the plain call reports it
     }
-    if (one_launch && n > 256) {
-        // Many token rows (the pipelined kernel's regime): one launch or member by member?  The members' tiles side by side may
-        // fill a round of workgroups that one member alone leaves half empty (384-768 token rows x 6144 features: one launch is
-        // 7-13 % faster per layer), or they may end in a mostly empty last round that three launches with a narrower tile avoid
-        // (1024 rows: 6 % slower).  What decides is rounds of workgroups x tile width for the best width either way, the
-        // quantity the pipelined kernel's launcher minimises; ties go to separate launches.  Both ways give the same bits.
+    const int wl = transa == LG_OP_TILED ? W_TILED : (transa ? W_NK : W_KN);
+    if (mode < 0 && one_launch && n > 64) {
+        constexpr double kLaunch = 1.5;  // microseconds between two launches
         const int cus = stream_info((hipStream_t)stream).cus;
-        const int tiles_m = (n + 255) / 256;
-        auto round_widths = [&](int members) {
-            long best = -1;
-            for (int nj = 4; nj >= 2; --nj) {
-                if (m % (64 * nj)) continue;
-                const long tiles = (long)tiles_m * (m / (64 * nj)) * members;
-                const long u = ((tiles + cus - 1) / cus) * nj;
-                if (best < 0 || u < best) best = u;
-            }
-            return best;
+        auto plan = [&](int members, int features) {
+            GemmArgs g{};
+            g.M = n; g.N = features; g.K = k;
+            g.X = (const half_t*)B; g.ldx = ldb;
+            g.W = grp.W[0]; g.ldw = lda;
+            g.Y = grp.Y[0]; g.ldy = grp.ldy[0];
+            g.epi = Epilogue{epilogue, grp.bias[0], epi_arg0, epi_arg1, epi_arg2, 0};
+            GemmGroup sub = grp;
+            sub.count = members;
+            return plan_gemm_tiles_f16(g, sub, wl, 1, (hipStream_t)stream);
         };
-        const long together = round_widths(count), apart = round_widths(1);
-        if (together > 0 && apart > 0 && together >= (long)count * apart) one_launch = false;
-        // A third plan for groups that are many full rounds plus a remainder (Q, K, V of 4096 rows x 6144 features: 72 columns
-        // of 256-wide tiles, 16 columns to a round of 256 workgroups, 8 left over): the members before the last as one launch
-        // of whole rounds of the widest tile, the last member's leading features as whole rounds too, and its remaining features
-        // as one round of 128-wide tiles -- instead of six rounds of 192-wide tiles either way (4.6-6.6 % faster, measured).
-        // Only taken when every launch but the last is whole rounds; pieces are addressed like any feature sub-range.
+        const TilePlan together = plan(count, m), apart = plan(1, m);
+        const double cost_apart = count * (apart.cost + kLaunch);
+        if (together.nsplit == 0 || (apart.nsplit != 0 && cost_apart < together.cost)) one_launch = false;
+        // A third way for groups that are many full rounds of workgroups plus a remainder (Q, K, V of 4096 rows x 6144 features: 72
+        // columns of 256-wide tiles, 16 columns to a round of 256 workgroups, 8 left over): the members before the last as one
+        // launch of whole rounds, the last member's leading features as whole rounds too, and its remaining features as one round
+        // of narrower tiles -- instead of six rounds of 192-wide tiles (4.6-6.6 % faster, measured).  Pieces are addressed like any
+        // feature sub-range.
         int split_at = 0;   // feature at which the last member is cut (0: no such plan)
+        const int tiles_m = (n + 255) / 256;
         const bool range_ok = epilogue == LG_EPI_NONE || epilogue == LG_EPI_BIAS || epilogue == LG_EPI_BIAS_GELU ||
                               (epilogue == LG_EPI_BIAS_HEADS && epi_arg1 > 0 && 256 % epi_arg1 == 0);
-        if (mode < 0 && range_ok && m % 256 == 0 && cus % tiles_m == 0 && (transa != LG_OP_TILED || lda == k)) {
+        if (range_ok && apart.nsplit == 1 && m % 256 == 0 && cus % tiles_m == 0 && (transa != LG_OP_TILED || lda == k)) {
             const int cols = m / 256, per_round = cus / tiles_m, rem = (count * cols) % per_round;
-            if (rem > 0 && rem < cols && ((count - 1) * cols) % per_round == 0 && (cols - rem) % per_round == 0 && 2 * rem * tiles_m <= cus)
-                split_at = (cols - rem) * 256;
+            if (rem > 0 && rem < cols && ((count - 1) * cols) % per_round == 0 && (cols - rem) % per_round == 0) {
+                const TilePlan lead = plan(count - 1, m), body = plan(1, (cols - rem) * 256), tail = plan(1, rem * 256);
+                const double pieces = lead.cost + body.cost + tail.cost + 3 * kLaunch;
+                if (lead.nsplit == 1 && body.nsplit == 1 && tail.nsplit == 1 && pieces < together.cost && pieces < cost_apart) split_at = (cols - rem) * 256;
+            }
         }
         // LG_GEMM_GROUP=1|0 in the environment (read once) forces one launch / member by member: a measurement knob
         static const int forced = [] { const char* e = getenv("LG_GEMM_GROUP"); return e ? atoi(e) : -1; }();
         if (forced == 0) { one_launch = false; split_at = 0; }
         else if (forced == 1) { one_launch = true; split_at = 0; }
-        if (mode == 0) one_launch = false;
-        else if (mode == 1) one_launch = true;
         if (split_at > 0) {
             int rc = count - 1 > 1 ? gemm_fused_grouped_f16_impl(1, transa, m, n, k, count - 1, A, lda, B, ldb, C, ldc, epilogue, bias, epi_arg0, epi_arg1,
                                                                  epilogue == LG_EPI_BIAS_HEADS && epi_arg2 == 0 ? m / epi_arg1 : epi_arg2, stream)
@@ -578,15 +583,8 @@ static int gemm_fused_grouped_f16_impl(int mode, int transa, int m, int n, int k
             g.Y = grp.Y[0]; g.ldy = grp.ldy[0]; g.strideY = 0;
             g.epi = Epilogue{epilogue, grp.bias[0], epi_arg0, epi_arg1, heads_total, 0};
             bool handled = false;
-            const int wl = transa == LG_OP_TILED ? W_TILED : (transa ? W_NK : W_KN);
-            int rc = launch_gemm_fast_f16(g, grp, wl, 1, (hipStream_t)stream, &handled);
+            int rc = launch_one_problem(g, grp, nullptr, wl, 1, (hipStream_t)stream, &handled);
             if (handled) return rc;
-            if (transa != 0) {
-                rc = launch_gemv_f16(g, grp, nullptr, wl, 1, (hipStream_t)stream, &handled);
-                if (handled) return rc;
-                rc = launch_gemm_skinny_f16(g, grp, nullptr, wl, 1, (hipStream_t)stream, &handled);
-                if (handled) return rc;
-            }
         }
     }
     for (int i = 0; i < count; ++i) {
@@ -641,37 +639,16 @@ int lg_gemm_fused_grouped_rows_f16(int transa, int m, int n, int k, int count, c
         grp.ldy[i] = ldc[i];
         grp.rows[i] = use_rows[i] ? 1 : 0;
     }
-    if (transa != 0) {
+    {
         GemmArgs g;
         g.M = n; g.N = m; g.K = k;
         g.X = (const half_t*)B; g.ldx = ldb; g.strideX = 0;
         g.W = grp.W[0]; g.ldw = lda; g.strideW = 0;
         g.Y = grp.Y[0]; g.ldy = grp.ldy[0]; g.strideY = 0;
         g.epi = Epilogue{LG_EPI_BIAS_HEADS_ROWS, grp.bias[0], 1, d, heads_total, grp.rows[0]};
-        const int wl = transa == LG_OP_TILED ? W_TILED : W_NK;
         bool handled = false;
-        int rc = launch_gemv_f16(g, grp, &rm, wl, 1, (hipStream_t)stream, &handled);
+        int rc = launch_one_problem(g, grp, &rm, transa == LG_OP_TILED ? W_TILED : (transa ? W_NK : W_KN), 1, (hipStream_t)stream, &handled);
         if (handled) return rc;
-        rc = launch_gemm_skinny_f16(g, grp, &rm, wl, 1, (hipStream_t)stream, &handled);
-        if (handled) return rc;
-    }
-    if (transa == 0) {
-        // weights stored [in, out]: one launch of the LDS-transposing weight-streaming kernel per member
-        bool all = true;
-        for (int i = 0; i < count && all; ++i) {
-            GemmArgs g;
-            g.M = n; g.N = m; g.K = k;
-            g.X = (const half_t*)B; g.ldx = ldb; g.strideX = 0;
-            g.W = grp.W[i]; g.ldw = lda; g.strideW = 0;
-            g.Y = grp.Y[i]; g.ldy = grp.ldy[i]; g.strideY = 0;
-            g.epi = Epilogue{LG_EPI_BIAS_HEADS_ROWS, grp.bias[i], 1, d, heads_total, grp.rows[i]};
-            bool handled = false;
-            int rc = launch_gemm_skinny_kn_f16(g, &rm, W_KN, 1, (hipStream_t)stream, &handled);
-            if (rc) return rc;
-            all = handled;
-            if (!handled && i > 0) { set_error("gemm_fused_grouped_rows_f16: members of one group must take the same kernel"); return LG_ERR_INVALID; }
-        }
-        if (all) return LG_OK;
     }
     // anything the weight-streaming kernels do not take: plain calls, one per member -- and one per token row for a member
     // whose rows go to their own places

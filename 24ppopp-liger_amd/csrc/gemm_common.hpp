@@ -168,9 +168,10 @@ __device__ __forceinline__ void barrier_keep_loads_in_flight() {
 typedef __attribute__((address_space(3))) void lds_void_t;
 typedef __attribute__((address_space(1))) const void gbl_void_t;
 
+template <int AUX = 0>  // cache policy bits of the instruction (2: non-temporal)
 __device__ __forceinline__ void load_lds16(const half_t* gptr, half_t* lds_wave_base) {
     // every lane supplies its own global address; the 64 x 16 bytes land contiguously at lds_wave_base
-    __builtin_amdgcn_global_load_lds((gbl_void_t*)gptr, (lds_void_t*)lds_wave_base, 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((gbl_void_t*)gptr, (lds_void_t*)lds_wave_base, 16, 0, AUX);
 }
 
 // swizzles: position (in 16-byte chunks) of logical chunk c in row r of the [rows][64] tiles; block (32 bytes) of
@@ -236,8 +237,17 @@ __device__ __forceinline__ void epilogue_geglu4(const GemmArgs& g, half_t* Yb, i
     }
 }
 
-// ---- split-K support shared by the weight-streaming and the pipelined kernel (gemm_skinny.hip) --------------------------
-constexpr int LG_EPI_PARTIAL = 100;  // kernel-internal: store the fp32 accumulators of K-slice `split` to partial[split][M][N]
+// ---- tile kernels (gemm_mid.hip): the choice made for a problem, or for `count` members of a group as one launch ---------------
+struct TilePlan {
+    double cost;   // estimated microseconds
+    int mi, nj;    // tile (32 mi) x (32 nj); the 256-row kernel: 256 x (64 nj)
+    int nsplit;    // K-slices (0: no tile kernel takes the problem)
+    bool fast;     // the 256-row kernel of gemm_fast.hip
+};
+TilePlan plan_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, int wlayout, int batch, hipStream_t stream);
+int launch_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled);
+
+// ---- split-K support of the weight-streaming kernel (gemm_skinny.hip) --------------------------
 // The fp32 partials live in the stream's workspace (StreamInfo::ws, allocated when the stream was created or attached); a
 // launcher never allocates: with no workspace, or one that is too small, it slices K less or not at all.
 // Y = epilogue(sum over the nsplit K-slices in slice order) of the fp32 partials [nsplit][M][N]

@@ -1,8 +1,8 @@
 // gemm_fast.hip -- pipelined 256x256x64 fp16 GEMM for gfx950 (the prefill shapes of the launch vector).
 //
 //   Y[M, N] = X[M, K] * W,  W row-major [K, N] (the reference's layout) or [N, K];  fp32 accumulate, optional fused
-//   epilogue.  Requires N % 128 == 0 (or % 192), K % 64 == 0, M > 64 (any M; a partial last row of tiles is padded) and 16-byte aligned operands; everything else goes to
-//   the generic kernel in gemm.hip.
+//   epilogue.  Requires N % 256 == 0 (or % 192), K % 64 == 0, any M (a partial last row of tiles is padded) and 16-byte aligned
+//   operands.  gemm_mid.hip chooses between this kernel (many rows of tiles) and tiles fitted to the token count.
 //
 // Structure (one workgroup = 8 waves = one 256x256 output tile, one workgroup per CU):
 //   * global -> LDS with direct-to-LDS loads (global_load_lds_dwordx4): no VGPR staging, each wave instruction fills
@@ -49,7 +49,7 @@ template <int NJ> __device__ __forceinline__ int unswz_kn(int k, int blk) {
 }
 
 template <int WL, int EPI, int NJ>
-__global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup grp, int tiles_m, int tiles_n, float* partial, int kt_per_split, int cus, int wide_store) {
+__global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup grp, int tiles_m, int tiles_n, int cus, int wide_store) {
     constexpr int FB_N = 64 * NJ;
     constexpr int X_TILE = FB_M * FB_K, W_TILE = FB_K * FB_N;  // halves per ring slot
     constexpr int WCH = (FB_K * FB_N) / 512 / 8;  // 1 KiB chunks of the W tile per wave (= NJ)
@@ -109,15 +109,10 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup
         g.ldy = grp.ldy[member];
     }
     const int m0 = tm * FB_M, n0 = tn * FB_N;
-    // K-slice of this workgroup (blockIdx.y; the whole K when the launch is not split): k-tiles [kt0, kt0 + ktiles)
-    const int split = blockIdx.y;
-    const int kt0 = split * kt_per_split;
-    const int ktiles = min(g.K / FB_K - kt0, kt_per_split);
-    const half_t* X = g.X + (int64_t)m0 * g.ldx + (int64_t)kt0 * FB_K;
+    const int ktiles = g.K / FB_K;
+    const half_t* X = g.X + (int64_t)m0 * g.ldx;
     // tiled weights: feature tile n0 / 16 starts n0 * K elements in, and a k-tile of 64 is two consecutive 512-element blocks
-    const half_t* W = (WL == W_KN)   ? g.W + n0 + (int64_t)kt0 * FB_K * g.ldw
-                      : (WL == W_NK) ? g.W + (int64_t)n0 * g.ldw + (int64_t)kt0 * FB_K
-                                     : g.W + (int64_t)n0 * g.ldw + (int64_t)kt0 * 1024;
+    const half_t* W = (WL == W_KN) ? g.W + n0 : g.W + (int64_t)n0 * g.ldw;
 
     // ---- per-lane global offsets of the 8 direct-to-LDS loads of one k-tile ---------------------------------------------
     // X tile (and W tile when [N, K]): 32 chunks of 1 KiB = 8 rows x 128 B; wave w fills chunks w, w+8, w+16, w+24.
@@ -281,18 +276,6 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup
     // ---- epilogue: acc[i][j][r] = Y[m0 + wm*128 + i*16 + l16][n0 + wn*16*NJ + j*16 + 4*lk + r] -----------------------------
     // Everything that depends only on the column (bias, head offset) or only on the row (batch / position split) is
     // computed once, so the 8 x NJ stores of a lane are not separated by dependent loads or integer divisions.
-    if (EPI == LG_EPI_PARTIAL) {
-        // split-K: the fp32 accumulators of this K-slice go to partial[split][M][N]; a second kernel sums the slices
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int m = m0 + wm * 128 + i * 16 + l16;
-            if (m >= g.M) continue;
-            float* prow = partial + ((int64_t)split * g.M + m) * g.N + n0 + wn * (16 * NJ) + 4 * lk;
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) *reinterpret_cast<float4_t*>(prow + j * 16) = acc[i][j];
-        }
-        return;
-    }
     if (EPI == LG_EPI_BIAS_GEGLU) {
         // the wave's 16-feature tiles are (gate, up) pairs (NJ even): out[m][(n / 32) * 16 + n % 16 ..] = gelu(gate + b) * (up + b)
         float bg[NJ / 2 + 1][4], bu[NJ / 2 + 1][4];
@@ -327,7 +310,7 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup
 #pragma unroll
     for (int j = 0; j < NJ; ++j) {
         const int n = n0 + wn * (16 * NJ) + j * 16 + 4 * lk;
-        if (EPI != LG_EPI_NONE && EPI != LG_EPI_PARTIAL) {
+        if (EPI != LG_EPI_NONE) {
             const half4_t bv = *reinterpret_cast<const half4_t*>(g.epi.bias + n);
 #pragma unroll
             for (int r = 0; r < 4; ++r) bias_v[j][r] = (float)bv[r];
@@ -411,27 +394,9 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup
 }
 
 template <int WL, int NJ>
-static int launch_fast_epi(const GemmArgs& g, const GemmGroup& grp, int tiles_m, int tiles_n, const StreamInfo& si, hipStream_t stream) {
-    const int tiles = tiles_m * tiles_n, ktiles = g.K / FB_K;
+static void launch_fast_epi(const GemmArgs& g, const GemmGroup& grp, int tiles_m, int tiles_n, const StreamInfo& si, hipStream_t stream) {
     const int cus = si.cus;
-    // At most 256 token rows (one row of tiles, the continuation of the weight-streaming kernel's regime): the time is set by
-    // how fast the weights stream in, so K is split over otherwise idle CUs (slices of >= 8 k-tiles, fp32 partials in the
-    // stream's workspace, summed in slice order by a second kernel that applies the epilogue; no more slices than the workspace
-    // holds, none on a stream without one).  Larger M never splits K, so that a token row's result does not depend on how many
-    // other rows are in the batch (each output is one sequential sum over k).
-    int nsplit = 1;
-    if (tiles_m == 1 && tiles <= cus / 2 && si.ws && grp.count == 1) {
-        nsplit = cus / tiles;
-        if (nsplit > ktiles / 8) nsplit = ktiles / 8;
-        if (nsplit > 16) nsplit = 16;
-        const size_t slice_bytes = (size_t)g.M * g.N * sizeof(float);
-        if ((size_t)nsplit * slice_bytes > si.ws_bytes) nsplit = (int)(si.ws_bytes / slice_bytes);
-        if (nsplit < 1) nsplit = 1;
-    }
-    int kt_per_split = (ktiles + nsplit - 1) / nsplit;
-    nsplit = (ktiles + kt_per_split - 1) / kt_per_split;
-    float* partial = nsplit > 1 ? si.ws : nullptr;
-    const dim3 grid(tiles, nsplit), block(F_THREADS);
+    const dim3 grid(tiles_m * tiles_n), block(F_THREADS);
     const size_t smem = lds_halves(NJ) * sizeof(half_t);
     // whole-row stores through LDS need 16-byte aligned rows (heads epilogue: rows of size_per_head halves)
     static const int wide_forced = [] { const char* e = getenv("LG_GEMM_WIDE_STORE"); return e ? atoi(e) : -1; }();
@@ -444,78 +409,37 @@ static int launch_fast_epi(const GemmArgs& g, const GemmGroup& grp, int tiles_m,
         /* set once per instantiation; the initialisation of a function-local static is thread-safe */              \
         static const hipError_t attr_rc = hipFuncSetAttribute((const void*)gemm_f16_fast<WL, E, NJ>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem); \
         (void)attr_rc;                                                                                              \
-        hipLaunchKernelGGL((gemm_f16_fast<WL, E, NJ>), grid, block, smem, stream, g, grp, tiles_m, tiles_n, partial, kt_per_split, cus, wide); \
+        hipLaunchKernelGGL((gemm_f16_fast<WL, E, NJ>), grid, block, smem, stream, g, grp, tiles_m, tiles_n, cus, wide); \
     } while (0)
-    if (nsplit > 1) {
-        LG_FAST(LG_EPI_PARTIAL);
-        launch_splitk_reduce(g, partial, nsplit, stream);
-    } else {
-        switch (g.epi.kind) {
-            case LG_EPI_NONE: LG_FAST(LG_EPI_NONE); break;
-            case LG_EPI_BIAS: LG_FAST(LG_EPI_BIAS); break;
-            case LG_EPI_BIAS_GELU: LG_FAST(LG_EPI_BIAS_GELU); break;
-            case LG_EPI_BIAS_GEGLU:
-                if constexpr (NJ % 2 == 0) LG_FAST(LG_EPI_BIAS_GEGLU);  // the launcher picks an even tile width for it
-                break;
-            default: LG_FAST(LG_EPI_BIAS_HEADS); break;
-        }
+    switch (g.epi.kind) {
+        case LG_EPI_NONE: LG_FAST(LG_EPI_NONE); break;
+        case LG_EPI_BIAS: LG_FAST(LG_EPI_BIAS); break;
+        case LG_EPI_BIAS_GELU: LG_FAST(LG_EPI_BIAS_GELU); break;
+        case LG_EPI_BIAS_GEGLU:
+            if constexpr (NJ % 2 == 0) LG_FAST(LG_EPI_BIAS_GEGLU);  // the plan picks an even tile width for it
+            break;
+        default: LG_FAST(LG_EPI_BIAS_HEADS); break;
     }
 #undef LG_FAST
-    return LG_OK;
 }
 
-int launch_gemm_fast_f16(const GemmArgs& g, const GemmGroup& grp, int wlayout, int batch, hipStream_t stream, bool* handled) {
-    *handled = false;
-    if (batch != 1) return LG_OK;
-    if (g.K % FB_K || g.M <= 0 || g.N <= 0 || g.K <= 0) return LG_OK;
-    // A partial last row of tiles computes (and discards) up to 255 extra token rows.  Even so this kernel is the faster one
-    // for every token count the weight-streaming kernel does not take (M = 128: 182 us vs 331 us in the generic kernel for a
-    // 16384 x 12288 weight), because with few token rows the time is set by how fast the weights stream in.
-    if (g.M <= 64) return LG_OK;
-    if (!aligned16(g.X) || (g.ldx % 8) || (g.ldw % 8)) return LG_OK;
-    if (g.ldx >= (1 << 22) || g.ldw >= (1 << 22)) return LG_OK;  // 256 rows x ld must fit the 31-bit tile offsets
-    if (wlayout == W_TILED && g.ldw != g.K) return LG_OK;
-    for (int i = 0; i < grp.count; ++i) {
-        if (!aligned16(grp.W[i]) || !aligned16(grp.Y[i])) return LG_OK;
-        if (g.epi.kind == LG_EPI_BIAS_HEADS ? (g.epi.d % 4 != 0) : (grp.ldy[i] % 4 != 0)) return LG_OK;
-        if (g.epi.kind != LG_EPI_NONE && (reinterpret_cast<uintptr_t>(grp.bias[i]) & 7u)) return LG_OK;  // 8-byte bias loads
-    }
-    if (grp.count > 1 && g.M <= FB_M) return LG_OK;  // one row of tiles may want K-slices, which take single problems only
-    // tile width: the one that needs the least work-rounds on the stream's CUs (rounds x tile width); ties go to the wider tile
-    const StreamInfo si = stream_info(stream);
-    const int tiles_m = (g.M + FB_M - 1) / FB_M;
-    int best_nj = 0;
-    long best_cost = 0;
-    for (int nj = 4; nj >= 2; --nj) {
-        if (g.N % (64 * nj)) continue;
-        if (nj == 3 && g.epi.kind == LG_EPI_BIAS_GEGLU) continue;  // a wave must hold whole (gate, up) pairs of 16-feature tiles
-        const long tiles = (long)tiles_m * (g.N / (64 * nj)) * grp.count;
-        // narrower tiles move more operand bytes per flop: about 3 % / 35 % more time per unit of width (measured)
-        const long cost = ((tiles + si.cus - 1) / si.cus) * nj * (nj == 4 ? 100 : nj == 3 ? 103 : 135);
-        if (!best_nj || cost < best_cost) { best_nj = nj; best_cost = cost; }
-    }
+// nj: tile width in units of 64 features (gemm_mid.hip chooses it)
+void launch_gemm_fast_tile(const GemmArgs& g, const GemmGroup& grp, int wlayout, int nj, const StreamInfo& si, hipStream_t stream) {
     // LG_GEMM_TILE_WIDTH=2|3|4 in the environment (read once) overrides the choice where that width divides N: a measurement knob
     // (256 x 128 tiles leave registers and LDS for a second kernel's waves on the same compute unit)
     static const int forced_nj = [] { const char* e = getenv("LG_GEMM_TILE_WIDTH"); return e ? atoi(e) : 0; }();
-    if (forced_nj >= 2 && forced_nj <= 4 && g.N % (64 * forced_nj) == 0 && !(forced_nj == 3 && g.epi.kind == LG_EPI_BIAS_GEGLU)) best_nj = forced_nj;
-    if (!best_nj) return LG_OK;
-    *handled = true;
-    const int tiles_n = g.N / (64 * best_nj) * grp.count;
-    int rc;
-    if (wlayout == W_TILED) {
-        if (best_nj == 4) rc = launch_fast_epi<W_TILED, 4>(g, grp, tiles_m, tiles_n, si, stream);
-        else if (best_nj == 3) rc = launch_fast_epi<W_TILED, 3>(g, grp, tiles_m, tiles_n, si, stream);
-        else rc = launch_fast_epi<W_TILED, 2>(g, grp, tiles_m, tiles_n, si, stream);
-    } else if (wlayout == W_NK) {
-        if (best_nj == 4) rc = launch_fast_epi<W_NK, 4>(g, grp, tiles_m, tiles_n, si, stream);
-        else if (best_nj == 3) rc = launch_fast_epi<W_NK, 3>(g, grp, tiles_m, tiles_n, si, stream);
-        else rc = launch_fast_epi<W_NK, 2>(g, grp, tiles_m, tiles_n, si, stream);
-    } else {
-        if (best_nj == 4) rc = launch_fast_epi<W_KN, 4>(g, grp, tiles_m, tiles_n, si, stream);
-        else if (best_nj == 3) rc = launch_fast_epi<W_KN, 3>(g, grp, tiles_m, tiles_n, si, stream);
-        else rc = launch_fast_epi<W_KN, 2>(g, grp, tiles_m, tiles_n, si, stream);
-    }
-    return rc != LG_OK ? rc : check_launch("gemm_f16_fast");
+    if (forced_nj >= 2 && forced_nj <= 4 && g.N % (64 * forced_nj) == 0 && !(forced_nj == 3 && g.epi.kind == LG_EPI_BIAS_GEGLU)) nj = forced_nj;
+    const int tiles_m = (g.M + FB_M - 1) / FB_M, tiles_n = g.N / (64 * nj) * grp.count;
+#define LG_FAST_WIDTHS(WL)                                                                   \
+    do {                                                                                     \
+        if (nj == 4) launch_fast_epi<WL, 4>(g, grp, tiles_m, tiles_n, si, stream);           \
+        else if (nj == 3) launch_fast_epi<WL, 3>(g, grp, tiles_m, tiles_n, si, stream);      \
+        else launch_fast_epi<WL, 2>(g, grp, tiles_m, tiles_n, si, stream);                   \
+    } while (0)
+    if (wlayout == W_TILED) LG_FAST_WIDTHS(W_TILED);
+    else if (wlayout == W_NK) LG_FAST_WIDTHS(W_NK);
+    else LG_FAST_WIDTHS(W_KN);
+#undef LG_FAST_WIDTHS
 }
 
 }  // namespace lg

@@ -1,0 +1,149 @@
+// gemm_mid.hip -- which tile, and how many K-slices, an fp16 GEMM takes: the instantiations of gemm_mid.hpp and the 256-row
+// kernel of gemm_fast.hip compared by a cost model, and the launch.
+#include "gemm_mid.hpp"
+
+namespace lg {
+
+#define LG_MID_DECL(L) bool launch_mid_##L(int mi, bool nt, const GemmArgs& g, const GemmGroup& grp, const RowMap& rm, const MidLaunch& l)
+LG_MID_DECL(kn_128); LG_MID_DECL(kn_192); LG_MID_DECL(kn_256);
+LG_MID_DECL(nk_96); LG_MID_DECL(nk_128); LG_MID_DECL(nk_192); LG_MID_DECL(nk_256);
+LG_MID_DECL(tiled_96); LG_MID_DECL(tiled_128); LG_MID_DECL(tiled_192); LG_MID_DECL(tiled_256);
+#undef LG_MID_DECL
+void launch_gemm_fast_tile(const GemmArgs& g, const GemmGroup& grp, int wlayout, int nj, const StreamInfo& si, hipStream_t stream);
+
+namespace {
+
+struct Tile { signed char mi, nj; };
+// the tiles that were the fastest, or within 1 % of it, for some problem of the sweep below; the 96-wide ones exist for K-contiguous weights
+constexpr Tile kTiles[] = {{1, 4}, {2, 4}, {3, 4}, {4, 4}, {6, 4}, {8, 4}, {2, 3}, {4, 3}, {4, 6}, {5, 6}, {6, 6}, {7, 6}, {8, 6}, {4, 8}, {5, 8}, {6, 8}, {7, 8}, {8, 8}};
+constexpr int kMinSliceTiles = 8;     // k-tiles of a K-slice at least: below that its ramp costs more than it hides
+constexpr int kMaxTiles = LG_ARRIVAL_COUNTERS / 2;
+
+// Microseconds of one launch.  Fitted to 556 problems (M 8 .. 2048, 17 weight shapes from 1024 x 1024 to 32768 x 12288, all three
+// layouts) x all tiles and slice counts, each measured with weights cycled out of the caches; picking by it costs 1 % against
+// the best measured choice on average.  Terms: a k-tile costs its matrix work or its loads; a workgroup cannot pull more than 69 GB/s
+// of weights and the chip 7.4 TB/s; what memory and matrix pipes do in the same time overlaps only in part; a K-slice meeting
+// costs a trip to the counter and the transfer of the sums.
+double tile_cost(int M, int N, int K, int count, int mi, int nj, int nsplit, int cus) {
+    const int tiles_m = (M + 32 * mi - 1) / (32 * mi), tiles_n = N / (32 * nj) * count, ktiles = K / MID_K;
+    const int kt = (ktiles + nsplit - 1) / nsplit;
+    const long wgs = (long)tiles_m * tiles_n * nsplit;
+    const double rounds = (double)((wgs + cus - 1) / cus);
+    const double work = kt * (0.13 + 0.0192 * mi * nj), loads = kt * (0.0673 + 0.0292 * (mi + nj));
+    const double compute = work > loads ? work : loads;
+    const double chip = 2.0 * N * K * count / (7.3735e6 * cus / 256.0) / rounds, own = kt * (64.0 * 32 * 2 / 69.42e3) * nj;
+    double round = compute > chip ? compute + 0.6025 * chip : chip + 0.6025 * compute;
+    if (round < own) round = own;
+    double us = 3.67 + rounds * round;
+    if (nsplit > 1) us += 2.13 + 0.1128 * mi * nj * (mi * nj <= 16 ? nsplit : 1);
+    return us;
+}
+// The 256-row kernel keeps two waves per SIMD and places tiles for many rows of tiles: 3 % faster than the same tile here when it
+// has several rounds of workgroups (4096 rows x 16384 x 12288: 1172 against 1230 us), level at one.
+constexpr double kFastFactor = 0.97;
+
+// whether K may be sliced: every output is one sequential sum over k, whatever else is in the batch, from 512 token rows on if
+// there are outputs enough for one 96 x 128 tile per compute unit of the chip
+bool may_slice(int M, int N) { return M < 512 || (int64_t)M * N < (int64_t)256 * 96 * 128; }
+
+}  // namespace
+
+static TilePlan plan_gemm_tiles(const GemmArgs& g, int count, int wlayout, bool fast_ok, const StreamInfo& si) {
+    TilePlan best{};
+    best.cost = 1e30;
+    const int cus = si.cus, ktiles = g.K / MID_K;
+    const bool heads = g.epi.kind == LG_EPI_BIAS_HEADS || g.epi.kind == LG_EPI_BIAS_HEADS_ROWS;
+    auto usable = [&](const Tile& t, int cnt, int sp) {
+        if (g.N % (32 * t.nj)) return false;
+        if (t.nj == 3 && (wlayout == W_KN || g.epi.kind == LG_EPI_BIAS_GEGLU)) return false;  // GeGLU: a wave must hold (gate, up) pairs
+        if (sp == 1) return true;
+        const int64_t tiles = (int64_t)((g.M + 32 * t.mi - 1) / (32 * t.mi)) * (g.N / (32 * t.nj)) * cnt;
+        if (t.mi * t.nj > 16 && sp > 2) return false;
+        return sp <= 8 && ktiles >= sp * kMinSliceTiles && (ktiles + sp - 1) / sp * (sp - 1) < ktiles && tiles <= kMaxTiles &&
+               (size_t)(tiles * sp) * (size_t)(t.mi * t.nj * 4096) <= si.ws_bytes;
+    };
+    // the best tile for a given number of members and slices (0: any number of slices that keeps one round of workgroups)
+    auto pick = [&](int cnt, int fixed) {
+        TilePlan p{};
+        p.cost = 1e30;
+        for (const Tile& t : kTiles) {
+            const long tiles = (long)((g.M + 32 * t.mi - 1) / (32 * t.mi)) * (g.N / (32 * t.nj)) * cnt;
+            const int fill = tiles > 0 ? (int)(cus / tiles) : 0;
+            const int tries[4] = {1, 2, fill > 8 ? 8 : fill, 5};
+            for (int c = 0; c < 4; ++c) {
+                const int sp = fixed ? fixed : tries[c];
+                if ((fixed && c) || sp < 1 || (c > 1 && sp <= 2) || (!fixed && sp > 1 && (!si.ws || tiles * sp > cus || !may_slice(g.M, g.N)))) continue;
+                if (!usable(t, cnt, sp)) continue;
+                const double us = tile_cost(g.M, g.N, g.K, cnt, t.mi, t.nj, sp, cus);
+                if (us < p.cost) p = TilePlan{us, t.mi, t.nj, sp, false};
+            }
+        }
+        return p;
+    };
+    // The projections of Q, K and V have the heads epilogue and come as one call or as three: how K is sliced, and with it every bit
+    // of the result, must not depend on which, so it is decided for the three together.
+    int slices = 0;
+    if (heads) {
+        slices = pick(3, 0).nsplit;
+        if (slices < 1) slices = 1;
+    }
+    best = pick(count, slices);
+    if (best.nsplit == 0 && slices > 1) best = pick(count, 1);
+    if (fast_ok && best.nsplit <= 1 && g.M > 64 && g.epi.kind != LG_EPI_BIAS_HEADS_ROWS)
+        for (int nj = 4; nj >= 3; --nj) {
+            if (g.N % (64 * nj) || (nj == 3 && g.epi.kind == LG_EPI_BIAS_GEGLU)) continue;
+            const double us = kFastFactor * tile_cost(g.M, g.N, g.K, count, 8, 2 * nj, 1, cus);
+            if (us < best.cost) best = TilePlan{us, 8, nj, 1, true};
+        }
+    return best;
+}
+
+// alignment and shape that the tile kernels need of every member
+static bool tiles_apply(const GemmArgs& g, const GemmGroup& grp, int wlayout, int batch) {
+    if (batch != 1 || g.K % MID_K || g.M <= 0 || g.N <= 0 || g.K <= 0) return false;
+    if (!aligned16(g.X) || (g.ldx % 8) || (g.ldw % 8)) return false;
+    if (g.ldx >= (1 << 22) || g.ldw >= (1 << 22)) return false;  // 256 rows x ld must fit the 31-bit tile offsets
+    if (wlayout == W_TILED && g.ldw != g.K) return false;
+    const bool heads = g.epi.kind == LG_EPI_BIAS_HEADS || g.epi.kind == LG_EPI_BIAS_HEADS_ROWS;
+    for (int i = 0; i < grp.count; ++i) {
+        if (!aligned16(grp.W[i]) || (reinterpret_cast<uintptr_t>(grp.Y[i]) & 7u)) return false;
+        if (heads ? (g.epi.d % 4 != 0) : (grp.ldy[i] % 4 != 0)) return false;
+        if (g.epi.kind != LG_EPI_NONE && (reinterpret_cast<uintptr_t>(grp.bias[i]) & 7u)) return false;  // 8-byte bias loads
+    }
+    return true;
+}
+
+TilePlan plan_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, int wlayout, int batch, hipStream_t stream) {
+    if (!tiles_apply(g, grp, wlayout, batch)) return TilePlan{};
+    bool fast_ok = true;  // whole rows of 16 bytes
+    for (int i = 0; i < grp.count; ++i) fast_ok = fast_ok && aligned16(grp.Y[i]);
+    return plan_gemm_tiles(g, grp.count, wlayout, fast_ok, stream_info(stream));
+}
+
+int launch_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled) {
+    *handled = false;
+    if (g.epi.kind == LG_EPI_BIAS_HEADS_ROWS && !rows) return LG_OK;
+    const TilePlan p = plan_gemm_tiles_f16(g, grp, wlayout, batch, stream);
+    if (p.nsplit == 0) return LG_OK;
+    const StreamInfo si = stream_info(stream);
+    *handled = true;
+    if (p.fast) {
+        launch_gemm_fast_tile(g, grp, wlayout, p.nj, si, stream);
+        return check_launch("gemm_f16_fast");
+    }
+    const int ktiles = g.K / MID_K, kt = (ktiles + p.nsplit - 1) / p.nsplit;
+    const MidLaunch l{(ktiles + kt - 1) / kt, kt, si, stream};
+    const RowMap rm = rows ? *rows : RowMap{};
+    const bool nt = g.M <= 32 * p.mi;
+    bool ok = false;
+    switch (p.nj) {
+        case 3: ok = wlayout == W_NK ? launch_mid_nk_96(p.mi, nt, g, grp, rm, l) : launch_mid_tiled_96(p.mi, nt, g, grp, rm, l); break;
+        case 4: ok = wlayout == W_KN ? launch_mid_kn_128(p.mi, nt, g, grp, rm, l) : wlayout == W_NK ? launch_mid_nk_128(p.mi, nt, g, grp, rm, l) : launch_mid_tiled_128(p.mi, nt, g, grp, rm, l); break;
+        case 6: ok = wlayout == W_KN ? launch_mid_kn_192(p.mi, nt, g, grp, rm, l) : wlayout == W_NK ? launch_mid_nk_192(p.mi, nt, g, grp, rm, l) : launch_mid_tiled_192(p.mi, nt, g, grp, rm, l); break;
+        case 8: ok = wlayout == W_KN ? launch_mid_kn_256(p.mi, nt, g, grp, rm, l) : wlayout == W_NK ? launch_mid_nk_256(p.mi, nt, g, grp, rm, l) : launch_mid_tiled_256(p.mi, nt, g, grp, rm, l); break;
+    }
+    if (!ok) { set_error("gemm_f16: no kernel for tile %d x %d", 32 * p.mi, 32 * p.nj); return LG_ERR_INVALID; }
+    return check_launch("gemm_f16_mid");
+}
+
+}  // namespace lg

@@ -1,0 +1,13 @@
+// gemm_mid_tiled_128.hip -- instantiations of gemm_mid.hpp for weights [out, in] in fragment blocks and tiles of 96 and 128 features.
+#include "gemm_mid.hpp"
+
+namespace lg {
+
+bool launch_mid_tiled_96(int mi, bool nt, const GemmArgs& g, const GemmGroup& grp, const RowMap& rm, const MidLaunch& l) {
+    return launch_mid_heights<W_TILED, 3, 2, 4>(mi, nt, g, grp, rm, l);
+}
+bool launch_mid_tiled_128(int mi, bool nt, const GemmArgs& g, const GemmGroup& grp, const RowMap& rm, const MidLaunch& l) {
+    return launch_mid_heights<W_TILED, 4, 1, 2, 3, 4, 6, 8>(mi, nt, g, grp, rm, l);
+}
+
+}  // namespace lg

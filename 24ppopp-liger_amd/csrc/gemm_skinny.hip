@@ -347,21 +347,26 @@ void launch_splitk_reduce(const GemmArgs& g, const float* partial, int nsplit, h
     }
 }
 
-// grp.count > 1: handled only if the unsliced kernels apply (the caller then falls back to one launch per member)
+static bool skinny_applies(const GemmArgs& g, const GemmGroup& grp, int wlayout, int batch) {
+    if (batch != 1 || (wlayout != W_NK && wlayout != W_TILED)) return false;
+    if (g.M <= 0 || g.M > 64 || g.N < 512 || g.K < 1024 || (g.K % SK_KC) || (g.N % 4)) return false;
+    if (wlayout == W_TILED && ((g.N % 16) || g.ldw != g.K)) return false;
+    return aligned16(g.X) && (g.ldx % 8) == 0 && (g.ldw % 8) == 0 && group_aligned(g, grp);
+}
+
+// The unsliced kernel, for a problem or a group as one launch
 int launch_gemm_skinny_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled) {
     *handled = false;
-    if (batch != 1 || (wlayout != W_NK && wlayout != W_TILED)) return LG_OK;
-    if (g.M <= 0 || g.M > 64 || g.N < 512 || g.K < 1024 || (g.K % SK_KC) || (g.N % 4)) return LG_OK;
-    if (wlayout == W_TILED && ((g.N % 16) || g.ldw != g.K)) return LG_OK;
-    if (!aligned16(g.X) || (g.ldx % 8) || (g.ldw % 8) || !group_aligned(g, grp)) return LG_OK;
+    if (!skinny_applies(g, grp, wlayout, batch)) return LG_OK;
     if (g.epi.kind == LG_EPI_BIAS_HEADS_ROWS && !rows) return LG_OK;
+    // GeGLU pairs features 16 apart, which sit in different waves here: left to the tile kernels
+    if (g.epi.kind == LG_EPI_BIAS_GEGLU) return LG_OK;
+    // Above 48 token rows the tile kernels read less of X per weight byte (12288 x 16384 weight at 64 rows: 64.0 against 75.5 us,
+    // 12288 x 6144: 29.9 against 32.1) unless the features fill the chip several times over (18432 x 12288: 86 against 77).
+    if (g.M > 48 && (int64_t)g.N * grp.count <= 16384) return LG_OK;
     const RowMap rm = rows ? *rows : RowMap{};
     const int mt = (g.M + 15) / 16;
-    // GeGLU pairs features 16 apart, which sit in different waves of the unsliced kernel: such problems take the sliced kernel
-    // below (one slice when N alone fills the chip), whose reduce step forms the product
-    const bool geglu = g.epi.kind == LG_EPI_BIAS_GEGLU;
-    const StreamInfo si = stream_info(stream);
-    const int cus = si.cus;  // compute units this stream's kernels run on: "one round of blocks" means this many
+    const int cus = stream_info(stream).cus;  // compute units this stream's kernels run on: "one round of blocks" means this many
     // Unsliced: the 16-feature tiles are dealt to one block per compute unit of the stream, 2 to 8 waves a block (the partly
     // filled last wave sits in the first blocks only).  That needs enough tiles to give most compute units two waves, whole
     // pipeline depths of chunks, and for the 2-wave block (four chunks deep) registers for one row tile only.  Problems with more
@@ -372,7 +377,7 @@ int launch_gemm_skinny_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap
         if (nwv > 8 && tiles >= 16 * cus) { nwv = 4; nblocks = (tiles + 3) / 4; }
         if (nwv == 7) { nwv = 8; nblocks = (tiles + 7) / 8; }
         const bool deep = nwv == 2;
-        if (!geglu && nwv >= 2 && nwv <= 8 && tiles >= cus * 3 / 2 && g.K % ((deep ? 4 : 2) * SK_KC) == 0 && (!deep || mt == 1) &&
+        if (nwv >= 2 && nwv <= 8 && tiles >= cus * 3 / 2 && g.K % ((deep ? 4 : 2) * SK_KC) == 0 && (!deep || mt == 1) &&
             (int64_t)(nwv - 1) * nblocks < tiles && tiles <= (int64_t)nwv * nblocks) {  // what the kernel's dealing assumes
             *handled = true;
             if (wlayout == W_TILED) launch_direct_nwv<true>(nwv, g, grp, rm, nblocks, stream);
@@ -380,8 +385,16 @@ int launch_gemm_skinny_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap
             return check_launch("gemm_f16_skinny");
         }
     }
-    if (wlayout == W_TILED) return LG_OK;  // the K-sliced kernel below reads [N, K] rows
-    if (grp.count > 1 || g.epi.kind == LG_EPI_BIAS_HEADS_ROWS) return LG_OK;  // the sliced kernels take plain single problems only
+    return LG_OK;
+}
+
+// The K-sliced kernel, for what neither the unsliced kernel nor the tile kernels take (features that are not a multiple of 96 or
+// 128): single problems with weights [N, K]
+int launch_gemm_skinny_sliced_f16(const GemmArgs& g, int wlayout, int batch, hipStream_t stream, bool* handled) {
+    *handled = false;
+    if (wlayout != W_NK || !skinny_applies(g, single_group(g), wlayout, batch) || g.epi.kind == LG_EPI_BIAS_HEADS_ROWS) return LG_OK;
+    const StreamInfo si = stream_info(stream);
+    const int cus = si.cus, mt = (g.M + 15) / 16;
     const int nblk = (g.N + SK_BN - 1) / SK_BN;
     // K-slices: as few as fill the chip.  One block of 4 waves keeps 64 KiB of weight loads in flight, which is enough for one
     // CU; more slices only add fp32 partials and reduce work (six GEMMs of a decode step at 32 token rows on 256 CUs: 344 us

@@ -56,11 +56,11 @@ StreamInfo stream_info(hipStream_t stream) {
         auto it = g_streams.find((void*)stream);
         if (it != g_streams.end()) return it->second;
     }
-    return StreamInfo{device_cu_count(), nullptr, 0};
+    return StreamInfo{device_cu_count(), nullptr, 0, nullptr};
 }
 
 static int register_stream(void* stream, int cus) {
-    StreamInfo info{cus > 0 ? cus : device_cu_count(), nullptr, 0};
+    StreamInfo info{cus > 0 ? cus : device_cu_count(), nullptr, 0, nullptr};
     {
         std::lock_guard<std::mutex> lk(g_streams_mu);
         auto it = g_streams.find(stream);
@@ -72,10 +72,19 @@ static int register_stream(void* stream, int cus) {
     // hipMalloc may synchronise the device, so it runs outside the lock; two threads that attach the same stream at the same
     // time both get here, and the one that finds the stream registered when it comes back frees its block again
     void* p = nullptr;
-    const int rc = rt(hipMalloc(&p, LG_SPLITK_WORKSPACE_BYTES), "hipMalloc (split-K workspace)");
+    constexpr size_t counter_bytes = LG_ARRIVAL_COUNTERS * sizeof(unsigned);
+    int rc = rt(hipMalloc(&p, LG_SPLITK_WORKSPACE_BYTES + counter_bytes), "hipMalloc (split-K workspace)");
     if (rc) return rc;
     info.ws = (float*)p;
     info.ws_bytes = LG_SPLITK_WORKSPACE_BYTES;
+    info.arrivals = (unsigned*)((char*)p + LG_SPLITK_WORKSPACE_BYTES);
+    // set once, here: every kernel that counts arrivals leaves its counters at zero
+    rc = rt(hipMemset(info.arrivals, 0, counter_bytes), "hipMemset (arrival counters)");
+    if (rc == LG_OK) rc = rt(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
+    if (rc) {
+        (void)hipFree(p);
+        return rc;
+    }
     {
         std::lock_guard<std::mutex> lk(g_streams_mu);
         auto it = g_streams.find(stream);
@@ -89,7 +98,7 @@ static int register_stream(void* stream, int cus) {
 }
 
 static int unregister_stream(void* stream) {
-    StreamInfo info{0, nullptr, 0};
+    StreamInfo info{0, nullptr, 0, nullptr};
     {
         std::lock_guard<std::mutex> lk(g_streams_mu);
         auto it = g_streams.find(stream);

@@ -9,8 +9,8 @@
  *     are thin runtime wrappers for host code that does not include HIP headers).  The one piece of device memory the
  *     library owns is a 64 MiB split-K workspace per stream, allocated by lg_stream_create* / lg_stream_attach and freed
  *     by lg_stream_destroy / lg_stream_detach -- the counterpart of the workspace a cuBLAS handle owns (context.h:20-29
- *     binds one handle per stream).  A GEMM on a stream the library was never told about still runs, on kernels that
- *     need no workspace (slower for fewer than 257 token rows);
+ *     binds one handle per stream).  A GEMM on a stream the library was never told about still runs, without slicing K
+ *     (slower for few and medium token counts);
  *   - several kernels work in place, exactly where the reference's do.
  * Differences: every function returns an int status instead of asserting --
  *   LG_OK, LG_ERR_INVALID (bad / unsupported shape or pointer), LG_ERR_LAUNCH (HIP error; text via
