@@ -3,18 +3,21 @@
 //   gemm_f16_generic   128x128x32 tiles, 4 waves (2x2), MFMA 16x16x32 f16 -> fp32, any shape / stride /
 //                      alignment, both weight layouts, optional fused epilogue.  Correctness workhorse
 //                      (edge tiles, decomposed sub-ranges, attention GEMMs, small models).
-//   gemm_f32_mfma      128x128x16 tiles on v_mfma_f32_32x32x2_f32 for the fp32 instantiation (any shape, both layouts);
+//   gemm_f32_mfma      128x128x16 tiles on v_mfma_f32_32x32x2_f32 for the fp32 instantiation (any shape, both layouts); problems
+//                      of few such tiles go to gemm_f32.hip;
 //   gemm_f32_generic   64x64x16 VALU tiles, kept as a cross-check.
 // The large aligned prefill shapes are routed to the pipelined kernels in gemm_fast.hip.
 #include <stdlib.h>
 
 #include "gemm_common.hpp"
+#include "gemm_f32.hpp"
 
 namespace lg {
 
 int launch_gemm_skinny_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled);
 int launch_gemv_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled);
 int launch_gemm_skinny_sliced_f16(const GemmArgs& g, int wlayout, int batch, hipStream_t stream, bool* handled);
+int launch_gemm_f32_direct(const GemmArgsF32& g, int wlayout, int batch, bool aligned, hipStream_t stream, bool* handled);
 
 // ---------------------------------------------------------------------------------------------------
 // fp16 generic kernel
@@ -202,13 +205,6 @@ static int gemm_f16_dispatch(GemmArgs g, int wlayout, int batch, hipStream_t str
 // ---------------------------------------------------------------------------------------------------
 // fp32 generic kernel (plumbing configuration): 64x64x16 tiles, 256 threads, 4x4 outputs per thread
 // ---------------------------------------------------------------------------------------------------
-struct GemmArgsF32 {
-    int M, N, K;
-    const float* X; int64_t ldx; int64_t strideX;
-    const float* W; int64_t ldw; int64_t strideW;
-    float* Y;       int64_t ldy; int64_t strideY;
-};
-
 template <int WL>
 __global__ __launch_bounds__(256) void gemm_f32_generic(GemmArgsF32 g) {
     __shared__ float As[16][64 + 4];  // [k][m]
@@ -390,6 +386,9 @@ static int gemm_f32_dispatch(const GemmArgsF32& g, int wlayout, int batch, hipSt
         if (grid.y > 65535 || grid.z > 65535) { set_error("gemm: problem too large for the grid"); return LG_ERR_INVALID; }
         const bool aligned = aligned16(g.X) && aligned16(g.W) && aligned16(g.Y) && (g.ldx % 4 == 0) && (g.ldw % 4 == 0) &&
                              (g.strideX % 4 == 0) && (g.strideW % 4 == 0) && (g.strideY % 4 == 0);
+        bool handled = false;
+        const int rc = launch_gemm_f32_direct(g, wlayout, batch, aligned, stream, &handled);
+        if (handled) return rc;
         if (wlayout == W_NK) {
             if (aligned) hipLaunchKernelGGL((gemm_f32_mfma<W_NK, true>), grid, dim3(256), 0, stream, g);
             else hipLaunchKernelGGL((gemm_f32_mfma<W_NK, false>), grid, dim3(256), 0, stream, g);

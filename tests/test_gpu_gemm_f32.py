@@ -1,0 +1,62 @@
+"""fp32 GEMM (gemm_f32.hpp and the 128 x 128 tiles of gemm.hip): edges of the tiles, remainders of k, matrices inside wider ones, unaligned
+pointers, batches.  Tolerance: the products are exact in the fp32 unit up to one rounding each, so the error of a sum of K terms is at
+most K 2^-24 of the sum of magnitudes; measured against that bound element by element."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+EPS = 2.0 ** -24
+
+
+def _case(dev, transa, M, N, K, batch=1, pad=0, shift=0, seed=0):
+    """Y [batch, M, N] inside a larger buffer: rows of N + pad, everything `shift` floats past a 16-byte boundary"""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(seed)
+    rows, cols = (K, N) if transa == 0 else (N, K)
+
+    def matrix(r, c):
+        ld = c + pad
+        flat = torch.randn(shift + batch * r * ld + 8, device="cuda", generator=gen)
+        return flat, flat[shift:shift + batch * r * ld].view(batch, r, ld)[:, :, :c], ld
+
+    fx, X, ldx = matrix(M, K)
+    fw, W, ldw = matrix(rows, cols)
+    fy, Y, ldy = matrix(M, N)
+    before = fy.clone()
+    Wk = W if transa == 0 else W.transpose(1, 2)
+    ref = torch.stack([X[b].double().cpu() @ Wk[b].double().cpu() for b in range(batch)])
+    mag = torch.stack([X[b].double().abs().cpu() @ Wk[b].double().abs().cpu() for b in range(batch)])
+    dev.call("lg_gemm_strided_batched_f32", transa, 0, N, M, K, W.data_ptr(), ldw, rows * ldw, X.data_ptr(), ldx, M * ldx, Y.data_ptr(), ldy, M * ldy, batch)
+    dev.sync()
+    assert bool(((Y.double().cpu() - ref).abs() <= K * EPS * mag).all())
+    first = Y.clone()
+    Y.copy_(before[shift:shift + batch * M * ldy].view(batch, M, ldy)[:, :, :N])
+    assert torch.equal(fy, before)          # nothing outside the output was written
+    return first, X, W
+
+
+@pytest.mark.parametrize("transa", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(1, 1, 1), (3, 5, 7), (16, 16, 16), (17, 15, 15), (15, 33, 64), (31, 31, 65), (64, 64, 63), (65, 66, 130), (64, 256, 1024),
+                                   (100, 257, 33), (127, 513, 200), (129, 130, 31), (200, 1000, 96), (333, 333, 64), (333, 1024, 512), (800, 1024, 128),
+                                   (1024, 2050, 64), (2048, 2048, 48), (512, 8200, 40)])
+def test_shapes(dev, transa, M, N, K):
+    _case(dev, transa, M, N, K)
+
+
+@pytest.mark.parametrize("transa", [0, 1])
+@pytest.mark.parametrize("M,N,K,batch,pad,shift", [(33, 47, 50, 1, 3, 1), (70, 66, 100, 3, 1, 0), (200, 200, 64, 16, 0, 0), (200, 64, 200, 16, 0, 2), (333, 64, 333, 4, 0, 0),
+                                                   (130, 260, 128, 2, 4, 0), (512, 512, 64, 40, 0, 0), (1000, 1030, 72, 4, 2, 3)])
+def test_strides_and_batches(dev, transa, M, N, K, batch, pad, shift):
+    _case(dev, transa, M, N, K, batch, pad, shift)
+
+
+def test_infinities_stay_in_their_rows(dev):
+    """Rows and k beyond the matrix are not multiplied in: an infinity in one token row leaves the others finite."""
+    M, N, K = 50, 70, 37
+    X, W, Y = torch.randn(M, K, device="cuda"), torch.randn(K, N, device="cuda"), torch.empty(M, N, device="cuda")
+    X[49, 36] = float("inf")
+    dev.call("lg_gemm_f32", 0, 0, N, M, K, W.data_ptr(), N, X.data_ptr(), K, Y.data_ptr(), N)
+    dev.sync()
+    assert bool(torch.isfinite(Y[:49]).all()) and not bool(torch.isfinite(Y[49]).any())
