@@ -518,12 +518,12 @@ static int gemm_fused_grouped_f16_impl(int mode, int transa, int m, int n, int k
         // columns of 256-wide tiles, 16 columns to a round of 256 workgroups, 8 left over): the members before the last as one
         // launch of whole rounds, the last member's leading features as whole rounds too, and its remaining features as one round
         // of narrower tiles -- instead of six rounds of 192-wide tiles (4.6-6.6 % faster, measured).  Pieces are addressed like any
-        // feature sub-range.
+        // feature sub-range.  Only where the order of a sum over k does not depend on the feature's place in its launch.
         int split_at = 0;   // feature at which the last member is cut (0: no such plan)
         const int tiles_m = (n + 255) / 256;
         const bool range_ok = epilogue == LG_EPI_NONE || epilogue == LG_EPI_BIAS || epilogue == LG_EPI_BIAS_GELU ||
                               (epilogue == LG_EPI_BIAS_HEADS && epi_arg1 > 0 && 256 % epi_arg1 == 0);
-        if (range_ok && apart.nsplit == 1 && m % 256 == 0 && cus % tiles_m == 0 && (transa != LG_OP_TILED || lda == k)) {
+        if (range_ok && n >= kSequentialRows && apart.nsplit == 1 && m % 256 == 0 && cus % tiles_m == 0 && (transa != LG_OP_TILED || lda == k)) {
             const int cols = m / 256, per_round = cus / tiles_m, rem = (count * cols) % per_round;
             if (rem > 0 && rem < cols && ((count - 1) * cols) % per_round == 0 && (cols - rem) % per_round == 0) {
                 const TilePlan lead = plan(count - 1, m), body = plan(1, (cols - rem) * 256), tail = plan(1, rem * 256);

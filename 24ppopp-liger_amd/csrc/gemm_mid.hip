@@ -44,7 +44,15 @@ constexpr double kFastFactor = 0.97;
 
 // whether K may be sliced: every output is one sequential sum over k, whatever else is in the batch, from 512 token rows on if
 // there are outputs enough for one 96 x 128 tile per compute unit of the chip
-bool may_slice(int M, int N) { return M < 512 || (int64_t)M * N < (int64_t)256 * 96 * 128; }
+bool may_slice(int M, int N) { return M < kSequentialRows || (int64_t)M * N < (int64_t)256 * 96 * 128; }
+
+// Where a workgroup starts in its loop over k.  If all start at the first k-tile, all of them read the same k of every weight row at
+// the same time: pieces of 128 bytes, a row apart, and where the row is a multiple of many memory channels they come from a few of
+// them.  Apart by 5 k-tiles, [out, in] weights 24576 x 12288 take 149 -> 107 us at 106 rows (the same as rows padded by 128 bytes),
+// 164 -> 140 at 200, 218 -> 193 at 384; 12288 x 24576 139 -> 120 at 106; 6144 x 12288 43.0 -> 41.9.  Fragment blocks, read in pieces
+// of 2 KiB, gain 0-3 % by 3 (16384 x 12288 at 80 rows 72.9 -> 70.8).  [in, out] rows are read over their whole length as it is: by 3,
+// 12288 x 16384 loses 3 %.  From 512 rows on every output is a sum in the order of k (may_slice).
+int mid_turn(int M, int wlayout) { return M >= kSequentialRows || wlayout == W_KN ? 0 : wlayout == W_NK ? 5 : 3; }
 
 }  // namespace
 
@@ -132,7 +140,7 @@ int launch_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap*
         return check_launch("gemm_f16_fast");
     }
     const int ktiles = g.K / MID_K, kt = (ktiles + p.nsplit - 1) / p.nsplit;
-    const MidLaunch l{(ktiles + kt - 1) / kt, kt, si, stream};
+    const MidLaunch l{(ktiles + kt - 1) / kt, kt, mid_turn(g.M, wlayout), si, stream};
     const RowMap rm = rows ? *rows : RowMap{};
     const bool nt = g.M <= 32 * p.mi;
     bool ok = false;

@@ -16,6 +16,9 @@
 //     (the schedule of gemm_fast.hip);
 //   * with one row of tiles every weight byte is read once, and the loads say so (non-temporal: 84 -> 73 us for a 16384 x 12288
 //     weight at 72 rows);
+//   * below 512 rows the workgroups of different feature blocks start their loop over k at different k-tiles, which spreads what
+//     they read at one time over the memory channels (mid_turn in gemm_mid.hip: up to 28 % of a GEMM).  Where it starts depends on
+//     the feature alone, not on the tile: a member of a group has the same bits as a call of its own;
 //   * K-slices meet in the kernel: the slice of a tile that arrives last adds the others' sums and applies the epilogue.  A second
 //     kernel for that cost 5-10 us per GEMM.
 // 16384 x 12288 weight (403 MB), before (gemm_fast.hip, K-slices summed by a second kernel) -> now: 80 rows 104 -> 73 us, 128 rows
@@ -27,9 +30,11 @@ namespace lg {
 
 constexpr int MID_K = 64;
 constexpr int MID_THREADS = 256;
+constexpr int MID_TURN_COLS = 768;  // features of such a block: a multiple of every tile width
 
 struct MidLaunch {  // what a launch of one of the instantiations needs besides the problem
     int nsplit, kt_per_split;
+    int turn;  // k-tiles by which the workgroups of neighbouring feature blocks are apart in their loop over k (0: all start at the first)
     StreamInfo si;
     hipStream_t stream;
 };
@@ -55,7 +60,7 @@ constexpr int CACHE_DEVICE = 16;
 constexpr int mid_max_splits(int mi, int nj) { return mi * nj <= 16 ? 8 : 2; }
 
 template <int WL, int MI, int NJ, int XS, int WS, bool NT>
-__global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmGroup grp, RowMap rm, int tiles_m, int tiles_n, float* partial, unsigned* arrivals, int nsplit, int kt_per_split, int wide_store) {
+__global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmGroup grp, RowMap rm, int tiles_m, int tiles_n, float* partial, unsigned* arrivals, int nsplit, int kt_per_split, int turn, int wide_store) {
     constexpr int TM = 32 * MI, TN = 32 * NJ;
     constexpr int X_TILE = TM * MID_K, W_TILE = TN * MID_K;  // halves per ring slot
     extern __shared__ __attribute__((aligned(16))) half_t smem[];  // X ring (XS tiles), then W ring (WS tiles)
@@ -122,9 +127,14 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
         }
     }
     const int64_t wstep = (WL == W_KN) ? (int64_t)MID_K * g.ldw : (WL == W_NK ? MID_K : 1024);
+    const int first = n0 / MID_TURN_COLS * turn % ktiles;
     // the tile index is clamped to the last one: the loop body is branch-free, the extra loads refill slots nobody reads
-    auto x_tile = [&](int kt) { return reinterpret_cast<const char*>(X + (int64_t)(kt < ktiles ? kt : ktiles - 1) * MID_K); };
-    auto w_tile = [&](int kt) { return reinterpret_cast<const char*>(W + (int64_t)(kt < ktiles ? kt : ktiles - 1) * wstep); };
+    auto at = [&](int kt) {
+        const int t = (kt < ktiles ? kt : ktiles - 1) + first;
+        return (int64_t)(t < ktiles ? t : t - ktiles);
+    };
+    auto x_tile = [&](int kt) { return reinterpret_cast<const char*>(X + at(kt) * MID_K); };
+    auto w_tile = [&](int kt) { return reinterpret_cast<const char*>(W + at(kt) * wstep); };
 
     constexpr int NLOAD = MI + NJ;
     constexpr bool XFIRST = WS > XS;  // the operand with the shallower ring is issued first in a phase
@@ -419,7 +429,7 @@ static void launch_mid_tile(const GemmArgs& g, const GemmGroup& grp, const RowMa
     static const hipError_t attr_rc = hipFuncSetAttribute((const void*)gemm_f16_mid<WL, MI, NJ, XS, WS, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     (void)attr_rc;
     hipLaunchKernelGGL((gemm_f16_mid<WL, MI, NJ, XS, WS, NT>), dim3(tiles_m * tiles_n * l.nsplit), dim3(MID_THREADS), smem, l.stream, g, grp, rm, tiles_m, tiles_n,
-                       l.si.ws, l.si.arrivals, l.nsplit, l.kt_per_split, wide);
+                       l.si.ws, l.si.arrivals, l.nsplit, l.kt_per_split, l.turn, wide);
 }
 
 // one instantiation per tile height MI of a list, with and without the non-temporal hint

@@ -151,3 +151,25 @@ def test_streams_of_their_own_and_a_stream_without_a_workspace(dev, po):
     assert dev.lib.lg_gemm_f16(TILED, 0, N, M, K, dW.data_ptr(), ld, dX[0].data_ptr(), K, y.data_ptr(), N, C.c_void_p(other.cuda_stream)) == 0
     dev.sync()
     assert max_rel_err(dev.down(y), ref[0]) < 1e-3
+
+
+@pytest.mark.parametrize("layout", [1, 2])
+@pytest.mark.parametrize("M,N,K", [(70, 3072, 448), (106, 1920, 2048), (200, 6144, 1088), (384, 4608, 192), (511, 2304, 4096)])
+def test_turned_loops(dev, po, layout, M, N, K):
+    """Feature blocks of 768 that start at different k-tiles: fewer k-tiles than the turns add up to, a last block that is not whole,
+    K-slices; and a member of a group of three has the bits of a call of its own, whichever tiles the two take."""
+    X = rnd(po, M * K, 21).reshape(M, K)
+    Ws = [rnd(po, K * N, 22 + i, 0.05).reshape(K, N) for i in range(3)]
+    dX, bias = dev.up(X, 1), dev.up(rnd(po, N, 25), 1)
+    dW = [weight(dev, W, layout)[0] for W in Ws]
+    one = [dev.empty((1, N // 128, M, 128), 1) for _ in range(3)]
+    for i in range(3):
+        dev.call("lg_gemm_fused_f16", layout, N, M, K, dW[i], K, dX, K, one[i], M, dev.capi.EPI_BIAS_HEADS, bias, M, 128, 0)
+    three = [dev.empty((1, N // 128, M, 128), 1) for _ in range(3)]
+    ptrs = lambda ts: (C.c_void_p * 3)(*[t.data_ptr() for t in ts])
+    dev.call("lg_gemm_fused_grouped_f16", layout, N, M, K, 3, ptrs(dW), K, dX, K, ptrs(three), (C.c_int * 3)(M, M, M), dev.capi.EPI_BIAS_HEADS, ptrs([bias] * 3), M, 128, 0)
+    want = [po.gemm(X, W, 1) + dev.down(bias) for W in Ws]
+    for i in range(3):
+        got = dev.down(one[i])
+        assert np.array_equal(got, dev.down(three[i]))
+        assert max_rel_err(got[0].transpose(1, 0, 2).reshape(M, N), want[i]) < 2e-3
