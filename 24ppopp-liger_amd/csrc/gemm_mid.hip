@@ -51,8 +51,12 @@ bool may_slice(int M, int N) { return M < kSequentialRows || (int64_t)M * N < (i
 // them.  Apart by 5 k-tiles, [out, in] weights 24576 x 12288 take 149 -> 107 us at 106 rows (the same as rows padded by 128 bytes),
 // 164 -> 140 at 200, 218 -> 193 at 384; 12288 x 24576 139 -> 120 at 106; 6144 x 12288 43.0 -> 41.9.  Fragment blocks, read in pieces
 // of 2 KiB, gain 0-3 % by 3 (16384 x 12288 at 80 rows 72.9 -> 70.8).  [in, out] rows are read over their whole length as it is: by 3,
-// 12288 x 16384 loses 3 %.  From 512 rows on every output is a sum in the order of k (may_slice).
-int mid_turn(int M, int wlayout) { return M >= kSequentialRows || wlayout == W_KN ? 0 : wlayout == W_NK ? 5 : 3; }
+// 12288 x 16384 loses 3 %.  Only where K may be sliced too
+// (fewer than 512 rows, K of two slices or more): everywhere else an output is a sum in the order of k, whatever computes it.
+int mid_turn(int M, int K, int wlayout) {
+    if (M >= kSequentialRows || K < 2 * kMinSliceTiles * MID_K) return 0;
+    return wlayout == W_NK ? 5 : wlayout == W_TILED ? 3 : 0;
+}
 
 }  // namespace
 
@@ -140,7 +144,7 @@ int launch_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap*
         return check_launch("gemm_f16_fast");
     }
     const int ktiles = g.K / MID_K, kt = (ktiles + p.nsplit - 1) / p.nsplit;
-    const MidLaunch l{(ktiles + kt - 1) / kt, kt, mid_turn(g.M, wlayout), si, stream};
+    const MidLaunch l{(ktiles + kt - 1) / kt, kt, mid_turn(g.M, g.K, wlayout), si, stream};
     const RowMap rm = rows ? *rows : RowMap{};
     const bool nt = g.M <= 32 * p.mi;
     bool ok = false;
