@@ -73,6 +73,10 @@ template <typename T> __device__ __forceinline__ float ldf(const T* p) { return 
 template <typename T> __device__ __forceinline__ void stf(T* p, float v) { *p = (T)v; }
 
 // 16-byte vector of T
+// at any alignment: global memory takes loads and stores of these as whole ones
+typedef half_t half4u_t __attribute__((ext_vector_type(4), aligned(2)));
+typedef half_t half8u_t __attribute__((ext_vector_type(8), aligned(2)));
+
 template <typename T> struct Vec16;
 template <> struct Vec16<float> {
     static constexpr int N = 4;

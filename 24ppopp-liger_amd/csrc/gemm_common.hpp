@@ -211,7 +211,7 @@ __device__ __forceinline__ void epilogue_store4(const GemmArgs& g, half_t* Yb, i
     }
     if (vec_ok && n + 3 < g.N) {
         half4_t o = {(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
-        *reinterpret_cast<half4_t*>(Yb + base) = o;
+        *reinterpret_cast<half4u_t*>(Yb + base) = o;
     } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r)
@@ -230,7 +230,7 @@ __device__ __forceinline__ void epilogue_geglu4(const GemmArgs& g, half_t* Yb, i
     const int64_t base = (int64_t)m * g.ldy + (n >> 5) * 16 + (n & 15);
     if (vec_ok) {
         half4_t o = {(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
-        *reinterpret_cast<half4_t*>(Yb + base) = o;
+        *reinterpret_cast<half4u_t*>(Yb + base) = o;
     } else {
 #pragma unroll
         for (int r = 0; r < 4; ++r) Yb[base + r] = (half_t)v[r];
