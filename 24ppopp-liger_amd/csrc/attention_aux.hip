@@ -114,12 +114,14 @@ static int launch_transpose(T* dst, const T* src, int batch, int seq, int head_n
 
 // ---- softmax (attention_kernels.cu:395-680) -----------------------------------------------------------
 //   t = qk*scalar + (1 - mask)*(-10000);  p = exp(t - max t);  out = p / (sum p + 1e-6)
-// One wave64 per row, the row held in registers as NC 16-byte vectors per lane.
+// One wave64 per row, the row held in registers as NC vectors of 16 bytes per lane, at any alignment (global memory takes such loads
+// and stores as whole ones; only the last vector of a row that is not whole goes element by element).  Bound by memory: 2 x 48 x 333
+// rows of 333 halves 22 us, 44 in one workgroup and three passes per row, which rows longer than 512 vectors still take.
 template <typename T, int NC>
 __global__ __launch_bounds__(256) void softmax_wave_kernel(T* buf, const T* __restrict__ mask, int seq, int head_num,
                                                            int64_t rows, float scalar) {
-    typedef Vec16<T> V;
-    constexpr int VN = V::N;
+    constexpr int VN = Vec16<T>::N;
+    typedef T vec_t __attribute__((ext_vector_type(VN), aligned(sizeof(T))));
     const int lane = threadIdx.x & 63;
     const int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
     if (row >= rows) return;
@@ -127,35 +129,35 @@ __global__ __launch_bounds__(256) void softmax_wave_kernel(T* buf, const T* __re
     const int sq = (int)(row % seq);
     T* p = buf + row * seq;
     const T* mrow = mask + (b * seq + sq) * (int64_t)seq;
-    const int nvec = seq / VN;
     float t[NC][VN];
     float mx = -1e20f;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-        const int v = lane + c * 64;
-        if (v < nvec) {
-            V a = *reinterpret_cast<const V*>(p + (int64_t)v * VN);
-            V m = *reinterpret_cast<const V*>(mrow + (int64_t)v * VN);
+        const int i = (lane + c * 64) * VN;  // this lane's first element of the vector
 #pragma unroll
-            for (int j = 0; j < VN; ++j) {
-                t[c][j] = a.get(j) * scalar + (1.0f - m.get(j)) * -10000.0f;
-                mx = fmaxf(mx, t[c][j]);
-            }
-        } else {
+        for (int j = 0; j < VN; ++j) t[c][j] = -1e20f;
+        if (i + VN <= seq) {
+            const vec_t a = *reinterpret_cast<const vec_t*>(p + i), m = *reinterpret_cast<const vec_t*>(mrow + i);
 #pragma unroll
-            for (int j = 0; j < VN; ++j) t[c][j] = -1e20f;
+            for (int j = 0; j < VN; ++j) t[c][j] = (float)a[j] * scalar + (1.0f - (float)m[j]) * -10000.0f;
+        } else if (i < seq) {
+#pragma unroll
+            for (int j = 0; j < VN; ++j)
+                if (i + j < seq) t[c][j] = ldf(p + i + j) * scalar + (1.0f - ldf(mrow + i + j)) * -10000.0f;
         }
+#pragma unroll
+        for (int j = 0; j < VN; ++j) mx = fmaxf(mx, t[c][j]);
     }
     mx = wave_max(mx);
     float sum = 0.f;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-        const int v = lane + c * 64;
-        if (v < nvec) {
+        const int i = (lane + c * 64) * VN;
+        if (i < seq) {
 #pragma unroll
             for (int j = 0; j < VN; ++j) {
                 t[c][j] = __expf(t[c][j] - mx);
-                sum += t[c][j];
+                if (i + j < seq) sum += t[c][j];
             }
         }
     }
@@ -163,17 +165,21 @@ __global__ __launch_bounds__(256) void softmax_wave_kernel(T* buf, const T* __re
     const float inv = 1.0f / (sum + 1e-6f);
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-        const int v = lane + c * 64;
-        if (v < nvec) {
-            V o;
+        const int i = (lane + c * 64) * VN;
+        if (i + VN <= seq) {
+            vec_t o;
 #pragma unroll
-            for (int j = 0; j < VN; ++j) o.set(j, t[c][j] * inv);
-            *reinterpret_cast<V*>(p + (int64_t)v * VN) = o;
+            for (int j = 0; j < VN; ++j) o[j] = (T)(t[c][j] * inv);
+            *reinterpret_cast<vec_t*>(p + i) = o;
+        } else if (i < seq) {
+#pragma unroll
+            for (int j = 0; j < VN; ++j)
+                if (i + j < seq) stf(p + i + j, t[c][j] * inv);
         }
     }
 }
 
-// any seq / alignment: one block per row, three passes
+// rows of any length: one block per row, three passes
 template <typename T>
 __global__ __launch_bounds__(256) void softmax_scalar_kernel(T* buf, const T* mask, int seq, int head_num, float scalar) {
     __shared__ float scratch[16];
@@ -202,9 +208,8 @@ static int launch_softmax(T* buf, const T* mask, int batch, int seq, int head_nu
     if (rows == 0) return LG_OK;
     scalar = (float)(T)scalar;  // the reference keeps the scalar as T (bert_layer.h:94)
     constexpr int VN = Vec16<T>::N;
-    const bool vec = (seq % VN == 0) && aligned16(buf) && aligned16(mask);
-    const int nvec = seq / VN;
-    if (vec && nvec <= 64 * 8) {
+    const int nvec = (seq + VN - 1) / VN;
+    if (nvec <= 64 * 8) {
         const int nc = (nvec + 63) / 64;
         const int64_t grid = (rows + 3) / 4;
         if (grid > 0x7fffffff) { set_error("attn_softmax: too many rows"); return LG_ERR_INVALID; }
