@@ -238,7 +238,7 @@ __device__ __forceinline__ void epilogue_geglu4(const GemmArgs& g, half_t* Yb, i
 }
 
 // ---- tile kernels (gemm_mid.hip): the choice made for a problem, or for `count` members of a group as one launch ---------------
-constexpr int kSequentialRows = 512;  // from so many token rows on every output is one sum in the order of k
+constexpr int kSequentialRows = 257;  // from so many token rows on every output is one sum in the order of k, whichever kernel computes it
 struct TilePlan {
     double cost;   // estimated microseconds
     int mi, nj;    // tile (32 mi) x (32 nj); the 256-row kernel: 256 x (64 nj)

@@ -42,17 +42,17 @@ double tile_cost(int M, int N, int K, int count, int mi, int nj, int nsplit, int
 // has several rounds of workgroups (4096 rows x 16384 x 12288: 1172 against 1230 us), level at one.
 constexpr double kFastFactor = 0.97;
 
-// whether K may be sliced: every output is one sequential sum over k, whatever else is in the batch, from 512 token rows on if
-// there are outputs enough for one 96 x 128 tile per compute unit of the chip
-bool may_slice(int M, int N) { return M < kSequentialRows || (int64_t)M * N < (int64_t)256 * 96 * 128; }
+// K is sliced, and loops over it are turned, up to 256 token rows only.  Above that every output is one sum in the order of k: a row's
+// bits do not depend on the rows and features around it in a call, on the layout or on the stream, so that a batch, its parts and the
+// ranges of a decomposed call agree.  The price is what slices would give there, in microseconds at 384 rows ([out, in] weights):
+// 6144 x 12288 79 -> 105, 12288 x 16384 140 -> 192, 16384 x 12288 157 -> 163, 2048 x 8192 30 -> 41 (256-row tiles: 160, 236, 197, 94).
 
 // Where a workgroup starts in its loop over k.  If all start at the first k-tile, all of them read the same k of every weight row at
 // the same time: pieces of 128 bytes, a row apart, and where the row is a multiple of many memory channels they come from a few of
 // them.  Apart by 5 k-tiles, [out, in] weights 24576 x 12288 take 149 -> 107 us at 106 rows (the same as rows padded by 128 bytes),
-// 164 -> 140 at 200, 218 -> 193 at 384; 12288 x 24576 139 -> 120 at 106; 6144 x 12288 43.0 -> 41.9.  Fragment blocks, read in pieces
+// 164 -> 140 at 200; 12288 x 24576 139 -> 120 at 106; 6144 x 12288 43.0 -> 41.9.  Fragment blocks, read in pieces
 // of 2 KiB, gain 0-3 % by 3 (16384 x 12288 at 80 rows 72.9 -> 70.8).  [in, out] rows are read over their whole length as it is: by 3,
-// 12288 x 16384 loses 3 %.  Only where K may be sliced too
-// (fewer than 512 rows, K of two slices or more): everywhere else an output is a sum in the order of k, whatever computes it.
+// 12288 x 16384 loses 3 %.  Only where K may be sliced too (up to 256 rows, K of two slices or more).
 int mid_turn(int M, int K, int wlayout) {
     if (M >= kSequentialRows || K < 2 * kMinSliceTiles * MID_K) return 0;
     return wlayout == W_NK ? 5 : wlayout == W_TILED ? 3 : 0;
@@ -84,7 +84,7 @@ static TilePlan plan_gemm_tiles(const GemmArgs& g, int count, int wlayout, bool 
             const int tries[4] = {1, 2, fill > 8 ? 8 : fill, 5};
             for (int c = 0; c < 4; ++c) {
                 const int sp = fixed ? fixed : tries[c];
-                if ((fixed && c) || sp < 1 || (c > 1 && sp <= 2) || (!fixed && sp > 1 && (!si.ws || tiles * sp > cus || !may_slice(g.M, g.N)))) continue;
+                if ((fixed && c) || sp < 1 || (c > 1 && sp <= 2) || (!fixed && sp > 1 && (!si.ws || tiles * sp > cus || g.M >= kSequentialRows))) continue;
                 if (!usable(t, cnt, sp)) continue;
                 const double us = tile_cost(g.M, g.N, g.K, cnt, t.mi, t.nj, sp, cus);
                 if (us < p.cost) p = TilePlan{us, t.mi, t.nj, sp, false};

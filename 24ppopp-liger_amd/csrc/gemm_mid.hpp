@@ -16,13 +16,13 @@
 //     (the schedule of gemm_fast.hip);
 //   * with one row of tiles every weight byte is read once, and the loads say so (non-temporal: 84 -> 73 us for a 16384 x 12288
 //     weight at 72 rows);
-//   * below 512 rows the workgroups of different feature blocks start their loop over k at different k-tiles, which spreads what
+//   * up to 256 rows the workgroups of different feature blocks start their loop over k at different k-tiles, which spreads what
 //     they read at one time over the memory channels (mid_turn in gemm_mid.hip: up to 28 % of a GEMM).  Where it starts depends on
 //     the feature alone, not on the tile: a member of a group has the same bits as a call of its own;
 //   * K-slices meet in the kernel: the slice of a tile that arrives last adds the others' sums and applies the epilogue.  A second
 //     kernel for that cost 5-10 us per GEMM.
 // 16384 x 12288 weight (403 MB), before (gemm_fast.hip, K-slices summed by a second kernel) -> now: 80 rows 104 -> 73 us, 128 rows
-// 108 -> 80, 256 rows 127 -> 108, 384 rows 187 -> 138 (1.12 PFLOP/s), 768 rows 264 -> 233 (1.33), 1536 rows 514 -> 457.
+// 108 -> 80, 256 rows 127 -> 108, 384 rows 187 -> 157 (0.98 PFLOP/s), 768 rows 264 -> 233 (1.33), 1536 rows 514 -> 457.
 #pragma once
 #include "gemm_common.hpp"
 

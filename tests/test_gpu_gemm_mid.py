@@ -173,3 +173,54 @@ def test_turned_loops(dev, po, layout, M, N, K):
         got = dev.down(one[i])
         assert np.array_equal(got, dev.down(three[i]))
         assert max_rel_err(got[0].transpose(1, 0, 2).reshape(M, N), want[i]) < 2e-3
+
+
+# on both sides of 512 rows and of 3 145 728 outputs, K long enough for slices; one block of 768 features and several
+@pytest.mark.parametrize("M,N,K", [(257, 1536, 2048), (300, 3072, 2048), (511, 2304, 4096), (513, 2304, 2048), (700, 4096, 2048), (768, 4096, 2048), (1024, 1024, 4096)])
+def test_above_256_rows_a_row_does_not_depend_on_its_call(dev, po, M, N, K):
+    """One sum in the order of k whatever computes it: a range of the rows (more than 256 of them), a range of the features and the
+    three layouts have the bits of the whole call."""
+    X, W = rnd(po, M * K, 51).reshape(M, K), rnd(po, K * N, 52, 0.05).reshape(K, N)
+    dX = dev.up(X, 1)
+    first = None
+    for layout in (0, 1, 2):
+        dW, ld = weight(dev, W, layout)
+
+        def gemm(rows, r0, n, n0):
+            y = dev.empty((rows, n), 1)
+            dev.call("lg_gemm_f16", layout, 0, n, rows, K, dW.data_ptr() + 2 * n0 * (1 if layout == 0 else K), ld, dX.data_ptr() + 2 * r0 * K, K, y, n)
+            return dev.down(y)
+
+        whole = gemm(M, 0, N, 0)
+        first = whole if layout == 0 else first
+        assert np.array_equal(whole, first)
+        assert np.array_equal(gemm(257, M - 257, N, 0), whole[M - 257:])
+        for n0 in (256, 768):
+            assert np.array_equal(gemm(M, 0, N - n0, n0), whole[:, n0:]) and np.array_equal(gemm(M, 0, n0, 0), whole[:, :n0])
+    assert max_rel_err(first, po.gemm(X, W, 1)) < 2e-3
+
+
+def test_on_a_stream_with_half_of_the_compute_units(dev, po):
+    """The plans are made for the units of the stream: above 256 rows the bits are those of the whole chip, up to 256 K is sliced
+    another way, always the same one."""
+    N, K = 3072, 4096
+    W = rnd(po, K * N, 53, 0.05).reshape(K, N)
+    dW, ld = weight(dev, W, TILED)
+    s = C.c_void_p()
+    assert dev.lib.lg_stream_create_cu_mask(C.byref(s), (C.c_uint * 8)(*[0xFFFFFFFF] * 4 + [0] * 4), 8) == 0, dev.capi.last_error()
+    try:
+        for M in (40, 200, 300):
+            X = rnd(po, M * K, 54 + M).reshape(M, K)
+            dX, whole = dev.up(X, 1), dev.empty((M, N), 1)
+            dev.call("lg_gemm_f16", TILED, 0, N, M, K, dW, ld, dX, K, whole, N)
+            outs = [dev.empty((M, N), 1) for _ in range(4)]
+            dev.sync()
+            for y in outs:
+                assert dev.lib.lg_gemm_f16(TILED, 0, N, M, K, dW.data_ptr(), ld, dX.data_ptr(), K, y.data_ptr(), N, s) == 0
+            got = [dev.down(y) for y in outs]
+            assert all(np.array_equal(g, got[0]) for g in got)
+            assert max_rel_err(got[0], po.gemm(X, W, 1)) < 2e-3
+            if M > 256:
+                assert np.array_equal(got[0], dev.down(whole))
+    finally:
+        assert dev.lib.lg_stream_destroy(s) == 0
