@@ -235,8 +235,8 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
     static_for<NDS>([&](auto uc) { read_unit(uc, std::integral_constant<int, 0>{}, 0u, 0u, a0, b0); });
     arrive(std::integral_constant<int, 0>{}, a0, b0);
 
-    int xslot = 0, wslot = 0;
-    for (int kt = 0; kt < ktiles; ++kt) {
+    int xslot = 0, wslot = 0, kt = 0;
+    do {
         const unsigned xb = (unsigned)(xslot * X_TILE * 2), wb = (unsigned)(wslot * W_TILE * 2);
         half_t* const xs = smem + xslot * X_TILE;
         half_t* const ws = wring + wslot * W_TILE;
@@ -250,8 +250,14 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
         phase(std::true_type{}, std::integral_constant<int, 1>{}, a1, b1, a0, b0, (unsigned)(xslot * X_TILE * 2), (unsigned)(wslot * W_TILE * 2), x_tile(kt + XS),
               w_tile(kt + WS), xs, ws);
         arrive(std::integral_constant<int, 0>{}, a0, b0);
-    }
-    asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");  // the clamped refills of the last iterations
+    } while (++kt < ktiles);
+    // The clamped refills of the last iterations land, and the last matrix instructions write their results: they are assembly, so the
+    // compiler does not wait for them by itself.  The accumulators are named after the wait so that nothing reads one before it.
+    asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[i][j]));
 
     // ---- epilogue: acc[i][j][r] = Y[m0 + wm*16*MI + i*16 + l16][n0 + wn*16*NJ + j*16 + 4*lk + r] ---------------------------
     // ---- K-slices: the slice of a tile that arrives last takes the others' fp32 sums from the stream's workspace (lane-contiguous),
