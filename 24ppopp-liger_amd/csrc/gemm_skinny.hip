@@ -363,7 +363,8 @@ int launch_gemm_skinny_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap
     if (g.epi.kind == LG_EPI_BIAS_GEGLU) return LG_OK;
     // Above 48 token rows the tile kernels read less of X per weight byte (12288 x 16384 weight at 64 rows: 64.0 against 75.5 us,
     // 12288 x 6144: 29.9 against 32.1) unless the features fill the chip several times over (18432 x 12288: 86 against 77).
-    if (g.M > 48 && (int64_t)g.N * grp.count <= 16384) return LG_OK;
+    // Features that none of their tiles divides stay here: there the sliced or the generic kernel would be next, or a call for every row.
+    if (g.M > 48 && (int64_t)g.N * grp.count <= 16384 && plan_gemm_tiles_f16(g, grp, wlayout, batch, stream).nsplit > 0) return LG_OK;
     const RowMap rm = rows ? *rows : RowMap{};
     const int mt = (g.M + 15) / 16;
     const int cus = stream_info(stream).cus;  // compute units this stream's kernels run on: "one round of blocks" means this many

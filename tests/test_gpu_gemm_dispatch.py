@@ -1,0 +1,90 @@
+"""Which launches a GEMM call makes, read from a graph that the call is captured into: calls that one kernel can take must not fall
+through to slower ways (a second kernel, a kernel on a fraction of the chip, a call for every token row)."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from tests.conftest import max_rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+class _KernelNode(C.Structure):
+    _fields_ = [("block", C.c_uint * 3), ("extra", C.c_void_p), ("func", C.c_void_p), ("grid", C.c_uint * 3), ("params", C.c_void_p), ("shared", C.c_uint)]
+
+
+@pytest.fixture
+def stream(dev):
+    p = C.c_void_p()
+    assert dev.lib.lg_stream_create(C.byref(p)) == 0
+    yield p
+    assert dev.lib.lg_stream_destroy(p) == 0
+
+
+def launches(dev, stream, name, *args):
+    """[workgroups] of the kernels that the call launches; the graph is then run once."""
+    hip, graph, run = dev.lib, C.c_void_p(), C.c_void_p()   # the HIP runtime that the library itself uses
+    dev.sync()
+    assert hip.hipStreamBeginCapture(stream, 0) == 0
+    rc = getattr(dev.lib, name)(*[C.c_void_p(a.data_ptr()) if hasattr(a, "data_ptr") else a for a in args], stream)
+    assert hip.hipStreamEndCapture(stream, C.byref(graph)) == 0 and rc == 0, dev.capi.last_error()
+    n = C.c_size_t()
+    assert hip.hipGraphGetNodes(graph, None, C.byref(n)) == 0
+    nodes, out = (C.c_void_p * n.value)(), []
+    assert hip.hipGraphGetNodes(graph, nodes, C.byref(n)) == 0
+    for node in nodes:
+        p = _KernelNode()
+        assert hip.hipGraphKernelNodeGetParams(C.c_void_p(node), C.byref(p)) == 0
+        out.append(p.grid[0] * p.grid[1] * p.grid[2])
+    assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, 0) == 0
+    assert hip.hipGraphLaunch(run, stream) == 0 and hip.hipStreamSynchronize(stream) == 0
+    assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
+    return out
+
+
+def rnd(po, n, tid, std=1.0):
+    return po.fill_normal(n, 0, tid, 0.0, std, 1)
+
+
+def weight(dev, W, layout):
+    """W [N, K] as the device matrix of layout 1 ([out, in]) or 2 (fragment blocks)"""
+    plain = dev.up(W, 1)
+    if layout == 1:
+        return plain
+    t = dev.empty((W.size,), 1)
+    dev.call("lg_weight_tile_f16", t, plain, W.shape[0], W.shape[1], 1, W.shape[1])
+    dev.sync()
+    return t
+
+
+# features that are a multiple of neither 96 nor 128, on both sides of the row count from which the tile kernels are preferred
+@pytest.mark.parametrize("layout", [1, 2])
+@pytest.mark.parametrize("M", [48, 49, 64])
+def test_features_no_tile_divides_stay_on_one_launch(dev, po, stream, layout, M):
+    N, K = 8224, 2048
+    X, W = rnd(po, M * K, 61).reshape(M, K), rnd(po, N * K, 62, 0.05).reshape(N, K)
+    dX, dW, y = dev.up(X, 1), weight(dev, W, layout), dev.empty((M, N), 1)
+    got = launches(dev, stream, "lg_gemm_f16", layout, 0, N, M, K, dW, K, dX, K, y, N)
+    assert len(got) == 1 and got[0] >= 128
+    assert max_rel_err(dev.down(y), po.gemm(X, np.ascontiguousarray(W.T), 1)) < 2e-3
+
+
+@pytest.mark.parametrize("layout", [1, 2])
+@pytest.mark.parametrize("M", [48, 49, 64])
+def test_projections_with_row_places_stay_on_one_launch(dev, po, stream, layout, M):
+    N, K, d = 2912, 2048, 32
+    h = N // d
+    X = rnd(po, M * K, 63).reshape(M, K)
+    Ws, bs = [rnd(po, N * K, 64 + i, 0.05).reshape(N, K) for i in range(3)], [rnd(po, N, 67 + i, 0.3) for i in range(3)]
+    dX, dW, dB = dev.up(X, 1), [weight(dev, W, layout) for W in Ws], [dev.up(b, 1) for b in bs]
+    out = [dev.empty((M, h, 1, d), 1) for _ in range(3)]
+    ptrs, ints = lambda ts: (C.c_void_p * 3)(*[t.data_ptr() for t in ts]), lambda v: (C.c_int * len(v))(*v)
+    slots = [(5 * r + 3) % M if M % 5 else M - 1 - r for r in range(M)]
+    got = launches(dev, stream, "lg_gemm_fused_grouped_rows_f16", layout, N, M, K, 3, ptrs(dW), K, dX, K, ptrs(out), ints([1, 1, 1]), ptrs(dB), d, h,
+                   ints([0, 1, 1]), ints(slots), ints([0] * M))
+    assert len(got) == 1 and got[0] >= 128
+    for i in range(3):
+        ref = po.round_f16(po.gemm(X, np.ascontiguousarray(Ws[i].T), 1) + bs[i]).reshape(M, h, 1, d)
+        res = dev.down(out[i])
+        assert max_rel_err(res[slots] if i else res, ref) < 2e-3
