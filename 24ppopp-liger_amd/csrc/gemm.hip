@@ -477,8 +477,9 @@ static int gemm_fused_grouped_f16_impl(int mode, int transa, int m, int n, int k
         set_error("gemm_fused_grouped_f16: count must be 1..%d and the pointer arrays non-null", LG_MAX_GROUP);
         return LG_ERR_INVALID;
     }
-    // One launch for the group, member by member, or in pieces: whichever the kernels' own estimate says is the fastest.  All
-    // ways give the same bits (the number of K-slices does not depend on it).
+    // One launch for the group, member by member, or in pieces: whichever the kernels' own estimate says is the fastest.  All ways
+    // give the same bits above 64 rows, and at any count with weights [in, out] (the number of K-slices does not depend on it); at
+    // 5-64 rows with weights [out, in] the weight-streaming kernel may take a group and not its members, in another order of the sum.
     GemmGroup grp{};
     grp.count = count;
     bool one_launch = m > 0 && n > 0 && k > 0 && count > 1 && B != nullptr;

@@ -248,6 +248,9 @@ struct TilePlan {
 TilePlan plan_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, int wlayout, int batch, hipStream_t stream);
 int launch_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled);
 
+// whether the weight-streaming kernel (gemm_skinny.hip) takes `count` members like this, which the tile kernels could take, as one launch
+bool skinny_takes_group(const GemmArgs& g, int count, int wlayout, int cus);
+
 // ---- split-K support of the weight-streaming kernel (gemm_skinny.hip) --------------------------
 // The fp32 partials live in the stream's workspace (StreamInfo::ws, allocated when the stream was created or attached); a
 // launcher never allocates: with no workspace, or one that is too small, it slices K less or not at all.

@@ -22,20 +22,21 @@ constexpr int kMaxTiles = LG_ARRIVAL_COUNTERS / 2;
 // Microseconds of one launch.  Fitted to 556 problems (M 8 .. 2048, 17 weight shapes from 1024 x 1024 to 32768 x 12288, all three
 // layouts) x all tiles and slice counts, each measured with weights cycled out of the caches; picking by it costs 1 % against
 // the best measured choice on average.  Terms: a k-tile costs its matrix work or its loads; a workgroup cannot pull more than 69 GB/s
-// of weights and the chip 7.4 TB/s; what memory and matrix pipes do in the same time overlaps only in part; a K-slice meeting
-// costs a trip to the counter and the transfer of the sums.
-double tile_cost(int M, int N, int K, int count, int mi, int nj, int nsplit, int cus) {
+// of weights (44 in pieces of 256 bytes: 128-wide tiles of [in, out] weights, few rows) and the chip 7.4 TB/s; what memory and matrix pipes do in the same time overlaps only in part; a K-slice meeting
+// costs a trip to the counter and the transfer of the sums, in every round (three projections of 64 rows x 4096 x 4096 in four slices, three
+// rounds: 40 us).
+double tile_cost(int M, int N, int K, int count, int mi, int nj, int nsplit, int wlayout, int cus) {
     const int tiles_m = (M + 32 * mi - 1) / (32 * mi), tiles_n = N / (32 * nj) * count, ktiles = K / MID_K;
     const int kt = (ktiles + nsplit - 1) / nsplit;
     const long wgs = (long)tiles_m * tiles_n * nsplit;
     const double rounds = (double)((wgs + cus - 1) / cus);
     const double work = kt * (0.13 + 0.0192 * mi * nj), loads = kt * (0.0673 + 0.0292 * (mi + nj));
     const double compute = work > loads ? work : loads;
-    const double chip = 2.0 * N * K * count / (7.3735e6 * cus / 256.0) / rounds, own = kt * (64.0 * 32 * 2 / 69.42e3) * nj;
+    const double chip = 2.0 * N * K * count / (7.3735e6 * cus / 256.0) / rounds, own = kt * (64.0 * 32 * 2 / (wlayout == W_KN && nj == 4 && M <= 64 ? 44e3 : 69.42e3)) * nj;
     double round = compute > chip ? compute + 0.6025 * chip : chip + 0.6025 * compute;
     if (round < own) round = own;
     double us = 3.67 + rounds * round;
-    if (nsplit > 1) us += 2.13 + 0.1128 * mi * nj * (mi * nj <= 16 ? nsplit : 1);
+    if (nsplit > 1) us += rounds * (2.13 + 0.1128 * mi * nj * (mi * nj <= 16 ? nsplit : 1));
     return us;
 }
 // The 256-row kernel keeps two waves per SIMD and places tiles for many rows of tiles: 3 % faster than the same tile here when it
@@ -86,25 +87,35 @@ static TilePlan plan_gemm_tiles(const GemmArgs& g, int count, int wlayout, bool 
                 const int sp = fixed ? fixed : tries[c];
                 if ((fixed && c) || sp < 1 || (c > 1 && sp <= 2) || (!fixed && sp > 1 && (!si.ws || tiles * sp > cus || g.M >= kSequentialRows))) continue;
                 if (!usable(t, cnt, sp)) continue;
-                const double us = tile_cost(g.M, g.N, g.K, cnt, t.mi, t.nj, sp, cus);
+                const double us = tile_cost(g.M, g.N, g.K, cnt, t.mi, t.nj, sp, wlayout, cus);
                 if (us < p.cost) p = TilePlan{us, t.mi, t.nj, sp, false};
             }
         }
         return p;
     };
-    // The projections of Q, K and V have the heads epilogue and come as one call or as three: how K is sliced, and with it every bit
-    // of the result, must not depend on which, so it is decided for the three together.
-    int slices = 0;
-    if (heads) {
-        slices = pick(3, 0).nsplit;
-        if (slices < 1) slices = 1;
+    // The members of a group (Q, K and V) come as one call or as several: how K is sliced, and with it every bit of the result, must not
+    // depend on which.  So it is decided for one member alone or, for the heads epilogue, as suits three best (they are what a decode
+    // step calls) among those slice counts with which a projection alone loses less than a half, above 64 rows (prompts, where it is as
+    // likely to come alone) a quarter.  Without that limit it left most of the chip idle under one that comes alone, in microseconds:
+    // 11 rows x 6144 x 12288 [in, out] 79 -> 31 (the three 93 -> 90), 64 rows x 4096 x 4096 30 -> 21 (33 -> 29), 96 rows x 3072 x 4096
+    // 30 -> 18.  Where the weight-streaming kernel takes the three, in another order of the sum anyway, a projection alone is
+    // sliced as suits it.
+    const TilePlan alone = pick(1, 0);
+    if (alone.nsplit == 0) return TilePlan{};
+    int slices = alone.nsplit;
+    if (heads && (alone.nsplit > 1 || pick(LG_MAX_GROUP, 0).nsplit > 1) && !skinny_takes_group(g, LG_MAX_GROUP, wlayout, cus)) {
+        const double most = (g.M <= 64 ? 1.5 : 1.25) * alone.cost;
+        double least = 1e30;
+        for (int sp = 1; sp <= 8; ++sp) {
+            const TilePlan a = pick(1, sp), t = pick(LG_MAX_GROUP, sp);
+            if (a.nsplit && t.nsplit && a.cost < most && t.cost < least) { least = t.cost; slices = sp; }
+        }
     }
     best = pick(count, slices);
-    if (best.nsplit == 0 && slices > 1) best = pick(count, 1);
     if (fast_ok && best.nsplit <= 1 && g.M > 64 && g.epi.kind != LG_EPI_BIAS_HEADS_ROWS)
         for (int nj = 4; nj >= 3; --nj) {
             if (g.N % (64 * nj) || (nj == 3 && g.epi.kind == LG_EPI_BIAS_GEGLU)) continue;
-            const double us = kFastFactor * tile_cost(g.M, g.N, g.K, count, 8, 2 * nj, 1, cus);
+            const double us = kFastFactor * tile_cost(g.M, g.N, g.K, count, 8, 2 * nj, 1, wlayout, cus);
             if (us < best.cost) best = TilePlan{us, 8, nj, 1, true};
         }
     return best;

@@ -354,39 +354,48 @@ static bool skinny_applies(const GemmArgs& g, const GemmGroup& grp, int wlayout,
     return aligned16(g.X) && (g.ldx % 8) == 0 && (g.ldw % 8) == 0 && group_aligned(g, grp);
 }
 
+// How the unsliced kernel deals a problem, or `count` members of a group as one launch, to the compute units: the 16-feature tiles go
+// to one block per compute unit of the stream, 2 to 8 waves a block (the partly filled last wave sits in the first blocks only).  That
+// needs enough tiles to give most compute units two waves, whole pipeline depths of chunks, and for the 2-wave block (four chunks
+// deep) registers for one row tile only.  Problems with more tiles than 8 waves a block take many rounds of 4-wave blocks, where the
+// partial last round no longer matters.  False: the kernel does not take it.
+static bool direct_blocks(const GemmArgs& g, int count, int cus, int* nwv, int* nblocks) {
+    // GeGLU pairs features 16 apart, which sit in different waves here: left to the tile kernels
+    if (g.epi.kind == LG_EPI_BIAS_GEGLU) return false;
+    const int tiles = (g.N + 15) / 16 * count;
+    *nwv = (tiles + cus - 1) / cus;
+    *nblocks = cus;
+    if (*nwv > 8 && tiles >= 16 * cus) { *nwv = 4; *nblocks = (tiles + 3) / 4; }
+    if (*nwv == 7) { *nwv = 8; *nblocks = (tiles + 7) / 8; }
+    const bool deep = *nwv == 2;
+    return *nwv >= 2 && *nwv <= 8 && tiles >= cus * 3 / 2 && g.K % ((deep ? 4 : 2) * SK_KC) == 0 && (!deep || g.M <= 16) &&
+           (int64_t)(*nwv - 1) * *nblocks < tiles && tiles <= (int64_t)*nwv * *nblocks;  // what the kernel's dealing assumes
+}
+
+// Above 48 token rows the tile kernels read less of X per weight byte, and slice K (12288 x 16384 weight at 64 rows: 64.0 against 75.5 us,
+// 12288 x 6144: 29.9 against 32.1), unless the features fill the chip several times over (18432 x 12288: 86 against 77).  For a group,
+// whose members the slices have to suit as well, the line lies lower (64 rows, fragment blocks: three times 3072 x 4096 20.7 against
+// 24.4, three times 4096 x 4096 29.0 against 26.0).
+static bool tiles_preferred(const GemmArgs& g, int count) { return g.M > 48 && (int64_t)g.N * count <= (count > 1 ? 10240 : 16384); }
+
+bool skinny_takes_group(const GemmArgs& g, int count, int wlayout, int cus) {
+    int nwv, nblocks;
+    return skinny_applies(g, single_group(g), wlayout, 1) && direct_blocks(g, count, cus, &nwv, &nblocks) && !tiles_preferred(g, count);
+}
+
 // The unsliced kernel, for a problem or a group as one launch
 int launch_gemm_skinny_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled) {
     *handled = false;
-    if (!skinny_applies(g, grp, wlayout, batch)) return LG_OK;
+    int nwv, nblocks;
+    if (!skinny_applies(g, grp, wlayout, batch) || !direct_blocks(g, grp.count, stream_info(stream).cus, &nwv, &nblocks)) return LG_OK;
     if (g.epi.kind == LG_EPI_BIAS_HEADS_ROWS && !rows) return LG_OK;
-    // GeGLU pairs features 16 apart, which sit in different waves here: left to the tile kernels
-    if (g.epi.kind == LG_EPI_BIAS_GEGLU) return LG_OK;
-    // Above 48 token rows the tile kernels read less of X per weight byte (12288 x 16384 weight at 64 rows: 64.0 against 75.5 us,
-    // 12288 x 6144: 29.9 against 32.1) unless the features fill the chip several times over (18432 x 12288: 86 against 77).
-    // Features that none of their tiles divides stay here: there the sliced or the generic kernel would be next, or a call for every row.
-    if (g.M > 48 && (int64_t)g.N * grp.count <= 16384 && plan_gemm_tiles_f16(g, grp, wlayout, batch, stream).nsplit > 0) return LG_OK;
+    // features that none of their tiles divides stay here: the sliced or the generic kernel would be next, or a call for every row
+    if (tiles_preferred(g, grp.count) && plan_gemm_tiles_f16(g, grp, wlayout, batch, stream).nsplit > 0) return LG_OK;
     const RowMap rm = rows ? *rows : RowMap{};
-    const int mt = (g.M + 15) / 16;
-    const int cus = stream_info(stream).cus;  // compute units this stream's kernels run on: "one round of blocks" means this many
-    // Unsliced: the 16-feature tiles are dealt to one block per compute unit of the stream, 2 to 8 waves a block (the partly
-    // filled last wave sits in the first blocks only).  That needs enough tiles to give most compute units two waves, whole
-    // pipeline depths of chunks, and for the 2-wave block (four chunks deep) registers for one row tile only.  Problems with more
-    // tiles than 8 waves a block take many rounds of 4-wave blocks, where the partial last round no longer matters.
-    {
-        const int tiles = (g.N + 15) / 16 * grp.count;
-        int nwv = (tiles + cus - 1) / cus, nblocks = cus;
-        if (nwv > 8 && tiles >= 16 * cus) { nwv = 4; nblocks = (tiles + 3) / 4; }
-        if (nwv == 7) { nwv = 8; nblocks = (tiles + 7) / 8; }
-        const bool deep = nwv == 2;
-        if (nwv >= 2 && nwv <= 8 && tiles >= cus * 3 / 2 && g.K % ((deep ? 4 : 2) * SK_KC) == 0 && (!deep || mt == 1) &&
-            (int64_t)(nwv - 1) * nblocks < tiles && tiles <= (int64_t)nwv * nblocks) {  // what the kernel's dealing assumes
-            *handled = true;
-            if (wlayout == W_TILED) launch_direct_nwv<true>(nwv, g, grp, rm, nblocks, stream);
-            else launch_direct_nwv<false>(nwv, g, grp, rm, nblocks, stream);
-            return check_launch("gemm_f16_skinny");
-        }
-    }
-    return LG_OK;
+    *handled = true;
+    if (wlayout == W_TILED) launch_direct_nwv<true>(nwv, g, grp, rm, nblocks, stream);
+    else launch_direct_nwv<false>(nwv, g, grp, rm, nblocks, stream);
+    return check_launch("gemm_f16_skinny");
 }
 
 // The K-sliced kernel, for what neither the unsliced kernel nor the tile kernels take (features that are not a multiple of 96 or

@@ -48,9 +48,9 @@ def rnd(po, n, tid, std=1.0):
 
 
 def weight(dev, W, layout):
-    """W [N, K] as the device matrix of layout 1 ([out, in]) or 2 (fragment blocks)"""
-    plain = dev.up(W, 1)
-    if layout == 1:
+    """W [N, K] as the device matrix of layout 0 ([in, out]), 1 ([out, in]) or 2 (fragment blocks)"""
+    plain = dev.up(np.ascontiguousarray(W.T) if layout == 0 else W, 1)
+    if layout != 2:
         return plain
     t = dev.empty((W.size,), 1)
     dev.call("lg_weight_tile_f16", t, plain, W.shape[0], W.shape[1], 1, W.shape[1])
@@ -88,3 +88,32 @@ def test_projections_with_row_places_stay_on_one_launch(dev, po, stream, layout,
         ref = po.round_f16(po.gemm(X, np.ascontiguousarray(Ws[i].T), 1) + bs[i]).reshape(M, h, 1, d)
         res = dev.down(out[i])
         assert max_rel_err(res[slots] if i else res, ref) < 2e-3
+
+
+@pytest.mark.parametrize("layout", [0, 1, 2])
+@pytest.mark.parametrize("M,N,K", [(11, 4096, 4096), (48, 3072, 4096), (64, 4096, 4096), (106, 4096, 2048), (200, 2048, 2048)])
+def test_a_member_alone_has_the_chip_and_the_bits_of_its_group(dev, po, stream, layout, M, N, K):
+    """How K is sliced does not depend on how many members come together: as one of three a member has the bits it has alone (except
+    where the weight-streaming kernel takes the three), and alone it has as many workgroups as a plain call, a projection (whose slices
+    have to suit three as well) a third of them at least."""
+    d = 128
+    X = rnd(po, M * K, 71).reshape(M, K)
+    Ws, bs = [rnd(po, N * K, 72 + i, 0.05).reshape(N, K) for i in range(3)], [rnd(po, N, 75 + i, 0.3) for i in range(3)]
+    dX, dW, dB = dev.up(X, 1), [weight(dev, W, layout) for W in Ws], [dev.up(b, 1) for b in bs]
+    ld = N if layout == 0 else K
+    ptrs = lambda ts: (C.c_void_p * 3)(*[t.data_ptr() for t in ts])
+    plain = launches(dev, stream, "lg_gemm_f16", layout, 0, N, M, K, dW[0], ld, dX, K, dev.empty((M, N), 1), N)
+    for epi, a0, a1, ldc in ((dev.capi.EPI_BIAS_HEADS, 1, d, 1), (dev.capi.EPI_BIAS, 0, 0, N), (dev.capi.EPI_BIAS_GELU, 0, 0, N)):
+        one, three = [[dev.empty((M, N), 1) for _ in range(3)] for _ in range(2)]
+        for i in range(3):
+            got = launches(dev, stream, "lg_gemm_fused_f16", layout, N, M, K, dW[i], ld, dX, K, one[i], ldc, epi, dB[i], a0, a1, 0)
+            assert len(got) == len(plain) and 3 * got[0] >= plain[0] and (epi == dev.capi.EPI_BIAS_HEADS or got == plain)
+        launches(dev, stream, "lg_gemm_fused_grouped_f16", layout, N, M, K, 3, ptrs(dW), ld, dX, K, ptrs(three), (C.c_int * 3)(ldc, ldc, ldc), epi, ptrs(dB), a0, a1, 0)
+        for i in range(3):
+            got, ref = dev.down(three[i]), dev.down(one[i])
+            if M > 64 or layout == 0:
+                assert np.array_equal(got, ref)
+            else:
+                assert max_rel_err(got, ref) < 1e-3
+            if epi != dev.capi.EPI_BIAS_GELU:
+                assert max_rel_err(ref, po.round_f16(po.gemm(X, np.ascontiguousarray(Ws[i].T), 1) + bs[i])) < 2e-3
