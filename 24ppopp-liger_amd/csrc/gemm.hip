@@ -491,19 +491,28 @@ static int gemm_fused_grouped_f16_impl(int mode, int transa, int m, int n, int k
         if (!A[i] || !C[i] || (epilogue != LG_EPI_NONE && !bias[i])) one_launch = false;  // the plain call reports it
     }
     const int wl = transa == LG_OP_TILED ? W_TILED : (transa ? W_NK : W_KN);
+    // a member of the group as a problem of its own, with some of its features
+    auto member = [&](int features) {
+        GemmArgs g{};
+        g.M = n; g.N = features; g.K = k;
+        g.X = (const half_t*)B; g.ldx = ldb;
+        g.W = grp.W[0]; g.ldw = lda;
+        g.Y = grp.Y[0]; g.ldy = grp.ldy[0];
+        g.epi = Epilogue{epilogue, grp.bias[0], epi_arg0, epi_arg1, epi_arg2, 0};
+        return g;
+    };
+    const int cus = stream_info((hipStream_t)stream).cus;
+    // Fragment blocks and few rows: member by member where the weight-streaming kernel takes a member but not the group, whose features
+    // are too many for one wave a feature tile (three times 12288 x 12288, 11 rows: 142 us, as tiles 159; x 4096, 32 rows: 60 and 67).
+    // At 48 rows, or with rows of [out, in], the tiles are level or ahead (x 4096, 48 rows: 63 and 59; [out, in], 11 rows: 71 and 64).
+    if (mode < 0 && one_launch && wl == W_TILED && n <= 32)
+        one_launch = !skinny_takes_group(member(m), 1, wl, cus) || skinny_takes_group(member(m), count, wl, cus);
     if (mode < 0 && one_launch && n > 64) {
         constexpr double kLaunch = 1.5;  // microseconds between two launches
-        const int cus = stream_info((hipStream_t)stream).cus;
         auto plan = [&](int members, int features) {
-            GemmArgs g{};
-            g.M = n; g.N = features; g.K = k;
-            g.X = (const half_t*)B; g.ldx = ldb;
-            g.W = grp.W[0]; g.ldw = lda;
-            g.Y = grp.Y[0]; g.ldy = grp.ldy[0];
-            g.epi = Epilogue{epilogue, grp.bias[0], epi_arg0, epi_arg1, epi_arg2, 0};
             GemmGroup sub = grp;
             sub.count = members;
-            return plan_gemm_tiles_f16(g, sub, wl, 1, (hipStream_t)stream);
+            return plan_gemm_tiles_f16(member(features), sub, wl, 1, (hipStream_t)stream);
         };
         const TilePlan together = plan(count, m), apart = plan(1, m);
         const double cost_apart = count * (apart.cost + kLaunch);

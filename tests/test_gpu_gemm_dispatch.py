@@ -117,3 +117,20 @@ def test_a_member_alone_has_the_chip_and_the_bits_of_its_group(dev, po, stream, 
                 assert max_rel_err(got, ref) < 1e-3
             if epi != dev.capi.EPI_BIAS_GELU:
                 assert max_rel_err(ref, po.round_f16(po.gemm(X, np.ascontiguousarray(Ws[i].T), 1) + bs[i])) < 2e-3
+
+
+@pytest.mark.parametrize("M", [5, 32])
+def test_members_of_many_features_are_weight_streaming_launches_of_their_own(dev, po, stream, M):
+    """Fragment blocks: three times 12288 features are more than one wave a feature tile can hold on the chip; one member is not."""
+    N, K, layout = 12288, 1024, 2
+    X, Ws, b = rnd(po, M * K, 81).reshape(M, K), [rnd(po, N * K, 82 + i, 0.05).reshape(N, K) for i in range(3)], rnd(po, N, 85, 0.3)
+    dX, dB, dW = dev.up(X, 1), dev.up(b, 1), [weight(dev, W, layout) for W in Ws]
+    one, three = [[dev.empty((M, N), 1) for _ in range(3)] for _ in range(2)]
+    ptrs = lambda ts: (C.c_void_p * 3)(*[t.data_ptr() for t in ts])
+    alone = [launches(dev, stream, "lg_gemm_fused_f16", layout, N, M, K, dW[i], K, dX, K, one[i], 1, dev.capi.EPI_BIAS_HEADS, dB, 1, 128, 0) for i in range(3)]
+    got = launches(dev, stream, "lg_gemm_fused_grouped_f16", layout, N, M, K, 3, ptrs(dW), K, dX, K, ptrs(three), (C.c_int * 3)(1, 1, 1), dev.capi.EPI_BIAS_HEADS,
+                   ptrs([dB] * 3), 1, 128, 0)
+    assert [len(a) for a in alone] == [1, 1, 1] and got == alone[0] + alone[1] + alone[2]
+    for i in range(3):
+        assert np.array_equal(dev.down(one[i]), dev.down(three[i]))
+    assert max_rel_err(dev.down(one[2]).reshape(M, N), po.round_f16(po.gemm(X, np.ascontiguousarray(Ws[2].T), 1) + b)) < 2e-3
