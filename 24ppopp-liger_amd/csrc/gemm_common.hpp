@@ -238,6 +238,7 @@ __device__ __forceinline__ void epilogue_geglu4(const GemmArgs& g, half_t* Yb, i
 }
 
 // ---- tile kernels (gemm_mid.hip): the choice made for a problem, or for `count` members of a group as one launch ---------------
+constexpr int MID_TURN_COLS = 768;    // features of a block whose workgroups start their loop over k together: a multiple of every tile width
 constexpr int kSequentialRows = 257;  // from so many token rows on every output is one sum in the order of k, whichever kernel computes it
 struct TilePlan {
     double cost;   // estimated microseconds

@@ -49,7 +49,7 @@ template <int NJ> __device__ __forceinline__ int unswz_kn(int k, int blk) {
 }
 
 template <int WL, int EPI, int NJ>
-__global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup grp, int tiles_m, int tiles_n, int cus, int wide_store) {
+__global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup grp, int tiles_m, int tiles_n, int turn, int cus, int wide_store) {
     constexpr int FB_N = 64 * NJ;
     constexpr int X_TILE = FB_M * FB_K, W_TILE = FB_K * FB_N;  // halves per ring slot
     constexpr int WCH = (FB_K * FB_N) / 512 / 8;  // 1 KiB chunks of the W tile per wave (= NJ)
@@ -144,10 +144,16 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup
     }
     const int64_t wstep = (WL == W_KN) ? (int64_t)FB_K * g.ldw : (WL == W_NK ? FB_K : 1024);
 
+    // Where the loop over k starts, as in the tiles of gemm_mid.hpp: members of one group may be computed by either kernel.
+    const int first = n0 / MID_TURN_COLS * turn % ktiles;
     // tile index clamped to the last one: the loop body is branch-free, the extra loads of the last iterations
     // refill slots nobody reads any more
-    auto x_tile = [&](int kt) { return reinterpret_cast<const char*>(X + (int64_t)(kt < ktiles ? kt : ktiles - 1) * FB_K); };
-    auto w_tile = [&](int kt) { return reinterpret_cast<const char*>(W + (int64_t)(kt < ktiles ? kt : ktiles - 1) * wstep); };
+    auto at = [&](int kt) {
+        const int t = (kt < ktiles ? kt : ktiles - 1) + first;
+        return (int64_t)(t < ktiles ? t : t - ktiles);
+    };
+    auto x_tile = [&](int kt) { return reinterpret_cast<const char*>(X + at(kt) * FB_K); };
+    auto w_tile = [&](int kt) { return reinterpret_cast<const char*>(W + at(kt) * wstep); };
     // load l of a k-tile: l < WCH -> chunk l of the W tile, else chunk l - WCH of the X tile (W first: it is needed first)
     auto issue_one = [&](int l, const char* xg, const char* wg, half_t* xs, half_t* ws) {
         if (l < WCH) load_lds16(reinterpret_cast<const half_t*>(wg + woff[l]), ws + (l * 8 + wave) * 512);
@@ -394,7 +400,7 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup
 }
 
 template <int WL, int NJ>
-static void launch_fast_epi(const GemmArgs& g, const GemmGroup& grp, int tiles_m, int tiles_n, const StreamInfo& si, hipStream_t stream) {
+static void launch_fast_epi(const GemmArgs& g, const GemmGroup& grp, int tiles_m, int tiles_n, int turn, const StreamInfo& si, hipStream_t stream) {
     const int cus = si.cus;
     const dim3 grid(tiles_m * tiles_n), block(F_THREADS);
     const size_t smem = lds_halves(NJ) * sizeof(half_t);
@@ -409,7 +415,7 @@ static void launch_fast_epi(const GemmArgs& g, const GemmGroup& grp, int tiles_m
         /* set once per instantiation; the initialisation of a function-local static is thread-safe */              \
         static const hipError_t attr_rc = hipFuncSetAttribute((const void*)gemm_f16_fast<WL, E, NJ>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem); \
         (void)attr_rc;                                                                                              \
-        hipLaunchKernelGGL((gemm_f16_fast<WL, E, NJ>), grid, block, smem, stream, g, grp, tiles_m, tiles_n, cus, wide); \
+        hipLaunchKernelGGL((gemm_f16_fast<WL, E, NJ>), grid, block, smem, stream, g, grp, tiles_m, tiles_n, turn, cus, wide); \
     } while (0)
     switch (g.epi.kind) {
         case LG_EPI_NONE: LG_FAST(LG_EPI_NONE); break;
@@ -424,7 +430,7 @@ static void launch_fast_epi(const GemmArgs& g, const GemmGroup& grp, int tiles_m
 }
 
 // nj: tile width in units of 64 features (gemm_mid.hip chooses it)
-void launch_gemm_fast_tile(const GemmArgs& g, const GemmGroup& grp, int wlayout, int nj, const StreamInfo& si, hipStream_t stream) {
+void launch_gemm_fast_tile(const GemmArgs& g, const GemmGroup& grp, int wlayout, int nj, int turn, const StreamInfo& si, hipStream_t stream) {
     // LG_GEMM_TILE_WIDTH=2|3|4 in the environment (read once) overrides the choice where that width divides N: a measurement knob
     // (256 x 128 tiles leave registers and LDS for a second kernel's waves on the same compute unit)
     static const int forced_nj = [] { const char* e = getenv("LG_GEMM_TILE_WIDTH"); return e ? atoi(e) : 0; }();
@@ -432,9 +438,9 @@ void launch_gemm_fast_tile(const GemmArgs& g, const GemmGroup& grp, int wlayout,
     const int tiles_m = (g.M + FB_M - 1) / FB_M, tiles_n = g.N / (64 * nj) * grp.count;
 #define LG_FAST_WIDTHS(WL)                                                                   \
     do {                                                                                     \
-        if (nj == 4) launch_fast_epi<WL, 4>(g, grp, tiles_m, tiles_n, si, stream);           \
-        else if (nj == 3) launch_fast_epi<WL, 3>(g, grp, tiles_m, tiles_n, si, stream);      \
-        else launch_fast_epi<WL, 2>(g, grp, tiles_m, tiles_n, si, stream);                   \
+        if (nj == 4) launch_fast_epi<WL, 4>(g, grp, tiles_m, tiles_n, turn, si, stream);           \
+        else if (nj == 3) launch_fast_epi<WL, 3>(g, grp, tiles_m, tiles_n, turn, si, stream);      \
+        else launch_fast_epi<WL, 2>(g, grp, tiles_m, tiles_n, turn, si, stream);                   \
     } while (0)
     if (wlayout == W_TILED) LG_FAST_WIDTHS(W_TILED);
     else if (wlayout == W_NK) LG_FAST_WIDTHS(W_NK);

@@ -9,7 +9,7 @@ LG_MID_DECL(kn_128); LG_MID_DECL(kn_192); LG_MID_DECL(kn_256);
 LG_MID_DECL(nk_96); LG_MID_DECL(nk_128); LG_MID_DECL(nk_192); LG_MID_DECL(nk_256);
 LG_MID_DECL(tiled_96); LG_MID_DECL(tiled_128); LG_MID_DECL(tiled_192); LG_MID_DECL(tiled_256);
 #undef LG_MID_DECL
-void launch_gemm_fast_tile(const GemmArgs& g, const GemmGroup& grp, int wlayout, int nj, const StreamInfo& si, hipStream_t stream);
+void launch_gemm_fast_tile(const GemmArgs& g, const GemmGroup& grp, int wlayout, int nj, int turn, const StreamInfo& si, hipStream_t stream);
 
 namespace {
 
@@ -151,7 +151,7 @@ int launch_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap*
     const StreamInfo si = stream_info(stream);
     *handled = true;
     if (p.fast) {
-        launch_gemm_fast_tile(g, grp, wlayout, p.nj, si, stream);
+        launch_gemm_fast_tile(g, grp, wlayout, p.nj, mid_turn(g.M, g.K, wlayout), si, stream);
         return check_launch("gemm_f16_fast");
     }
     const int ktiles = g.K / MID_K, kt = (ktiles + p.nsplit - 1) / p.nsplit;

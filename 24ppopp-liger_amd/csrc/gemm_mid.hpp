@@ -30,7 +30,6 @@ namespace lg {
 
 constexpr int MID_K = 64;
 constexpr int MID_THREADS = 256;
-constexpr int MID_TURN_COLS = 768;  // features of such a block: a multiple of every tile width
 
 struct MidLaunch {  // what a launch of one of the instantiations needs besides the problem
     int nsplit, kt_per_split;

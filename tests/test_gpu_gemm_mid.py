@@ -154,7 +154,7 @@ def test_streams_of_their_own_and_a_stream_without_a_workspace(dev, po):
 
 
 @pytest.mark.parametrize("layout", [1, 2])
-@pytest.mark.parametrize("M,N,K", [(70, 3072, 960), (106, 1920, 2048), (200, 6144, 1088), (384, 4608, 1024), (511, 2304, 4096)])
+@pytest.mark.parametrize("M,N,K", [(70, 3072, 960), (106, 1920, 2048), (200, 6144, 1088), (240, 12288, 1024), (256, 11264, 1024), (384, 4608, 1024), (511, 2304, 4096)])
 def test_turned_loops(dev, po, layout, M, N, K):
     """Feature blocks of 768 that start at different k-tiles (from 16 k-tiles on): fewer k-tiles than the turns add up to, a last block that is not whole,
     K-slices; and a member of a group of three has the bits of a call of its own, whichever tiles the two take."""
