@@ -253,119 +253,121 @@ __global__ __launch_bounds__(256) void gemm_f32_generic(GemmArgsF32 g) {
 }
 
 // ---------------------------------------------------------------------------------------------------
-// fp32 on the matrix cores: 128 x 128 x 16 tiles, 4 waves (2 x 2), v_mfma_f32_32x32x2_f32
+// fp32 on the matrix cores: 128 x 128 x 16 tiles, 8 waves (2 x 4), v_mfma_f32_16x16x4_f32
 // ---------------------------------------------------------------------------------------------------
 // The reference instantiates every layer for float through cublasGemmEx(..., CUDA_R_32F, ...) (context.h:49-55,
-// linear.h:47-49,99-101).  A wave owns 64 x 64 outputs = 2 x 2 MFMA tiles (64 accumulator registers); operands are swapped as
-// in the fp16 kernels (the weight tile is the A operand), so a lane ends up with 4 consecutive output features of one token
-// row: acc[i][j][v] = Y[token 32 i + lane % 32][feature 32 j + 8 (v / 4) + 4 (lane / 32) + v % 4].  Both tiles sit in LDS
-// k-major ([16][128 + 32] floats): a wave-wide operand read is two runs of 32 consecutive floats, 32 banks apart.
-typedef float float16v_t __attribute__((ext_vector_type(16)));
-constexpr int SB_M = 128, SB_N = 128, SB_K = 16, SB_PITCH = 128 + 32;
+// linear.h:47-49,99-101).  A wave owns 64 x 32 outputs = 4 x 2 MFMA tiles; operands are swapped as in the fp16 kernels (the weight
+// tile is the A operand), so a lane ends up with 4 consecutive output features of one token row:
+// acc[i][j][v] = Y[token 16 i + lane % 16][feature 16 j + 4 (lane / 16) + v].  An output is summed as in gemm_f32.hpp, quarter of K by
+// quarter, with the same instruction and the same k in each of its slots, so that the bits of a row do not depend on which of
+// the two kernels its call takes; that costs a second set of accumulators, and 8 waves instead of 4 leave room for it with four
+// waves on a SIMD.  Rows of 16 k sit in LDS 20 floats apart: a lane's four k are one 16-byte read, and the 16 rows of such a read
+// cover all banks once.  [K, N] weights stay k-major, 132 floats a row: the four k of a read are 16 banks apart.  Two buffers, one
+// barrier for every 16 k.  Against one sum over the whole of K in 4 waves of half the registers, microseconds: 800 x 4096 x 1024
+// 88 -> 81, 1600 x 4096 x 1024 148 -> 145, 4096 x 1024 x 1024 80 -> 83, 4096 x 4096 x 1024 263 -> 285 (120 TFLOP/s: two workgroups share
+// a compute unit, not three), 64 times 512 x 512 x 64 29 -> 33; error against 64-bit sums half as large (K = 1024: 5.7e-7 -> 2.9e-7).
+constexpr int SB_M = 128, SB_N = 128, SB_K = SF_K, SB_ROW = SB_K + 4, SB_PITCH = 128 + 4, SB_THREADS = 512;
 
 template <int WL, bool ALIGNED>
-__global__ __launch_bounds__(256) void gemm_f32_mfma(GemmArgsF32 g) {
-    __shared__ __attribute__((aligned(16))) float Xs[SB_K * SB_PITCH];
-    __shared__ __attribute__((aligned(16))) float Ws[SB_K * SB_PITCH];
+__global__ __launch_bounds__(SB_THREADS, 4) void gemm_f32_mfma(GemmArgsF32 g) {
+    constexpr int W_TILE = WL == W_NK ? SB_N * SB_ROW : SB_K * SB_PITCH;
+    __shared__ __attribute__((aligned(16))) float Xs[2][SB_M * SB_ROW];
+    __shared__ __attribute__((aligned(16))) float Ws[2][W_TILE];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int wm = wave >> 1, wn = wave & 1;
+    const int wm = wave >> 2, wn = wave & 3;
     const int m0 = blockIdx.y * SB_M, n0 = blockIdx.x * SB_N;
     const float* X = g.X + (int64_t)blockIdx.z * g.strideX;
     const float* W = g.W + (int64_t)blockIdx.z * g.strideW;
     float* Y = g.Y + (int64_t)blockIdx.z * g.strideY;
 
-    float16v_t acc[2][2];
+    // 4 consecutive floats p[0..3] with `valid` of them inside the matrix
+    auto load4f = [](const float* p, int valid) {
+        float4_t r = {0.f, 0.f, 0.f, 0.f};
+        if (ALIGNED && valid >= 4) return *reinterpret_cast<const float4_t*>(p);
+        if (valid > 0) {
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
-#pragma unroll
-        for (int j = 0; j < 2; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-
-    // 8 consecutive floats p[0..7] with `valid` of them inside the matrix
-    auto load8f = [](const float* p, int valid, float (&r)[8]) {
-        if (ALIGNED && valid >= 8) {
-            const float4_t a = *reinterpret_cast<const float4_t*>(p), b = *reinterpret_cast<const float4_t*>(p + 4);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) { r[i] = a[i]; r[4 + i] = b[i]; }
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) r[i] = i < valid ? p[i] : 0.f;
+            for (int i = 0; i < 4; ++i)
+                if (i < valid) r[i] = p[i];
         }
+        return r;
     };
-    float rx[8], rw[8];
+    float4_t rx, rw;
+    const int row = tid >> 2, kq = (tid & 3) * 4;    // rows of 16 k: thread = (row, quarter of the k)
+    const int kr = tid >> 5, ns = (tid & 31) * 4;    // [K, N] weights: 16 k-rows x 128 features; thread = (k, 4 consecutive features)
     auto gload = [&](int k0) {
-        {   // X tile: 128 token rows x 16 k; thread = (row, half of the k range)
-            const int row = tid >> 1, kh = (tid & 1) * 8;
-            const int m = m0 + row, k = k0 + kh;
-            load8f(X + (int64_t)m * g.ldx + k, m < g.M ? g.K - k : 0, rx);
-        }
-        if (WL == W_NK) {
-            const int row = tid >> 1, kh = (tid & 1) * 8;
-            const int n = n0 + row, k = k0 + kh;
-            load8f(W + (int64_t)n * g.ldw + k, n < g.N ? g.K - k : 0, rw);
-        } else {  // [K, N]: 16 k-rows x 128 features; thread = (k, 8 consecutive features)
-            const int kr = tid >> 4, ns = (tid & 15) * 8;
-            const int k = k0 + kr, n = n0 + ns;
-            load8f(W + (int64_t)k * g.ldw + n, k < g.K ? g.N - n : 0, rw);
-        }
+        rx = load4f(X + (int64_t)(m0 + row) * g.ldx + k0 + kq, m0 + row < g.M ? g.K - k0 - kq : 0);
+        if (WL == W_NK) rw = load4f(W + (int64_t)(n0 + row) * g.ldw + k0 + kq, n0 + row < g.N ? g.K - k0 - kq : 0);
+        else rw = load4f(W + (int64_t)(k0 + kr) * g.ldw + n0 + ns, k0 + kr < g.K ? g.N - n0 - ns : 0);
     };
-    auto lstore = [&]() {
-        {
-            const int row = tid >> 1, kh = (tid & 1) * 8;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) Xs[(kh + i) * SB_PITCH + row] = rx[i];
-        }
-        if (WL == W_NK) {
-            const int row = tid >> 1, kh = (tid & 1) * 8;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) Ws[(kh + i) * SB_PITCH + row] = rw[i];
-        } else {
-            const int kr = tid >> 4, ns = (tid & 15) * 8;
-            *reinterpret_cast<float4_t*>(&Ws[kr * SB_PITCH + ns]) = float4_t{rw[0], rw[1], rw[2], rw[3]};
-            *reinterpret_cast<float4_t*>(&Ws[kr * SB_PITCH + ns + 4]) = float4_t{rw[4], rw[5], rw[6], rw[7]};
-        }
+    auto lstore = [&](int buf) {
+        *reinterpret_cast<float4_t*>(&Xs[buf][row * SB_ROW + kq]) = rx;
+        *reinterpret_cast<float4_t*>(WL == W_NK ? &Ws[buf][row * SB_ROW + kq] : &Ws[buf][kr * SB_PITCH + ns]) = rw;
     };
 
-    const int l32 = lane & 31, lh = lane >> 5;
-    gload(0);
-    for (int k0 = 0; k0 < g.K; k0 += SB_K) {
-        __syncthreads();
-        lstore();
-        __syncthreads();
-        if (k0 + SB_K < g.K) gload(k0 + SB_K);
+    const int l16 = lane & 15, lk = lane >> 4;
+    float4_t acc[4][2], total[4][2];
+    const int chunks = (g.K + SB_K - 1) / SB_K, quarter = f32_quarter(g.K);
+    int c = 0;
+    auto chunk = [&](auto first, float4_t (&sum)[4][2]) {  // first of its quarter: the sums start from zero
+        const int buf = c & 1;
+        lstore(buf);
+        __syncthreads();  // the other buffer is refilled after the next one: every wave is done with it by then
+        if (++c < chunks) gload(c * SB_K);
+        float4_t x[4], w[2];  // k 4 lk .. 4 lk + 3 of row 16 i + l16
 #pragma unroll
-        for (int ks = 0; ks < SB_K / 2; ++ks) {
-            float a[2], b[2];
+        for (int i = 0; i < 4; ++i) x[i] = *reinterpret_cast<const float4_t*>(&Xs[buf][(wm * 64 + i * 16 + l16) * SB_ROW + 4 * lk]);
 #pragma unroll
-            for (int i = 0; i < 2; ++i) a[i] = Xs[(ks * 2 + lh) * SB_PITCH + wm * 64 + i * 32 + l32];
+        for (int j = 0; j < 2; ++j) {
+            if (WL == W_NK) {
+                w[j] = *reinterpret_cast<const float4_t*>(&Ws[buf][(wn * 32 + j * 16 + l16) * SB_ROW + 4 * lk]);
+            } else {
 #pragma unroll
-            for (int j = 0; j < 2; ++j) b[j] = Ws[(ks * 2 + lh) * SB_PITCH + wn * 64 + j * 32 + l32];
-#pragma unroll
-            for (int i = 0; i < 2; ++i)
-#pragma unroll
-                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(b[j], a[i], acc[i][j], 0, 0, 0);
+                for (int r = 0; r < 4; ++r) w[j][r] = Ws[buf][(4 * lk + r) * SB_PITCH + wn * 32 + j * 16 + l16];
+            }
         }
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const float4_t before = decltype(first)::value && r == 0 ? float4_t{0.f, 0.f, 0.f, 0.f} : sum[i][j];
+                    sum[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][r], x[i][r], before, 0, 0, 0);
+                }
+    };
+    gload(0);
+    chunk(std::true_type{}, total);
+#pragma unroll 1
+    while (c < quarter) chunk(std::false_type{}, total);
+#pragma unroll 1
+    for (int q = 1; q < SF_WAVES; ++q) {
+        const int end = min(chunks, (q + 1) * quarter);
+        if (c >= end) break;  // (a wave of gemm_f32.hpp without chunks adds zero)
+        chunk(std::true_type{}, acc);
+#pragma unroll 1
+        while (c < end) chunk(std::false_type{}, acc);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) total[i][j] += acc[i][j];
     }
     const bool vec_ok = ALIGNED && (g.ldy % 4 == 0);
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int m = m0 + wm * 64 + i * 32 + l32;
+    for (int i = 0; i < 4; ++i) {
+        const int m = m0 + wm * 64 + i * 16 + l16;
         if (m >= g.M) continue;
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < 2; ++j) {
+            const int n = n0 + wn * 32 + j * 16 + 4 * lk;
+            float* p = Y + (int64_t)m * g.ldy + n;
+            if (vec_ok && n + 3 < g.N) {
+                *reinterpret_cast<float4_t*>(p) = total[i][j];
+            } else {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const int n = n0 + wn * 64 + j * 32 + 8 * q + 4 * lh;
-                float* p = Y + (int64_t)m * g.ldy + n;
-                if (vec_ok && n + 3 < g.N) {
-                    *reinterpret_cast<float4_t*>(p) = float4_t{acc[i][j][4 * q], acc[i][j][4 * q + 1], acc[i][j][4 * q + 2], acc[i][j][4 * q + 3]};
-                } else {
-#pragma unroll
-                    for (int r = 0; r < 4; ++r)
-                        if (n + r < g.N) p[r] = acc[i][j][4 * q + r];
-                }
+                for (int r = 0; r < 4; ++r)
+                    if (n + r < g.N) p[r] = total[i][j][r];
             }
+        }
     }
 }
 
@@ -383,11 +385,11 @@ static int gemm_f32_dispatch(const GemmArgsF32& g, int wlayout, int batch, hipSt
         const int rc = launch_gemm_f32_direct(g, wlayout, batch, aligned, stream, &handled);
         if (handled) return rc;
         if (wlayout == W_NK) {
-            if (aligned) hipLaunchKernelGGL((gemm_f32_mfma<W_NK, true>), grid, dim3(256), 0, stream, g);
-            else hipLaunchKernelGGL((gemm_f32_mfma<W_NK, false>), grid, dim3(256), 0, stream, g);
+            if (aligned) hipLaunchKernelGGL((gemm_f32_mfma<W_NK, true>), grid, dim3(SB_THREADS), 0, stream, g);
+            else hipLaunchKernelGGL((gemm_f32_mfma<W_NK, false>), grid, dim3(SB_THREADS), 0, stream, g);
         } else {
-            if (aligned) hipLaunchKernelGGL((gemm_f32_mfma<W_KN, true>), grid, dim3(256), 0, stream, g);
-            else hipLaunchKernelGGL((gemm_f32_mfma<W_KN, false>), grid, dim3(256), 0, stream, g);
+            if (aligned) hipLaunchKernelGGL((gemm_f32_mfma<W_KN, true>), grid, dim3(SB_THREADS), 0, stream, g);
+            else hipLaunchKernelGGL((gemm_f32_mfma<W_KN, false>), grid, dim3(SB_THREADS), 0, stream, g);
         }
         return check_launch("gemm_f32");
     }

@@ -6,15 +6,16 @@
 // most, which the caches deliver without LDS.  What bounds the path is how the work is dealt out -- the 128 x 128 tiles that this
 // replaces left a layer of hidden 1024 and 800 tokens on 56 of 256 compute units and one of hidden 256 on two -- and, inside a
 // workgroup, the latency of the loads.  So:
-//   * the four waves of a workgroup own the same tile and share K: chunks of 16 k go to them in turn (two neighbours use the two
-//     halves of a cache line), no wave waits for another until the end, and even a 16 x 16 tile has four SIMDs at work;
+//   * the four waves of a workgroup own the same tile and take a quarter of K each, no wave waits for another until the end, and
+//     even a 16 x 16 tile has four SIMDs at work;
 //   * a wave keeps D chunks of both operands in flight in registers;
 //   * a lane loads 4 consecutive k of one row as 16 bytes ([N, K] weights, X) and feeds one of them to each of four matrix
 //     instructions -- any assignment of k to instruction slots will do if both operands agree; of [K, N] weights it loads NJ
 //     consecutive features, one for each tile column, so tile column j holds features NJ c + j;
 //   * the four sums of an output meet in LDS, added in wave order, and leave as whole rows.
-// Every tile size adds the same products in the same order, so a result does not depend on the tile, the batch around a row or the
-// feature range around a column.
+// Every tile size, and the 128 x 128 kernel of gemm.hip, adds the same products in the same order: within a quarter of K by chunks of 16
+// k, in a chunk by the slots of the matrix instruction, then the four quarters.  So a result does not depend on the tile, the batch
+// around a row or the feature range around a column.
 #pragma once
 #include "gemm_common.hpp"
 
@@ -35,6 +36,8 @@ template <> struct FloatU<4> { typedef float type __attribute__((ext_vector_type
 typedef FloatU<4>::type float4u_t;
 
 constexpr int SF_WAVES = 4, SF_THREADS = 64 * SF_WAVES, SF_K = 16;  // k of a chunk
+// chunks in a quarter of K; the last ones may hold fewer, or none
+__host__ __device__ inline int f32_quarter(int K) { return ((K + SF_K - 1) / SF_K + SF_WAVES - 1) / SF_WAVES; }
 
 template <int WL, int MI, int NJ, int D>
 __global__ __launch_bounds__(SF_THREADS, 2) void gemm_f32_direct(GemmArgsF32 g, int tiles_m, int tiles_n) {
@@ -122,12 +125,12 @@ __global__ __launch_bounds__(SF_THREADS, 2) void gemm_f32_direct(GemmArgsF32 g, 
                 }
     };
 
-    const int chunks = g.K / SF_K;
-    const int mine = (chunks - wave + SF_WAVES - 1) / SF_WAVES;  // this wave's chunks: wave, wave + 4, ...
+    const int chunks = g.K / SF_K, quarter = f32_quarter(g.K);
+    const int first = wave * quarter, mine = min(chunks - first, quarter);  // this wave's whole chunks: first, first + 1, ...
     if (mine > 0) {
         Chunk c[D];
         // the chunk index is clamped to the last one: loads past it are not used
-        auto at = [&](int t) { return (int64_t)(wave + SF_WAVES * min(t, mine - 1)) * SF_K; };
+        auto at = [&](int t) { return (int64_t)(first + min(t, mine - 1)) * SF_K; };
 #pragma unroll
         for (int d = 0; d < D; ++d) load(c[d], at(d));
         for (int t = 0; t < mine; t += D) {
@@ -140,7 +143,7 @@ __global__ __launch_bounds__(SF_THREADS, 2) void gemm_f32_direct(GemmArgsF32 g, 
             }
         }
     }
-    if (g.K % SF_K != 0 && wave == chunks % SF_WAVES) {
+    if (g.K % SF_K != 0 && wave == chunks / quarter) {
         Chunk c;
         load_tail(c, (int64_t)chunks * SF_K);
         multiply(c);

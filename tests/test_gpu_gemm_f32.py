@@ -60,3 +60,28 @@ def test_infinities_stay_in_their_rows(dev):
     dev.call("lg_gemm_f32", 0, 0, N, M, K, W.data_ptr(), N, X.data_ptr(), K, Y.data_ptr(), N)
     dev.sync()
     assert bool(torch.isfinite(Y[:49]).all()) and not bool(torch.isfinite(Y[49]).any())
+
+
+# shapes whose parts take smaller tiles than the whole, in both kernels; K with whole quarters, with a remainder and with fewer chunks than quarters
+@pytest.mark.parametrize("transa", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(800, 4096, 1024), (1600, 1024, 1000), (1000, 4100, 333), (2048, 2048, 40), (1300, 2050, 17)])
+def test_a_row_does_not_depend_on_its_call(dev, transa, M, N, K):
+    """Rows and features of a decomposed call have the bits of the whole: every tile of both kernels sums in the same order."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(1)
+    X = torch.randn(M, K, device="cuda", generator=gen)
+    W = torch.randn(*((K, N) if transa == 0 else (N, K)), device="cuda", generator=gen)
+    ldw = W.shape[1]
+
+    def gemm(m0, m, n0, n):
+        Y = torch.empty(m, n, device="cuda")
+        dev.call("lg_gemm_f32", transa, 0, n, m, K, W.data_ptr() + 4 * n0 * (1 if transa == 0 else K), ldw, X.data_ptr() + 4 * m0 * K, K, Y.data_ptr(), n)
+        dev.sync()
+        return Y
+
+    torch.cuda.synchronize()
+    whole = gemm(0, M, 0, N)
+    for m0, m in ((0, M // 2), (M // 2, M - M // 2), (M - 200, 200), (3, 64), (5, 1)):
+        assert torch.equal(gemm(m0, m, 0, N), whole[m0:m0 + m])
+    for n0, n in ((0, N // 4), (N // 4, N - N // 4), (N - 130, 130), (7, 16)):
+        assert torch.equal(gemm(0, M, n0, n), whole[:, n0:n0 + n])
