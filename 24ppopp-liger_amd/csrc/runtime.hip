@@ -78,9 +78,15 @@ static int register_stream(void* stream, int cus) {
     info.ws = (float*)p;
     info.ws_bytes = LG_SPLITK_WORKSPACE_BYTES;
     info.arrivals = (unsigned*)((char*)p + LG_SPLITK_WORKSPACE_BYTES);
-    // set once, here: every kernel that counts arrivals leaves its counters at zero
-    rc = rt(hipMemset(info.arrivals, 0, counter_bytes), "hipMemset (arrival counters)");
-    if (rc == LG_OK) rc = rt(hipStreamSynchronize(nullptr), "hipStreamSynchronize");
+    // Set once, here: every kernel that counts arrivals leaves its counters at zero.  On a stream of its own: the null stream waits for
+    // the work of every blocking stream, and ends a capture that is open on one.
+    hipStream_t own = nullptr;
+    rc = rt(hipStreamCreateWithFlags(&own, hipStreamNonBlocking), "hipStreamCreateWithFlags");
+    if (rc == LG_OK) {
+        rc = rt(hipMemsetAsync(info.arrivals, 0, counter_bytes, own), "hipMemsetAsync (arrival counters)");
+        if (rc == LG_OK) rc = rt(hipStreamSynchronize(own), "hipStreamSynchronize");
+        (void)hipStreamDestroy(own);
+    }
     if (rc) {
         (void)hipFree(p);
         return rc;

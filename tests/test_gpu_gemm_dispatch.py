@@ -134,3 +134,13 @@ def test_members_of_many_features_are_weight_streaming_launches_of_their_own(dev
     for i in range(3):
         assert np.array_equal(dev.down(one[i]), dev.down(three[i]))
     assert max_rel_err(dev.down(one[2]).reshape(M, N), po.round_f16(po.gemm(X, np.ascontiguousarray(Ws[2].T), 1) + b)) < 2e-3
+
+
+def test_a_stream_can_be_made_while_another_is_captured(dev):
+    """The set-up of a stream's workspace keeps off the null stream: a (relaxed) capture that is open on a blocking stream goes on."""
+    hip, s, graph, made = dev.lib, C.c_void_p(), C.c_void_p(), C.c_void_p()
+    dev.sync()
+    assert hip.hipStreamCreate(C.byref(s)) == 0 and hip.hipStreamBeginCapture(s, 2) == 0
+    rc = dev.lib.lg_stream_create(C.byref(made))
+    assert hip.hipStreamEndCapture(s, C.byref(graph)) == 0 and rc == 0, dev.capi.last_error()
+    assert dev.lib.lg_stream_destroy(made) == 0 and hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(s) == 0
