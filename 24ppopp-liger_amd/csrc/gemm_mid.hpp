@@ -30,6 +30,7 @@ namespace lg {
 
 constexpr int MID_K = 64;
 constexpr int MID_THREADS = 256;
+constexpr int MID_MAX_SPINS = 1 << 21;
 
 struct MidLaunch {  // what a launch of one of the instantiations needs besides the problem
     int nsplit, kt_per_split;
@@ -261,7 +262,9 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
     // ---- epilogue: acc[i][j][r] = Y[m0 + wm*16*MI + i*16 + l16][n0 + wn*16*NJ + j*16 + 4*lk + r] ---------------------------
     // ---- K-slices: the slice of a tile that arrives last takes the others' fp32 sums from the stream's workspace (lane-contiguous),
     // adds all of them in slice order and goes on to the epilogue.  Nobody waits for a workgroup that may not be running: the wait
-    // below is for slices that have already arrived and are storing.  The counters are back at zero when the launch ends.
+    // below is for slices that have already arrived and are storing, microseconds.  It is bounded (a second or so) for a caller who
+    // breaks the rule that one launch runs at a time on a workspace (a captured graph replayed on two streams at once): wrong sums
+    // then, but the launch ends.  The counters are back at zero when the launch ends.
     if (nsplit > 1) {
         constexpr int SLICE = MI * NJ * MID_THREADS * 16;  // bytes
         // Small tiles: every slice stores its sums, then counts itself in (one trip to the counter).  Large ones: a slice first learns
@@ -295,7 +298,8 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
                 return;
             }
             if (tid == 0) {
-                while (__hip_atomic_load(stored, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (unsigned)nsplit - 1) __builtin_amdgcn_s_sleep(1);
+                for (int spins = 0; spins < MID_MAX_SPINS && __hip_atomic_load(stored, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != (unsigned)nsplit - 1; ++spins)
+                    __builtin_amdgcn_s_sleep(1);
                 __hip_atomic_store(stored, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
             }
             __syncthreads();

@@ -10,7 +10,8 @@
  *     library owns is a 64 MiB split-K workspace per stream, allocated by lg_stream_create* / lg_stream_attach and freed
  *     by lg_stream_destroy / lg_stream_detach -- the counterpart of the workspace a cuBLAS handle owns (context.h:20-29
  *     binds one handle per stream).  A GEMM on a stream the library was never told about still runs, without slicing K
- *     (slower for few and medium token counts);
+ *     (slower for few and medium token counts).  A captured launch keeps the workspace of the stream it was captured on:
+ *     replay it there, or while that stream is idle, and not twice at the same time;
  *   - several kernels work in place, exactly where the reference's do.
  * Differences: every function returns an int status instead of asserting --
  *   LG_OK, LG_ERR_INVALID (bad / unsupported shape or pointer), LG_ERR_LAUNCH (HIP error; text via

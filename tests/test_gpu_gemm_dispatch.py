@@ -4,6 +4,7 @@ import ctypes as C
 
 import numpy as np
 import pytest
+import torch
 
 from tests.conftest import max_rel_err
 
@@ -22,8 +23,8 @@ def stream(dev):
     assert dev.lib.lg_stream_destroy(p) == 0
 
 
-def launches(dev, stream, name, *args):
-    """[workgroups] of the kernels that the call launches; the graph is then run once."""
+def launches(dev, stream, name, *args, replays=1, between=None):
+    """[workgroups] of the kernels that the call launches; the graph is then run, with `between` after each replay."""
     hip, graph, run = dev.lib, C.c_void_p(), C.c_void_p()   # the HIP runtime that the library itself uses
     dev.sync()
     assert hip.hipStreamBeginCapture(stream, 0) == 0
@@ -38,7 +39,10 @@ def launches(dev, stream, name, *args):
         assert hip.hipGraphKernelNodeGetParams(C.c_void_p(node), C.byref(p)) == 0
         out.append(p.grid[0] * p.grid[1] * p.grid[2])
     assert hip.hipGraphInstantiate(C.byref(run), graph, None, None, 0) == 0
-    assert hip.hipGraphLaunch(run, stream) == 0 and hip.hipStreamSynchronize(stream) == 0
+    for _ in range(replays):
+        assert hip.hipGraphLaunch(run, stream) == 0 and hip.hipStreamSynchronize(stream) == 0
+        if between:
+            between()
     assert hip.hipGraphExecDestroy(run) == 0 and hip.hipGraphDestroy(graph) == 0
     return out
 
@@ -144,3 +148,25 @@ def test_a_stream_can_be_made_while_another_is_captured(dev):
     rc = dev.lib.lg_stream_create(C.byref(made))
     assert hip.hipStreamEndCapture(s, C.byref(graph)) == 0 and rc == 0, dev.capi.last_error()
     assert dev.lib.lg_stream_destroy(made) == 0 and hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(s) == 0
+
+
+@pytest.mark.parametrize("M,N,K", [(11, 4096, 4096), (200, 4096, 4096), (256, 6144, 12288)])
+def test_sliced_launches_replayed_between_eager_ones(dev, po, stream, M, N, K):
+    """K-slices that meet in small tiles and in large ones: every replay, and the plain calls between them on the same workspace, end
+    with the counters where they were and have the same bits."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(5)
+    dX, dW = torch.randn(M, K, device="cuda", generator=gen).half(), (torch.randn(N * K, device="cuda", generator=gen) * 0.02).half()
+    y, z = dev.empty((M, N), 1), dev.empty((M, N), 1)
+    seen = []
+
+    def between():
+        assert dev.lib.lg_gemm_f16(2, 0, N, M, K, dW.data_ptr(), K, dX.data_ptr(), K, z.data_ptr(), N, stream) == 0
+        dev.sync()
+        seen.append((y.clone(), z.clone()))
+        y.fill_(0.0)
+        z.fill_(0.0)
+        dev.sync()
+
+    assert len(launches(dev, stream, "lg_gemm_f16", 2, 0, N, M, K, dW, K, dX, K, y, N, replays=4, between=between)) == 1
+    assert all(torch.equal(a, seen[0][0]) and torch.equal(b, seen[0][0]) for a, b in seen) and bool(seen[0][0].any())
