@@ -256,6 +256,6 @@ bool skinny_takes_group(const GemmArgs& g, int count, int wlayout, int cus);
 // The fp32 partials live in the stream's workspace (StreamInfo::ws, allocated when the stream was created or attached); a
 // launcher never allocates: with no workspace, or one that is too small, it slices K less or not at all.
 // Y = epilogue(sum over the nsplit K-slices in slice order) of the fp32 partials [nsplit][M][N]
-void launch_splitk_reduce(const GemmArgs& g, const float* partial, int nsplit, hipStream_t stream, const RowMap* rows = nullptr);
+void launch_splitk_reduce(const GemmArgs& g, const float* partial, int nsplit, hipStream_t stream);
 
 }  // namespace lg

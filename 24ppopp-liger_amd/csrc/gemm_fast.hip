@@ -29,8 +29,8 @@ namespace lg {
 
 constexpr int FB_M = 256, FB_K = 64;
 constexpr int F_THREADS = 512;
-// The tile is 256 x (64 * NJ) outputs: NJ = 4 -> 256 x 256, NJ = 3 -> 256 x 192, NJ = 2 -> 256 x 128 (used when it needs fewer rounds of 256
-// workgroups, e.g. N = 6144: 512 tiles = 2 full rounds instead of 384 tiles = 1.5 rounds)
+// The tile is 256 x (64 * NJ) outputs: NJ = 4 -> 256 x 256, NJ = 3 -> 256 x 192; NJ = 2 -> 256 x 128 only on demand (LG_GEMM_TILE_WIDTH,
+// below): gemm_mid.hip never prefers it
 // LDS: a ring of 3 X tiles and a ring of 2 W tiles (256-wide: 96 + 64 KiB = the whole 160 KiB of a CU)
 constexpr int X_STAGES = 3, W_STAGES = 2;
 constexpr int lds_halves(int NJ) { return X_STAGES * FB_M * FB_K + W_STAGES * FB_K * 64 * NJ; }
@@ -431,8 +431,8 @@ static void launch_fast_epi(const GemmArgs& g, const GemmGroup& grp, int tiles_m
 
 // nj: tile width in units of 64 features (gemm_mid.hip chooses it)
 void launch_gemm_fast_tile(const GemmArgs& g, const GemmGroup& grp, int wlayout, int nj, int turn, const StreamInfo& si, hipStream_t stream) {
-    // LG_GEMM_TILE_WIDTH=2|3|4 in the environment (read once) overrides the choice where that width divides N: a measurement knob
-    // (256 x 128 tiles leave registers and LDS for a second kernel's waves on the same compute unit)
+    // LG_GEMM_TILE_WIDTH=2|3|4 in the environment (read once) overrides the width where it divides N, for the problems that come here: a
+    // measurement knob (256 x 128 tiles leave registers and LDS for a second kernel's waves on the same compute unit)
     static const int forced_nj = [] { const char* e = getenv("LG_GEMM_TILE_WIDTH"); return e ? atoi(e) : 0; }();
     if (forced_nj >= 2 && forced_nj <= 4 && g.N % (64 * forced_nj) == 0 && !(forced_nj == 3 && g.epi.kind == LG_EPI_BIAS_GEGLU)) nj = forced_nj;
     const int tiles_m = (g.M + FB_M - 1) / FB_M, tiles_n = g.N / (64 * nj) * grp.count;

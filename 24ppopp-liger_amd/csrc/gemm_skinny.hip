@@ -290,7 +290,7 @@ static void launch_direct_nwv(int nwv, const GemmArgs& g, const GemmGroup& grp, 
 
 // sums the K-slices and applies the epilogue; one thread per 4 consecutive output columns
 template <int EPI>
-__global__ __launch_bounds__(256) void gemm_skinny_reduce_kernel(GemmArgs g, const float* partial, int nsplit, RowMap rm) {
+__global__ __launch_bounds__(256) void gemm_skinny_reduce_kernel(GemmArgs g, const float* partial, int nsplit) {
     const int64_t quads = (int64_t)g.M * ((g.N + 3) / 4);
     for (int64_t q = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; q < quads; q += (int64_t)gridDim.x * blockDim.x) {
         const int nq = (g.N + 3) / 4;
@@ -304,7 +304,7 @@ __global__ __launch_bounds__(256) void gemm_skinny_reduce_kernel(GemmArgs g, con
                 for (int r = 0; r < 4 && n + r < g.N; ++r) s[r] += p[r];
             }
         }
-        epilogue_store4<EPI>(g, g.Y, m, n, s, true, &rm);
+        epilogue_store4<EPI>(g, g.Y, m, n, s, true);
     }
 }
 
@@ -325,7 +325,7 @@ __global__ __launch_bounds__(256) void gemm_skinny_reduce_geglu_kernel(GemmArgs 
     }
 }
 
-void launch_splitk_reduce(const GemmArgs& g, const float* partial, int nsplit, hipStream_t stream, const RowMap* rows) {
+void launch_splitk_reduce(const GemmArgs& g, const float* partial, int nsplit, hipStream_t stream) {
     const dim3 block(256);
     if (g.epi.kind == LG_EPI_BIAS_GEGLU) {
         const int64_t gq = (int64_t)g.M * (g.N / 8);
@@ -337,13 +337,11 @@ void launch_splitk_reduce(const GemmArgs& g, const float* partial, int nsplit, h
     const int64_t quads = (int64_t)g.M * ((g.N + 3) / 4);
     int rgrid = (int)((quads + 255) / 256);
     if (rgrid > 4096) rgrid = 4096;
-    const RowMap rm = rows ? *rows : RowMap{};
     switch (g.epi.kind) {
-        case LG_EPI_NONE: hipLaunchKernelGGL((gemm_skinny_reduce_kernel<LG_EPI_NONE>), dim3(rgrid), block, 0, stream, g, partial, nsplit, rm); break;
-        case LG_EPI_BIAS: hipLaunchKernelGGL((gemm_skinny_reduce_kernel<LG_EPI_BIAS>), dim3(rgrid), block, 0, stream, g, partial, nsplit, rm); break;
-        case LG_EPI_BIAS_GELU: hipLaunchKernelGGL((gemm_skinny_reduce_kernel<LG_EPI_BIAS_GELU>), dim3(rgrid), block, 0, stream, g, partial, nsplit, rm); break;
-        case LG_EPI_BIAS_HEADS_ROWS: hipLaunchKernelGGL((gemm_skinny_reduce_kernel<LG_EPI_BIAS_HEADS_ROWS>), dim3(rgrid), block, 0, stream, g, partial, nsplit, rm); break;
-        default: hipLaunchKernelGGL((gemm_skinny_reduce_kernel<LG_EPI_BIAS_HEADS>), dim3(rgrid), block, 0, stream, g, partial, nsplit, rm); break;
+        case LG_EPI_NONE: hipLaunchKernelGGL((gemm_skinny_reduce_kernel<LG_EPI_NONE>), dim3(rgrid), block, 0, stream, g, partial, nsplit); break;
+        case LG_EPI_BIAS: hipLaunchKernelGGL((gemm_skinny_reduce_kernel<LG_EPI_BIAS>), dim3(rgrid), block, 0, stream, g, partial, nsplit); break;
+        case LG_EPI_BIAS_GELU: hipLaunchKernelGGL((gemm_skinny_reduce_kernel<LG_EPI_BIAS_GELU>), dim3(rgrid), block, 0, stream, g, partial, nsplit); break;
+        default: hipLaunchKernelGGL((gemm_skinny_reduce_kernel<LG_EPI_BIAS_HEADS>), dim3(rgrid), block, 0, stream, g, partial, nsplit); break;
     }
 }
 
