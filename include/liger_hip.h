@@ -211,10 +211,10 @@ int lg_gemm_fused_f16(int transa, int m, int n, int k, const void* A, int lda, c
 /* `count` (1..3) lg_gemm_fused_f16 calls that share B (the token rows), the shape, lda and the epilogue arguments
  * and differ in A[i], C[i], ldc[i] and bias[i]: the Q, K and V projections of a decode step (linear.h:99-101 issued
  * three times by bert_layer.h:127-137; also the column blocks of one packed [H, 3 Hl] weight: A[i] = the block's first
- * column or row, lda = the packed matrix's).  Few-token problems with weights [out, in] run as ONE launch of the
- * weight-streaming kernels, problems of more than 256 token rows as ONE launch of the pipelined kernel (either weight
- * layout); anything else is executed as `count` plain calls.  Results are those of the plain calls up to the order of the
- * fp32 sum over k (the one launch may use another block width).  No reference counterpart. */
+ * column or row, lda = the packed matrix's).  Runs as ONE launch, as `count` plain calls, or as a few launches over feature
+ * ranges, whichever the kernels' estimate says is the fastest (either weight layout).  Results are those of the plain calls,
+ * bit for bit above 64 token rows and at any count with weights [in, out]; at 5-64 rows with weights [out, in] up to the order
+ * of the fp32 sum over k.  No reference counterpart. */
 int lg_gemm_fused_grouped_f16(int transa, int m, int n, int k, int count, const void* const* A, int lda, const void* B,
                               int ldb, void* const* C, const int* ldc, int epilogue, const void* const* bias,
                               int epi_arg0, int epi_arg1, int epi_arg2, void* stream);
