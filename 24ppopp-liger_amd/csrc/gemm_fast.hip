@@ -144,16 +144,12 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup
     }
     const int64_t wstep = (WL == W_KN) ? (int64_t)FB_K * g.ldw : (WL == W_NK ? FB_K : 1024);
 
-    // Where the loop over k starts, as in the tiles of gemm_mid.hpp: members of one group may be computed by either kernel.
+    // Where the loop over k starts, as in the tiles of gemm_mid.hpp: members of one group may be computed by either kernel.  The loop goes
+    // round: its body is branch-free, the extra loads of the last iterations refill slots nobody reads any more with the first k-tiles.
     const int first = n0 / MID_TURN_COLS * turn % ktiles;
-    // tile index clamped to the last one: the loop body is branch-free, the extra loads of the last iterations
-    // refill slots nobody reads any more
-    auto at = [&](int kt) {
-        const int t = (kt < ktiles ? kt : ktiles - 1) + first;
-        return (int64_t)(t < ktiles ? t : t - ktiles);
-    };
-    auto x_tile = [&](int kt) { return reinterpret_cast<const char*>(X + at(kt) * FB_K); };
-    auto w_tile = [&](int kt) { return reinterpret_cast<const char*>(W + at(kt) * wstep); };
+    auto next = [&](int t) { return t + 1 == ktiles ? 0 : t + 1; };
+    auto x_tile = [&](int t) { return reinterpret_cast<const char*>(X + (int64_t)t * FB_K); };
+    auto w_tile = [&](int t) { return reinterpret_cast<const char*>(W + (int64_t)t * wstep); };
     // load l of a k-tile: l < WCH -> chunk l of the W tile, else chunk l - WCH of the X tile (W first: it is needed first)
     auto issue_one = [&](int l, const char* xg, const char* wg, half_t* xs, half_t* ws) {
         if (l < WCH) load_lds16(reinterpret_cast<const half_t*>(wg + woff[l]), ws + (l * 8 + wave) * 512);
@@ -241,10 +237,13 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup
     };
 
     // prologue: X0 W0 X1 W1 X2; everything but X2 must have landed before the first fragments are read
+    int tw = first, tx = first;  // the k-tiles that are fetched next
     for (int t = 0; t < 3; ++t) {
 #pragma unroll
         for (int l = (t < 2 ? 0 : WCH); l < NLOAD; ++l)
-            issue_one(l, x_tile(t), w_tile(t), xring + t * X_TILE, wring + (t & 1) * W_TILE);
+            issue_one(l, x_tile(tx), w_tile(tx), xring + t * X_TILE, wring + (t & 1) * W_TILE);
+        tw = tx;
+        tx = next(tx);
     }
     asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
     __syncthreads();
@@ -265,8 +264,10 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup
         __syncthreads();
         // every wave is past tile kt: its W slot takes W(kt+2), its X slot X(kt+3); tile kt+1's first fragments stream
         // in under the MFMAs of the second k-step
-        phase(std::true_type{}, std::integral_constant<int, 1>{}, a1, b1, a0, b0, xring + xnext * X_TILE, wring + (wslot ^ 1) * W_TILE, 0, x_tile(kt + 3),
-              w_tile(kt + 2), xs, ws);
+        phase(std::true_type{}, std::integral_constant<int, 1>{}, a1, b1, a0, b0, xring + xnext * X_TILE, wring + (wslot ^ 1) * W_TILE, 0, x_tile(tx),
+              w_tile(tw), xs, ws);
+        tw = tx;
+        tx = next(tx);
         xslot = xnext;
         xnext = (xnext == X_STAGES - 1) ? 0 : xnext + 1;
     }
