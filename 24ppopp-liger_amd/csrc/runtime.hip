@@ -78,12 +78,18 @@ static int register_stream(void* stream, int cus) {
     info.ws = (float*)p;
     info.ws_bytes = LG_SPLITK_WORKSPACE_BYTES;
     info.arrivals = (unsigned*)((char*)p + LG_SPLITK_WORKSPACE_BYTES);
-    // Set once, here: every kernel that counts arrivals leaves its counters at zero.  On a stream of its own: the null stream waits for
-    // the work of every blocking stream, and ends a capture that is open on one.
-    hipStream_t own = nullptr;
-    rc = rt(hipStreamCreateWithFlags(&own, hipStreamNonBlocking), "hipStreamCreateWithFlags");
-    if (rc == LG_OK) {
-        rc = rt(hipMemsetAsync(info.arrivals, 0, counter_bytes, own), "hipMemsetAsync (arrival counters)");
+    // Set once, here: every kernel that counts arrivals leaves its counters at zero.  The stream's own order puts it before the first
+    // of them.  Not on the null stream, which waits for the work of every blocking stream and ends a capture that is open on one, and not
+    // into a capture: those two get a stream for the purpose (a stream more takes part in the sharing of hardware queues).
+    hipStream_t clear = (hipStream_t)stream, own = nullptr;
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    if (clear && hipStreamIsCapturing(clear, &capture) != hipSuccess) capture = hipStreamCaptureStatusInvalidated;
+    if (!clear || capture != hipStreamCaptureStatusNone) {
+        rc = rt(hipStreamCreateWithFlags(&own, hipStreamNonBlocking), "hipStreamCreateWithFlags");
+        clear = own;
+    }
+    if (rc == LG_OK) rc = rt(hipMemsetAsync(info.arrivals, 0, counter_bytes, clear), "hipMemsetAsync (arrival counters)");
+    if (own) {
         if (rc == LG_OK) rc = rt(hipStreamSynchronize(own), "hipStreamSynchronize");
         (void)hipStreamDestroy(own);
     }

@@ -140,14 +140,24 @@ def test_members_of_many_features_are_weight_streaming_launches_of_their_own(dev
     assert max_rel_err(dev.down(one[2]).reshape(M, N), po.round_f16(po.gemm(X, np.ascontiguousarray(Ws[2].T), 1) + b)) < 2e-3
 
 
-def test_a_stream_can_be_made_while_another_is_captured(dev):
-    """The set-up of a stream's workspace keeps off the null stream: a (relaxed) capture that is open on a blocking stream goes on."""
-    hip, s, graph, made = dev.lib, C.c_void_p(), C.c_void_p(), C.c_void_p()
-    dev.sync()
-    assert hip.hipStreamCreate(C.byref(s)) == 0 and hip.hipStreamBeginCapture(s, 2) == 0
-    rc = dev.lib.lg_stream_create(C.byref(made))
-    assert hip.hipStreamEndCapture(s, C.byref(graph)) == 0 and rc == 0, dev.capi.last_error()
-    assert dev.lib.lg_stream_destroy(made) == 0 and hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(s) == 0
+def test_a_stream_can_be_made_known_while_one_is_captured(dev):
+    """The set-up of a stream's workspace keeps off the null stream and out of captures: a (relaxed) capture that is open on a blocking
+    stream goes on, with nothing in it, when a stream is created, when the stream that is captured is attached, and the null stream."""
+    hip = dev.lib
+    for case in ("create", "attach captured", "attach null"):
+        s, graph, made, n = C.c_void_p(), C.c_void_p(), C.c_void_p(), C.c_size_t(7)
+        dev.lib.lg_stream_detach(None)
+        dev.sync()
+        assert hip.hipStreamCreate(C.byref(s)) == 0 and hip.hipStreamBeginCapture(s, 2) == 0
+        rc = dev.lib.lg_stream_create(C.byref(made)) if case == "create" else dev.lib.lg_stream_attach(s if case == "attach captured" else None, 0)
+        assert hip.hipStreamEndCapture(s, C.byref(graph)) == 0 and rc == 0, dev.capi.last_error()
+        assert hip.hipGraphGetNodes(graph, None, C.byref(n)) == 0 and n.value == 0
+        if made:
+            assert dev.lib.lg_stream_destroy(made) == 0
+        if case == "attach captured":
+            assert dev.lib.lg_stream_detach(s) == 0
+        assert hip.hipGraphDestroy(graph) == 0 and hip.hipStreamDestroy(s) == 0
+    assert dev.lib.lg_stream_attach(C.c_void_p(dev.stream), 0) == 0     # as the fixture left it
 
 
 @pytest.mark.parametrize("M,N,K", [(11, 4096, 4096), (200, 4096, 4096), (256, 6144, 12288)])
