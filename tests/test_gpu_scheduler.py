@@ -261,6 +261,7 @@ def test_batched_decode_steps_teacher_forced_against_the_oracle(dev, po, host, m
             state[slot] = x
             forced[r] = x[0]
         t = torch.from_numpy(forced).cuda().half()
+        torch.cuda.synchronize()               # converted on torch's stream, copied on the step's
         dev.capi.call("lg_memcpy_d2d_async", rows_ptr, t.data_ptr(), t.numel() * 2, stream)
         dev.capi.call("lg_stream_synchronize", stream)
         worst["steps"] += 1
