@@ -24,7 +24,7 @@ def early_accumulator_uses(body):
     return [l for l in lines[last + 1:drain] if re.search(r"\ba\[?\d", l)]
 
 
-def test_the_checker_sees_an_accumulator_read_before_the_drain():
+def test_an_accumulator_read_before_the_drain_is_seen():
     body = "v_mfma_f32_16x16x32_f16 a[0:3], v[0:3], v[4:7], a[0:3]\n%s\ts_waitcnt vmcnt(0)\n\ts_nop 15\n\ts_nop 15\n\tv_accvgpr_read_b32 v0, a0\n"
     assert early_accumulator_uses(body % "") == []
     assert len(early_accumulator_uses(body % "\tscratch_store_dwordx4 off, a[192:195], off offset:8 ; 16-byte Folded Spill\n")) == 1
