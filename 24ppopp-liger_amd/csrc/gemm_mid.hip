@@ -22,9 +22,9 @@ constexpr int kMaxTiles = LG_ARRIVAL_COUNTERS / 2;
 // Microseconds of one launch.  Fitted to 556 problems (M 8 .. 2048, 17 weight shapes from 1024 x 1024 to 32768 x 12288, all three
 // layouts) x all tiles and slice counts, each measured with weights cycled out of the caches; picking by it costs 1 % against
 // the best measured choice on average.  Terms: a k-tile costs its matrix work or its loads; a workgroup cannot pull more than 69 GB/s
-// of weights (44 in pieces of 256 bytes: 128-wide tiles of [in, out] weights, few rows) and the chip 7.4 TB/s; what memory and matrix pipes do in the same time overlaps only in part; a K-slice meeting
-// costs a trip to the counter and the transfer of the sums, in every round (three projections of 64 rows x 4096 x 4096 in four slices, three
-// rounds: 40 us).
+// of weights (44 in pieces of 256 bytes: 128-wide tiles of [in, out] weights, few rows) and the chip 7.4 TB/s; what memory and matrix
+// pipes do in the same time overlaps only in part; a K-slice meeting costs a trip to the counter and the transfer of the sums, in
+// every round (three projections of 64 rows x 4096 x 4096 in four slices, three rounds: 40 us).
 double tile_cost(int M, int N, int K, int count, int mi, int nj, int nsplit, int wlayout, int cus) {
     const int tiles_m = (M + 32 * mi - 1) / (32 * mi), tiles_n = N / (32 * nj) * count, ktiles = K / MID_K;
     const int kt = (ktiles + nsplit - 1) / nsplit;
@@ -32,7 +32,8 @@ double tile_cost(int M, int N, int K, int count, int mi, int nj, int nsplit, int
     const double rounds = (double)((wgs + cus - 1) / cus);
     const double work = kt * (0.13 + 0.0192 * mi * nj), loads = kt * (0.0673 + 0.0292 * (mi + nj));
     const double compute = work > loads ? work : loads;
-    const double chip = 2.0 * N * K * count / (7.3735e6 * cus / 256.0) / rounds, own = kt * (64.0 * 32 * 2 / (wlayout == W_KN && nj == 4 && M <= 64 ? 44e3 : 69.42e3)) * nj;
+    const double rate = wlayout == W_KN && nj == 4 && M <= 64 ? 44e3 : 69.42e3;
+    const double chip = 2.0 * N * K * count / (7.3735e6 * cus / 256.0) / rounds, own = kt * (64.0 * 32 * 2 / rate) * nj;
     double round = compute > chip ? compute + 0.6025 * chip : chip + 0.6025 * compute;
     if (round < own) round = own;
     double us = 3.67 + rounds * round;
@@ -112,7 +113,8 @@ static TilePlan plan_gemm_tiles(const GemmArgs& g, int count, int wlayout, bool 
         }
     }
     best = pick(count, slices);
-    if (fast_ok && best.nsplit <= 1 && g.M > 64 && g.epi.kind != LG_EPI_BIAS_HEADS_ROWS)
+    // (where members are sliced and the slices of a group do not fit the workspace, the group is not taken as one launch)
+    if (fast_ok && slices == 1 && g.M > 64 && g.epi.kind != LG_EPI_BIAS_HEADS_ROWS)
         for (int nj = 4; nj >= 3; --nj) {
             if (g.N % (64 * nj) || (nj == 3 && g.epi.kind == LG_EPI_BIAS_GEGLU)) continue;
             const double us = kFastFactor * tile_cost(g.M, g.N, g.K, count, 8, 2 * nj, 1, wlayout, cus);

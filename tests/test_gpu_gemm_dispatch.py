@@ -180,3 +180,20 @@ def test_sliced_launches_replayed_between_eager_ones(dev, po, stream, M, N, K):
 
     assert len(launches(dev, stream, "lg_gemm_f16", 2, 0, N, M, K, dW, K, dX, K, y, N, replays=4, between=between)) == 1
     assert all(torch.equal(a, seen[0][0]) and torch.equal(b, seen[0][0]) for a, b in seen) and bool(seen[0][0].any())
+
+
+def test_a_group_whose_slices_do_not_fit_has_the_bits_of_its_members(dev, stream):
+    """Members in two K-slices, three of which need more than the workspace: the group must not go to an unsliced kernel instead."""
+    M, N, K = 256, 12288, 4096
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(6)
+    dX = torch.randn(M, K, device="cuda", generator=gen).half()
+    dW = [(torch.randn(N * K, device="cuda", generator=gen) * 0.02).half() for _ in range(3)]
+    dB = torch.randn(N, device="cuda", generator=gen).half()
+    one, three = [[dev.empty((M, N), 1) for _ in range(3)] for _ in range(2)]
+    ptrs = lambda ts: (C.c_void_p * 3)(*[t.data_ptr() for t in ts])
+    for i in range(3):
+        launches(dev, stream, "lg_gemm_fused_f16", 0, N, M, K, dW[i], N, dX, K, one[i], N, dev.capi.EPI_BIAS, dB, 0, 0, 0)
+    launches(dev, stream, "lg_gemm_fused_grouped_f16", 0, N, M, K, 3, ptrs(dW), N, dX, K, ptrs(three), (C.c_int * 3)(N, N, N), dev.capi.EPI_BIAS, ptrs([dB] * 3), 0, 0, 0)
+    for i in range(3):
+        assert torch.equal(one[i], three[i]) and bool(torch.isfinite(one[i]).all())
