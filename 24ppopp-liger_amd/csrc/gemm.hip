@@ -506,8 +506,9 @@ static int gemm_fused_grouped_f16_impl(int mode, int transa, int m, int n, int k
     const int cus = stream_info((hipStream_t)stream).cus;
     // Fragment blocks and few rows: member by member where the weight-streaming kernel takes a member but not the group, whose features
     // are too many for one wave a feature tile (three times 12288 x 12288, 11 rows: 142 us, as tiles 159; x 4096, 32 rows: 60 and 67).
-    // At 48 rows, or with rows of [out, in], the tiles are level or ahead (x 4096, 48 rows: 63 and 59; [out, in], 11 rows: 71 and 64).
-    if (mode < 0 && one_launch && wl == W_TILED && n <= 32)
+    // At 48 rows, with more features or with rows of [out, in], the tiles are level or ahead (x 4096, 48 rows: 63 and 59; 16384 x 4096, 11
+    // rows: 80 and 68; [out, in], 12288 x 4096, 11 rows: 71 and 64).
+    if (mode < 0 && one_launch && wl == W_TILED && n <= 32 && m <= 12288)
         one_launch = !skinny_takes_group(member(m), 1, wl, cus) || skinny_takes_group(member(m), count, wl, cus);
     if (mode < 0 && one_launch && n > 64) {
         constexpr double kLaunch = 1.5;  // microseconds between two launches
