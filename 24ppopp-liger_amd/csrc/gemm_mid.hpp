@@ -14,15 +14,19 @@
 //   * both operands go global -> LDS with direct-to-LDS loads into rings of 2 to 6 k-tiles (as many as 160 KiB hold), one barrier
 //     per k-tile; fragments are double-buffered in registers and read by hand-issued LDS reads between the matrix instructions
 //     (the schedule of gemm_fast.hip);
-//   * with one row of tiles every weight byte is read once, and the loads say so (non-temporal: 84 -> 73 us for a 16384 x 12288
-//     weight at 72 rows);
+//   * a compute unit has 32 KiB of loads on their way at most, and they come back in order: X, from the L2 in 0.1 us, waits behind W,
+//     from memory in 0.5 us and more.  Taken in turns, 60 GB/s of both together reach a compute unit, and that bounded most
+//     prompts (384 rows x 12288 x 16384: 174 us of loads alone, 98 with W from the L2).  So W goes out for two k-tiles at a time and
+//     then X for two (loads alone 147 us); tiles whose rings are too short for that spread their loads over both k-steps at least;
+//   * with one or two rows of tiles every weight byte is read about once, and the loads say so (non-temporal: 84 -> 73 us for a
+//     16384 x 12288 weight at 72 rows);
 //   * up to 256 rows the workgroups of different feature blocks start their loop over k at different k-tiles, which spreads what
 //     they read at one time over the memory channels (mid_turn in gemm_mid.hip: up to 28 % of a GEMM).  Where it starts depends on
 //     the feature alone, not on the tile: a member of a group has the same bits as a call of its own;
 //   * K-slices meet in the kernel: the slice of a tile that arrives last adds the others' sums and applies the epilogue.  A second
 //     kernel for that cost 5-10 us per GEMM.
-// 16384 x 12288 weight (403 MB), before (gemm_fast.hip, K-slices summed by a second kernel) -> now: 80 rows 104 -> 73 us, 128 rows
-// 108 -> 80, 256 rows 127 -> 108, 384 rows 187 -> 157 (0.98 PFLOP/s), 768 rows 264 -> 233 (1.33), 1536 rows 514 -> 457.
+// 16384 x 12288 weight (403 MB), fragment blocks, all loads of a k-tile under its second k-step -> now: 80 rows 71 -> 69 us, 128 rows
+// 80 -> 76, 256 rows 112 -> 100, 384 rows 150 -> 132 (1.17 PFLOP/s), 666 rows 241 -> 222, 1000 rows 310 -> 290 (1.39).
 #pragma once
 #include "gemm_common.hpp"
 
@@ -54,12 +58,16 @@ __device__ __forceinline__ void mfma16_acc(float4_t& c, half8_t a, half8_t b) {
 }
 
 typedef int int4_t __attribute__((ext_vector_type(4)));
+
+// When the loads of later k-tiles are issued: half of a k-tile's under its second k-step and half under the next one's first, or for two
+// k-tiles at a time, W before X
+enum { MID_SPREAD, MID_PAIRS };
 // cache policy of the K-slices' sums: written through to, and read from, the level that all XCDs share
 constexpr int CACHE_DEVICE = 16;
 // most K-slices of a tile (their sums are held in registers 64 fragments at a time)
 constexpr int mid_max_splits(int mi, int nj) { return mi * nj <= 16 ? 8 : 2; }
 
-template <int WL, int MI, int NJ, int XS, int WS, bool NT>
+template <int WL, int MI, int NJ, int XS, int WS, int ORDER, bool NT>
 __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmGroup grp, RowMap rm, int tiles_m, int tiles_n, float* partial, unsigned* arrivals, int nsplit, int kt_per_split, int turn, int wide_store) {
     constexpr int TM = 32 * MI, TN = 32 * NJ;
     constexpr int X_TILE = TM * MID_K, W_TILE = TN * MID_K;  // halves per ring slot
@@ -138,11 +146,14 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
 
     constexpr int NLOAD = MI + NJ;
     constexpr bool XFIRST = WS > XS;  // the operand with the shallower ring is issued first in a phase
+    auto issue_x = [&](int i, const char* xg, half_t* xs) { load_lds16(reinterpret_cast<const half_t*>(xg + xoff[i]), xs + (i * 4 + wave) * 512); };
+    auto issue_w = [&](int i, const char* wg, half_t* ws) { load_lds16<NT ? 2 : 0>(reinterpret_cast<const half_t*>(wg + woff[i]), ws + (i * 4 + wave) * 512); };
+    // load l of the NLOAD of one k-tile of each operand
     auto issue_one = [&](int l, const char* xg, const char* wg, half_t* xs, half_t* ws) {
         const bool is_x = XFIRST ? l < MI : l >= NJ;
         const int i = is_x ? (XFIRST ? l : l - NJ) : (XFIRST ? l - MI : l);
-        if (is_x) load_lds16(reinterpret_cast<const half_t*>(xg + xoff[i < MI ? i : 0]), xs + (i * 4 + wave) * 512);
-        else load_lds16<NT ? 2 : 0>(reinterpret_cast<const half_t*>(wg + woff[i < NJ ? i : 0]), ws + (i * 4 + wave) * 512);
+        if (is_x) issue_x(i < MI ? i : 0, xg, xs);
+        else issue_w(i < NJ ? i : 0, wg, ws);
     };
 
     float4_t acc[MI][NJ];
@@ -195,21 +206,18 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
     };
     constexpr int NMFMA = MI * NJ;
     constexpr int DS_SPAN = NMFMA * 3 / 4;
-    // One phase = the MFMAs of one k-step with the LDS reads of the next and, if LOADS, the loads of a later k-tile between them
-    auto phase = [&](auto with_loads, auto kstep, half8_t (&ma)[MI], half8_t (&mb)[NJ], half8_t (&ra)[MI], half8_t (&rb)[NJ], unsigned rx, unsigned rw,
-                     const char* xg, const char* wg, half_t* lxs, half_t* lws) {
-        constexpr bool LOADS = decltype(with_loads)::value;
+    // One phase = the MFMAs of one k-step with the LDS reads of the next and NL loads of later k-tiles between them
+    auto phase = [&](auto loads, auto kstep, half8_t (&ma)[MI], half8_t (&mb)[NJ], half8_t (&ra)[MI], half8_t (&rb)[NJ], unsigned rx, unsigned rw, auto&& load) {
+        constexpr int NL = decltype(loads)::value;
         constexpr int KS = decltype(kstep)::value;
         static_for<NMFMA>([&](auto mc) {
             constexpr int m = decltype(mc)::value;
             constexpr int i = m / NJ, j = m % NJ;
             mfma16_acc(acc[i][j], mb[j], ma[i]);
-            if constexpr (LOADS) {
-                static_for<NLOAD>([&](auto lc) {
-                    constexpr int l = decltype(lc)::value;
-                    if constexpr (l * NMFMA / NLOAD == m) issue_one(l, xg, wg, lxs, lws);
-                });
-            }
+            static_for<NL>([&](auto lc) {
+                constexpr int l = decltype(lc)::value;
+                if constexpr (l * NMFMA / NL == m) load(l);
+            });
             static_for<NDS>([&](auto uc) {
                 constexpr int u = decltype(uc)::value;
                 if constexpr (u * DS_SPAN / NDS == m) read_unit(uc, std::integral_constant<int, KS ^ 1>{}, rx, rw, ra, rb);
@@ -217,40 +225,107 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
             __builtin_amdgcn_sched_barrier(0);
         });
     };
-
-    // prologue: tiles 0 .. in the order the loop would have issued them
-    constexpr int SMAX = XS > WS ? XS : WS, SMIN = XS < WS ? XS : WS;
-    constexpr int NDEEP = XS == WS ? 0 : (XS > WS ? MI : NJ);  // loads of the deeper ring that may stay in flight besides whole tiles
-    static_for<SMAX>([&](auto tc) {
-        constexpr int t = decltype(tc)::value;
-#pragma unroll
-        for (int l = 0; l < NLOAD; ++l) {
-            const bool is_x = XFIRST ? l < MI : l >= NJ;
-            if (is_x ? t < XS : t < WS) issue_one(l, x_tile(t), w_tile(t), smem + t * X_TILE, wring + t * W_TILE);
-        }
-    });
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SMIN - 1) * NLOAD + NDEEP) : "memory");
-    barrier_keep_loads_in_flight();
+    using Step0 = std::integral_constant<int, 0>;
+    using Step1 = std::integral_constant<int, 1>;
+    auto x_at = [](int slot) { return (unsigned)(slot * X_TILE * 2); };
+    auto w_at = [](int slot) { return (unsigned)(slot * W_TILE * 2); };
     half8_t a0[MI], b0[NJ], a1[MI], b1[NJ];
-    static_for<NDS>([&](auto uc) { read_unit(uc, std::integral_constant<int, 0>{}, 0u, 0u, a0, b0); });
-    arrive(std::integral_constant<int, 0>{}, a0, b0);
-
-    int xslot = 0, wslot = 0, kt = 0;
-    do {
-        const unsigned xb = (unsigned)(xslot * X_TILE * 2), wb = (unsigned)(wslot * W_TILE * 2);
-        half_t* const xs = smem + xslot * X_TILE;
-        half_t* const ws = wring + wslot * W_TILE;
-        phase(std::false_type{}, std::integral_constant<int, 0>{}, a0, b0, a1, b1, xb, wb, nullptr, nullptr, nullptr, nullptr);
-        // all of tile kt is in this wave's registers and tile kt + 1 has landed; later tiles may stay in flight
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SMIN - 2) * NLOAD + NDEEP) : "memory");
-        arrive(std::integral_constant<int, 1>{}, a1, b1);
+    // tile kt + 1 has landed for every wave but IN_FLIGHT of this wave's loads, which are later, and this wave has all of tile kt in registers
+    auto publish = [&](auto in_flight) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(decltype(in_flight)::value) : "memory");
+        arrive(Step1{}, a1, b1);
         barrier_keep_loads_in_flight();
-        xslot = xslot == XS - 1 ? 0 : xslot + 1;
-        wslot = wslot == WS - 1 ? 0 : wslot + 1;
-        phase(std::true_type{}, std::integral_constant<int, 1>{}, a1, b1, a0, b0, (unsigned)(xslot * X_TILE * 2), (unsigned)(wslot * W_TILE * 2), x_tile(kt + XS),
-              w_tile(kt + WS), xs, ws);
-        arrive(std::integral_constant<int, 0>{}, a0, b0);
-    } while (++kt < ktiles);
+    };
+    int kt = 0;
+    if constexpr (ORDER == MID_PAIRS) {
+        // Every second k-tile the W tiles of two k-tiles go out together, and then their X tiles.
+        static_assert(XS == WS && XS >= 3, "one ring depth for both operands");
+        constexpr int S = XS;
+        constexpr int EVEN = (S - 2) * MI + (S - 3) * NJ, ODD = (S - 2) * NJ + (S - 3) * MI;  // loads issued after those of tile kt + 1
+#pragma unroll
+        for (int t = 0; t < S - 1; ++t) {
+#pragma unroll
+            for (int i = 0; i < MI; ++i) issue_x(i, x_tile(t), smem + t * X_TILE);
+#pragma unroll
+            for (int i = 0; i < NJ; ++i) issue_w(i, w_tile(t), wring + t * W_TILE);
+        }
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((S - 2) * NLOAD) : "memory");
+        barrier_keep_loads_in_flight();
+        static_for<NDS>([&](auto uc) { read_unit(uc, Step0{}, 0u, 0u, a0, b0); });
+        arrive(Step0{}, a0, b0);
+        int prev = S - 1, slot = 0, next = 1;
+        auto advance = [&] {
+            prev = slot;
+            slot = next;
+            next = next == S - 1 ? 0 : next + 1;
+        };
+        for (;;) {
+            {   // even k-tile: the second X tile of the last pair, then a pair of W tiles, into the slots of k-tiles kt - 1 and kt
+                const char* xg = x_tile(kt - 1 + S);
+                half_t* const xs = smem + prev * X_TILE;
+                phase(std::integral_constant<int, MI>{}, Step0{}, a0, b0, a1, b1, x_at(slot), w_at(slot), [&](int l) { issue_x(l, xg, xs); });
+                publish(std::integral_constant<int, EVEN>{});
+                const char* wg0 = w_tile(kt - 1 + S);
+                const char* wg1 = w_tile(kt + S);
+                half_t* const ws0 = wring + prev * W_TILE;
+                half_t* const ws1 = wring + slot * W_TILE;
+                phase(std::integral_constant<int, 2 * NJ>{}, Step1{}, a1, b1, a0, b0, x_at(next), w_at(next),
+                      [&](int l) { l < NJ ? issue_w(l, wg0, ws0) : issue_w(l - NJ, wg1, ws1); });
+                arrive(Step0{}, a0, b0);
+            }
+            if (++kt >= ktiles) break;
+            advance();
+            {   // odd k-tile: the first X tile of the pair
+                phase(std::integral_constant<int, 0>{}, Step0{}, a0, b0, a1, b1, x_at(slot), w_at(slot), [](int) {});
+                publish(std::integral_constant<int, ODD>{});
+                const char* xg = x_tile(kt - 1 + S);
+                half_t* const xs = smem + prev * X_TILE;
+                phase(std::integral_constant<int, MI>{}, Step1{}, a1, b1, a0, b0, x_at(next), w_at(next), [&](int l) { issue_x(l, xg, xs); });
+                arrive(Step0{}, a0, b0);
+            }
+            if (++kt >= ktiles) break;
+            advance();
+        }
+    } else {
+        // The loads of k-tiles kt + XS and kt + WS go out once tile kt is done with: half of them under its second k-step and half under the
+        // first k-step of the next.
+        constexpr int SMAX = XS > WS ? XS : WS, SMIN = XS < WS ? XS : WS;
+        constexpr int NDEEP = XS == WS ? 0 : (XS > WS ? MI : NJ);  // loads of the deeper ring that may stay in flight besides whole tiles
+        constexpr int NOW = NLOAD / 2;
+        // prologue: tiles 0 .. in the order the loop would have issued them
+        static_for<SMAX>([&](auto tc) {
+            constexpr int t = decltype(tc)::value;
+#pragma unroll
+            for (int l = 0; l < NLOAD; ++l) {
+                const bool is_x = XFIRST ? l < MI : l >= NJ;
+                if (l >= NOW && t == (is_x ? XS : WS) - 1) continue;
+                if (is_x ? t < XS : t < WS) issue_one(l, x_tile(t), w_tile(t), smem + t * X_TILE, wring + t * W_TILE);
+            }
+        });
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((SMIN - 1) * NLOAD + NDEEP - (NLOAD - NOW)) : "memory");
+        barrier_keep_loads_in_flight();
+        static_for<NDS>([&](auto uc) { read_unit(uc, Step0{}, 0u, 0u, a0, b0); });
+        arrive(Step0{}, a0, b0);
+        int xslot = 0, wslot = 0, xprev = XS - 1, wprev = WS - 1;
+        do {
+            const char* xg0 = x_tile(kt - 1 + XS);
+            const char* wg0 = w_tile(kt - 1 + WS);
+            half_t* const xs0 = smem + xprev * X_TILE;
+            half_t* const ws0 = wring + wprev * W_TILE;
+            phase(std::integral_constant<int, NLOAD - NOW>{}, Step0{}, a0, b0, a1, b1, x_at(xslot), w_at(wslot), [&](int l) { issue_one(l + NOW, xg0, wg0, xs0, ws0); });
+            publish(std::integral_constant<int, (SMIN - 2) * NLOAD + NDEEP>{});
+            const char* xg = x_tile(kt + XS);
+            const char* wg = w_tile(kt + WS);
+            half_t* const xs = smem + xslot * X_TILE;
+            half_t* const ws = wring + wslot * W_TILE;
+            xprev = xslot;
+            wprev = wslot;
+            xslot = xslot == XS - 1 ? 0 : xslot + 1;
+            wslot = wslot == WS - 1 ? 0 : wslot + 1;
+            phase(std::integral_constant<int, NOW>{}, Step1{}, a1, b1, a0, b0, x_at(xslot), w_at(wslot), [&](int l) { issue_one(l, xg, wg, xs, ws); });
+            arrive(Step0{}, a0, b0);
+        } while (++kt < ktiles);
+    }
     // The clamped refills of the last iterations land, and the last matrix instructions write their results: they are assembly, so the
     // compiler does not wait for them by itself.  The accumulators are named after the wait so that nothing reads one before it.
     asm volatile("s_waitcnt vmcnt(0)\n\ts_nop 15\n\ts_nop 15" ::: "memory");
@@ -419,13 +494,19 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
     }
 }
 
-// ring depths: as many k-tiles as 160 KiB hold, at most 6
-constexpr int mid_xs(int mi, int nj) { return 6 * (mi + nj) <= 40 ? 6 : 4 * (mi + nj) <= 40 ? 4 : 3 * (mi + nj) <= 40 || 3 * mi + 2 * nj <= 40 ? 3 : 2; }
-constexpr int mid_ws(int mi, int nj) { return 6 * (mi + nj) <= 40 ? 6 : 4 * (mi + nj) <= 40 ? 4 : 3 * (mi + nj) <= 40 ? 3 : 3 * mi + 2 * nj <= 40 ? 2 : 3; }
+// Ring depths: as many k-tiles as 160 KiB hold, at most 6.  Where they do not hold 3 of both: W, which comes from memory, gets the third
+// (6 x 8 and 7 x 8: 0.90 of the time before, with 3 of X 0.94), but for 256 rows, where it makes no difference up to two rows of tiles and X
+// gains by it above.
+constexpr int mid_depth(int mi, int nj) { return 6 * (mi + nj) <= 40 ? 6 : 4 * (mi + nj) <= 40 ? 4 : 3 * (mi + nj) <= 40 ? 3 : 2; }
+constexpr int mid_xs(int mi, int nj) { return mid_depth(mi, nj) > 2 ? mid_depth(mi, nj) : mi == 8 ? 3 : 2; }
+constexpr int mid_ws(int mi, int nj) { return mid_depth(mi, nj) > 2 ? mid_depth(mi, nj) : mi == 8 ? 2 : 3; }
+// Against all loads under the second k-step, over the problems that a tile is good for: in pairs 0.89 (6 x 4), 0.91 (4 x 3, 8 x 4), 0.95 (3 x 4,
+// 4 x 4), 0.97-1.0 (the others of depth 4 and 6: bound by memory, or by few workgroups); at depth 3 spread 0.89-0.99, in pairs up to 1.05.
+constexpr int mid_order(int mi, int nj) { return mid_depth(mi, nj) > 3 || nj == 4 ? MID_PAIRS : MID_SPREAD; }
 
 template <int WL, int MI, int NJ, bool NT>
 static void launch_mid_tile(const GemmArgs& g, const GemmGroup& grp, const RowMap& rm, const MidLaunch& l) {
-    constexpr int XS = mid_xs(MI, NJ), WS = mid_ws(MI, NJ);
+    constexpr int XS = mid_xs(MI, NJ), WS = mid_ws(MI, NJ), ORDER = mid_order(MI, NJ);
     const int tiles_m = (g.M + 32 * MI - 1) / (32 * MI), tiles_n = g.N / (32 * NJ) * grp.count;
     constexpr size_t ring = (size_t)(XS * MI + WS * NJ) * 32 * MID_K * sizeof(half_t), tile = (size_t)(32 * MI) * (32 * NJ + 8) * sizeof(half_t);
     constexpr size_t smem = ring > tile ? ring : tile;
@@ -435,9 +516,9 @@ static void launch_mid_tile(const GemmArgs& g, const GemmGroup& grp, const RowMa
     for (int i = 0; i < grp.count; ++i)
         if (!aligned16(grp.Y[i]) || (g.epi.kind == LG_EPI_BIAS_HEADS || g.epi.kind == LG_EPI_BIAS_HEADS_ROWS ? (g.epi.d % 8 != 0) : (grp.ldy[i] % 8 != 0))) wide = 0;
     // set once per instantiation; the initialisation of a function-local static is thread-safe
-    static const hipError_t attr_rc = hipFuncSetAttribute((const void*)gemm_f16_mid<WL, MI, NJ, XS, WS, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    static const hipError_t attr_rc = hipFuncSetAttribute((const void*)gemm_f16_mid<WL, MI, NJ, XS, WS, ORDER, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     (void)attr_rc;
-    hipLaunchKernelGGL((gemm_f16_mid<WL, MI, NJ, XS, WS, NT>), dim3(tiles_m * tiles_n * l.nsplit), dim3(MID_THREADS), smem, l.stream, g, grp, rm, tiles_m, tiles_n,
+    hipLaunchKernelGGL((gemm_f16_mid<WL, MI, NJ, XS, WS, ORDER, NT>), dim3(tiles_m * tiles_n * l.nsplit), dim3(MID_THREADS), smem, l.stream, g, grp, rm, tiles_m, tiles_n,
                        l.si.ws, l.si.arrivals, l.nsplit, l.kt_per_split, l.turn, wide);
 }
 

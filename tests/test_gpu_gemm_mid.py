@@ -54,6 +54,22 @@ def test_gemm_at_the_edges_of_the_tiles(dev, po, layout, M, N, K):
         assert np.array_equal(dev.down(dY)[:M], got[:M])
 
 
+# fewer k-tiles than a ring is deep, as many and more, even and odd: loads go out for pairs of k-tiles, and the loop may end in either half of one
+@pytest.mark.parametrize("layout", [0, 1, 2])
+@pytest.mark.parametrize("M,N", [(20, 768), (96, 3072), (190, 6144), (250, 12288), (384, 3072), (500, 4608), (1100, 3072)])
+def test_every_number_of_k_tiles(dev, po, layout, M, N):
+    K = 13 * 64
+    X, W = rnd(po, M * K, 13).reshape(M, K), rnd(po, K * N, 14, 0.05).reshape(K, N)
+    dX = dev.up(X, 1)
+    for kt in (1, 2, 3, 4, 5, 6, 7, 8, 13):
+        k = 64 * kt
+        dW, ld = weight(dev, np.ascontiguousarray(W[:k]), layout)
+        dY = dev.empty((M, N), 1)
+        dev.call("lg_gemm_f16", layout, 0, N, M, k, dW, ld, dX, K, dY, N)
+        ref = (torch.from_numpy(X[:, :k]).cuda().float() @ torch.from_numpy(W[:k]).cuda().float()).cpu().numpy()
+        assert max_rel_err(dev.down(dY), ref) < 2e-3, kt
+
+
 @pytest.mark.parametrize("layout", [0, 1, 2])
 @pytest.mark.parametrize("M,S,h,d", [(72, 24, 8, 128), (90, 45, 8, 96), (130, 65, 16, 12), (48, 1, 32, 128), (300, 300, 6, 64)])
 def test_fused_epilogues(dev, po, layout, M, S, h, d):
