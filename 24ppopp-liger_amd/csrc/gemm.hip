@@ -6,7 +6,7 @@
 //   gemm_f32_mfma      128x128x16 tiles on v_mfma_f32_32x32x2_f32 for the fp32 instantiation (any shape, both layouts); problems
 //                      of few such tiles go to gemm_f32.hip;
 //   gemm_f32_generic   64x64x16 VALU tiles, kept as a cross-check.
-// The large aligned prefill shapes are routed to the pipelined kernels in gemm_fast.hip.
+// Aligned problems are routed to the tile kernels of gemm_mid.hpp and the weight-streaming ones.
 #include <stdlib.h>
 
 #include "gemm_common.hpp"

@@ -242,9 +242,8 @@ constexpr int MID_TURN_COLS = 768;    // features of a block whose workgroups st
 constexpr int kSequentialRows = 257;  // from so many token rows on every output is one sum in the order of k, whichever kernel computes it
 struct TilePlan {
     double cost;   // estimated microseconds
-    int mi, nj;    // tile (32 mi) x (32 nj); the 256-row kernel: 256 x (64 nj)
+    int mi, nj;    // tile (32 mi) x (32 nj)
     int nsplit;    // K-slices (0: no tile kernel takes the problem)
-    bool fast;     // the 256-row kernel of gemm_fast.hip
 };
 TilePlan plan_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, int wlayout, int batch, hipStream_t stream);
 int launch_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled);

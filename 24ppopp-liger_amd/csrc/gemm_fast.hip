@@ -1,12 +1,17 @@
-// gemm_fast.hip -- pipelined 256x256x64 fp16 GEMM for gfx950 (the prefill shapes of the launch vector).
+// gemm_fast.hip -- fp16 GEMM in tiles of 256 x 128 for a compute unit that is shared (gfx950).
 //
 //   Y[M, N] = X[M, K] * W,  W row-major [K, N] (the reference's layout) or [N, K];  fp32 accumulate, optional fused
-//   epilogue.  Requires N % 256 == 0 (or % 192), K % 64 == 0, any M (a partial last row of tiles is padded) and 16-byte aligned
-//   operands.  gemm_mid.hip chooses between this kernel (many rows of tiles) and tiles fitted to the token count.
+//   epilogue.  Requires N % 128 == 0, K % 64 == 0, any M (a partial last row of tiles is padded) and 16-byte aligned
+//   operands.
 //
-// Structure (one workgroup = 8 waves = one 256x256 output tile, one workgroup per CU):
+// The tiles of gemm_mid.hpp take the whole of a compute unit's LDS and are the faster ones (4096 rows x 16384 x 12288, fragment blocks:
+// 1141 us, this kernel's structure at 256 x 256 1170; [in, out] 1198 and 1249).  At 256 x 128 with 8 waves this one leaves 32 KiB
+// of LDS and a third wave's registers on every SIMD to a kernel on another stream: gemm_mid.hip launches it where LG_GEMM_TILE_WIDTH=2
+// asks for it, to measure such pairs of streams.
+//
+// Structure (one workgroup = 8 waves = one output tile, one workgroup per CU):
 //   * global -> LDS with direct-to-LDS loads (global_load_lds_dwordx4): no VGPR staging, each wave instruction fills
-//     1 KiB of LDS; two LDS stages (2 x 64 KiB);
+//     1 KiB of LDS;
 //   * software pipeline with ONE barrier per k-tile, placed between the tile's two k-steps: fragments are double
 //     buffered in registers, so when a wave reaches the barrier the whole of tile t is already in its registers.  After
 //     the barrier tile t's stage is free and is refilled with tile t+2 (a full iteration ahead of its use), the first
@@ -16,7 +21,7 @@
 //   * LDS layouts are XOR-swizzled through the *global* address each lane loads from (the LDS position of a lane's
 //     16 bytes is fixed by the instruction), so that both the 16-byte fragment reads of X and the transposed 8-byte
 //     reads of a [K, N] weight tile are spread over the banks;
-//   * wave grid 2 (M) x 4 (N): each wave owns 128 x 64 outputs = 8 x 4 MFMA 16x16x32 tiles, 128 fp32 accumulators;
+//   * wave grid 2 (M) x 4 (N): each wave owns 128 x 32 outputs = 8 x 2 MFMA 16x16x32 tiles, 64 fp32 accumulators;
 //     operands are swapped in the MFMA so that a lane ends up with 4 consecutive output columns of one row;
 //   * workgroup ids are remapped so that the 32 workgroups resident on one XCD (ids congruent mod 8) form a compact
 //     4 x 8 block of tiles and share their X / W panels in that XCD's L2.
@@ -29,9 +34,8 @@ namespace lg {
 
 constexpr int FB_M = 256, FB_K = 64;
 constexpr int F_THREADS = 512;
-// The tile is 256 x (64 * NJ) outputs: NJ = 4 -> 256 x 256, NJ = 3 -> 256 x 192; NJ = 2 -> 256 x 128 only on demand (LG_GEMM_TILE_WIDTH,
-// below): gemm_mid.hip never prefers it
-// LDS: a ring of 3 X tiles and a ring of 2 W tiles (256-wide: 96 + 64 KiB = the whole 160 KiB of a CU)
+// The tile is 256 x (64 * NJ) outputs.  LDS: a ring of 3 X tiles and a ring of 2 W tiles (96 + 32 KiB)
+constexpr int FB_NJ = 2;
 constexpr int X_STAGES = 3, W_STAGES = 2;
 constexpr int lds_halves(int NJ) { return X_STAGES * FB_M * FB_K + W_STAGES * FB_K * 64 * NJ; }
 
@@ -49,7 +53,7 @@ template <int NJ> __device__ __forceinline__ int unswz_kn(int k, int blk) {
 }
 
 template <int WL, int EPI, int NJ>
-__global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup grp, int tiles_m, int tiles_n, int turn, int cus, int wide_store) {
+__global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup grp, int tiles_m, int tiles_n, int cus, int wide_store) {
     constexpr int FB_N = 64 * NJ;
     constexpr int X_TILE = FB_M * FB_K, W_TILE = FB_K * FB_N;  // halves per ring slot
     constexpr int WCH = (FB_K * FB_N) / 512 / 8;  // 1 KiB chunks of the W tile per wave (= NJ)
@@ -144,9 +148,7 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup
     }
     const int64_t wstep = (WL == W_KN) ? (int64_t)FB_K * g.ldw : (WL == W_NK ? FB_K : 1024);
 
-    // Where the loop over k starts, as in the tiles of gemm_mid.hpp: members of one group may be computed by either kernel.  The loop goes
-    // round: its body is branch-free, the extra loads of the last iterations refill slots nobody reads any more with the first k-tiles.
-    const int first = n0 / MID_TURN_COLS * turn % ktiles;
+    // The loop's body is branch-free: the extra loads of the last iterations refill slots nobody reads any more with the first k-tiles.
     auto next = [&](int t) { return t + 1 == ktiles ? 0 : t + 1; };
     auto x_tile = [&](int t) { return reinterpret_cast<const char*>(X + (int64_t)t * FB_K); };
     auto w_tile = [&](int t) { return reinterpret_cast<const char*>(W + (int64_t)t * wstep); };
@@ -237,7 +239,7 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup
     };
 
     // prologue: X0 W0 X1 W1 X2; everything but X2 must have landed before the first fragments are read
-    int tw = first, tx = first;  // the k-tiles that are fetched next
+    int tw = 0, tx = 0;  // the k-tiles that are fetched next
     for (int t = 0; t < 3; ++t) {
 #pragma unroll
         for (int l = (t < 2 ? 0 : WCH); l < NLOAD; ++l)
@@ -401,7 +403,7 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup
 }
 
 template <int WL, int NJ>
-static void launch_fast_epi(const GemmArgs& g, const GemmGroup& grp, int tiles_m, int tiles_n, int turn, const StreamInfo& si, hipStream_t stream) {
+static void launch_fast_epi(const GemmArgs& g, const GemmGroup& grp, int tiles_m, int tiles_n, const StreamInfo& si, hipStream_t stream) {
     const int cus = si.cus;
     const dim3 grid(tiles_m * tiles_n), block(F_THREADS);
     const size_t smem = lds_halves(NJ) * sizeof(half_t);
@@ -416,7 +418,7 @@ static void launch_fast_epi(const GemmArgs& g, const GemmGroup& grp, int tiles_m
         /* set once per instantiation; the initialisation of a function-local static is thread-safe */              \
         static const hipError_t attr_rc = hipFuncSetAttribute((const void*)gemm_f16_fast<WL, E, NJ>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem); \
         (void)attr_rc;                                                                                              \
-        hipLaunchKernelGGL((gemm_f16_fast<WL, E, NJ>), grid, block, smem, stream, g, grp, tiles_m, tiles_n, turn, cus, wide); \
+        hipLaunchKernelGGL((gemm_f16_fast<WL, E, NJ>), grid, block, smem, stream, g, grp, tiles_m, tiles_n, cus, wide); \
     } while (0)
     switch (g.epi.kind) {
         case LG_EPI_NONE: LG_FAST(LG_EPI_NONE); break;
@@ -430,23 +432,11 @@ static void launch_fast_epi(const GemmArgs& g, const GemmGroup& grp, int tiles_m
 #undef LG_FAST
 }
 
-// nj: tile width in units of 64 features (gemm_mid.hip chooses it)
-void launch_gemm_fast_tile(const GemmArgs& g, const GemmGroup& grp, int wlayout, int nj, int turn, const StreamInfo& si, hipStream_t stream) {
-    // LG_GEMM_TILE_WIDTH=2|3|4 in the environment (read once) overrides the width where it divides N, for the problems that come here: a
-    // measurement knob (256 x 128 tiles leave registers and LDS for a second kernel's waves on the same compute unit)
-    static const int forced_nj = [] { const char* e = getenv("LG_GEMM_TILE_WIDTH"); return e ? atoi(e) : 0; }();
-    if (forced_nj >= 2 && forced_nj <= 4 && g.N % (64 * forced_nj) == 0 && !(forced_nj == 3 && g.epi.kind == LG_EPI_BIAS_GEGLU)) nj = forced_nj;
-    const int tiles_m = (g.M + FB_M - 1) / FB_M, tiles_n = g.N / (64 * nj) * grp.count;
-#define LG_FAST_WIDTHS(WL)                                                                   \
-    do {                                                                                     \
-        if (nj == 4) launch_fast_epi<WL, 4>(g, grp, tiles_m, tiles_n, turn, si, stream);           \
-        else if (nj == 3) launch_fast_epi<WL, 3>(g, grp, tiles_m, tiles_n, turn, si, stream);      \
-        else launch_fast_epi<WL, 2>(g, grp, tiles_m, tiles_n, turn, si, stream);                   \
-    } while (0)
-    if (wlayout == W_TILED) LG_FAST_WIDTHS(W_TILED);
-    else if (wlayout == W_NK) LG_FAST_WIDTHS(W_NK);
-    else LG_FAST_WIDTHS(W_KN);
-#undef LG_FAST_WIDTHS
+void launch_gemm_fast_tile(const GemmArgs& g, const GemmGroup& grp, int wlayout, const StreamInfo& si, hipStream_t stream) {
+    const int tiles_m = (g.M + FB_M - 1) / FB_M, tiles_n = g.N / (64 * FB_NJ) * grp.count;
+    if (wlayout == W_TILED) launch_fast_epi<W_TILED, FB_NJ>(g, grp, tiles_m, tiles_n, si, stream);
+    else if (wlayout == W_NK) launch_fast_epi<W_NK, FB_NJ>(g, grp, tiles_m, tiles_n, si, stream);
+    else launch_fast_epi<W_KN, FB_NJ>(g, grp, tiles_m, tiles_n, si, stream);
 }
 
 }  // namespace lg

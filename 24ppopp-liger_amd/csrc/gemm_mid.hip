@@ -1,5 +1,8 @@
-// gemm_mid.hip -- which tile, and how many K-slices, an fp16 GEMM takes: the instantiations of gemm_mid.hpp and the 256-row
-// kernel of gemm_fast.hip compared by a cost model, and the launch.
+// gemm_mid.hip -- which tile, and how many K-slices, an fp16 GEMM takes: the instantiations of gemm_mid.hpp compared by a cost model,
+// and the launch.
+#include <math.h>
+#include <stdlib.h>
+
 #include "gemm_mid.hpp"
 
 namespace lg {
@@ -9,7 +12,7 @@ LG_MID_DECL(kn_128); LG_MID_DECL(kn_192); LG_MID_DECL(kn_256);
 LG_MID_DECL(nk_96); LG_MID_DECL(nk_128); LG_MID_DECL(nk_192); LG_MID_DECL(nk_256);
 LG_MID_DECL(tiled_96); LG_MID_DECL(tiled_128); LG_MID_DECL(tiled_192); LG_MID_DECL(tiled_256);
 #undef LG_MID_DECL
-void launch_gemm_fast_tile(const GemmArgs& g, const GemmGroup& grp, int wlayout, int nj, int turn, const StreamInfo& si, hipStream_t stream);
+void launch_gemm_fast_tile(const GemmArgs& g, const GemmGroup& grp, int wlayout, const StreamInfo& si, hipStream_t stream);
 
 namespace {
 
@@ -40,9 +43,6 @@ double tile_cost(int M, int N, int K, int count, int mi, int nj, int nsplit, int
     if (nsplit > 1) us += rounds * (2.13 + 0.1128 * mi * nj * (mi * nj <= 16 ? nsplit : 1));
     return us;
 }
-// The 256-row kernel keeps two waves per SIMD and places tiles for many rows of tiles: 3 % faster than the same tile here when it
-// has several rounds of workgroups (4096 rows x 16384 x 12288: 1172 against 1230 us), level at one.
-constexpr double kFastFactor = 0.97;
 
 // K is sliced, and loops over it are turned, up to 256 token rows only.  Above that every output is one sum in the order of k: a row's
 // bits do not depend on the rows and features around it in a call, on the layout or on the stream, so that a batch, its parts and the
@@ -62,9 +62,7 @@ int mid_turn(int M, int K, int wlayout) {
 
 }  // namespace
 
-static TilePlan plan_gemm_tiles(const GemmArgs& g, int count, int wlayout, bool fast_ok, const StreamInfo& si) {
-    TilePlan best{};
-    best.cost = 1e30;
+static TilePlan plan_gemm_tiles(const GemmArgs& g, int count, int wlayout, const StreamInfo& si) {
     const int cus = si.cus, ktiles = g.K / MID_K;
     const bool heads = g.epi.kind == LG_EPI_BIAS_HEADS || g.epi.kind == LG_EPI_BIAS_HEADS_ROWS;
     auto usable = [&](const Tile& t, int cnt, int sp) {
@@ -89,7 +87,7 @@ static TilePlan plan_gemm_tiles(const GemmArgs& g, int count, int wlayout, bool 
                 if ((fixed && c) || sp < 1 || (c > 1 && sp <= 2) || (!fixed && sp > 1 && (!si.ws || tiles * sp > cus || g.M >= kSequentialRows))) continue;
                 if (!usable(t, cnt, sp)) continue;
                 const double us = tile_cost(g.M, g.N, g.K, cnt, t.mi, t.nj, sp, wlayout, cus);
-                if (us < p.cost) p = TilePlan{us, t.mi, t.nj, sp, false};
+                if (us < p.cost) p = TilePlan{us, t.mi, t.nj, sp};
             }
         }
         return p;
@@ -112,15 +110,8 @@ static TilePlan plan_gemm_tiles(const GemmArgs& g, int count, int wlayout, bool 
             if (a.nsplit && t.nsplit && a.cost < most && t.cost < least) { least = t.cost; slices = sp; }
         }
     }
-    best = pick(count, slices);
     // (where members are sliced and the slices of a group do not fit the workspace, the group is not taken as one launch)
-    if (fast_ok && slices == 1 && g.M > 64 && g.epi.kind != LG_EPI_BIAS_HEADS_ROWS)
-        for (int nj = 4; nj >= 3; --nj) {
-            if (g.N % (64 * nj) || (nj == 3 && g.epi.kind == LG_EPI_BIAS_GEGLU)) continue;
-            const double us = kFastFactor * tile_cost(g.M, g.N, g.K, count, 8, 2 * nj, 1, wlayout, cus);
-            if (us < best.cost) best = TilePlan{us, 8, nj, 1, true};
-        }
-    return best;
+    return pick(count, slices);
 }
 
 // alignment and shape that the tile kernels need of every member
@@ -140,21 +131,28 @@ static bool tiles_apply(const GemmArgs& g, const GemmGroup& grp, int wlayout, in
 
 TilePlan plan_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, int wlayout, int batch, hipStream_t stream) {
     if (!tiles_apply(g, grp, wlayout, batch)) return TilePlan{};
-    bool fast_ok = true;  // whole rows of 16 bytes
-    for (int i = 0; i < grp.count; ++i) fast_ok = fast_ok && aligned16(grp.Y[i]);
-    return plan_gemm_tiles(g, grp.count, wlayout, fast_ok, stream_info(stream));
+    return plan_gemm_tiles(g, grp.count, wlayout, stream_info(stream));
 }
 
 int launch_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled) {
     *handled = false;
     if (g.epi.kind == LG_EPI_BIAS_HEADS_ROWS && !rows) return LG_OK;
-    const TilePlan p = plan_gemm_tiles_f16(g, grp, wlayout, batch, stream);
+    TilePlan p = plan_gemm_tiles_f16(g, grp, wlayout, batch, stream);
     if (p.nsplit == 0) return LG_OK;
     const StreamInfo si = stream_info(stream);
     *handled = true;
-    if (p.fast) {
-        launch_gemm_fast_tile(g, grp, wlayout, p.nj, mid_turn(g.M, g.K, wlayout), si, stream);
-        return check_launch("gemm_f16_fast");
+    // LG_GEMM_TILE_WIDTH=2|3|4 in the environment (read once) overrides the width of 256-row tiles, in units of 64 features, where it
+    // divides N: a measurement knob.  2 takes the kernel of gemm_fast.hip, which leaves registers and LDS for a second kernel's waves on
+    // the same compute unit.
+    static const int width = [] { const char* e = getenv("LG_GEMM_TILE_WIDTH"); return e ? atoi(e) : 0; }();
+    if (width >= 2 && width <= 4 && p.mi == 8 && g.M >= kSequentialRows && g.N % (64 * width) == 0) {
+        bool whole_rows = true;  // of 16 bytes
+        for (int i = 0; i < grp.count; ++i) whole_rows = whole_rows && aligned16(grp.Y[i]);
+        if (width > 2 && !(width == 3 && g.epi.kind == LG_EPI_BIAS_GEGLU)) p.nj = 2 * width;
+        else if (width == 2 && whole_rows && g.epi.kind != LG_EPI_BIAS_HEADS_ROWS) {
+            launch_gemm_fast_tile(g, grp, wlayout, si, stream);
+            return check_launch("gemm_f16_fast");
+        }
     }
     const int ktiles = g.K / MID_K, kt = (ktiles + p.nsplit - 1) / p.nsplit;
     const MidLaunch l{(ktiles + kt - 1) / kt, kt, mid_turn(g.M, g.K, wlayout), si, stream};

@@ -1,19 +1,15 @@
-// gemm_mid.hpp -- fp16 GEMM whose tile is fitted to the token count (gfx950): everything between a few token rows and the full
-// prefill batches of gemm_fast.hip.
+// gemm_mid.hpp -- fp16 GEMM whose tile is fitted to the token count (gfx950): everything from a few token rows to full prefill batches.
 //
 //   Y[M, N] = X[M, K] * W, any weight layout, fp32 accumulate, fused epilogue, groups; K % 64 == 0, N a multiple of the tile width.
 //
 // What bounds it depends on M.  Up to about 200 token rows it is the stream of weights from memory, above that the matrix pipes --
-// provided that the tiles cover the token rows without much padding and that there is one workgroup for every compute unit.  The
-// 256-row tiles of gemm_fast.hip do neither for a prompt or a large decode batch, and their 128-wide variant spends 208 KiB of LDS
-// traffic on 1024 cycles of matrix work.  So here:
+// provided that the tiles cover the token rows without much padding and that there is one workgroup for every compute unit.  So here:
 //   * the tile is (32 MI) x (32 NJ), MI = 1 .. 8 and NJ = 3, 4, 6, 8, chosen per problem (gemm_mid.hip), and K may be sliced;
 //   * a workgroup is 4 waves, one per SIMD, in a 2 x 2 grid: a wave multiplies (16 MI) x (16 NJ) outputs, which costs
 //     (MI + NJ) / (MI NJ) LDS reads per matrix instruction -- half to two thirds of what 8 waves of half the size read.  The
 //     accumulators are AGPRs and named as such in the instruction: left to itself the compiler moves them back and forth;
 //   * both operands go global -> LDS with direct-to-LDS loads into rings of 2 to 6 k-tiles (as many as 160 KiB hold), one barrier
-//     per k-tile; fragments are double-buffered in registers and read by hand-issued LDS reads between the matrix instructions
-//     (the schedule of gemm_fast.hip);
+//     per k-tile; fragments are double-buffered in registers and read by hand-issued LDS reads between the matrix instructions;
 //   * a compute unit has 32 KiB of loads on their way at most, and they come back in order: X, from the L2 in 0.1 us, waits behind W,
 //     from memory in 0.5 us and more.  Taken in turns, 60 GB/s of both together reach a compute unit, and that bounded most
 //     prompts (384 rows x 12288 x 16384: 174 us of loads alone, 98 with W from the L2).  So W goes out for two k-tiles at a time and
@@ -43,7 +39,9 @@ struct MidLaunch {  // what a launch of one of the instantiations needs besides 
     hipStream_t stream;
 };
 
-// block position of a [64 k][32 NJ n] weight tile (see gemm_fast.hip): the 192-wide tile rotates, the others XOR
+// block position of a [64 k][32 NJ n] weight tile: which logical 32-byte block sits at position `pos` of row k, and where block `blk` sits.
+// Power-of-two widths XOR.  The 192-wide tile has 12 blocks to a row and rotates: its rows are 96 dwords apart, so rows k and k + 2 (and k + 8,
+// k + 10: the other half of the 32 lanes that one transposed read serves together) would share banks.
 template <int NJ> __device__ __forceinline__ int mid_swz_kn(int k, int pos) {
     if (NJ == 6) { const int b = pos + ((k >> 1) & 1) + 2 * ((k >> 3) & 1); return b >= 12 ? b - 12 : b; }
     return swz_b(k, pos);
@@ -68,7 +66,7 @@ constexpr int CACHE_DEVICE = 16;
 constexpr int mid_max_splits(int mi, int nj) { return mi * nj <= 16 ? 8 : 2; }
 
 template <int WL, int MI, int NJ, int XS, int WS, int ORDER, bool NT>
-__global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmGroup grp, RowMap rm, int tiles_m, int tiles_n, float* partial, unsigned* arrivals, int nsplit, int kt_per_split, int turn, int wide_store) {
+__global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmGroup grp, RowMap rm, int tiles_m, int tiles_n, float* partial, unsigned* arrivals, int nsplit, int kt_per_split, int turn, int wide_store, int region) {
     constexpr int TM = 32 * MI, TN = 32 * NJ;
     constexpr int X_TILE = TM * MID_K, W_TILE = TN * MID_K;  // halves per ring slot
     extern __shared__ __attribute__((aligned(16))) half_t smem[];  // X ring (XS tiles), then W ring (WS tiles)
@@ -82,7 +80,16 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
     // Workgroup ids are dealt to the 8 XCDs in turn; every XCD takes a contiguous run of (K-slice, tile column, tile row) with the
     // row fastest, so the workgroups that share a weight panel run next to each other on one XCD and fetch it from memory once.
     int tm, tn, split;
-    {
+    if (region) {
+        // Many rows of tiles: the workgroups of a round (one per compute unit, P on each XCD) cover RM x RN tiles, as near to a square as the
+        // tile counts allow, and each XCD 4 x P / 4 of them: a round reads 32 operand panels and an XCD 12 of them, where the run above
+        // makes it 18 (16 rows of tiles).  Fills cost power, which is what bounds these: 4096 rows x 12288 x 16384 1187 -> 1134 us
+        const int P = region >> 8, RM = region & 255, pw = P >> 2, RN = 8 * P / RM, xcols = RN / pw;
+        const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, round = slot / P, in = slot % P, regions_n = tiles_n / RN;
+        tm = (round / regions_n) * RM + (xcd / xcols) * 4 + (in & 3);
+        tn = (round % regions_n) * RN + (xcd % xcols) * pw + (in >> 2);
+        split = 0;
+    } else {
         const int total = gridDim.x, q = total >> 3, r = total & 7;
         const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
         const int id = xcd * q + min(xcd, r) + slot;
@@ -440,7 +447,7 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
         }
         return;
     }
-    // The tile goes through LDS and leaves in whole rows (gemm_fast.hip); rows that are not 16-byte aligned leave 8 bytes at a time.
+    // The tile goes through LDS and leaves in whole rows; rows that are not 16-byte aligned leave 8 bytes at a time.
     constexpr int PITCH = TN + 8;
     barrier_keep_loads_in_flight();  // every wave has read its last fragments
 #pragma unroll
@@ -518,8 +525,14 @@ static void launch_mid_tile(const GemmArgs& g, const GemmGroup& grp, const RowMa
     // set once per instantiation; the initialisation of a function-local static is thread-safe
     static const hipError_t attr_rc = hipFuncSetAttribute((const void*)gemm_f16_mid<WL, MI, NJ, XS, WS, ORDER, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     (void)attr_rc;
+    int region = 0;
+    const int P = l.si.cus >> 3, pw = P >> 2;
+    if (l.nsplit == 1 && pw >= 1 && P % 4 == 0) {
+        region = tiles_m % 16 == 0 && tiles_n % (2 * pw) == 0 ? 16 : tiles_m % 8 == 0 && tiles_n % (4 * pw) == 0 ? 8 : 0;
+        if (region) region |= P << 8;
+    }
     hipLaunchKernelGGL((gemm_f16_mid<WL, MI, NJ, XS, WS, ORDER, NT>), dim3(tiles_m * tiles_n * l.nsplit), dim3(MID_THREADS), smem, l.stream, g, grp, rm, tiles_m, tiles_n,
-                       l.si.ws, l.si.arrivals, l.nsplit, l.kt_per_split, l.turn, wide);
+                       l.si.ws, l.si.arrivals, l.nsplit, l.kt_per_split, l.turn, wide, region);
 }
 
 // one instantiation per tile height MI of a list, with and without the non-temporal hint
