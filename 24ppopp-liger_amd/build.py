@@ -26,7 +26,7 @@ HIP_FLAGS = [
 ]
 HIP_SOURCES = ["runtime.hip", "elementwise.hip", "attention_aux.hip", "gemm.hip", "gemm_fast.hip", "gemm_skinny.hip", "gemm_skinny_kn.hip", "gemm_mid.hip",
                "gemm_mid_kn_192.hip", "gemm_mid_kn_256.hip", "gemm_mid_nk_128.hip", "gemm_mid_nk_192.hip", "gemm_mid_nk_256.hip",
-               "gemm_mid_tiled_128.hip", "gemm_mid_tiled_192.hip", "gemm_mid_tiled_256.hip", "gemm_f32.hip", "gemv.hip", "attention.hip",
+               "gemm_mid_tiled_128.hip", "gemm_mid_tiled_192.hip", "gemm_mid_tiled_256.hip", "gemm_f32.hip", "gemm_f32_split.hip", "gemv.hip", "attention.hip",
                "attention_prefill.hip", "ceilings.hip", "weight_layout.hip"]
 
 

@@ -3,8 +3,8 @@
 //   gemm_f16_generic   128x128x32 tiles, 4 waves (2x2), MFMA 16x16x32 f16 -> fp32, any shape / stride /
 //                      alignment, both weight layouts, optional fused epilogue.  Correctness workhorse
 //                      (edge tiles, decomposed sub-ranges, attention GEMMs, small models).
-//   gemm_f32_mfma      128x128x16 tiles on v_mfma_f32_32x32x2_f32 for the fp32 instantiation (any shape, both layouts); problems
-//                      of few such tiles go to gemm_f32.hip;
+//   gemm_f32_mfma      128x128x16 tiles on v_mfma_f32_16x16x4_f32 for the fp32 instantiation (any shape, both layouts); problems
+//                      of few such tiles go to gemm_f32.hip, those of K >= 256 in whole chunks of 32 to gemm_f32_split.hip;
 //   gemm_f32_generic   64x64x16 VALU tiles, kept as a cross-check.
 // Aligned problems are routed to the tile kernels of gemm_mid.hpp and the weight-streaming ones.
 #include <stdlib.h>
@@ -17,6 +17,7 @@ namespace lg {
 int launch_gemm_skinny_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled);
 int launch_gemv_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled);
 int launch_gemm_skinny_sliced_f16(const GemmArgs& g, int wlayout, int batch, hipStream_t stream, bool* handled);
+int launch_gemm_f32_split(const GemmArgsF32& g, int wlayout, int batch, bool aligned, hipStream_t stream, bool* handled);
 int launch_gemm_f32_direct(const GemmArgsF32& g, int wlayout, int batch, bool aligned, hipStream_t stream, bool* handled);
 
 // ---------------------------------------------------------------------------------------------------
@@ -382,7 +383,9 @@ static int gemm_f32_dispatch(const GemmArgsF32& g, int wlayout, int batch, hipSt
         const bool aligned = aligned16(g.X) && aligned16(g.W) && aligned16(g.Y) && (g.ldx % 4 == 0) && (g.ldw % 4 == 0) &&
                              (g.strideX % 4 == 0) && (g.strideW % 4 == 0) && (g.strideY % 4 == 0);
         bool handled = false;
-        const int rc = launch_gemm_f32_direct(g, wlayout, batch, aligned, stream, &handled);
+        int rc = launch_gemm_f32_split(g, wlayout, batch, aligned, stream, &handled);
+        if (handled) return rc;
+        rc = launch_gemm_f32_direct(g, wlayout, batch, aligned, stream, &handled);
         if (handled) return rc;
         if (wlayout == W_NK) {
             if (aligned) hipLaunchKernelGGL((gemm_f32_mfma<W_NK, true>), grid, dim3(SB_THREADS), 0, stream, g);

@@ -11,7 +11,7 @@ constexpr TileF32 kTilesF32[] = {{1, 1, 0.0016, 0.0030}, {1, 2, 0.0030, 0.0045},
 // Estimated microseconds, fitted to 54 problems (M 8 .. 4096, K 32 .. 4096, batches up to 128, both layouts) x all tiles.
 // 64 x 64 tiles of this kernel reach 82 TFLOP/s on a full chip (their operands come through the first-level cache), the 128 x 128
 // tiles of gemm.hip 105-125, but only once there is one of them for every compute unit, and half of that if rows are not 16-byte
-// aligned: 800 x 1024 x 1024 80 us there, 23 here; 800 x 4096 x 1024 81 and 102; 64 x 256 x 1024 79 and 5.  Both sum in the same
+// aligned (K of 1024, which gemm_f32_split.hip takes now: 800 x 1024 80 us there, 23 here; 800 x 4096 81 and 102).  Both sum in the same
 // order, so the choice changes no bit of a result.
 double direct_cost(const TileF32& t, double tiles, int K, int cus) {
     const double load = (tiles + 0.25 * cus) / cus, fixed = 0.09 * t.mi * t.nj;  // fixed: the sums of the waves meet

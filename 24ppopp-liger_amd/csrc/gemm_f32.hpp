@@ -1,4 +1,5 @@
 // gemm_f32.hpp -- fp32 GEMM for few output tiles (gfx950): v_mfma_f32_16x16x4_f32, operands straight from global memory to registers.
+// Of K below 256 or not in chunks of 32; the others are the bf16 unit's (gemm_f32_split.hpp).
 //
 //   Y[M, N] = X[M, K] * W, W as [K, N] or [N, K]; any shape, stride and (4-byte) alignment; batched by strides.
 //

@@ -1,0 +1,52 @@
+// gemm_f32_split.hip -- which tile of gemm_f32_split.hpp an fp32 GEMM takes.
+#include "gemm_f32_split.hpp"
+
+namespace lg {
+
+namespace {
+
+struct TileSplit { int mi, nj; double alone_k, alone, shared_k, shared, ahead; };  // microseconds, for each k and besides
+// A tile on a compute unit of its own, and for each round of tiles when they are more than the compute units; `ahead`: what part of a round the
+// last one costs on top of its tiles.  Fitted to 448 problems (M 8 .. 4096, N 64 .. 4096, K 256 .. 4096, both layouts) x all tiles, within
+// 8 %; picking by it costs 0.6 % on average.  8 x 8: the 128 x 128 kernel.
+constexpr TileSplit kTilesSplit[] = {{1, 1, 0.00190, 0.07, 0.00186, 0.36, 0.37}, {1, 2, 0.00273, 0.39, 0.00267, 0.66, 0.48}, {2, 2, 0.00385, 1.01, 0.00400, 0.83, 0.58},
+                                     {2, 4, 0.00625, 1.70, 0.00746, 2.54, 0.48}, {4, 4, 0.00968, 3.01, 0.01176, 4.38, 0.46}, {8, 8, 0.04555, 2.05, 0.04189, 2.11, 1.00}};
+
+template <int WL>
+void launch(const TileSplit& t, bool staged, const GemmArgsF32& g, int batch, hipStream_t stream) {
+    switch (t.mi * 8 + t.nj) {
+        case 1 * 8 + 1: staged ? launch_f32_split_tile<WL, 1, 1, true>(g, batch, stream) : launch_f32_split_tile<WL, 1, 1, false>(g, batch, stream); break;
+        case 1 * 8 + 2: staged ? launch_f32_split_tile<WL, 1, 2, true>(g, batch, stream) : launch_f32_split_tile<WL, 1, 2, false>(g, batch, stream); break;
+        case 2 * 8 + 2: staged ? launch_f32_split_tile<WL, 2, 2, true>(g, batch, stream) : launch_f32_split_tile<WL, 2, 2, false>(g, batch, stream); break;
+        case 2 * 8 + 4: staged ? launch_f32_split_tile<WL, 2, 4, true>(g, batch, stream) : launch_f32_split_tile<WL, 2, 4, false>(g, batch, stream); break;
+        case 4 * 8 + 4: staged ? launch_f32_split_tile<WL, 4, 4, true>(g, batch, stream) : launch_f32_split_tile<WL, 4, 4, false>(g, batch, stream); break;
+        default: launch_f32_split128<WL>(g, batch, stream); break;
+    }
+}
+
+}  // namespace
+
+// The choice of this path looks at K alone: rows and features of a decomposed call have the bits of the whole.
+int launch_gemm_f32_split(const GemmArgsF32& g, int wlayout, int batch, bool aligned, hipStream_t stream, bool* handled) {
+    *handled = false;
+    if (g.K < 256 || g.K % FS_K) return LG_OK;
+    const int cus = stream_info(stream).cus;
+    const TileSplit* best = nullptr;
+    double best_us = 1e30;
+    for (const TileSplit& t : kTilesSplit) {
+        const double tiles = (double)((g.M + 16 * t.mi - 1) / (16 * t.mi)) * ((g.N + 16 * t.nj - 1) / (16 * t.nj)) * batch;
+        if (tiles > 1e9 || (wlayout == W_KN && t.nj > 1 && t.nj < 8 && g.N < 16 * t.nj)) continue;  // [K, N] weights are loaded nj features at a time
+        const double alone = g.K * t.alone_k + t.alone, shared = tiles > cus ? (tiles / cus + t.ahead) * (g.K * t.shared_k + t.shared) : 0.0;
+        const double us = alone > shared ? alone : shared;
+        if (us < best_us) { best_us = us; best = &t; }
+    }
+    if (!best) return LG_OK;
+    *handled = true;
+    // direct-to-LDS loads are whole 16-byte vectors at 16-byte addresses, also where the last tile column of [K, N] weights is moved back
+    const bool staged = aligned && (wlayout == W_NK || (g.N >= 16 && g.N % 4 == 0));
+    if (wlayout == W_NK) launch<W_NK>(*best, staged, g, batch, stream);
+    else launch<W_KN>(*best, staged, g, batch, stream);
+    return check_launch("gemm_f32_split");
+}
+
+}  // namespace lg

@@ -85,3 +85,47 @@ def test_a_row_does_not_depend_on_its_call(dev, transa, M, N, K):
         assert torch.equal(gemm(m0, m, 0, N), whole[m0:m0 + m])
     for n0, n in ((0, N // 4), (N // 4, N - N // 4), (N - 130, 130), (7, 16)):
         assert torch.equal(gemm(0, M, n0, n), whole[:, n0:n0 + n])
+
+
+# K of the bf16 kernels (256 and more, whole chunks of 32; fewer chunks than slices, slices of unequal length), every tile, its edges, and
+# operands that only the unaligned path takes
+@pytest.mark.parametrize("transa", [0, 1])
+@pytest.mark.parametrize("M,N,K,batch,pad,shift", [(1, 1, 256, 1, 0, 0), (17, 20, 256, 1, 0, 0), (15, 33, 288, 1, 0, 0), (33, 66, 544, 1, 2, 1), (64, 256, 1024, 1, 0, 0),
+                                                   (65, 260, 320, 3, 0, 0), (200, 1001, 512, 1, 3, 0), (200, 1004, 512, 1, 0, 0), (800, 1024, 256, 1, 0, 0),
+                                                   (1000, 2050, 320, 1, 0, 2), (1030, 4100, 288, 1, 0, 0), (333, 64, 352, 40, 0, 0)])
+def test_split_products(dev, transa, M, N, K, batch, pad, shift):
+    _case(dev, transa, M, N, K, batch, pad, shift)
+
+
+@pytest.mark.parametrize("transa", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(40, 70, 512), (300, 1024, 256), (1100, 2048, 256)])
+def test_split_of_what_bf16_does_not_hold(dev, transa, M, N, K):
+    """Infinities, NaN, the largest numbers, sums that overflow and rows of tiny numbers come out as from fp32 products; what else shares a
+    tile with them keeps its accuracy."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(2)
+    X, W, Y = torch.randn(M, K, device="cuda", generator=gen), torch.randn(K, N, device="cuda", generator=gen), torch.empty(M, N, device="cuda")
+    X[0, 5], X[1, 7], X[2, 9] = float("inf"), float("nan"), -float("inf")
+    W[5] = torch.where(W[5].abs() < 0.25, torch.ones_like(W[5]), W[5])     # an infinity times a number, times one (exact in hi), never times 0
+    X[3] = 0.0
+    X[3, 11] = 3.4e38                                                      # hi rounds to infinity
+    W[11] = W[11].clamp(-1.0, 1.0)
+    X[4], X[5] = 2.0 ** 120 * X[4].abs() + 2.0 ** 120, X[5] * 2.0 ** -118  # overflows where a column sums up; below the smallest bf16 in lo
+    W[:, 0] = W[:, 0].abs() + 2.0 ** 7
+    W[:, 1] *= 2.0 ** -116
+    Wd = W if transa == 0 else W.t().contiguous()
+    dev.call("lg_gemm_f32", transa, 0, N, M, K, Wd.data_ptr(), N if transa == 0 else K, X.data_ptr(), K, Y.data_ptr(), N)
+    dev.sync()
+    ref, mag = X.double().cpu() @ W.double().cpu(), X.double().abs().cpu() @ W.double().abs().cpu()
+    got = Y.double().cpu()
+    assert torch.equal(got[0], ref[0]) and bool(torch.isnan(got[1]).all()) and torch.equal(got[2], ref[2])     # infinities with their signs
+    assert float(ref[4, 0]) > 3.5e38 and float(got[4, 0]) == float("inf")
+    inside = (ref.abs() < 3.4e38) & (mag < 3.4e38)
+    tiny = K * 2.0 ** -149                                                  # products below the smallest fp32 number
+    assert bool(((got - ref).abs() <= K * EPS * mag + tiny)[inside].all())
+
+
+@pytest.mark.parametrize("transa", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(4096, 1024, 256), (1600, 4096, 320), (800, 1024, 1024)])
+def test_a_row_of_a_split_product_does_not_depend_on_its_call(dev, transa, M, N, K):
+    test_a_row_does_not_depend_on_its_call(dev, transa, M, N, K)
