@@ -22,23 +22,25 @@ constexpr Tile kTiles[] = {{1, 4}, {2, 4}, {3, 4}, {4, 4}, {6, 4}, {8, 4}, {2, 3
 constexpr int kMinSliceTiles = 8;     // k-tiles of a K-slice at least: below that its ramp costs more than it hides
 constexpr int kMaxTiles = LG_ARRIVAL_COUNTERS / 2;
 
-// Microseconds of one launch.  Fitted to 15000 measurements (M 9 .. 4096, 16 weight shapes from 1024 x 1024 to 32768 x 12288, all three
-// layouts, the tiles and slice counts worth trying, weights cycled out of the caches); picking by it costs 0.6 % against the best
-// measured choice on average (the worst 18 %: 8192 x 2048 [in, out] at 106 rows, 16.5 against 14.0 us).  Terms: a k-tile costs its
-// matrix work or its loads, of which the weights' weigh the most (they come from memory, and a compute unit has no more than 32 KiB on
-// their way at a time); a last round that is partly empty runs faster, at a higher clock; the chip reads 7.7 TB/s, which overlaps
-// with the rest as in sqrt(a^2 + b^2); K-slices that meet cost a trip to the counter and the transfer of the sums in every round, and
-// rounds of short loops their ramps.
-double tile_cost(int M, int N, int K, int count, int mi, int nj, int nsplit, int cus) {
+// Microseconds of one launch.  Fitted to 556 problems (M 8 .. 2048, 17 weight shapes from 1024 x 1024 to 32768 x 12288, all three
+// layouts) x all tiles and slice counts, each measured with weights cycled out of the caches; picking by it costs 1 % against
+// the best measured choice on average.  Terms: a k-tile costs its matrix work or its loads; a workgroup cannot pull more than 69 GB/s
+// of weights (44 in pieces of 256 bytes: 128-wide tiles of [in, out] weights, few rows) and the chip 7.4 TB/s; what memory and matrix
+// pipes do in the same time overlaps only in part; a K-slice meeting costs a trip to the counter and the transfer of the sums, in
+// every round (three projections of 64 rows x 4096 x 4096 in four slices, three rounds: 40 us).
+double tile_cost(int M, int N, int K, int count, int mi, int nj, int nsplit, int wlayout, int cus) {
     const int tiles_m = (M + 32 * mi - 1) / (32 * mi), tiles_n = N / (32 * nj) * count, ktiles = K / MID_K;
     const int kt = (ktiles + nsplit - 1) / nsplit;
     const long wgs = (long)tiles_m * tiles_n * nsplit;
     const double rounds = (double)((wgs + cus - 1) / cus);
-    const double work = kt * (0.185 + 0.0201 * mi * nj), loads = kt * (0.0073 + 0.0111 * mi + 0.0714 * nj);
-    const double own = (work > loads ? work : loads) * (0.774 + 0.226 * wgs / (rounds * cus));
-    const double chip = 2.0 * N * K * count / (7.68e6 * cus / 256.0) / rounds;
-    double us = 4.37 + rounds * sqrt(own * own + chip * chip);
-    if (nsplit > 1) us += rounds * (mi * nj <= 16 ? 1.0 + 0.086 * mi * nj * nsplit : 6.5 + 0.0245 * mi * nj) + 5.5 * (rounds - 1);
+    const double work = kt * (0.13 + 0.0192 * mi * nj), loads = kt * (0.0673 + 0.0292 * (mi + nj));
+    const double compute = work > loads ? work : loads;
+    const double rate = wlayout == W_KN && nj == 4 && M <= 64 ? 44e3 : 69.42e3;
+    const double chip = 2.0 * N * K * count / (7.3735e6 * cus / 256.0) / rounds, own = kt * (64.0 * 32 * 2 / rate) * nj;
+    double round = compute > chip ? compute + 0.6025 * chip : chip + 0.6025 * compute;
+    if (round < own) round = own;
+    double us = 3.67 + rounds * round;
+    if (nsplit > 1) us += rounds * (2.13 + 0.1128 * mi * nj * (mi * nj <= 16 ? nsplit : 1));
     return us;
 }
 
@@ -84,7 +86,7 @@ static TilePlan plan_gemm_tiles(const GemmArgs& g, int count, int wlayout, const
                 const int sp = fixed ? fixed : tries[c];
                 if ((fixed && c) || sp < 1 || (c > 1 && sp <= 2) || (!fixed && sp > 1 && (!si.ws || tiles * sp > cus || g.M >= kSequentialRows))) continue;
                 if (!usable(t, cnt, sp)) continue;
-                const double us = tile_cost(g.M, g.N, g.K, cnt, t.mi, t.nj, sp, cus);
+                const double us = tile_cost(g.M, g.N, g.K, cnt, t.mi, t.nj, sp, wlayout, cus);
                 if (us < p.cost) p = TilePlan{us, t.mi, t.nj, sp};
             }
         }
