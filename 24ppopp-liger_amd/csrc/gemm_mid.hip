@@ -157,10 +157,12 @@ int launch_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap*
     const int ktiles = g.K / MID_K, kt = (ktiles + p.nsplit - 1) / p.nsplit;
     const MidLaunch l{(ktiles + kt - 1) / kt, kt, mid_turn(g.M, g.K, wlayout), si, stream};
     const RowMap rm = rows ? *rows : RowMap{};
-    // Weights that one row of tiles reads, or two whose workgroups run side by side on an XCD, need not stay in the L2: the non-temporal hint
-    // is worth 7 % and 4 % with fragment blocks, 7 % and 2 % with [out, in], 5 % and nothing with [in, out], and costs up to 4 % from
-    // three rows of tiles on.
-    const bool nt = g.M <= 32 * p.mi * (wlayout == W_KN ? 1 : 2);
+    // Weights that one row of tiles reads, or two whose workgroups run side by side on an XCD, need not stay in the L2: coming from memory, the
+    // non-temporal hint is worth 7 % and 4 % with fragment blocks, 7 % and 2 % with [out, in], 5 % and nothing with [in, out], and costs up to
+    // 4 % from three rows of tiles on.  Weights that the 256 MiB memory-side cache still holds from the last step lose by it (at two rows
+    // 6144 x 2048 5 %, 12288 x 4096 20 %): two rows take it for weights that the cache cannot hold.
+    const bool large = (int64_t)g.N * g.K * grp.count * (int64_t)sizeof(half_t) >= (int64_t)256 << 20;
+    const bool nt = g.M <= 32 * p.mi || (g.M <= 64 * p.mi && wlayout != W_KN && large);
     bool ok = false;
     switch (p.nj) {
         case 3: ok = wlayout == W_NK ? launch_mid_nk_96(p.mi, nt, g, grp, rm, l) : launch_mid_tiled_96(p.mi, nt, g, grp, rm, l); break;

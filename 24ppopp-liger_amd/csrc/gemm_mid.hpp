@@ -57,9 +57,9 @@ __device__ __forceinline__ void mfma16_acc(float4_t& c, half8_t a, half8_t b) {
 
 typedef int int4_t __attribute__((ext_vector_type(4)));
 
-// When the loads of later k-tiles are issued: half of a k-tile's under its second k-step and half under the next one's first, or for two
-// k-tiles at a time, W before X
-enum { MID_SPREAD, MID_PAIRS };
+// When the loads of later k-tiles are issued: all of a k-tile's under its second k-step, half of them there and half under the next k-tile's
+// first, or for two k-tiles at a time, W before X
+enum { MID_BURST, MID_SPREAD, MID_PAIRS };
 // cache policy of the K-slices' sums: written through to, and read from, the level that all XCDs share
 constexpr int CACHE_DEVICE = 16;
 // most K-slices of a tile (their sums are held in registers 64 fragments at a time)
@@ -81,7 +81,7 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
     // row fastest, so the workgroups that share a weight panel run next to each other on one XCD and fetch it from memory once.
     int tm, tn, split;
     if (region) {
-        // Many rows of tiles: the workgroups of a round (one per compute unit, P on each XCD) cover RM x RN tiles, as near to a square as the
+        // Many rows of 256-row tiles: the workgroups of a round (one per compute unit, P on each XCD) cover RM x RN tiles, as near to a square as the
         // tile counts allow, and each XCD 4 x P / 4 of them: a round reads 32 operand panels and an XCD 12 of them, where the run above
         // makes it 18 (16 rows of tiles).  Fills cost power, which is what bounds these: 4096 rows x 12288 x 16384 1187 -> 1134 us
         const int P = region >> 8, RM = region & 255, pw = P >> 2, RN = 8 * P / RM, xcols = RN / pw;
@@ -294,11 +294,11 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
             advance();
         }
     } else {
-        // The loads of k-tiles kt + XS and kt + WS go out once tile kt is done with: half of them under its second k-step and half under the
-        // first k-step of the next.
+        // The loads of k-tiles kt + XS and kt + WS go out once tile kt is done with: NOW of them under its second k-step and the others under
+        // the first k-step of the next.
         constexpr int SMAX = XS > WS ? XS : WS, SMIN = XS < WS ? XS : WS;
         constexpr int NDEEP = XS == WS ? 0 : (XS > WS ? MI : NJ);  // loads of the deeper ring that may stay in flight besides whole tiles
-        constexpr int NOW = NLOAD / 2;
+        constexpr int NOW = ORDER == MID_BURST ? NLOAD : NLOAD / 2;
         // prologue: tiles 0 .. in the order the loop would have issued them
         static_for<SMAX>([&](auto tc) {
             constexpr int t = decltype(tc)::value;
@@ -509,11 +509,14 @@ constexpr int mid_xs(int mi, int nj) { return mid_depth(mi, nj) > 2 ? mid_depth(
 constexpr int mid_ws(int mi, int nj) { return mid_depth(mi, nj) > 2 ? mid_depth(mi, nj) : mi == 8 ? 2 : 3; }
 // Against all loads under the second k-step, over the problems that a tile is good for: in pairs 0.89 (6 x 4), 0.91 (4 x 3, 8 x 4), 0.95 (3 x 4,
 // 4 x 4), 0.97-1.0 (the others of depth 4 and 6: bound by memory, or by few workgroups); at depth 3 spread 0.89-0.99, in pairs up to 1.05.
-constexpr int mid_order(int mi, int nj) { return mid_depth(mi, nj) > 3 || nj == 4 ? MID_PAIRS : MID_SPREAD; }
+// 1 x 4 with weights contiguous along k, from two rows of tiles on: in pairs 1.00-1.04, spread 1.00-1.05 ([in, out]: in pairs 0.93-1.0).
+constexpr int mid_order(int wl, int mi, int nj) {
+    return mi == 1 && nj == 4 && wl != W_KN ? MID_BURST : mid_depth(mi, nj) > 3 || nj == 4 ? MID_PAIRS : MID_SPREAD;
+}
 
 template <int WL, int MI, int NJ, bool NT>
 static void launch_mid_tile(const GemmArgs& g, const GemmGroup& grp, const RowMap& rm, const MidLaunch& l) {
-    constexpr int XS = mid_xs(MI, NJ), WS = mid_ws(MI, NJ), ORDER = mid_order(MI, NJ);
+    constexpr int XS = mid_xs(MI, NJ), WS = mid_ws(MI, NJ), ORDER = mid_order(WL, MI, NJ);
     const int tiles_m = (g.M + 32 * MI - 1) / (32 * MI), tiles_n = g.N / (32 * NJ) * grp.count;
     constexpr size_t ring = (size_t)(XS * MI + WS * NJ) * 32 * MID_K * sizeof(half_t), tile = (size_t)(32 * MI) * (32 * NJ + 8) * sizeof(half_t);
     constexpr size_t smem = ring > tile ? ring : tile;
@@ -527,7 +530,7 @@ static void launch_mid_tile(const GemmArgs& g, const GemmGroup& grp, const RowMa
     (void)attr_rc;
     int region = 0;
     const int P = l.si.cus >> 3, pw = P >> 2;
-    if (l.nsplit == 1 && pw >= 1 && P % 4 == 0) {
+    if (MI == 8 && l.nsplit == 1 && pw >= 1 && P % 4 == 0) {
         region = tiles_m % 16 == 0 && tiles_n % (2 * pw) == 0 ? 16 : tiles_m % 8 == 0 && tiles_n % (4 * pw) == 0 ? 8 : 0;
         if (region) region |= P << 8;
     }
