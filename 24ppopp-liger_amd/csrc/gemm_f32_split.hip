@@ -42,8 +42,9 @@ int launch_gemm_f32_split(const GemmArgsF32& g, int wlayout, int batch, bool ali
     }
     if (!best) return LG_OK;
     *handled = true;
-    // direct-to-LDS loads are whole 16-byte vectors at 16-byte addresses, also where the last tile column of [K, N] weights is moved back
-    const bool staged = aligned && (wlayout == W_NK || (g.N >= 16 && g.N % 4 == 0));
+    // direct-to-LDS loads are whole 16-byte vectors at 16-byte addresses, also where the last tile column of [K, N] weights is moved back;
+    // they address the up to 64 rows of a tile by 32-bit element offsets
+    const bool staged = aligned && g.ldx < (1 << 25) && g.ldw < (1 << 25) && (wlayout == W_NK || (g.N >= 16 && g.N % 4 == 0));
     if (wlayout == W_NK) launch<W_NK>(*best, staged, g, batch, stream);
     else launch<W_KN>(*best, staged, g, batch, stream);
     return check_launch("gemm_f32_split");

@@ -129,3 +129,20 @@ def test_split_of_what_bf16_does_not_hold(dev, transa, M, N, K):
 @pytest.mark.parametrize("M,N,K", [(4096, 1024, 256), (1600, 4096, 320), (800, 1024, 1024)])
 def test_a_row_of_a_split_product_does_not_depend_on_its_call(dev, transa, M, N, K):
     test_a_row_does_not_depend_on_its_call(dev, transa, M, N, K)
+
+
+@pytest.mark.parametrize("M,N", [(64, 16384), (33, 512)])
+def test_rows_far_apart(dev, M, N):
+    """Rows further apart than 32-bit offsets within a tile reach: the same bits as rows next to each other."""
+    K, ld = 256, (1 << 27) + 4
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(3)
+    X, W = torch.randn(M, K, device="cuda", generator=gen), torch.randn(K, N, device="cuda", generator=gen)
+    far = torch.empty((M - 1) * ld + K, device="cuda").as_strided((M, K), (ld, 1))
+    far.copy_(X)
+    near, got = torch.empty(M, N, device="cuda"), torch.empty(M, N, device="cuda")
+    torch.cuda.synchronize()
+    dev.call("lg_gemm_f32", 0, 0, N, M, K, W.data_ptr(), N, X.data_ptr(), K, near.data_ptr(), N)
+    dev.call("lg_gemm_f32", 0, 0, N, M, K, W.data_ptr(), N, far.data_ptr(), ld, got.data_ptr(), N)
+    dev.sync()
+    assert torch.equal(near, got)
