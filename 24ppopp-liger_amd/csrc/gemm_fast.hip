@@ -39,19 +39,6 @@ constexpr int FB_NJ = 2;
 constexpr int X_STAGES = 3, W_STAGES = 2;
 constexpr int lds_halves(int NJ) { return X_STAGES * FB_M * FB_K + W_STAGES * FB_K * 64 * NJ; }
 
-// [64 k][64 NJ n] weight tile: which logical 32-byte block sits at block position `pos` of row k (swz_kn), and at which position
-// logical block `blk` sits (unswz_kn).  Power-of-two widths XOR (an involution); the 192-wide tile has 12 blocks to a row and
-// rotates instead: its rows are 96 dwords apart, so rows k and k + 2 (and k + 8, k + 10: the other half of the 32 lanes that one
-// transposed read serves together) would share banks, and a rotation by ((k >> 1) & 1) + 2 ((k >> 3) & 1) blocks separates them.
-template <int NJ> __device__ __forceinline__ int swz_kn(int k, int pos) {
-    if (NJ == 3) { const int b = pos + ((k >> 1) & 1) + 2 * ((k >> 3) & 1); return b >= 12 ? b - 12 : b; }
-    return swz_b(k, pos);
-}
-template <int NJ> __device__ __forceinline__ int unswz_kn(int k, int blk) {
-    if (NJ == 3) { const int p = blk - ((k >> 1) & 1) - 2 * ((k >> 3) & 1); return p < 0 ? p + 12 : p; }
-    return swz_b(k, blk);
-}
-
 template <int WL, int EPI, int NJ>
 __global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup grp, int tiles_m, int tiles_n, int cus, int wide_store) {
     constexpr int FB_N = 64 * NJ;
@@ -138,11 +125,10 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup
             woff[i] = (unsigned)(row * (int)g.ldw + c * 8) * 2u;
         } else {
             // W tile [64 k][FB_N n]: a k-row is FB_N / 8 lanes wide, chunk q = 64 / (FB_N / 8) consecutive k-rows
-            // (the 192-wide tile has 24 lanes to a k-row, so a chunk's lanes straddle rows: every lane finds its own row and place)
             constexpr int LPR = FB_N / 8;
             const int f = q * 64 + lane;
             const int k = f / LPR, p = f % LPR;
-            const int blk = swz_kn<NJ>(k, p >> 1);
+            const int blk = swz_b(k, p >> 1);
             woff[i] = (unsigned)(k * (int)g.ldw + (blk * 2 + (p & 1)) * 8) * 2u;
         }
     }
@@ -173,7 +159,7 @@ __global__ __launch_bounds__(F_THREADS) void gemm_f16_fast(GemmArgs g, GemmGroup
     for (int u = 0; u < NJ; ++u) {
         const int blk = wn * NJ + u;             // 32-byte block = 16 output columns
         const int k = lk * 8 + (l16 >> 2);       // this lane's source row of the first 4x16 read
-        wfrag[u] = k * FB_N + unswz_kn<NJ>(k, blk) * 16 + (l16 & 3) * 4;
+        wfrag[u] = k * FB_N + swz_b(k, blk) * 16 + (l16 & 3) * 4;
     }
     auto read_unit = [&](const half_t* xs, const half_t* ws, int ks, int u, half8_t (&a)[8], half8_t (&b)[NJ], int set) {
         if (u >= NJ) {
@@ -424,9 +410,7 @@ static void launch_fast_epi(const GemmArgs& g, const GemmGroup& grp, int tiles_m
         case LG_EPI_NONE: LG_FAST(LG_EPI_NONE); break;
         case LG_EPI_BIAS: LG_FAST(LG_EPI_BIAS); break;
         case LG_EPI_BIAS_GELU: LG_FAST(LG_EPI_BIAS_GELU); break;
-        case LG_EPI_BIAS_GEGLU:
-            if constexpr (NJ % 2 == 0) LG_FAST(LG_EPI_BIAS_GEGLU);  // the plan picks an even tile width for it
-            break;
+        case LG_EPI_BIAS_GEGLU: LG_FAST(LG_EPI_BIAS_GEGLU); break;
         default: LG_FAST(LG_EPI_BIAS_HEADS); break;
     }
 #undef LG_FAST
