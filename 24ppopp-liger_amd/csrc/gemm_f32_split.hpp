@@ -7,12 +7,14 @@
 // six roundings of the sum for every 32 k instead of 32.  Error against 64-bit sums, relative in the 2-norm, before (gemm_f32.hpp) -> now:
 // N(0, 1) times N(0, 0.02) K = 256 1.5e-7 -> 7.0e-8, 1024 2.9e-7 -> 1.6e-7, 4096 5.8e-7 -> 3.5e-7; uniform in 0 .. 1 K = 256 6.9e-8 -> 4.8e-8,
 // 4096 2.2e-7 -> 9.6e-8; the largest error of an element in units of 2^-24 of its sum of magnitudes 2.6 -> 1.3.
-// The split does not fit infinities, magnitudes of which hi rounds to infinity, and operands so small that lo falls below the smallest
-// bf16.  A tile with a sum that is not finite, or in which all that a lane has split of a row is below 2^-80 (and not zero), is computed
-// again on the fp32 unit, in the same slices.  (Single elements below 2^-110 beside larger ones of their row lose at most 2^-126 each.)
+// The parts are those of 2^23 times a number: a multiple of 2^-126, as every fp32 number is one of 2^-149, so that no part is below the smallest
+// normal bf16 and the split is exact however small an element is beside the others.  The sums are 2^46 times the result and are scaled back
+// at the end.  An output that is not finite then (infinities and NaN, magnitudes from 2^105, sums from 2^82) is computed again on the fp32
+// unit, in the same slices; the other outputs of its tile stay as they are.
 //
-// Every tile sums in the same order, so a result does not depend on the tile, the batch around a row or the feature range around a column:
-// K in eight slices of whole chunks of 32, in a slice chunk by chunk the six products, the slices one after the other.
+// Every tile sums in the same order, so an output depends on its row and its column alone: not on the tile, the batch around the row or the
+// feature range around the column, whatever these hold.
+// K goes in eight slices of whole chunks of 32, in a slice chunk by chunk the six products, the slices one after the other.
 //   * gemm_f32_split: (16 MI) x (16 NJ) tiles, a slice for each of 8 waves, no wave waits for another until the end.  A wave brings a chunk of
 //     its slice to LDS of its own with direct-to-LDS loads (whole rows; straight to registers, as unaligned operands go, they
 //     come in pieces of 16 bytes a lane, 800 x 4096 x 1024 85 instead of 65 us), takes it apart in registers and multiplies while
@@ -33,20 +35,23 @@ typedef __bf16 bf16x2_t __attribute__((ext_vector_type(2)));
 typedef float float2_t __attribute__((ext_vector_type(2)));
 
 constexpr int FS_WAVES = 8, FS_THREADS = 64 * FS_WAVES, FS_K = 32;  // k of a chunk
-constexpr float FS_SMALL = 0x1p-80f;
+constexpr float FS_SCALE = 0x1p23f, FS_UNSCALE = 0x1p-46f;
 
-// v[0..7] = hi + mid + lo, each rounded to bf16 from what the one before leaves: exact but for results below the smallest bf16
+// 2^23 v[0..7] = hi + mid + lo, each rounded to bf16 from what the one before leaves: exact for every finite v below 2^105.
 struct Split { bf16x8_t hi, mid, lo; };
 __device__ __forceinline__ Split split8(const float (&v)[8]) {
-    union { bf16x8_t b; unsigned u[4]; } h, m, l;
+    union { bf16x8_t b; bf16x2_t p[4]; } h, m, l;
+    auto rest = [&](float2_t a, bf16x2_t part) {
+        const unsigned bits = __builtin_bit_cast(unsigned, part);
+        return float2_t{a[0] - __builtin_bit_cast(float, bits << 16), a[1] - __builtin_bit_cast(float, bits & 0xffff0000u)};
+    };
 #pragma unroll
     for (int p = 0; p < 4; ++p) {
-        const float a = v[2 * p], b = v[2 * p + 1];
-        h.u[p] = __builtin_bit_cast(unsigned, __builtin_convertvector(float2_t{a, b}, bf16x2_t));
-        const float ra = a - __builtin_bit_cast(float, h.u[p] << 16), rb = b - __builtin_bit_cast(float, h.u[p] & 0xffff0000u);
-        m.u[p] = __builtin_bit_cast(unsigned, __builtin_convertvector(float2_t{ra, rb}, bf16x2_t));
-        const float sa = ra - __builtin_bit_cast(float, m.u[p] << 16), sb = rb - __builtin_bit_cast(float, m.u[p] & 0xffff0000u);
-        l.u[p] = __builtin_bit_cast(unsigned, __builtin_convertvector(float2_t{sa, sb}, bf16x2_t));
+        const float2_t a = {v[2 * p] * FS_SCALE, v[2 * p + 1] * FS_SCALE};
+        h.p[p] = __builtin_convertvector(a, bf16x2_t);
+        const float2_t r = rest(a, h.p[p]);
+        m.p[p] = __builtin_convertvector(r, bf16x2_t);
+        l.p[p] = __builtin_convertvector(rest(r, m.p[p]), bf16x2_t);
     }
     return Split{h.b, m.b, l.b};
 }
@@ -55,13 +60,13 @@ __device__ __forceinline__ Split split8(const float (&v)[8]) {
 __device__ __forceinline__ int split_k(int r) { return r < 4 ? r : r + 12; }
 
 // the six products that matter, small ones first; the weights are the A operand: acc[i][j][v] = token 16 i + l16, feature 4 lk + v of tile column j
-template <int MI, int NJ>
-__device__ __forceinline__ void split_multiply(float4_t (&acc)[MI][NJ], const Split (&xs)[MI], const Split (&ws)[NJ]) {
+template <int MI, int NJ, int JG>
+__device__ __forceinline__ void split_multiply(float4_t (&acc)[MI][NJ], const Split (&xs)[MI], const Split (&ws)[JG], int j0) {
     auto product = [&](auto wpart, auto xpart) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wpart(ws[j]), xpart(xs[i]), acc[i][j], 0, 0, 0);
+            for (int j = 0; j < JG; ++j) acc[i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wpart(ws[j]), xpart(xs[i]), acc[i][j0 + j], 0, 0, 0);
     };
     auto hi = [](const Split& s) { return s.hi; };
     auto mid = [](const Split& s) { return s.mid; };
@@ -73,7 +78,7 @@ __device__ __forceinline__ void split_multiply(float4_t (&acc)[MI][NJ], const Sp
     product(hi, mid);
     product(hi, hi);
 }
-// the same products in the fp32 unit, for operands that the split does not fit
+// the same products in the fp32 unit, for outputs that the scaled sums do not reach
 template <int MI, int NJ>
 __device__ __forceinline__ void plain_multiply(float4_t (&acc)[MI][NJ], const float (&x)[MI][8], const float (&w)[NJ][8]) {
 #pragma unroll
@@ -83,20 +88,7 @@ __device__ __forceinline__ void plain_multiply(float4_t (&acc)[MI][NJ], const fl
 #pragma unroll
             for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[j][r], x[i][r], acc[i][j], 0, 0, 0);
 }
-// whether the largest magnitude of what a lane has split of a row says that the split may not have fitted
-__device__ __forceinline__ bool split_unfit(float largest) { return largest > 0.f && largest < FS_SMALL; }
-// whether sums have overflowed, or an infinity, which splits into infinity and NaN, has come in
-template <int MI, int NJ>
-__device__ __forceinline__ bool not_finite(const float4_t (&sum)[MI][NJ]) {
-    float zero = 0.f;
-#pragma unroll
-    for (int i = 0; i < MI; ++i)
-#pragma unroll
-        for (int j = 0; j < NJ; ++j)
-#pragma unroll
-            for (int v = 0; v < 4; ++v) zero = fmaf(sum[i][j][v], 0.f, zero);
-    return !(zero == 0.f);
-}
+__device__ __forceinline__ bool finite(float v) { return fabsf(v) <= __FLT_MAX__; }
 
 template <int WL, int MI, int NJ, bool STAGED>
 __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split(GemmArgsF32 g, int tiles_m, int tiles_n) {
@@ -169,51 +161,45 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split(GemmArgsF32 g, i
         }
     };
     float4_t acc[MI][NJ];
-    auto clear = [&] {
+    auto clear = [](float4_t (&sum)[MI][NJ]) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < NJ; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+            for (int j = 0; j < NJ; ++j) sum[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
     };
-    clear();
-    float xmax[MI], wmax[NJ];
+    clear(acc);
+    // all of X is taken apart, W a few tile columns at a time: registers
+    constexpr int JG = MI == 4 || NJ == 1 ? 1 : 2;
+    Split xs[MI];
+    auto multiply = [&](const float (&w)[NJ][8]) {
 #pragma unroll
-    for (int i = 0; i < MI; ++i) xmax[i] = 0.f;
+        for (int j = 0; j < NJ; j += JG) {
+            Split ws[JG];
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) wmax[j] = 0.f;
-    auto largest = [](float m, const float (&v)[8]) {
-#pragma unroll
-        for (int r = 0; r < 8; ++r) m = fmaxf(m, fabsf(v[r]));
-        return m;
+            for (int u = 0; u < JG; ++u) ws[u] = split8(w[j + u]);
+            split_multiply<MI, NJ, JG>(acc, xs, ws, j);
+        }
     };
-    Split xs[MI], ws[NJ];
-    auto split = [&](const Chunk& c) {
-#pragma unroll
-        for (int i = 0; i < MI; ++i) { xmax[i] = largest(xmax[i], c.x[i]); xs[i] = split8(c.x[i]); }
-#pragma unroll
-        for (int j = 0; j < NJ; ++j) { wmax[j] = largest(wmax[j], c.w[j]); ws[j] = split8(c.w[j]); }
-    };
-    auto multiply = [&] { split_multiply<MI, NJ>(acc, xs, ws); };
 
     const int chunks = g.K / FS_K, part = (chunks + FS_WAVES - 1) / FS_WAVES;
     const int first = wave * part, mine = min(chunks - first, part);  // this wave's chunks: first, first + 1, ...
     if constexpr (STAGED) {
         float* const xl = lds + wave * CHUNK;
         float* const wl = xl + X_CHUNK;
-        unsigned xo[2 * MI], wo[2 * NJ];  // element offsets of the 1 KiB pieces
+        constexpr int WPIECES = WL == W_NK ? 2 * NJ : 1, PIECE_K = 16 / NJ;  // [K, N] weights: a piece is PIECE_K rows, the pieces are alike
+        unsigned xo[2 * MI], wo[WPIECES];  // element offsets in the 1 KiB pieces
 #pragma unroll
         for (int i = 0; i < 2 * MI; ++i) {
             const int row = i * 8 + (lane >> 3);
             xo[i] = (unsigned)min(row, g.M - 1 - m0) * (unsigned)g.ldx + swz_a(row, lane & 7) * 4;
         }
 #pragma unroll
-        for (int i = 0; i < 2 * NJ; ++i) {
+        for (int i = 0; i < WPIECES; ++i) {
             if (WL == W_NK) {
                 const int row = i * 8 + (lane >> 3);
                 wo[i] = (unsigned)min(row, g.N - 1 - n0) * (unsigned)g.ldw + swz_a(row, lane & 7) * 4;
             } else {
-                const int f = i * 64 + lane;
-                wo[i] = (unsigned)(f / (4 * NJ)) * (unsigned)g.ldw + f % (4 * NJ) * 4;
+                wo[i] = (unsigned)(lane / (4 * NJ)) * (unsigned)g.ldw + lane % (4 * NJ) * 4;
             }
         }
         const float* const xb = X + (int64_t)m0 * g.ldx;
@@ -224,7 +210,10 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split(GemmArgsF32 g, i
 #pragma unroll
             for (int i = 0; i < 2 * MI; ++i) load_lds16(reinterpret_cast<const half_t*>(xk + xo[i]), reinterpret_cast<half_t*>(xl + i * 256));
 #pragma unroll
-            for (int i = 0; i < 2 * NJ; ++i) load_lds16(reinterpret_cast<const half_t*>(wk + wo[i]), reinterpret_cast<half_t*>(wl + i * 256));
+            for (int i = 0; i < 2 * NJ; ++i) {
+                const float* const p = WL == W_NK ? wk + wo[WL == W_NK ? i : 0] : wk + (int64_t)(i * PIECE_K) * g.ldw + wo[0];
+                load_lds16(reinterpret_cast<const half_t*>(p), reinterpret_cast<half_t*>(wl + i * 256));
+            }
         };
         auto read8 = [&](float (&v)[8], const float* base) {
 #pragma unroll
@@ -241,97 +230,97 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split(GemmArgsF32 g, i
             for (int i = 0; i < MI; ++i) {
                 float v[8];
                 read8(v, xl + i * 16 * FS_K);
-                xmax[i] = largest(xmax[i], v);
                 xs[i] = split8(v);
             }
+            float w[NJ][8];
             if constexpr (WL == W_NK) {
 #pragma unroll
-                for (int j = 0; j < NJ; ++j) {
-                    float v[8];
-                    read8(v, wl + j * 16 * FS_K);
-                    wmax[j] = largest(wmax[j], v);
-                    ws[j] = split8(v);
-                }
+                for (int j = 0; j < NJ; ++j) read8(w[j], wl + j * 16 * FS_K);
             } else {
-                float v[NJ][8];
 #pragma unroll
                 for (int r = 0; r < 8; ++r) {
                     typedef float rowvec_t __attribute__((ext_vector_type(NJ > 1 ? NJ : 2)));
                     const float* const p = wl + (4 * lk + split_k(r)) * TN + NJ * l16;
-                    if constexpr (NJ == 1) v[0][r] = *p;
+                    if constexpr (NJ == 1) w[0][r] = *p;
                     else {
                         const rowvec_t q = *reinterpret_cast<const rowvec_t*>(p);
 #pragma unroll
-                        for (int j = 0; j < NJ; ++j) v[j][r] = q[j];
+                        for (int j = 0; j < NJ; ++j) w[j][r] = q[j];
                     }
                 }
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) { wmax[j] = largest(wmax[j], v[j]); ws[j] = split8(v[j]); }
             }
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // everything has been read: the next chunk may land
             __builtin_amdgcn_sched_barrier(0);
             if (t + 1 < mine) fetch(first + t + 1);
-            multiply();
+            multiply(w);
             __builtin_amdgcn_sched_barrier(0);
         }
     } else if (mine > 0) {
         Chunk c;
         load(c, (int64_t)first * FS_K);
         for (int t = 0; t < mine; ++t) {
-            split(c);
+#pragma unroll
+            for (int i = 0; i < MI; ++i) xs[i] = split8(c.x[i]);
+            float w[NJ][8];
+#pragma unroll
+            for (int j = 0; j < NJ; ++j)
+#pragma unroll
+                for (int r = 0; r < 8; ++r) w[j][r] = c.w[j][r];
             load(c, (int64_t)(first + min(t + 1, mine - 1)) * FS_K);
             __builtin_amdgcn_sched_barrier(0);
-            multiply();
+            multiply(w);
             __builtin_amdgcn_sched_barrier(0);
         }
     }
-    bool bad = not_finite<MI, NJ>(acc);
+
+    // ---- the eight sums of an output meet, 16 token rows at a time; if one is not finite, those outputs are summed in the fp32 unit -----
+    unsigned bad = 0;  // of this thread's outputs, 4 of each 16 rows
+    for (bool again = false;; again = true) {
 #pragma unroll
-    for (int i = 0; i < MI; ++i) bad = bad || split_unfit(xmax[i]);
+        for (int i = 0; i < MI; ++i) {
+            float* const mybuf = sums + (wave * 16 + l16) * PITCH;
+            if (STAGED || i > 0 || again) __syncthreads();
+            if constexpr (WL == W_NK || NJ == 1) {
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) bad = bad || split_unfit(wmax[j]);
-    if (__syncthreads_or(bad)) {
-        clear();
+                for (int j = 0; j < NJ; ++j) *reinterpret_cast<float4_t*>(mybuf + j * 16 + 4 * lk) = acc[i][j];
+            } else {
+                typedef float rowvec_t __attribute__((ext_vector_type(NJ)));
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    rowvec_t o;
+#pragma unroll
+                    for (int j = 0; j < NJ; ++j) o[j] = acc[i][j][v];
+                    *reinterpret_cast<rowvec_t*>(mybuf + NJ * (4 * lk + v)) = o;
+                }
+            }
+            __syncthreads();
+            const int row = tid / (TN / 4), col = tid % (TN / 4) * 4;
+            const int m = m0 + i * 16 + row, n = n0 + col;
+            if (row < 16 && m < g.M && n < g.N) {
+                float4_t v = *reinterpret_cast<const float4_t*>(&sums[row * PITCH + col]);
+#pragma unroll
+                for (int s = 1; s < FS_WAVES; ++s) v += *reinterpret_cast<const float4_t*>(&sums[(s * 16 + row) * PITCH + col]);
+                float* const p = Y + (int64_t)m * g.ldy + n;
+                if (!again) {
+                    v *= FS_UNSCALE;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) bad |= (finite(v[r]) ? 0u : 1u) << (4 * i + r);
+                }
+                if (n >= nlo && n + 3 < g.N && !again) {
+                    *reinterpret_cast<float4u_t*>(p) = v;
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (n + r >= nlo && n + r < g.N && (!again || (bad >> (4 * i + r) & 1))) p[r] = v[r];
+                }
+            }
+        }
+        if (again || !__syncthreads_or(bad != 0)) break;
+        clear(acc);
         for (int t = 0; t < mine; ++t) {
             Chunk c;
             load(c, (int64_t)(first + t) * FS_K);
             plain_multiply<MI, NJ>(acc, c.x, c.w);
-        }
-    }
-
-    // ---- the eight sums of an output meet, 16 token rows at a time ----------------------------------------------------------
-#pragma unroll
-    for (int i = 0; i < MI; ++i) {
-        float* const mybuf = sums + (wave * 16 + l16) * PITCH;
-        if (STAGED || i > 0) __syncthreads();
-        if constexpr (WL == W_NK || NJ == 1) {
-#pragma unroll
-            for (int j = 0; j < NJ; ++j) *reinterpret_cast<float4_t*>(mybuf + j * 16 + 4 * lk) = acc[i][j];
-        } else {
-            typedef float rowvec_t __attribute__((ext_vector_type(NJ)));
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                rowvec_t o;
-#pragma unroll
-                for (int j = 0; j < NJ; ++j) o[j] = acc[i][j][v];
-                *reinterpret_cast<rowvec_t*>(mybuf + NJ * (4 * lk + v)) = o;
-            }
-        }
-        __syncthreads();
-        const int row = tid / (TN / 4), col = tid % (TN / 4) * 4;
-        const int m = m0 + i * 16 + row, n = n0 + col;
-        if (row < 16 && m < g.M && n < g.N) {
-            float4_t v = *reinterpret_cast<const float4_t*>(&sums[row * PITCH + col]);
-#pragma unroll
-            for (int s = 1; s < FS_WAVES; ++s) v += *reinterpret_cast<const float4_t*>(&sums[(s * 16 + row) * PITCH + col]);
-            float* const p = Y + (int64_t)m * g.ldy + n;
-            if (n >= nlo && n + 3 < g.N) {
-                *reinterpret_cast<float4u_t*>(p) = v;
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (n + r >= nlo && n + r < g.N) p[r] = v[r];
-            }
         }
     }
 }
@@ -380,13 +369,13 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split128(GemmArgsF32 g
     const int xkb = lane & 3, wkb = WL == W_NK ? xkb : wave & 3;
     const int xrow = 16 * wave + (lane >> 2), wrow = WL == W_NK ? xrow : (wave >> 2) * 64 + lane;
     const float* const xp = X + (int64_t)min(m0 + xrow, g.M - 1) * g.ldx + 4 * xkb;
-    const float* const wp = WL == W_NK ? W + (int64_t)min(n0 + wrow, g.N - 1) * g.ldw + 4 * wkb : W + (int64_t)(4 * wkb) * g.ldw + min(n0 + wrow, g.N - 1);
+    const unsigned wfeature = min(n0 + wrow, g.N - 1);
+    const float* const wp = WL == W_NK ? W + (int64_t)wfeature * g.ldw + 4 * wkb : W + (int64_t)(4 * wkb) * g.ldw;
     char* const xdst = lds128 + (xrow >> 4) * FT_BLOCK + xkb * 320 + (xrow & 15) * 16;
     char* const wdst = lds128 + 3 * FT_PART + (wrow >> 4) * FT_BLOCK + wkb * 320 + (wrow & 15) * 16;
 
     const int chunks = g.K / FS_K, part = (chunks + FS_WAVES - 1) / FS_WAVES;
     struct Raw { float x[8], w[8]; };
-    float xmax = 0.f, wmax = 0.f;
     auto gload = [&](Raw& raw, int c) {  // a whole chunk
         const int64_t k0 = (int64_t)c * FS_K;
 #pragma unroll
@@ -402,15 +391,10 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split128(GemmArgsF32 g
         }
         if (WL == W_KN) {
 #pragma unroll
-            for (int r = 0; r < 8; ++r) raw.w[r] = wp[(k0 + split_k(r)) * g.ldw];
+            for (int r = 0; r < 8; ++r) raw.w[r] = (wp + (k0 + split_k(r)) * g.ldw)[wfeature];
         }
     };
     auto stage = [&](const Raw& raw, int buf) {
-#pragma unroll
-        for (int r = 0; r < 8; ++r) {
-            xmax = fmaxf(xmax, fabsf(raw.x[r]));
-            wmax = fmaxf(wmax, fabsf(raw.w[r]));
-        }
         const Split x = split8(raw.x), w = split8(raw.w);
         char* const xd = xdst + buf * FT_CHUNK;
         char* const wd = wdst + buf * FT_CHUNK;
@@ -465,7 +449,7 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split128(GemmArgsF32 g
         fetch(f, c & 1);
         stage(raw, (c + 1) & 1);
         gload(raw, c + 2);
-        split_multiply<FT_MI, FT_NJ>(acc, f.x, f.w);
+        split_multiply<FT_MI, FT_NJ, FT_NJ>(acc, f.x, f.w, 0);
         // the reads first, then three vector operations of the split under every matrix instruction
         __builtin_amdgcn_sched_group_barrier(0x100, 3 * (FT_MI + FT_NJ), 0);
 #pragma unroll
@@ -480,48 +464,62 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split128(GemmArgsF32 g
     for (; c < chunks; ++c) {
         fetch(f, c & 1);
         if (c + 1 < chunks) stage(raw, (c + 1) & 1);
-        split_multiply<FT_MI, FT_NJ>(acc, f.x, f.w);
+        split_multiply<FT_MI, FT_NJ, FT_NJ>(acc, f.x, f.w, 0);
         end_chunk(c == chunks - 1);
         __syncthreads();
     }
-    if (__syncthreads_or(split_unfit(xmax) || split_unfit(wmax) || not_finite<FT_MI, FT_NJ>(total))) {
-        left = part;
+    unsigned bad = 0;  // the outputs of this lane that are not finite, which the fp32 unit sums again
+    for (bool again = false;; again = true) {
+#pragma unroll
+        for (int i = 0; i < FT_MI; ++i) {
+            const int m = m0 + wm * 64 + i * 16 + l16;
+#pragma unroll
+            for (int j = 0; j < FT_NJ; ++j) {
+                const int n = n0 + wn * 32 + j * 16 + 4 * lk, bit = 4 * (i * FT_NJ + j);
+                float* const p = Y + (int64_t)m * g.ldy + n;
+                if (!again) {
+                    total[i][j] *= FS_UNSCALE;
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) bad |= (finite(total[i][j][r]) ? 0u : 1u) << (bit + r);
+                }
+                if (m >= g.M) continue;
+                if (n + 3 < g.N && !again) {
+                    *reinterpret_cast<float4u_t*>(p) = total[i][j];
+                } else {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (n + r < g.N && (!again || (bad >> (bit + r) & 1))) p[r] = total[i][j][r];
+                }
+            }
+        }
+        if (again || !__any(bad != 0)) break;
 #pragma unroll
         for (int i = 0; i < FT_MI; ++i)
 #pragma unroll
             for (int j = 0; j < FT_NJ; ++j) total[i][j] = float4_t{-0.f, -0.f, -0.f, -0.f};
-        for (c = 0; c < chunks; ++c) {
+        for (c = 0; c < chunks; ++c) {  // acc is zero
+            const int64_t k0 = (int64_t)c * FS_K + 4 * lk;
             float x[FT_MI][8], w[FT_NJ][8];
+            auto row8 = [](float (&v)[8], const float* p) {
 #pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                const int64_t k = (int64_t)c * FS_K + 4 * lk + split_k(r);
+                for (int h = 0; h < 2; ++h) {
+                    const float4u_t q = *reinterpret_cast<const float4u_t*>(p + 16 * h);
 #pragma unroll
-                for (int i = 0; i < FT_MI; ++i) x[i][r] = X[(int64_t)min(m0 + wm * 64 + i * 16 + l16, g.M - 1) * g.ldx + k];
-#pragma unroll
-                for (int j = 0; j < FT_NJ; ++j) {
-                    const int64_t n = min(n0 + wn * 32 + j * 16 + l16, g.N - 1);
-                    w[j][r] = W[WL == W_NK ? n * g.ldw + k : k * g.ldw + n];
+                    for (int r = 0; r < 4; ++r) v[4 * h + r] = q[r];
                 }
+            };
+#pragma unroll
+            for (int i = 0; i < FT_MI; ++i) row8(x[i], X + (int64_t)min(m0 + wm * 64 + i * 16 + l16, g.M - 1) * g.ldx + k0);
+#pragma unroll
+            for (int j = 0; j < FT_NJ; ++j) {
+                const int64_t n = min(n0 + wn * 32 + j * 16 + l16, g.N - 1);
+                if constexpr (WL == W_NK) row8(w[j], W + n * g.ldw + k0);
+                else
+#pragma unroll
+                    for (int r = 0; r < 8; ++r) w[j][r] = W[(k0 + split_k(r)) * g.ldw + n];
             }
             plain_multiply<FT_MI, FT_NJ>(acc, x, w);
             end_chunk(c == chunks - 1);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < FT_MI; ++i) {
-        const int m = m0 + wm * 64 + i * 16 + l16;
-        if (m >= g.M) continue;
-#pragma unroll
-        for (int j = 0; j < FT_NJ; ++j) {
-            const int n = n0 + wn * 32 + j * 16 + 4 * lk;
-            float* const p = Y + (int64_t)m * g.ldy + n;
-            if (n + 3 < g.N) {
-                *reinterpret_cast<float4u_t*>(p) = total[i][j];
-            } else {
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    if (n + r < g.N) p[r] = total[i][j][r];
-            }
         }
     }
 }

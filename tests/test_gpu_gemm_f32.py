@@ -146,3 +146,65 @@ def test_rows_far_apart(dev, M, N):
     dev.call("lg_gemm_f32", 0, 0, N, M, K, W.data_ptr(), N, far.data_ptr(), ld, got.data_ptr(), N)
     dev.sync()
     assert torch.equal(near, got)
+
+
+def _gemm(dev, transa, X, W, m0=0, m=None, n0=0, n=None):
+    """Rows m0 .. and features n0 .. of X [M, K] times W ([K, N], or [N, K] if transa)"""
+    K = X.shape[1]
+    m, n = m or X.shape[0] - m0, n or W.shape[0 if transa else 1] - n0
+    Y = torch.empty(m, n, device="cuda")
+    torch.cuda.synchronize()
+    dev.call("lg_gemm_f32", transa, 0, n, m, K, W.data_ptr() + 4 * n0 * (K if transa else 1), W.shape[1], X.data_ptr() + 4 * m0 * K, K, Y.data_ptr(), n)
+    dev.sync()
+    return Y
+
+
+def _same(a, b):
+    return bool(((a == b) | (a.isnan() & b.isnan())).all())
+
+
+# small tiles, 64 x 64 and 128 x 128 ones, whose slices are 1, 2 and 4 chunks
+@pytest.mark.parametrize("transa", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(40, 72, 256), (300, 1024, 512), (4096, 1024, 256), (1100, 4096, 1024)])
+def test_bits_of_an_output_depend_on_its_row_and_column_alone(dev, transa, M, N, K):
+    """Rows and features that the bf16 parts do not hold (infinities, NaN, large numbers, sums that overflow) leave their tile's other outputs
+    alone, and a row with a slice of tiny numbers has the bits of a call of its own."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(4)
+    X, W = torch.randn(M, K, device="cuda", generator=gen), torch.randn(*((N, K) if transa else (K, N)), device="cuda", generator=gen)
+    X[1, :32] *= 2.0 ** -90         # one slice of tiny numbers, or a part of one, in an ordinary row
+    X[2, 32:40] *= 2.0 ** -120
+    plain = _gemm(dev, transa, X, W)
+    for r in range(4):
+        assert _same(_gemm(dev, transa, X, W, r, 1), plain[r:r + 1])
+        assert _same(_gemm(dev, transa, X, W, r, 33), plain[r:r + 33])
+    bad, col = X.clone(), W.clone()
+    bad[5, 3], bad[7, 4], bad[8, 5], bad[9] = float("inf"), float("nan"), 3.0e38, bad[9] * 2.0 ** 120
+    bad[M - 1] *= 2.0 ** -100
+    (col[6] if transa else col[:, 6])[:] *= 2.0 ** 110
+    got = _gemm(dev, transa, bad, col)
+    rows, cols = torch.ones(M, dtype=torch.bool, device="cuda"), torch.ones(N, dtype=torch.bool, device="cuda")
+    rows[[5, 7, 8, 9, M - 1]], cols[6] = False, False
+    assert _same(got[rows][:, cols], plain[rows][:, cols])
+    for r in (5, 8, 9, M - 1):
+        assert _same(_gemm(dev, transa, bad, col, r, 1), got[r:r + 1])
+    assert _same(_gemm(dev, transa, bad, col, 10, 30, 0, 17), got[10:40, :17])
+
+
+@pytest.mark.parametrize("transa", [0, 1])
+@pytest.mark.parametrize("M,N", [(48, 80), (1100, 2048)])
+def test_tiny_elements_beside_ordinary_ones(dev, transa, M, N):
+    """One element of each row is 2^e times an ordinary one and all that a feature, which is zero elsewhere, sees.  The sum
+    rounds its partial products, of which one or two are of the size of the whole: 2^-23 each at most."""
+    K = 256
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(5)
+    for e in (-100, -112, -118, -124, -140):
+        for w in (1.0, 2.0 ** min(-e, 125)):
+            X, W = torch.ones(M, K, device="cuda"), torch.zeros(K, N, device="cuda")
+            X[:, 77] = (1 + torch.rand(M, device="cuda", generator=gen)) * 2.0 ** e
+            W[77] = (1 + torch.rand(N, device="cuda", generator=gen)) * w
+            ref = X.double() @ W.double()
+            for x, y, r in ((X, W, ref), (W.t().contiguous(), X.t().contiguous(), ref.t())):      # as token rows, and as features
+                got = _gemm(dev, transa, x, y.t().contiguous() if transa else y).double()
+                assert bool(((got - r).abs() <= 4 * EPS * r.abs() + 2.0 ** -149).all()), (e, w)
