@@ -19,7 +19,7 @@ void launch(const TileSplit& t, bool staged, const GemmArgsF32& g, int batch, hi
         case 1 * 8 + 2: staged ? launch_f32_split_tile<WL, 1, 2, true>(g, batch, stream) : launch_f32_split_tile<WL, 1, 2, false>(g, batch, stream); break;
         case 2 * 8 + 2: staged ? launch_f32_split_tile<WL, 2, 2, true>(g, batch, stream) : launch_f32_split_tile<WL, 2, 2, false>(g, batch, stream); break;
         case 2 * 8 + 4: staged ? launch_f32_split_tile<WL, 2, 4, true>(g, batch, stream) : launch_f32_split_tile<WL, 2, 4, false>(g, batch, stream); break;
-        case 4 * 8 + 4: staged ? launch_f32_split_tile<WL, 4, 4, true>(g, batch, stream) : launch_f32_split_tile<WL, 4, 4, false>(g, batch, stream); break;
+        case 4 * 8 + 4: launch_f32_split_tile<WL, 4, 4, true>(g, batch, stream); break;
         default: launch_f32_split128<WL>(g, batch, stream); break;
     }
 }
@@ -30,21 +30,22 @@ void launch(const TileSplit& t, bool staged, const GemmArgsF32& g, int batch, hi
 int launch_gemm_f32_split(const GemmArgsF32& g, int wlayout, int batch, bool aligned, hipStream_t stream, bool* handled) {
     *handled = false;
     if (g.K < 256 || g.K % FS_K) return LG_OK;
+    // direct-to-LDS loads are whole 16-byte vectors at 16-byte addresses, also where the last tile column of [K, N] weights is moved back;
+    // they address the up to 64 rows of a tile by 32-bit element offsets
+    const bool staged = aligned && g.ldx < (1 << 25) && g.ldw < (1 << 25) && (wlayout == W_NK || (g.N >= 16 && g.N % 4 == 0));
     const int cus = stream_info(stream).cus;
     const TileSplit* best = nullptr;
     double best_us = 1e30;
     for (const TileSplit& t : kTilesSplit) {
         const double tiles = (double)((g.M + 16 * t.mi - 1) / (16 * t.mi)) * ((g.N + 16 * t.nj - 1) / (16 * t.nj)) * batch;
         if (tiles > 1e9 || (wlayout == W_KN && t.nj > 1 && t.nj < 8 && g.N < 16 * t.nj)) continue;  // [K, N] weights are loaded nj features at a time
+        if (t.mi == 4 && !staged) continue;  // its sums leave no registers for a chunk on its way
         const double alone = g.K * t.alone_k + t.alone, shared = tiles > cus ? (tiles / cus + t.ahead) * (g.K * t.shared_k + t.shared) : 0.0;
         const double us = alone > shared ? alone : shared;
         if (us < best_us) { best_us = us; best = &t; }
     }
     if (!best) return LG_OK;
     *handled = true;
-    // direct-to-LDS loads are whole 16-byte vectors at 16-byte addresses, also where the last tile column of [K, N] weights is moved back;
-    // they address the up to 64 rows of a tile by 32-bit element offsets
-    const bool staged = aligned && g.ldx < (1 << 25) && g.ldw < (1 << 25) && (wlayout == W_NK || (g.N >= 16 && g.N % 4 == 0));
     if (wlayout == W_NK) launch<W_NK>(*best, staged, g, batch, stream);
     else launch<W_KN>(*best, staged, g, batch, stream);
     return check_launch("gemm_f32_split");

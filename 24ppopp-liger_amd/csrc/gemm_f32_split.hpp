@@ -3,10 +3,12 @@
 //   Y[M, N] = X[M, K] * W, W as [K, N] or [N, K]; any M, N, stride and (4-byte) alignment; batched by strides.
 //
 // The fp32 matrix instruction does 64 flop a cycle, the bf16 one 1024.  Every fp32 number is the sum of three bf16 numbers (8 bits of
-// significand each; hi, mid, lo), so a product is nine bf16 products, of which the six of more than 2^-24 of it count: 170 flop a cycle, and
-// six roundings of the sum for every 32 k instead of 32.  Error against 64-bit sums, relative in the 2-norm, before (gemm_f32.hpp) -> now:
-// N(0, 1) times N(0, 0.02) K = 256 1.5e-7 -> 7.0e-8, 1024 2.9e-7 -> 1.6e-7, 4096 5.8e-7 -> 3.5e-7; uniform in 0 .. 1 K = 256 6.9e-8 -> 4.8e-8,
-// 4096 2.2e-7 -> 9.6e-8; the largest error of an element in units of 2^-24 of its sum of magnitudes 2.6 -> 1.3.
+// significand each; hi, mid, lo), so a product is nine bf16 products, of which the ninth, of two lo parts, is below 2^-35 of it and left out: 128
+// flop a cycle.  The products of two hi parts have a sum of their own, which rounds once in 32 k instead of 32 times; what the other seven
+// round is 2^-8 of that; the two meet at the end of a slice of K.  (All in one sum, and without the products of mid and lo, rows of
+// few nonzeros lost: one nonzero 2.5e-8 -> 3.5e-8.)  Error against 64-bit sums, relative in the 2-norm, before (gemm_f32.hpp) -> now, N(0, 1)
+// operands: K = 256 1.5e-7 -> 6.8e-8, 1024 2.9e-7 -> 8.5e-8, 4096 5.7e-7 -> 1.4e-7; uniform in 0 .. 1 K = 1024 1.17e-7 -> 5.1e-8; rows of one
+// nonzero 2.53e-8 in both, of eight 5.15e-8 -> 5.25e-8, of 32 6.9e-8 -> 6.1e-8.
 // The parts are those of 2^23 times a number: a multiple of 2^-126, as every fp32 number is one of 2^-149, so that no part is below the smallest
 // normal bf16 and the split is exact however small an element is beside the others.  The sums are 2^46 times the result and are scaled back
 // at the end.  An output that is not finite then (infinities and NaN, magnitudes from 2^105, sums from 2^82) is computed again on the fp32
@@ -14,17 +16,18 @@
 //
 // Every tile sums in the same order, so an output depends on its row and its column alone: not on the tile, the batch around the row or the
 // feature range around the column, whatever these hold.
-// K goes in eight slices of whole chunks of 32, in a slice chunk by chunk the six products, the slices one after the other.
+// K goes in eight slices of whole chunks of 32, in a slice chunk by chunk the eight products, the slices one after the other.
 //   * gemm_f32_split: (16 MI) x (16 NJ) tiles, a slice for each of 8 waves, no wave waits for another until the end.  A wave brings a chunk of
 //     its slice to LDS of its own with direct-to-LDS loads (whole rows; straight to registers, as unaligned operands go, they
 //     come in pieces of 16 bytes a lane, 800 x 4096 x 1024 85 instead of 65 us), takes it apart in registers and multiplies while
 //     the next one lands.
 //   * gemm_f32_split128: 128 x 128 tiles, the slices in turn; 8 waves share the operands, which are taken apart once on their way to LDS.
-// What bounds the small tiles is the traffic of their operands (64 x 64: 9 TB/s from the L2), the large ones LDS (192 KiB a chunk) and
-// vector operations beside the matrix unit (0.77 PFLOP/s of bf16).
-// Before (fp32 unit) -> now, us, [in, out]: 64 x 256 x 1024 5.1 -> 5.0, 800 x 1024 x 1024 24.7 -> 18.5, 800 x 4096 x 1024 83 -> 58, 800 x 1024 x
-// 4096 73 -> 49, 4096 x 4096 x 1024 285 -> 220, 4096 x 4096 x 4096 1100 -> 800 (172 TFLOP/s); 8 rows pay 0.4 for the passage through LDS (8 x
-// 1024 x 1024 4.6 -> 5.0), [out, in] weights gain there (64 x 256 x 1024 6.3 -> 4.8).
+// What bounds the small tiles is taking operands apart (a lane spends 52 vector operations on its eight k of a row) and the traffic of the
+// operands, the large ones the matrix unit with vector operations and LDS (192 KiB a chunk) beside it (0.9 PFLOP/s of bf16).
+// Before (fp32 unit) -> now, us, [in, out]: 64 x 256 x 1024 5.25 -> 5.2, 800 x 1024 x 1024 22.6 -> 18.1, 800 x 4096 x 1024 81 -> 58, 800 x 1024 x
+// 4096 73 -> 55, 4096 x 1024 x 4096 308 -> 230, 4096 x 4096 x 4096 1100 -> 1000; up to 8 rows pay 0.5 at K = 1024 and 1.3 at 4096 (8 x 1024 x 1024
+// 4.7 -> 5.2), [out, in] weights gain there (8 x 1024 x 4096 14.1 -> 10.7).  The choice looks at K alone, so that a row has the same bits
+// in every call; the price of that is here.
 #pragma once
 #include "gemm_f32.hpp"
 
@@ -59,24 +62,27 @@ __device__ __forceinline__ Split split8(const float (&v)[8]) {
 // the r-th of the eight k of a chunk that a lane multiplies, from 4 lk on: four in either half of the chunk, so that four lanes read 64 bytes of a row
 __device__ __forceinline__ int split_k(int r) { return r < 4 ? r : r + 12; }
 
-// the six products that matter, small ones first; the weights are the A operand: acc[i][j][v] = token 16 i + l16, feature 4 lk + v of tile column j
+// The products of a chunk, small ones first; those of two hi parts have a sum of their own, so that its one rounding in a chunk is all that
+// large products pay.  The weights are the A operand: acc[i][j][v] = token 16 i + l16, feature 4 lk + v of tile column j
 template <int MI, int NJ, int JG>
-__device__ __forceinline__ void split_multiply(float4_t (&acc)[MI][NJ], const Split (&xs)[MI], const Split (&ws)[JG], int j0) {
-    auto product = [&](auto wpart, auto xpart) {
+__device__ __forceinline__ void split_multiply(float4_t (&acc)[MI][NJ], float4_t (&low)[MI][NJ], const Split (&xs)[MI], const Split (&ws)[JG], int j0) {
+    auto product = [&](float4_t (&sum)[MI][NJ], auto wpart, auto xpart) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
 #pragma unroll
-            for (int j = 0; j < JG; ++j) acc[i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wpart(ws[j]), xpart(xs[i]), acc[i][j0 + j], 0, 0, 0);
+            for (int j = 0; j < JG; ++j) sum[i][j0 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wpart(ws[j]), xpart(xs[i]), sum[i][j0 + j], 0, 0, 0);
     };
     auto hi = [](const Split& s) { return s.hi; };
     auto mid = [](const Split& s) { return s.mid; };
     auto lo = [](const Split& s) { return s.lo; };
-    product(lo, hi);
-    product(hi, lo);
-    product(mid, mid);
-    product(mid, hi);
-    product(hi, mid);
-    product(hi, hi);
+    product(low, lo, mid);
+    product(low, mid, lo);
+    product(low, lo, hi);
+    product(low, hi, lo);
+    product(low, mid, mid);
+    product(low, mid, hi);
+    product(low, hi, mid);
+    product(acc, hi, hi);
 }
 // the same products in the fp32 unit, for outputs that the scaled sums do not reach
 template <int MI, int NJ>
@@ -160,7 +166,7 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split(GemmArgsF32 g, i
             }
         }
     };
-    float4_t acc[MI][NJ];
+    float4_t acc[MI][NJ], low[MI][NJ];
     auto clear = [](float4_t (&sum)[MI][NJ]) {
 #pragma unroll
         for (int i = 0; i < MI; ++i)
@@ -168,6 +174,7 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split(GemmArgsF32 g, i
             for (int j = 0; j < NJ; ++j) sum[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
     };
     clear(acc);
+    clear(low);
     // all of X is taken apart, W a few tile columns at a time: registers
     constexpr int JG = MI == 4 || NJ == 1 ? 1 : 2;
     Split xs[MI];
@@ -177,7 +184,7 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split(GemmArgsF32 g, i
             Split ws[JG];
 #pragma unroll
             for (int u = 0; u < JG; ++u) ws[u] = split8(w[j + u]);
-            split_multiply<MI, NJ, JG>(acc, xs, ws, j);
+            split_multiply<MI, NJ, JG>(acc, low, xs, ws, j);
         }
     };
 
@@ -272,6 +279,10 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split(GemmArgsF32 g, i
             __builtin_amdgcn_sched_barrier(0);
         }
     }
+#pragma unroll
+    for (int i = 0; i < MI; ++i)
+#pragma unroll
+        for (int j = 0; j < NJ; ++j) acc[i][j] += low[i][j];
 
     // ---- the eight sums of an output meet, 16 token rows at a time; if one is not finite, those outputs are summed in the fp32 unit -----
     unsigned bad = 0;  // of this thread's outputs, 4 of each 16 rows
@@ -415,12 +426,12 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split128(GemmArgsF32 g
 #pragma unroll
         for (int i = 0; i < FT_MI; ++i) f.x[i] = Split{part_of(xb + i * FT_BLOCK, 0), part_of(xb + i * FT_BLOCK, 1), part_of(xb + i * FT_BLOCK, 2)};
     };
-    float4_t acc[FT_MI][FT_NJ], total[FT_MI][FT_NJ];
+    float4_t acc[FT_MI][FT_NJ], low[FT_MI][FT_NJ], total[FT_MI][FT_NJ];
 #pragma unroll
     for (int i = 0; i < FT_MI; ++i)
 #pragma unroll
         for (int j = 0; j < FT_NJ; ++j) {
-            acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+            acc[i][j] = low[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
             total[i][j] = float4_t{-0.f, -0.f, -0.f, -0.f};  // x + -0 is x
         }
     int left = part;  // chunks before the slice ends
@@ -431,8 +442,8 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split128(GemmArgsF32 g
         for (int i = 0; i < FT_MI; ++i)
 #pragma unroll
             for (int j = 0; j < FT_NJ; ++j) {
-                total[i][j] += acc[i][j];
-                acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+                total[i][j] += acc[i][j] + low[i][j];
+                acc[i][j] = low[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
             }
     };
 
@@ -449,11 +460,11 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split128(GemmArgsF32 g
         fetch(f, c & 1);
         stage(raw, (c + 1) & 1);
         gload(raw, c + 2);
-        split_multiply<FT_MI, FT_NJ, FT_NJ>(acc, f.x, f.w, 0);
+        split_multiply<FT_MI, FT_NJ, FT_NJ>(acc, low, f.x, f.w, 0);
         // the reads first, then three vector operations of the split under every matrix instruction
         __builtin_amdgcn_sched_group_barrier(0x100, 3 * (FT_MI + FT_NJ), 0);
 #pragma unroll
-        for (int m = 0; m < 6 * FT_MI * FT_NJ; ++m) {
+        for (int m = 0; m < 8 * FT_MI * FT_NJ; ++m) {
             __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
             __builtin_amdgcn_sched_group_barrier(0x002, 3, 0);
         }
@@ -464,7 +475,7 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split128(GemmArgsF32 g
     for (; c < chunks; ++c) {
         fetch(f, c & 1);
         if (c + 1 < chunks) stage(raw, (c + 1) & 1);
-        split_multiply<FT_MI, FT_NJ, FT_NJ>(acc, f.x, f.w, 0);
+        split_multiply<FT_MI, FT_NJ, FT_NJ>(acc, low, f.x, f.w, 0);
         end_chunk(c == chunks - 1);
         __syncthreads();
     }
@@ -497,7 +508,7 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split128(GemmArgsF32 g
         for (int i = 0; i < FT_MI; ++i)
 #pragma unroll
             for (int j = 0; j < FT_NJ; ++j) total[i][j] = float4_t{-0.f, -0.f, -0.f, -0.f};
-        for (c = 0; c < chunks; ++c) {  // acc is zero
+        for (c = 0; c < chunks; ++c) {  // acc and low are zero
             const int64_t k0 = (int64_t)c * FS_K + 4 * lk;
             float x[FT_MI][8], w[FT_NJ][8];
             auto row8 = [](float (&v)[8], const float* p) {

@@ -208,3 +208,27 @@ def test_tiny_elements_beside_ordinary_ones(dev, transa, M, N):
             for x, y, r in ((X, W, ref), (W.t().contiguous(), X.t().contiguous(), ref.t())):      # as token rows, and as features
                 got = _gemm(dev, transa, x, y.t().contiguous() if transa else y).double()
                 assert bool(((got - r).abs() <= 4 * EPS * r.abs() + 2.0 ** -149).all()), (e, w)
+
+
+@pytest.mark.parametrize("transa", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(256, 256, 256), (256, 512, 1024), (1024, 2048, 1024), (256, 256, 4096)])
+def test_sparse_rows(dev, transa, M, N, K):
+    """Rows of few nonzeros: no further from 64-bit sums (5 %: eight slices meet instead of four) than the same products summed in fp32 by quarters
+    of K, as the fp32 unit's kernels do, and a single one correct to a rounding (and a 16th: the small products are 2^-8 of the whole and
+    round seven times)."""
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(6)
+    for nonzeros in (1, 2, 3, 8, 32):
+        at = torch.rand(M, K, device="cuda", generator=gen).argsort(1)[:, :nonzeros].sort(1).values
+        x, W = torch.randn(M, nonzeros, device="cuda", generator=gen), torch.randn(K, N, device="cuda", generator=gen)
+        X = torch.zeros(M, K, device="cuda").scatter_(1, at, x)
+        ref, quarters = X.double() @ W.double(), torch.zeros(4, M, N, device="cuda")
+        for j in range(nonzeros):
+            product = x[:, j:j + 1].double() * W[at[:, j]].double()
+            for q in range(4):
+                quarters[q] = torch.where((at[:, j] * 4 // K == q)[:, None], (quarters[q].double() + product).float(), quarters[q])
+        fp32 = (quarters[0] + quarters[1] + quarters[2] + quarters[3]).double()
+        got = _gemm(dev, transa, X, W.t().contiguous() if transa else W).double()
+        assert float((got - ref).norm()) <= 1.05 * float((fp32 - ref).norm()), nonzeros
+        if nonzeros == 1:
+            assert bool(((got - ref).abs() <= (1 + 2.0 ** -4) * EPS * ref.abs()).all())
