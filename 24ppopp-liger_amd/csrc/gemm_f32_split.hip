@@ -7,10 +7,10 @@ namespace {
 
 struct TileSplit { int mi, nj; double alone_k, alone, shared_k, shared, ahead; };  // microseconds, for each k and besides
 // A tile on a compute unit of its own, and for each round of tiles when they are more than the compute units; `ahead`: what part of a round the
-// last one costs on top of its tiles.  Fitted to 448 problems (M 8 .. 4096, N 64 .. 4096, K 256 .. 4096, both layouts) x all tiles, within
-// 8 %; picking by it costs 0.6 % on average.  8 x 8: the 128 x 128 kernel.
-constexpr TileSplit kTilesSplit[] = {{1, 1, 0.00190, 0.07, 0.00186, 0.36, 0.37}, {1, 2, 0.00273, 0.39, 0.00267, 0.66, 0.48}, {2, 2, 0.00385, 1.01, 0.00400, 0.83, 0.58},
-                                     {2, 4, 0.00625, 1.70, 0.00746, 2.54, 0.48}, {4, 4, 0.00968, 3.01, 0.01176, 4.38, 0.46}, {8, 8, 0.04555, 2.05, 0.04189, 2.11, 1.00}};
+// last one costs on top of its tiles.  Fitted to 798 problems (M 1 .. 4096, N 64 .. 4096, K 256 .. 4096, both layouts, batches) x all tiles:
+// picking by it costs 0.4 % on average, at worst 26 %.  8 x 8: the 128 x 128 kernel.
+constexpr TileSplit kTilesSplit[] = {{1, 1, 0.00190, 0.07, 0.00186, 0.36, 0.37}, {1, 2, 0.00273, 0.39, 0.00267, 0.66, 0.48}, {2, 2, 0.00385, 1.01, 0.00396, 0.83, 0.55},
+                                     {2, 4, 0.00625, 1.70, 0.00746, 2.54, 0.48}, {4, 4, 0.01120, 2.85, 0.01252, 4.38, 0.42}, {8, 8, 0.04864, 2.05, 0.03597, 2.11, 1.00}};
 
 template <int WL>
 void launch(const TileSplit& t, bool staged, const GemmArgsF32& g, int batch, hipStream_t stream) {

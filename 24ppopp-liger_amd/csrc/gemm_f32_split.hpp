@@ -22,12 +22,13 @@
 //     come in pieces of 16 bytes a lane, 800 x 4096 x 1024 85 instead of 65 us), takes it apart in registers and multiplies while
 //     the next one lands.
 //   * gemm_f32_split128: 128 x 128 tiles, the slices in turn; 8 waves share the operands, which are taken apart once on their way to LDS.
-// What bounds the small tiles is taking operands apart (a lane spends 52 vector operations on its eight k of a row) and the traffic of the
-// operands, the large ones the matrix unit with vector operations and LDS (192 KiB a chunk) beside it (0.9 PFLOP/s of bf16).
-// Before (fp32 unit) -> now, us, [in, out]: 64 x 256 x 1024 5.25 -> 5.2, 800 x 1024 x 1024 22.6 -> 18.1, 800 x 4096 x 1024 81 -> 58, 800 x 1024 x
-// 4096 73 -> 55, 4096 x 1024 x 4096 308 -> 230, 4096 x 4096 x 4096 1100 -> 1000; up to 8 rows pay 0.5 at K = 1024 and 1.3 at 4096 (8 x 1024 x 1024
-// 4.7 -> 5.2), [out, in] weights gain there (8 x 1024 x 4096 14.1 -> 10.7).  The choice looks at K alone, so that a row has the same bits
-// in every call; the price of that is here.
+// What bounds the small tiles is taking operands apart (a lane spends 36 to 52 vector operations on its eight k of a row) and the traffic of the
+// operands, the large ones the matrix unit with vector operations and LDS (192 KiB a chunk) beside it (1.0 PFLOP/s of bf16).
+// Before (fp32 unit) -> now, us, [in, out]: 64 x 256 x 1024 5.2 -> 4.8, 800 x 1024 x 1024 22.5 -> 18.0, 800 x 4096 x 1024 81 -> 58, 800 x 1024 x
+// 4096 73 -> 56, 4096 x 1024 x 4096 306 -> 232, 4096 x 4096 x 4096 1100 -> 900 (153 TFLOP/s); up to 8 rows pay 0.4 at K = 1024 and 0.5 at 4096 (8 x
+// 1024 x 1024 4.4 -> 4.8), [out, in] weights gain there (8 x 1024 x 4096 14.1 -> 10.2).  The choice looks at K alone, so that a row has the
+// same bits in every call; those rows are the price.  Outputs summed again double the time of their tiles: 800 x 1024 x 1024 18 -> 39 with an
+// infinity in one row or in all, 4096 x 4096 x 4096 900 -> 990 and 2080.
 #pragma once
 #include "gemm_f32.hpp"
 
@@ -40,12 +41,24 @@ typedef float float2_t __attribute__((ext_vector_type(2)));
 constexpr int FS_WAVES = 8, FS_THREADS = 64 * FS_WAVES, FS_K = 32;  // k of a chunk
 constexpr float FS_SCALE = 0x1p23f, FS_UNSCALE = 0x1p-46f;
 
+// -1 as bf16 in one half of a register
+__device__ __forceinline__ unsigned minus_one(int shift) {
+    unsigned v;
+    asm("s_mov_b32 %0, %1" : "=s"(v) : "i"(0xbf80u << shift));
+    return v;
+}
+
 // 2^23 v[0..7] = hi + mid + lo, each rounded to bf16 from what the one before leaves: exact for every finite v below 2^105.
+// DOT: the rest is a two-term dot product with (-1, 0) or (0, -1), one instruction instead of two.  Tiles up to 32 x 32, whose time is the
+// splitting, gain 2-9 % by it (8 x 1024 x 4096 11.5 -> 10.7 us); the 128 x 128 one loses 18-20 %, 64 x 64 1 %.
 struct Split { bf16x8_t hi, mid, lo; };
+template <bool DOT>
 __device__ __forceinline__ Split split8(const float (&v)[8]) {
     union { bf16x8_t b; bf16x2_t p[4]; } h, m, l;
+    const bf16x2_t first = __builtin_bit_cast(bf16x2_t, minus_one(0)), second = __builtin_bit_cast(bf16x2_t, minus_one(16));
     auto rest = [&](float2_t a, bf16x2_t part) {
         const unsigned bits = __builtin_bit_cast(unsigned, part);
+        if (DOT) return float2_t{__builtin_amdgcn_fdot2_f32_bf16(part, first, a[0], false), __builtin_amdgcn_fdot2_f32_bf16(part, second, a[1], false)};
         return float2_t{a[0] - __builtin_bit_cast(float, bits << 16), a[1] - __builtin_bit_cast(float, bits & 0xffff0000u)};
     };
 #pragma unroll
@@ -177,13 +190,14 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split(GemmArgsF32 g, i
     clear(low);
     // all of X is taken apart, W a few tile columns at a time: registers
     constexpr int JG = MI == 4 || NJ == 1 ? 1 : 2;
+    constexpr bool DOT = MI * NJ <= 4;
     Split xs[MI];
     auto multiply = [&](const float (&w)[NJ][8]) {
 #pragma unroll
         for (int j = 0; j < NJ; j += JG) {
             Split ws[JG];
 #pragma unroll
-            for (int u = 0; u < JG; ++u) ws[u] = split8(w[j + u]);
+            for (int u = 0; u < JG; ++u) ws[u] = split8<DOT>(w[j + u]);
             split_multiply<MI, NJ, JG>(acc, low, xs, ws, j);
         }
     };
@@ -237,7 +251,7 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split(GemmArgsF32 g, i
             for (int i = 0; i < MI; ++i) {
                 float v[8];
                 read8(v, xl + i * 16 * FS_K);
-                xs[i] = split8(v);
+                xs[i] = split8<DOT>(v);
             }
             float w[NJ][8];
             if constexpr (WL == W_NK) {
@@ -267,7 +281,7 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split(GemmArgsF32 g, i
         load(c, (int64_t)first * FS_K);
         for (int t = 0; t < mine; ++t) {
 #pragma unroll
-            for (int i = 0; i < MI; ++i) xs[i] = split8(c.x[i]);
+            for (int i = 0; i < MI; ++i) xs[i] = split8<DOT>(c.x[i]);
             float w[NJ][8];
 #pragma unroll
             for (int j = 0; j < NJ; ++j)
@@ -406,7 +420,7 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split128(GemmArgsF32 g
         }
     };
     auto stage = [&](const Raw& raw, int buf) {
-        const Split x = split8(raw.x), w = split8(raw.w);
+        const Split x = split8<false>(raw.x), w = split8<false>(raw.w);
         char* const xd = xdst + buf * FT_CHUNK;
         char* const wd = wdst + buf * FT_CHUNK;
         *reinterpret_cast<bf16x8_t*>(xd) = x.hi;
