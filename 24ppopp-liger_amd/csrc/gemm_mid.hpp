@@ -81,13 +81,27 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
     // row fastest, so the workgroups that share a weight panel run next to each other on one XCD and fetch it from memory once.
     int tm, tn, split;
     if (region) {
-        // Many rows of 256-row tiles: the workgroups of a round (one per compute unit, P on each XCD) cover RM x RN tiles, as near to a square as the
-        // tile counts allow, and each XCD 4 x P / 4 of them: a round reads 32 operand panels and an XCD 12 of them, where the run above
-        // makes it 18 (16 rows of tiles).  Fills cost power, which is what bounds these: 4096 rows x 12288 x 16384 1187 -> 1134 us
+        // Many rows of tall tiles: the workgroups of a round (one per compute unit, P on each XCD) cover RM x RN tiles, as near to a square as the
+        // tile counts allow, and each XCD 4 x P / 4 of them: a round reads 32 operand panels and an XCD 12 of them, where the run below
+        // makes it 18 (16 rows of tiles).  Fills cost power, which is what bounds these: 4096 rows x 12288 x 16384 1187 -> 1134 us.
+        // RM = 4: any number of blocks of 4 x P / 4 tiles one after the other, from top to bottom; the last round may lack some, and its
+        // workgroups have nothing to do (5120 rows x 12288 x 16384 [out, in] 1851 -> 1527 us, 16384 x 12288 1489 -> 1442, 3072 x 12288 x 16384
+        // 958 -> 911; blocks from left to right, which make a round read all of W's panels: 1612, 1527, 935).
         const int P = region >> 8, RM = region & 255, pw = P >> 2, RN = 8 * P / RM, xcols = RN / pw;
-        const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, round = slot / P, in = slot % P, regions_n = tiles_n / RN;
-        tm = (round / regions_n) * RM + (xcd / xcols) * 4 + (in & 3);
-        tn = (round % regions_n) * RN + (xcd % xcols) * pw + (in >> 2);
+        const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3, round = slot / P, in = slot % P;
+        int bm, bn;  // the block, in units of 4 and pw tiles
+        if (RM > 4) {
+            const int regions_n = tiles_n / RN;
+            bm = round / regions_n * (RM / 4) + xcd / xcols;
+            bn = round % regions_n * xcols + xcd % xcols;
+        } else {
+            const int block = round * 8 + xcd, blocks_m = tiles_m >> 2;
+            bm = block % blocks_m;
+            bn = block / blocks_m;
+        }
+        tm = bm * 4 + (in & 3);
+        tn = bn * pw + (in >> 2);
+        if (tn >= tiles_n) return;
         split = 0;
     } else {
         const int total = gridDim.x, q = total >> 3, r = total & 7;
@@ -528,13 +542,21 @@ static void launch_mid_tile(const GemmArgs& g, const GemmGroup& grp, const RowMa
     // set once per instantiation; the initialisation of a function-local static is thread-safe
     static const hipError_t attr_rc = hipFuncSetAttribute((const void*)gemm_f16_mid<WL, MI, NJ, XS, WS, ORDER, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     (void)attr_rc;
+    // Tiles of 160 to 224 rows are placed where they make more than one round (2560 rows x 12288 x 16384 822 -> 788 us, 5120 x 4096 x 4096 152 ->
+    // 142); in one round it gains nothing (1280 x 8192 x 2048 41 -> 41.5), and smaller tiles lose by it.
     int region = 0;
+    int64_t blocks = (int64_t)tiles_m * tiles_n * l.nsplit;
     const int P = l.si.cus >> 3, pw = P >> 2;
-    if (MI == 8 && l.nsplit == 1 && pw >= 1 && P % 4 == 0) {
-        region = tiles_m % 16 == 0 && tiles_n % (2 * pw) == 0 ? 16 : tiles_m % 8 == 0 && tiles_n % (4 * pw) == 0 ? 8 : 0;
+    if ((MI == 8 || (MI >= 5 && blocks > 8 * P)) && l.nsplit == 1 && pw >= 1 && P % 4 == 0) {
+        if (tiles_m % 16 == 0 && tiles_n % (2 * pw) == 0) region = 16;
+        else if (tiles_m % 8 == 0 && tiles_n % (4 * pw) == 0) region = 8;
+        else if (tiles_m % 4 == 0 && tiles_n % pw == 0) {
+            region = 4;
+            blocks = (blocks + 8 * P - 1) / (8 * P) * (8 * P);
+        }
         if (region) region |= P << 8;
     }
-    hipLaunchKernelGGL((gemm_f16_mid<WL, MI, NJ, XS, WS, ORDER, NT>), dim3(tiles_m * tiles_n * l.nsplit), dim3(MID_THREADS), smem, l.stream, g, grp, rm, tiles_m, tiles_n,
+    hipLaunchKernelGGL((gemm_f16_mid<WL, MI, NJ, XS, WS, ORDER, NT>), dim3((unsigned)blocks), dim3(MID_THREADS), smem, l.stream, g, grp, rm, tiles_m, tiles_n,
                        l.si.ws, l.si.arrivals, l.nsplit, l.kt_per_split, l.turn, wide, region);
 }
 

@@ -240,3 +240,31 @@ def test_on_a_stream_with_half_of_the_compute_units(dev, po):
                 assert np.array_equal(got[0], dev.down(whole))
     finally:
         assert dev.lib.lg_stream_destroy(s) == 0
+
+
+# 256-row tiles in rounds of 16, 8 and 4 rows of tiles, a last round that is not whole and no rounds; lower tiles in more than one round
+@pytest.mark.parametrize("layout", [0, 1, 2])
+@pytest.mark.parametrize("M,N", [(4000, 2048), (2048, 4096), (1024, 8192), (5000, 6144), (5000, 3072), (2500, 8192), (1536, 12288)])
+def test_placement_on_the_xcds(dev, layout, M, N):
+    """Every tile is computed, whichever workgroups do it: on the whole chip and on a stream with half of it, whose rounds are half as large."""
+    K = 192
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(8)
+    X, W = torch.randn(M, K, device="cuda", generator=gen).half(), (0.05 * torch.randn(K, N, device="cuda", generator=gen)).half()
+    ref, w, ld = X.float() @ W.float(), W, N
+    if layout:
+        w, ld = W.t().contiguous(), K
+    if layout == TILED:
+        plain, w = w, torch.empty_like(w)
+        dev.call("lg_weight_tile_f16", w, plain, N, K, 1, K)
+    s, ys = C.c_void_p(), [torch.full((M, N), 7e4, device="cuda", dtype=torch.float32).half() for _ in range(2)]
+    assert dev.lib.lg_stream_create_cu_mask(C.byref(s), (C.c_uint * 8)(*[0xFFFFFFFF] * 4 + [0] * 4), 8) == 0, dev.capi.last_error()
+    try:
+        dev.sync()
+        for y, stream in zip(ys, (C.c_void_p(dev.stream), s)):
+            assert dev.lib.lg_gemm_f16(layout, 0, N, M, K, w.data_ptr(), ld, X.data_ptr(), K, y.data_ptr(), N, stream) == 0
+            dev.sync()
+            assert float((y.float() - ref).abs().max()) < 2e-3 * float(ref.abs().max())
+    finally:
+        assert dev.lib.lg_stream_destroy(s) == 0
+    assert torch.equal(*ys)
