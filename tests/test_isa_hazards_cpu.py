@@ -16,7 +16,7 @@ import pytest
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 PKG = os.path.join(ROOT, "24ppopp-liger_amd")
-SOURCES = ["gemm_fast.hip", "gemm_skinny_kn.hip", "attention_prefill.hip", "ceilings.hip"]   # every file that issues LDS reads by hand
+SOURCES = ["gemm_fast.hip", "gemm_skinny_kn.hip", "attention_prefill.hip", "ceilings.hip"]   # those of gemm_mid.hpp: tests/test_isa_hazards_mid_cpu.py
 
 
 def _build_recipe():
