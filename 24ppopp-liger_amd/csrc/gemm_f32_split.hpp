@@ -27,7 +27,8 @@
 // Before (fp32 unit) -> now, us, [in, out]: 64 x 256 x 1024 5.2 -> 4.8, 800 x 1024 x 1024 22.5 -> 18.0, 800 x 4096 x 1024 81 -> 58, 800 x 1024 x
 // 4096 73 -> 56, 4096 x 1024 x 4096 306 -> 232, 4096 x 4096 x 4096 1100 -> 900 (153 TFLOP/s); up to 8 rows pay 0.4 at K = 1024 and 0.5 at 4096 (8 x
 // 1024 x 1024 4.4 -> 4.8), [out, in] weights gain there (8 x 1024 x 4096 14.1 -> 10.2).  The choice looks at K alone, so that a row has the
-// same bits in every call; those rows are the price.  Outputs summed again double the time of their tiles: 800 x 1024 x 1024 18 -> 39 with an
+// same bits in every call; those rows are the price, and unaligned operands of up to 333 rows (800 x 1024 x 1024 22.7 -> 20.2, but 64 x 1024 x 1024 5.6 ->
+// 6.4, 200 x 1024 x 256 4.7 -> 5.6).  Outputs summed again double the time of their tiles: 800 x 1024 x 1024 18 -> 39 with an
 // infinity in one row or in all, 4096 x 4096 x 4096 900 -> 990 and 2080.
 #pragma once
 #include "gemm_f32.hpp"
@@ -274,6 +275,17 @@ __global__ __launch_bounds__(FS_THREADS, 2) void gemm_f32_split(GemmArgsF32 g, i
             __builtin_amdgcn_sched_barrier(0);
             if (t + 1 < mine) fetch(first + t + 1);
             multiply(w);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    } else if constexpr (MI == 4) {
+        // its sums leave no registers for a chunk on its way: the other wave of the SIMD multiplies meanwhile (800 x 1024 x 1024 20.2 us, in tiles of
+        // 32 x 64 30.7)
+        for (int t = 0; t < mine; ++t) {
+            Chunk c;
+            load(c, (int64_t)(first + t) * FS_K);
+#pragma unroll
+            for (int i = 0; i < MI; ++i) xs[i] = split8<DOT>(c.x[i]);
+            multiply(c.w);
             __builtin_amdgcn_sched_barrier(0);
         }
     } else if (mine > 0) {

@@ -191,6 +191,24 @@ def test_bits_of_an_output_depend_on_its_row_and_column_alone(dev, transa, M, N,
     assert _same(_gemm(dev, transa, bad, col, 10, 30, 0, 17), got[10:40, :17])
 
 
+# every tile of operands that go through registers: 16 x 16 up to 128 x 128, with and without rows and features beyond the matrix
+@pytest.mark.parametrize("transa", [0, 1])
+@pytest.mark.parametrize("M,N,K", [(8, 72, 256), (64, 1000, 288), (200, 1030, 256), (333, 1024, 1024), (801, 1030, 512), (800, 1024, 1024), (1100, 1026, 1024),
+                                   (3000, 2048, 288)])
+def test_unaligned_rows_have_the_bits_of_aligned_ones(dev, transa, M, N, K):
+    _, X, W = _case(dev, transa, M, N, K, pad=1, shift=1)
+    odd = torch.empty(M, N, device="cuda")
+    dev.call("lg_gemm_f32", transa, 0, N, M, K, W.data_ptr(), W.stride(1), X.data_ptr(), X.stride(1), odd.data_ptr(), N)
+    pad = -W.shape[2] % 4
+    aligned = torch.zeros(W.shape[1], W.shape[2] + pad, device="cuda")
+    aligned[:, :W.shape[2]] = W[0]
+    Y, x = torch.empty(M, N + -N % 4, device="cuda"), X[0].contiguous()
+    torch.cuda.synchronize()
+    dev.call("lg_gemm_f32", transa, 0, N, M, K, aligned.data_ptr(), aligned.shape[1], x.data_ptr(), K, Y.data_ptr(), Y.shape[1])
+    dev.sync()
+    assert torch.equal(odd, Y[:, :N])
+
+
 @pytest.mark.parametrize("transa", [0, 1])
 @pytest.mark.parametrize("M,N", [(48, 80), (1100, 2048)])
 def test_tiny_elements_beside_ordinary_ones(dev, transa, M, N):
