@@ -526,13 +526,15 @@ constexpr int mid_ws(int mi, int nj) { return mid_depth(mi, nj) > 2 ? mid_depth(
 // Against all loads under the second k-step, over the problems that a tile is good for: in pairs 0.89 (6 x 4), 0.91 (4 x 3, 8 x 4), 0.95 (3 x 4,
 // 4 x 4), 0.97-1.0 (the others of depth 4 and 6: bound by memory, or by few workgroups); at depth 3 spread 0.89-0.99, in pairs up to 1.05.
 // 1 x 4 with weights contiguous along k, from two rows of tiles on: in pairs 1.00-1.04, spread 1.00-1.05 ([in, out]: in pairs 0.93-1.0).
+// 4 x 6 with weights [in, out] above 256 rows: in pairs 1.00-1.07 (978 rows x 6144 x 12288 146 -> 156 us, 1968 x 9216 x 12288 433 -> 461), spread 0.99-1.05;
+// up to 256 rows, with its K-slices, in pairs 0.95-0.98.
 constexpr int mid_order(int wl, int mi, int nj) {
     return mi == 1 && nj == 4 && wl != W_KN ? MID_BURST : mid_depth(mi, nj) > 3 || nj == 4 ? MID_PAIRS : MID_SPREAD;
 }
 
-template <int WL, int MI, int NJ, bool NT>
-static void launch_mid_tile(const GemmArgs& g, const GemmGroup& grp, const RowMap& rm, const MidLaunch& l) {
-    constexpr int XS = mid_xs(MI, NJ), WS = mid_ws(MI, NJ), ORDER = mid_order(WL, MI, NJ);
+template <int WL, int MI, int NJ, int ORDER, bool NT>
+static void launch_mid_order(const GemmArgs& g, const GemmGroup& grp, const RowMap& rm, const MidLaunch& l) {
+    constexpr int XS = mid_xs(MI, NJ), WS = mid_ws(MI, NJ);
     const int tiles_m = (g.M + 32 * MI - 1) / (32 * MI), tiles_n = g.N / (32 * NJ) * grp.count;
     constexpr size_t ring = (size_t)(XS * MI + WS * NJ) * 32 * MID_K * sizeof(half_t), tile = (size_t)(32 * MI) * (32 * NJ + 8) * sizeof(half_t);
     constexpr size_t smem = ring > tile ? ring : tile;
@@ -560,6 +562,13 @@ static void launch_mid_tile(const GemmArgs& g, const GemmGroup& grp, const RowMa
     }
     hipLaunchKernelGGL((gemm_f16_mid<WL, MI, NJ, XS, WS, ORDER, NT>), dim3((unsigned)blocks), dim3(MID_THREADS), smem, l.stream, g, grp, rm, tiles_m, tiles_n,
                        l.si.ws, l.si.arrivals, l.nsplit, l.kt_per_split, l.turn, wide, region);
+}
+
+template <int WL, int MI, int NJ, bool NT>
+static void launch_mid_tile(const GemmArgs& g, const GemmGroup& grp, const RowMap& rm, const MidLaunch& l) {
+    if constexpr (WL == W_KN && MI == 4 && NJ == 6 && !NT)
+        if (g.M >= kSequentialRows) return launch_mid_order<WL, MI, NJ, MID_BURST, NT>(g, grp, rm, l);
+    launch_mid_order<WL, MI, NJ, mid_order(WL, MI, NJ), NT>(g, grp, rm, l);
 }
 
 // one instantiation per tile height MI of a list, with and without the non-temporal hint

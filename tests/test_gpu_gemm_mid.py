@@ -268,3 +268,20 @@ def test_placement_on_the_xcds(dev, layout, M, N):
     finally:
         assert dev.lib.lg_stream_destroy(s) == 0
     assert torch.equal(*ys)
+
+
+# 128 x 192 tiles with weights [in, out] above 256 rows have an order of the loads of their own: fewer k-tiles than a ring is deep, as many and more
+@pytest.mark.parametrize("M,N", [(389, 12288), (512, 12288), (978, 6144)])
+def test_128_x_192_tiles_of_in_out_weights(dev, M, N):
+    gen = torch.Generator(device="cuda")
+    gen.manual_seed(9)
+    for K in (64, 128, 192, 256, 320, 384, 576, 1088):
+        X, W = torch.randn(M, K, device="cuda", generator=gen).half(), (0.05 * torch.randn(K, N, device="cuda", generator=gen)).half()
+        t, Y = W.t().contiguous(), [torch.full((M, N), 7e4, device="cuda", dtype=torch.float32).half() for _ in range(2)]
+        torch.cuda.synchronize()
+        dev.call("lg_gemm_f16", 0, 0, N, M, K, W.data_ptr(), N, X.data_ptr(), K, Y[0].data_ptr(), N)
+        dev.call("lg_gemm_f16", 1, 0, N, M, K, t.data_ptr(), K, X.data_ptr(), K, Y[1].data_ptr(), N)
+        dev.sync()
+        ref = X.float() @ W.float()
+        assert float((Y[0].float() - ref).abs().max()) < 2e-3 * float(ref.abs().max())
+        assert torch.equal(*Y)
