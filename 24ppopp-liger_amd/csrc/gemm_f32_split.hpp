@@ -25,11 +25,11 @@
 // What bounds the small tiles is taking operands apart (a lane spends 36 to 52 vector operations on its eight k of a row) and the traffic of the
 // operands, the large ones the matrix unit with vector operations and LDS (192 KiB a chunk) beside it (1.0 PFLOP/s of bf16).
 // Before (fp32 unit) -> now, us, [in, out]: 64 x 256 x 1024 5.2 -> 4.8, 800 x 1024 x 1024 22.5 -> 18.0, 800 x 4096 x 1024 81 -> 58, 800 x 1024 x
-// 4096 73 -> 56, 4096 x 1024 x 4096 306 -> 232, 4096 x 4096 x 4096 1100 -> 900 (153 TFLOP/s); up to 8 rows pay 0.4 at K = 1024 and 0.5 at 4096 (8 x
-// 1024 x 1024 4.4 -> 4.8), [out, in] weights gain there (8 x 1024 x 4096 14.1 -> 10.2).  The choice looks at K alone, so that a row has the
-// same bits in every call; those rows are the price, and unaligned operands of up to 333 rows (800 x 1024 x 1024 22.7 -> 20.2, but 64 x 1024 x 1024 5.6 ->
-// 6.4, 200 x 1024 x 256 4.7 -> 5.6).  Outputs summed again double the time of their tiles: 800 x 1024 x 1024 18 -> 39 with an
-// infinity in one row or in all, 4096 x 4096 x 4096 900 -> 990 and 2080.
+// 4096 73 -> 56, 4096 x 1024 x 4096 306 -> 228, 4096 x 4096 x 4096 1150 -> 960 ([out, in] 920: 150 TFLOP/s); up to 8 rows pay 0.4 at K = 1024 and 0.5
+// at 4096 (8 x 1024 x 1024 4.4 -> 4.8), [out, in] weights gain there (8 x 1024 x 4096 14.1 -> 10.2).  The choice looks at K alone, so that a row
+// has the same bits in every call; those rows are the price, and some unaligned operands with few tiles (800 x 1024 x 1024 22.7 -> 20.2, but
+// 64 x 1024 x 1024 5.6 -> 6.4, 200 x 1024 x 256 4.7 -> 5.6).  Outputs summed again double the time of their tiles: 800 x 1024 x 1024 18 -> 39
+// with an infinity in one row or in all, 4096 x 4096 x 4096 900 -> 990 and 2080 (on a faster box).
 #pragma once
 #include "gemm_f32.hpp"
 
