@@ -29,7 +29,7 @@
 // at 4096 (8 x 1024 x 1024 4.4 -> 4.8), [out, in] weights gain there (8 x 1024 x 4096 14.1 -> 10.2).  The choice looks at K alone, so that a row
 // has the same bits in every call; those rows are the price, and some unaligned operands with few tiles (800 x 1024 x 1024 22.7 -> 20.2, but
 // 64 x 1024 x 1024 5.6 -> 6.4, 200 x 1024 x 256 4.7 -> 5.6).  Outputs summed again double the time of their tiles: 800 x 1024 x 1024 18 -> 39
-// with an infinity in one row or in all, 4096 x 4096 x 4096 900 -> 990 and 2080 (on a faster box).
+// with an infinity in one row or in all, 4096 x 4096 x 4096 900 -> 990 and 2080 (another card).
 #pragma once
 #include "gemm_f32.hpp"
 
