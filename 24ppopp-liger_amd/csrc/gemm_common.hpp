@@ -50,7 +50,7 @@ struct GemmArgs {
 };
 
 // Up to three problems that share X and the shape and differ in weight, bias and destination (the Q, K and V projections of a
-// decode step): the weight-streaming kernels run them as one launch, blockIdx.y selecting the problem.
+// decode step): one launch computes them all.
 constexpr int LG_MAX_GROUP = 3;
 struct GemmGroup {
     int count;  // 1 = plain launch (the GemmArgs' own W / Y / bias / ldy are used)
@@ -60,16 +60,6 @@ struct GemmGroup {
     int64_t ldy[LG_MAX_GROUP];
     int rows[LG_MAX_GROUP];  // LG_EPI_BIAS_HEADS_ROWS: whether the member's token rows follow the RowMap
 };
-__device__ __forceinline__ void select_group(GemmArgs& g, const GemmGroup& grp) {
-    if (grp.count > 1) {
-        const int gi = blockIdx.y;
-        g.W = grp.W[gi];
-        g.Y = grp.Y[gi];
-        g.epi.bias = grp.bias[gi];
-        g.ldy = grp.ldy[gi];
-        g.epi.rows = grp.rows[gi];
-    }
-}
 
 // host side: a plain launch seen as a group of one
 inline GemmGroup single_group(const GemmArgs& g) {
@@ -180,6 +170,22 @@ __device__ __forceinline__ int swz_a(int row, int c) { return c ^ ((row >> 1) & 
 // the 32 lanes served together by one transposed read touch rows k0..k0+3 and k0+8..k0+11: eight distinct XOR values
 __device__ __forceinline__ int swz_b(int k, int blk) { return blk ^ ((k & 3) | ((k >> 1) & 4)); }
 
+// Where an epilogue puts column n of token row m, in elements.
+template <int EPI>
+__device__ __forceinline__ int64_t output_offset(const Epilogue& epi, int64_t ldy, int mapped, int m, int n, const RowMap* rm) {
+    if (EPI == LG_EPI_BIAS_HEADS_ROWS) {
+        // one token per sequence: row m -> [slot, head, pos, e] with ldy rows reserved per (slot, head)
+        const int b = mapped ? rm->slot[m] : m, s = mapped ? rm->pos[m] : 0;
+        return (((int64_t)b * epi.heads_total + n / epi.d) * ldy + s) * (int64_t)epi.d + n % epi.d;
+    }
+    if (EPI == LG_EPI_BIAS_HEADS) {
+        // [M = b*seq + s, N = head*d + e]  ->  [b, head, s, e] with ldy rows reserved per (b, head)
+        const int b = m / epi.seq, s = m % epi.seq;
+        return (((int64_t)b * epi.heads_total + n / epi.d) * ldy + s) * (int64_t)epi.d + n % epi.d;
+    }
+    return (int64_t)m * ldy + n;
+}
+
 // Applies the epilogue to 4 consecutive output columns n..n+3 of token row m and stores them.
 template <int EPI>
 __device__ __forceinline__ void epilogue_store4(const GemmArgs& g, half_t* Yb, int m, int n, float4_t acc, bool vec_ok,
@@ -195,20 +201,7 @@ __device__ __forceinline__ void epilogue_store4(const GemmArgs& g, half_t* Yb, i
 #pragma unroll
         for (int r = 0; r < 4; ++r) v[r] = gelu_tanh(v[r]);
     }
-    int64_t base;
-    if (EPI == LG_EPI_BIAS_HEADS_ROWS) {
-        // one token per sequence: row m -> [slot, head, pos, e] with ldy rows reserved per (slot, head)
-        const int b = g.epi.rows ? rm->slot[m] : m, s = g.epi.rows ? rm->pos[m] : 0;
-        const int head = n / g.epi.d, e = n % g.epi.d;
-        base = (((int64_t)b * g.epi.heads_total + head) * g.ldy + s) * (int64_t)g.epi.d + e;
-    } else if (EPI == LG_EPI_BIAS_HEADS) {
-        // [M = b*seq + s, N = head*d + e]  ->  [b, head, s, e] with ldy rows reserved per (b, head)
-        const int b = m / g.epi.seq, s = m % g.epi.seq;
-        const int head = n / g.epi.d, e = n % g.epi.d;
-        base = (((int64_t)b * g.epi.heads_total + head) * g.ldy + s) * (int64_t)g.epi.d + e;  // n..n+3 stay inside one head (d % 4 == 0)
-    } else {
-        base = (int64_t)m * g.ldy + n;
-    }
+    const int64_t base = output_offset<EPI>(g.epi, g.ldy, g.epi.rows, m, n, rm);  // n..n+3 stay inside one head (d % 4 == 0)
     if (vec_ok && n + 3 < g.N) {
         half4_t o = {(half_t)v[0], (half_t)v[1], (half_t)v[2], (half_t)v[3]};
         *reinterpret_cast<half4u_t*>(Yb + base) = o;

@@ -3,24 +3,31 @@
 //   Y[M, N] = X[M, K] * W^T with W stored [N, K], M <= 4.
 // Every weight byte is used for 2*M flops, so the kernel is nothing but an HBM stream of W with the arithmetic on the
 // vector ALUs (v_dot2_f32_f16); what matters is how the stream is issued:
-//   * a wave owns 4 consecutive output features and walks their weight rows along k: one wave instruction reads 1 KiB of
-//     ONE row (64 lanes x 16 bytes, fully contiguous), 16 such loads (4 rows x 4 k-steps) are kept in flight per lane in a
-//     rolling pipeline (a fragment's registers are reloaded as soon as it has been multiplied);
-//   * a block (4 waves = 16 features) covers the whole of K, so there are no K-slices, no fp32 partials and no second
-//     kernel: lanes accumulate in fp32, one butterfly sum per output at the end, epilogue (bias / GELU / head-transposed
-//     store) applied in place;
-//   * the M token rows are staged once per block in LDS (M * K * 2 bytes) and shared by the 4 weight rows of every wave;
-//     the first weight loads are issued before that staging so that the stream starts at once.
-// Each output is one fixed-order fp32 sum (per-lane partial sums over k in an order fixed by the output's position, then a
-// butterfly), independent of the other token rows.
+//   * one block per compute unit, which stays until the end; its waves (8 where that deals the features evenly) own a feature at a
+//     time and walk its weight row from one end to the other, 4 KiB at a time, and then the row of the next feature: a wave is one
+//     sequential stream, and a compute unit has 8 x 4 KiB on their way, which is all it can have;
+//   * the loads are marked non-temporal where the weights are more than the caches keep;
+//   * a feature's row is summed by one wave, so there are no K-slices, no fp32 partials and no second kernel: lanes accumulate in
+//     fp32, one butterfly sum per output at the end, epilogue (bias / GELU / head-transposed store) applied in place.  The loads of
+//     the next feature are on their way by then;
+//   * the M token rows are staged once per block in LDS (M * K * 2 bytes); the first weight loads are issued before that.
+// Blocks of 4 waves that each walked 4 rows side by side, as many as the features made, left HBM pages after every KiB and drained at
+// every change of blocks: with weights cycled through memory, in microseconds,
+// 16384 x 12288 68.3 -> 60.7 (6.63 TB/s), 12288 x 6144 27.0 -> 25.1, 4096 x 4096 9.8 -> 8.5, 1024 x 4096 6.4 -> 4.7; at 4 token rows 12288 x 16384
+// 72.5 -> 63.8 (in gemm_skinny.hip before, as the rows did not fit the LDS share of one block of several), 4096 x 4096 13.5 -> 10.2.
+// Each output is one fixed-order fp32 sum (per-lane partial sums over k in an order fixed by the feature, then a butterfly),
+// independent of the other token rows and of the other members of a group.
+#include <limits.h>
+#include <stdlib.h>
+
 #include "gemm_common.hpp"
 
 namespace lg {
 
-constexpr int GV_ROWS = 4;          // weight rows (output features) per wave
-constexpr int GV_U = 4;             // k-steps in flight per row
-constexpr int GV_KSTEP = 512;       // halves per wave instruction and row (64 lanes x 8)
-constexpr int GV_MAX_LDS = 65536;   // bytes of staged X per block
+constexpr int GV_U = 4;             // k-steps in flight
+constexpr int GV_KSTEP = 512;       // halves per wave instruction (64 lanes x 8)
+constexpr int GV_MAX_WAVES = 12;
+constexpr int GV_MAX_LDS = 160 * 1024;   // bytes of staged X per block
 
 __device__ __forceinline__ float dot8(half8_t w, half8_t x, float acc) {
 #pragma unroll
@@ -29,74 +36,79 @@ __device__ __forceinline__ float dot8(half8_t w, half8_t x, float acc) {
     return acc;
 }
 
-// MR = staged token rows (1, 2 or 4; rows >= M are zero)
-template <int MR, int EPI>
-__global__ __launch_bounds__(256) void gemv_nk_kernel(GemmArgs g, GemmGroup members, RowMap rm) {
+// MR = staged token rows (1, 2 or 4; rows >= M are zero); the members' features follow each other
+template <int MR, int EPI, bool NT>
+__global__ __launch_bounds__(GV_MAX_WAVES * 64) void gemv_nk_kernel(GemmArgs g, GemmGroup members, RowMap rm) {
     extern __shared__ __attribute__((aligned(16))) half_t xs[];  // [MR][K]
-    select_group(g, members);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    const int n0 = (blockIdx.x * 4 + wave) * GV_ROWS;
-    const int K = g.K;
-    const int ksteps = K / GV_KSTEP;  // the launcher guarantees K % (GV_KSTEP * GV_U) == 0
+    const int tid = threadIdx.x, lane = tid & 63, threads = blockDim.x;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int K = g.K, features = g.N * members.count, step = gridDim.x * (threads >> 6);
+    const int groups = K / (GV_KSTEP * GV_U);  // the launcher guarantees whole groups
+    auto load = [](const half_t* p) {
+        const half8_t* v = reinterpret_cast<const half8_t*>(p);
+        return NT ? __builtin_nontemporal_load(v) : *v;
+    };
+    // the weight row of a feature (those beyond the last are read as the last and never stored), and the group its walk starts at: with
+    // a power-of-two row pitch (K = 16384) rows walked in phase would hit the same memory channels at the same time
+    auto row_of = [&](int f) {
+        const int c = min(f, features - 1), member = c / g.N;
+        return (members.count > 1 ? members.W[member] : g.W) + (int64_t)(c - member * g.N) * g.ldw + lane * 8;
+    };
+    auto start_of = [&](int f) { return f % g.N % groups; };
 
-    // weight rows of this wave (rows beyond N are clamped and never stored)
-    const half_t* wrow[GV_ROWS];
+    int f = blockIdx.x * (threads >> 6) + wave;
+    const half_t* row = row_of(f);
+    int grp = start_of(f);
+    half8_t wv[GV_U];  // the stream starts before X is staged
 #pragma unroll
-    for (int r = 0; r < GV_ROWS; ++r) wrow[r] = g.W + (int64_t)min(n0 + r, g.N - 1) * g.ldw + lane * 8;
+    for (int u = 0; u < GV_U; ++u) wv[u] = load(row + (int64_t)(grp * GV_U + u) * GV_KSTEP);
 
-    // Every wave walks k in groups of GV_U k-steps, starting at its own group and wrapping around: with a power-of-two row
-    // pitch (K = 16384) rows that are walked in phase would all hit the same memory channels at the same time.
-    const int groups = ksteps / GV_U;
-    int grp = (blockIdx.x * 4 + wave) % groups;
-
-    // the stream starts before X is staged
-    half8_t wv[GV_U][GV_ROWS];
-#pragma unroll
-    for (int u = 0; u < GV_U; ++u)
-#pragma unroll
-        for (int r = 0; r < GV_ROWS; ++r) wv[u][r] = *reinterpret_cast<const half8_t*>(wrow[r] + (int64_t)(grp * GV_U + u) * GV_KSTEP);
-
-    for (int v = tid; v < MR * (K / 8); v += 256) {
-        const int row = v / (K / 8), c = v % (K / 8);
+    for (int v = tid; v < MR * (K / 8); v += threads) {
+        const int r = v / (K / 8), c = v % (K / 8);
         half8_t val = half8_t{0, 0, 0, 0, 0, 0, 0, 0};
-        if (row < g.M) val = *reinterpret_cast<const half8_t*>(g.X + (int64_t)row * g.ldx + c * 8);
-        *reinterpret_cast<half8_t*>(&xs[row * K + c * 8]) = val;
+        if (r < g.M) val = *reinterpret_cast<const half8_t*>(g.X + (int64_t)r * g.ldx + c * 8);
+        *reinterpret_cast<half8_t*>(&xs[r * K + c * 8]) = val;
     }
     __syncthreads();
 
-    float acc[GV_ROWS][MR];
+    for (; f < features; f += step) {
+        const int member = f / g.N, n = f - member * g.N;
+        const half_t* bias = members.count > 1 ? members.bias[member] : g.epi.bias;
+        const float b = EPI == LG_EPI_NONE ? 0.f : (float)bias[n];  // on its way before it is needed
+        float acc[MR];
 #pragma unroll
-    for (int r = 0; r < GV_ROWS; ++r)
+        for (int m = 0; m < MR; ++m) acc[m] = 0.f;
+        for (int it = 0; it < groups; ++it) {
+            const int cur = grp;
+            if (it + 1 < groups) {
+                grp = grp + 1 == groups ? 0 : grp + 1;
+            } else {
+                row = row_of(f + step);
+                grp = start_of(f + step);
+            }
 #pragma unroll
-        for (int m = 0; m < MR; ++m) acc[r][m] = 0.f;
-
-    for (int it = 0; it < groups; ++it) {
-        // the group after the last one is the last one again: every load is unconditional
-        const int next = (it + 1 < groups) ? (grp + 1 == groups ? 0 : grp + 1) : grp;
+            for (int u = 0; u < GV_U; ++u) {
 #pragma unroll
-        for (int u = 0; u < GV_U; ++u) {
-            half8_t xv[MR];
-#pragma unroll
-            for (int m = 0; m < MR; ++m) xv[m] = *reinterpret_cast<const half8_t*>(&xs[m * K + (grp * GV_U + u) * GV_KSTEP + lane * 8]);
-#pragma unroll
-            for (int r = 0; r < GV_ROWS; ++r) {
-#pragma unroll
-                for (int m = 0; m < MR; ++m) acc[r][m] = dot8(wv[u][r], xv[m], acc[r][m]);
-                wv[u][r] = *reinterpret_cast<const half8_t*>(wrow[r] + (int64_t)(next * GV_U + u) * GV_KSTEP);
+                for (int m = 0; m < MR; ++m)
+                    acc[m] = dot8(wv[u], *reinterpret_cast<const half8_t*>(&xs[m * K + (cur * GV_U + u) * GV_KSTEP + lane * 8]), acc[m]);
+                wv[u] = load(row + (int64_t)(grp * GV_U + u) * GV_KSTEP);
+                asm volatile("" ::: "memory");  // the load stays where it is written: the others are on their way beside it
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
-        grp = next;
-    }
-
+        float v = 0.f;
 #pragma unroll
-    for (int m = 0; m < MR; ++m) {
-#pragma unroll
-        for (int q = 0; q < GV_ROWS / 4; ++q) {
-            float4_t out;
-#pragma unroll
-            for (int r = 0; r < 4; ++r) out[r] = wave_sum(acc[q * 4 + r][m]);
-            if (lane == 0 && m < g.M) epilogue_store4<EPI>(g, g.Y, m, n0 + q * 4, out, true, &rm);
+        for (int m = 0; m < MR; ++m) {
+            const float s = wave_sum(acc[m]);
+            v = lane == m ? s : v;
         }
+        if (lane >= g.M) continue;
+        if (EPI != LG_EPI_NONE) v += b;
+        if (EPI == LG_EPI_BIAS_GELU) v = gelu_tanh(v);
+        half_t* const Y = members.count > 1 ? members.Y[member] : g.Y;
+        const int64_t ldy = members.count > 1 ? members.ldy[member] : g.ldy;
+        const int mapped = members.count > 1 ? members.rows[member] : g.epi.rows;
+        Y[output_offset<EPI>(g.epi, ldy, mapped, lane, n, &rm)] = (half_t)v;
     }
 }
 
@@ -112,13 +124,29 @@ int launch_gemv_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows,
     if (g.epi.kind == LG_EPI_BIAS_GEGLU) return LG_OK;  // pairs features 16 apart: left to the tile kernels
     *handled = true;
     const RowMap rm = rows ? *rows : RowMap{};
-    const dim3 grid((g.N + 4 * GV_ROWS - 1) / (4 * GV_ROWS), grp.count), block(256);
-#define LG_GV(MR_, E_)                                                                                              \
+    // waves of a block: as many as give no compute unit more features than the others, 8 if that is a tie
+    const int cus = stream_info(stream).cus, features = g.N * grp.count;
+    int waves = 1, most = INT_MAX;
+    for (int w = 1; w <= GV_MAX_WAVES; ++w) {
+        const int rounds = (features + cus * w - 1) / (cus * w), per_cu = rounds * w;
+        if (per_cu < most || (per_cu == most && abs(w - 8) <= abs(waves - 8))) { most = per_cu; waves = w; }
+    }
+    // Weights of 64 MiB and more come from memory whatever was read before (a layer has several such), and the non-temporal hint is worth
+    // 6-10 % there (12288 x 16384 67.3 -> 59.9 us; 12288 x 4096, 96 MiB, 19.3 -> 18.0, and 16.5 -> 17.3 where it is the only weight and
+    // the memory-side cache holds it); below, what the caches still hold counts for more (4096 x 4096 8.5 -> 8.4, repeated 5.1 -> 7.4).
+    const bool nt = (int64_t)features * g.K * (int64_t)sizeof(half_t) >= (int64_t)64 << 20;
+    const dim3 grid((features + waves - 1) / waves < cus ? (features + waves - 1) / waves : cus), block(64 * waves);
+#define LG_GV_NT(MR_, E_, NT_)                                                                                      \
     do {                                                                                                            \
         /* set once per instantiation; the initialisation of a function-local static is thread-safe */              \
-        static const hipError_t attr_rc = hipFuncSetAttribute((const void*)gemv_nk_kernel<MR_, E_>, hipFuncAttributeMaxDynamicSharedMemorySize, GV_MAX_LDS); \
+        static const hipError_t attr_rc = hipFuncSetAttribute((const void*)gemv_nk_kernel<MR_, E_, NT_>, hipFuncAttributeMaxDynamicSharedMemorySize, GV_MAX_LDS); \
         (void)attr_rc;                                                                                              \
-        hipLaunchKernelGGL((gemv_nk_kernel<MR_, E_>), grid, block, smem, stream, g, grp, rm);                              \
+        hipLaunchKernelGGL((gemv_nk_kernel<MR_, E_, NT_>), grid, block, smem, stream, g, grp, rm);                  \
+    } while (0)
+#define LG_GV(MR_, E_)                       \
+    do {                                     \
+        if (nt) LG_GV_NT(MR_, E_, true);     \
+        else LG_GV_NT(MR_, E_, false);       \
     } while (0)
 #define LG_GV_MR(E_)                                 \
     switch (mr) {                                    \
@@ -135,6 +163,7 @@ int launch_gemv_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows,
     }
 #undef LG_GV_MR
 #undef LG_GV
+#undef LG_GV_NT
     return check_launch("gemv_f16");
 }
 
