@@ -16,8 +16,11 @@ void launch_gemm_fast_tile(const GemmArgs& g, const GemmGroup& grp, int wlayout,
 namespace {
 
 struct Tile { signed char mi, nj; };
-// the tiles that were the fastest, or within 1 % of it, for some problem of the sweep below; the 96-wide ones exist for K-contiguous weights
-constexpr Tile kTiles[] = {{1, 4}, {2, 4}, {3, 4}, {4, 4}, {6, 4}, {8, 4}, {2, 3}, {4, 3}, {4, 6}, {5, 6}, {6, 6}, {7, 6}, {8, 6}, {4, 8}, {5, 8}, {6, 8}, {7, 8}, {8, 8}};
+// the tiles that were the fastest, or within 1 % of it, for some problem of the sweep below; the 96-wide ones exist for K-contiguous weights,
+// those of 160 rows and more for token counts above 256 that wider tiles cover with fewer workgroups than compute units (12288 features are 128
+// columns of 96, two rows of them a full round): 384 rows x 12288 x 16384 151 -> 139 us, 420 rows 190 -> 154, 500 rows 192 -> 182.  Within a
+// layer less is left of it, as more compute units at work lower the clock: two layers of 384 rows 1157 -> 1141 us.
+constexpr Tile kTiles[] = {{1, 4}, {2, 4}, {3, 4}, {4, 4}, {6, 4}, {8, 4}, {2, 3}, {4, 3}, {5, 3}, {6, 3}, {7, 3}, {8, 3}, {4, 6}, {5, 6}, {6, 6}, {7, 6}, {8, 6}, {4, 8}, {5, 8}, {6, 8}, {7, 8}, {8, 8}};
 constexpr int kMinSliceTiles = 8;     // k-tiles of a K-slice at least: below that its ramp costs more than it hides
 constexpr int kMaxTiles = LG_ARRIVAL_COUNTERS / 2;
 
@@ -71,6 +74,7 @@ static TilePlan plan_gemm_tiles(const GemmArgs& g, int count, int wlayout, const
     auto usable = [&](const Tile& t, int cnt, int sp) {
         if (g.N % (32 * t.nj)) return false;
         if (t.nj == 3 && (wlayout == W_KN || g.epi.kind == LG_EPI_BIAS_GEGLU)) return false;  // GeGLU: a wave must hold (gate, up) pairs
+        if (t.nj == 3 && t.mi > 4 && g.M < kSequentialRows) return false;  // nothing gained where K may be sliced
         if (sp == 1) return true;
         const int64_t tiles = (int64_t)((g.M + 32 * t.mi - 1) / (32 * t.mi)) * (g.N / (32 * t.nj)) * cnt;
         if (t.mi * t.nj > 16 && sp > 2) return false;

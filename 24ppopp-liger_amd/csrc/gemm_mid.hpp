@@ -499,14 +499,13 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
         return (int64_t)m * g.ldy + n;
     };
     constexpr int CPR = TN / 8;                         // 16-byte chunks per tile row
-    constexpr int ITERS = TM * CPR / MID_THREADS;
-    static_assert(TM * CPR % MID_THREADS == 0, "every thread stores the same number of chunks");
+    constexpr int ITERS = (TM * CPR + MID_THREADS - 1) / MID_THREADS;  // (160 and 224 rows of 96: not a whole number of chunks a thread)
 #pragma unroll 4
     for (int it = 0; it < ITERS; ++it) {
         const int c = it * MID_THREADS + tid;
         const int row = c / CPR, cc = c % CPR;
         const int m = m0 + row, n = n0 + cc * 8;
-        if (m >= g.M) continue;
+        if (m >= g.M || (TM * CPR % MID_THREADS && row >= TM)) continue;
         const half8_t o = *reinterpret_cast<const half8_t*>(&smem[row * PITCH + cc * 8]);
         if (wide_store) {
             *reinterpret_cast<half8_t*>(g.Y + dest(m, n)) = o;

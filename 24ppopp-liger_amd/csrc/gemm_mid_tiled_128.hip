@@ -4,7 +4,7 @@
 namespace lg {
 
 bool launch_mid_tiled_96(int mi, bool nt, const GemmArgs& g, const GemmGroup& grp, const RowMap& rm, const MidLaunch& l) {
-    return launch_mid_heights<W_TILED, 3, 2, 4>(mi, nt, g, grp, rm, l);
+    return launch_mid_heights<W_TILED, 3, 2, 4, 5, 6, 7, 8>(mi, nt, g, grp, rm, l);
 }
 bool launch_mid_tiled_128(int mi, bool nt, const GemmArgs& g, const GemmGroup& grp, const RowMap& rm, const MidLaunch& l) {
     return launch_mid_heights<W_TILED, 4, 1, 2, 3, 4, 6, 8>(mi, nt, g, grp, rm, l);
