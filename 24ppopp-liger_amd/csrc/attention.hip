@@ -109,8 +109,7 @@ __global__ __launch_bounds__(256) void attn_decode_kernel(const half_t* __restri
             for (int c = 0; c < CPL; ++c)
 #pragma unroll
                 for (int j = 0; j < 8; ++j) p = fmaf(qf[c][j], (float)kv[u][c][j], p);
-#pragma unroll
-            for (int o = LPK / 2; o > 0; o >>= 1) p += __shfl_xor(p, o, 64);
+            p = lanes_sum<LPK>(p);
             const int key = base + u * KPL + grp;
             s[u] = (key < w_end) ? p : -1e30f;
             m_new = fmaxf(m_new, s[u]);

@@ -28,7 +28,6 @@ constexpr int PF_BC = 64;   // keys per LDS tile
 // x, v_permlane16_swap leaves {row 0, row 0, row 2, row 2} in the first and {row 1, row 1, row 3, row 3} in the second
 // (rows of 16 lanes), v_permlane32_swap {low half, low half} and {high half, high half}.  Plain VALU operations: no trip
 // through the LDS crossbar (ds_bpermute) in the middle of the softmax's dependent chain.
-typedef unsigned uint2_t __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float max_of_swapped(uint2_t r) {
     float m;
     asm("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(r[0]), "v"(r[1]));  // by hand: fmaxf would first canonicalise both bit-cast inputs
@@ -322,8 +321,9 @@ __global__ __launch_bounds__(64 * NW, NW == 4 ? 2 : 1) void attn_prefill_kernel(
 #pragma unroll
     for (int qt = 0; qt < 2; ++qt) {
         float l = l_run[qt];
-        l += __shfl_xor(l, 16, 64);
-        l += __shfl_xor(l, 32, 64);
+        auto sum = [](float a, float b) { return a + b; };
+        l = lane_step<16, false>(l, sum);
+        l = lane_step<32, false>(l, sum);
         const float inv = 1.0f / (l + 1e-6f);
         const int q = qw + qt * 16 + l16;
         if (q >= seq) continue;
