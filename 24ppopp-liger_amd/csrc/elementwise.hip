@@ -1,7 +1,7 @@
 // elementwise.hip -- bias+GELU, bias+residual and the LayerNorm family for gfx950.
 //
 // All of these are HBM-bound.  The vector kernels move 16 bytes per lane per access, keep one row
-// in registers (one HBM read, one HBM write per element) and reduce with wave64 shuffles; statistics
+// in registers (one HBM read, one HBM write per element) and reduce with wave64 butterflies; statistics
 // are two-pass in fp32 exactly as the reference computes them (cuda_kernels.cu:463-508):
 //   mean = sum(x)/n,  var = sum((x-mean)^2)/n,  y = (x-mean) * rsqrt(var + 1e-6) * gamma + beta.
 #include "common.hpp"
@@ -18,9 +18,9 @@ enum LnMode { LN_PLAIN = 0, LN_ADD_INPLACE = 1, LN_ADD_STORE = 2 };
 //                   as the reference kernel does (cuda_kernels.cu:377-408)
 // EARLY: gamma and beta are loaded with the row instead of after its statistics.  With fewer rows than fill the chip nothing hides
 // their way from memory (they are cold: a step reads a layer's weights in between), and the registers they hold cost nothing: rows of
-// 12288 halves 8.2 -> 6.3 us for 1, 8.3 -> 6.5 for 106, 9.7 -> 8.8 for 384.  The sums are the same, in the same order.
+// 12288 halves (in 256 threads) 8.2 -> 6.3 us for 1, 8.3 -> 6.5 for 106, 9.7 -> 8.8 for 384.  The sums are the same, in the same order.
 template <typename T, int MODE, int NV, bool EARLY>
-__global__ __launch_bounds__(256) void ln_vec_kernel(const T* __restrict__ src, const T* __restrict__ add,
+__global__ __launch_bounds__(512) void ln_vec_kernel(const T* __restrict__ src, const T* __restrict__ add,
                                                      const T* __restrict__ bias, const T* __restrict__ gamma,
                                                      const T* __restrict__ beta, T* sum_out, T* dst, int n) {
     typedef Vec16<T> V;
@@ -157,19 +157,21 @@ static int launch_ln(const T* src, const T* add, const T* bias, const T* gamma, 
                         (MODE == LN_PLAIN || (aligned16(add) && aligned16(bias))) &&
                         (MODE != LN_ADD_STORE || aligned16(sum_out));
     const int nvec = n / VN;
-    if (vec_ok && nvec <= 256 * 16) {
-        int block = ((nvec + 63) / 64) * 64;
-        if (block > 256) block = 256;
-        const int nv = (nvec + block - 1) / block;
+    if (vec_ok && nvec <= 512 * 8) {
+        // Up to two vectors a thread hide what the reductions wait for; rows that leave more to 256 threads take 512 (rows of 12288 halves: 32 of them
+        // 4.1 -> 3.6 us, 4096 33.4 -> 31.2; 4096 rows of 4096 would go from 11.9 to 13.1).  By the row's length alone: a row's bits do
+        // not depend on how many there are.
+        const int most = nvec > 2 * 256 ? 512 : 256;
+        const int nv = (nvec + most - 1) / most;
+        const int block = ((nvec + nv - 1) / nv + 63) / 64 * 64;
         const bool early = m <= 2 * stream_info(stream).cus;  // two workgroups on a compute unit: registers do not limit how many run
 #define LG_LN_LAUNCH(NVV) launch_ln_vec<T, MODE, NVV>(early, src, add, bias, gamma, beta, sum_out, dst, m, n, block, stream)
         if (nv <= 1) LG_LN_LAUNCH(1);
         else if (nv <= 2) LG_LN_LAUNCH(2);
+        else if (nv <= 3) LG_LN_LAUNCH(3);
         else if (nv <= 4) LG_LN_LAUNCH(4);
         else if (nv <= 6) LG_LN_LAUNCH(6);
-        else if (nv <= 8) LG_LN_LAUNCH(8);
-        else if (nv <= 12) LG_LN_LAUNCH(12);
-        else LG_LN_LAUNCH(16);
+        else LG_LN_LAUNCH(8);
 #undef LG_LN_LAUNCH
     } else {
         hipLaunchKernelGGL((ln_scalar_kernel<T, MODE>), dim3(m), dim3(256), 0, stream, src, add, bias, gamma, beta,
