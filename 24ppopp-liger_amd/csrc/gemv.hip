@@ -15,7 +15,8 @@
 // every change of blocks: with weights cycled through memory, in microseconds,
 // 16384 x 12288 68.3 -> 60.7 (6.63 TB/s), 12288 x 6144 27.0 -> 25.1, 4096 x 4096 9.8 -> 8.5, 1024 x 4096 6.4 -> 4.7; at 4 token rows 12288 x 16384
 // 72.5 -> 63.8 (in gemm_skinny.hip before, as the rows did not fit the LDS share of one block of several), 4096 x 4096 13.5 -> 10.2.
-// Each output is one fixed-order fp32 sum (per-lane partial sums over k in an order fixed by the feature, then a butterfly),
+// Each output is one fixed-order fp32 sum (four partial sums per lane over k in an order fixed by the feature, then a butterfly; with one per
+// lane 0.17 % of the outputs at K = 12288 were not the fp16 nearest to the 64-bit sum, with four 0.10 %, at the same time),
 // independent of the other token rows and of the other members of a group.
 #include <limits.h>
 #include <stdlib.h>
@@ -75,9 +76,11 @@ __global__ __launch_bounds__(GV_MAX_WAVES * 64) void gemv_nk_kernel(GemmArgs g, 
         const int member = f / g.N, n = f - member * g.N;
         const half_t* bias = members.count > 1 ? members.bias[member] : g.epi.bias;
         const float b = EPI == LG_EPI_NONE ? 0.f : (float)bias[n];  // on its way before it is needed
-        float acc[MR];
+        float acc[MR][GV_U];  // a sum for each piece of a group: shorter chains round less
 #pragma unroll
-        for (int m = 0; m < MR; ++m) acc[m] = 0.f;
+        for (int m = 0; m < MR; ++m)
+#pragma unroll
+            for (int u = 0; u < GV_U; ++u) acc[m][u] = 0.f;
         for (int it = 0; it < groups; ++it) {
             const int cur = grp;
             if (it + 1 < groups) {
@@ -90,7 +93,7 @@ __global__ __launch_bounds__(GV_MAX_WAVES * 64) void gemv_nk_kernel(GemmArgs g, 
             for (int u = 0; u < GV_U; ++u) {
 #pragma unroll
                 for (int m = 0; m < MR; ++m)
-                    acc[m] = dot8(wv[u], *reinterpret_cast<const half8_t*>(&xs[m * K + (cur * GV_U + u) * GV_KSTEP + lane * 8]), acc[m]);
+                    acc[m][u] = dot8(wv[u], *reinterpret_cast<const half8_t*>(&xs[m * K + (cur * GV_U + u) * GV_KSTEP + lane * 8]), acc[m][u]);
                 wv[u] = load(row + (int64_t)(grp * GV_U + u) * GV_KSTEP);
                 asm volatile("" ::: "memory");  // the load stays where it is written: the others are on their way beside it
                 __builtin_amdgcn_sched_barrier(0);
@@ -99,7 +102,8 @@ __global__ __launch_bounds__(GV_MAX_WAVES * 64) void gemv_nk_kernel(GemmArgs g, 
         float v = 0.f;
 #pragma unroll
         for (int m = 0; m < MR; ++m) {
-            const float s = wave_sum(acc[m]);
+            static_assert(GV_U == 4, "four partial sums");
+            const float s = wave_sum((acc[m][0] + acc[m][1]) + (acc[m][2] + acc[m][3]));
             v = lane == m ? s : v;
         }
         if (lane >= g.M) continue;
