@@ -522,7 +522,9 @@ static int gemm_fused_grouped_f16_impl(int mode, int transa, int m, int n, int k
         };
         const TilePlan together = plan(count, m), apart = plan(1, m);
         const double cost_apart = count * (apart.cost + kLaunch);
-        if (together.nsplit == 0 || (apart.nsplit != 0 && cost_apart < together.cost)) one_launch = false;
+        // (in pairs of slices three of a kind are one launch wherever the plan has them, which the estimate of four slices alone, on the low
+        // side, would not choose: 80 rows, fragment blocks of three times 6144 x 12288, in a layer 105 us, apart 130)
+        if (together.nsplit == 0 || (!together.pairs && apart.nsplit != 0 && cost_apart < together.cost)) one_launch = false;
         // A third way for groups that are many full rounds of workgroups plus a remainder (Q, K, V of 4096 rows x 6144 features: 72
         // columns of 256-wide tiles, 16 columns to a round of 256 workgroups, 8 left over): the members before the last as one
         // launch of whole rounds, the last member's leading features as whole rounds too, and its remaining features as one round

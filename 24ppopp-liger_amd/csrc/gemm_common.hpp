@@ -236,7 +236,8 @@ constexpr int kSequentialRows = 257;  // from so many token rows on every output
 struct TilePlan {
     double cost;   // estimated microseconds
     int mi, nj;    // tile (32 mi) x (32 nj)
-    int nsplit;    // K-slices (0: no tile kernel takes the problem)
+    int nsplit;    // workgroups that share the k of a tile (0: no tile kernel takes the problem)
+    bool pairs;    // each of them computes two of four K-slices
 };
 TilePlan plan_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, int wlayout, int batch, hipStream_t stream);
 int launch_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap* rows, int wlayout, int batch, hipStream_t stream, bool* handled);

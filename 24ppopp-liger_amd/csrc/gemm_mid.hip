@@ -95,7 +95,7 @@ static TilePlan plan_gemm_tiles(const GemmArgs& g, int count, int wlayout, const
                 if (!usable(t, cnt, sp)) continue;
                 const double factor = t.mi == 8 && t.nj >= 6 && g.M >= kSequentialRows ? kTallFactor : 1.0;
                 const double us = factor * tile_cost(g.M, g.N, g.K, cnt, t.mi, t.nj, sp, wlayout, cus);
-                if (us < p.cost) p = TilePlan{us, t.mi, t.nj, sp};
+                if (us < p.cost) p = TilePlan{us, t.mi, t.nj, sp, false};
             }
         }
         return p;
@@ -116,6 +116,19 @@ static TilePlan plan_gemm_tiles(const GemmArgs& g, int count, int wlayout, const
         for (int sp = 1; sp <= 8; ++sp) {
             const TilePlan a = pick(1, sp), t = pick(LG_MAX_GROUP, sp);
             if (a.nsplit && t.nsplit && a.cost < most && t.cost < least) { least = t.cost; slices = sp; }
+        }
+    }
+    // Where three want two slices and one four, both have them: the sums of four slices are added as two pairs, and the workgroups of a group
+    // compute a pair each.  6144 x 12288 alone, in two slices -> four: [out, in] 96 rows 42.4 -> 38.1 us, 128 rows 46.5 -> 39.7, fragment
+    // blocks 41.0 -> 37.0 and 43.6 -> 40.1; a layer of 106 rows with three projections 413 -> 391.  The three of 80 rows as one launch, a
+    // pair of slices to a workgroup instead of one slice: fragment blocks 100 -> 105, the step around them unchanged.  (Pairs need the loop
+    // over k to take an even number of k-tiles for each slice.)
+    if (heads && wlayout != W_KN && slices == 2 && alone.nsplit >= 4 && ktiles % 8 == 0) {
+        const TilePlan one = pick(1, 4);
+        TilePlan three = pick(LG_MAX_GROUP, 2);
+        if (one.nsplit == 4 && three.mi == MID_PAIR_MI && three.nj == MID_PAIR_NJ) {
+            three.pairs = true;
+            return count == 1 ? one : count == LG_MAX_GROUP ? three : TilePlan{};
         }
     }
     // (where members are sliced and the slices of a group do not fit the workspace, the group is not taken as one launch)
@@ -163,7 +176,7 @@ int launch_gemm_tiles_f16(const GemmArgs& g, const GemmGroup& grp, const RowMap*
         }
     }
     const int ktiles = g.K / MID_K, kt = (ktiles + p.nsplit - 1) / p.nsplit;
-    const MidLaunch l{(ktiles + kt - 1) / kt, kt, mid_turn(g.M, g.K, wlayout), si, stream};
+    const MidLaunch l{(ktiles + kt - 1) / kt, kt, mid_turn(g.M, g.K, wlayout), p.pairs, si, stream};
     const RowMap rm = rows ? *rows : RowMap{};
     // Weights that one row of tiles reads, or two whose workgroups run side by side on an XCD, need not stay in the L2: coming from memory, the
     // non-temporal hint is worth 7 % and 4 % with fragment blocks, 7 % and 2 % with [out, in], 5 % and nothing with [in, out], and costs up to

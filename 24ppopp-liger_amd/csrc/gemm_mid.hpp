@@ -35,6 +35,7 @@ constexpr int MID_MAX_SPINS = 1 << 21;
 struct MidLaunch {  // what a launch of one of the instantiations needs besides the problem
     int nsplit, kt_per_split;
     int turn;  // k-tiles by which the workgroups of neighbouring feature blocks are apart in their loop over k (0: all start at the first)
+    bool pairs;  // a workgroup computes two of four K-slices, one after the other
     StreamInfo si;
     hipStream_t stream;
 };
@@ -62,10 +63,14 @@ typedef int int4_t __attribute__((ext_vector_type(4)));
 enum { MID_BURST, MID_SPREAD, MID_PAIRS };
 // cache policy of the K-slices' sums: written through to, and read from, the level that all XCDs share
 constexpr int CACHE_DEVICE = 16;
+// the tile that comes with two K-slices to a workgroup as well, for K-contiguous weights
+constexpr int MID_PAIR_MI = 4, MID_PAIR_NJ = 6;
 // most K-slices of a tile (their sums are held in registers 64 fragments at a time)
 constexpr int mid_max_splits(int mi, int nj) { return mi * nj <= 16 ? 8 : 2; }
 
-template <int WL, int MI, int NJ, int XS, int WS, int ORDER, bool NT>
+// PAIR: a workgroup takes two K-slices of equal length, one after the other, and adds their sums.  It starts at the k-tile at which a single
+// slice of both would start, in the first or the second, so that the starts are spread as far apart.
+template <int WL, int MI, int NJ, int XS, int WS, int ORDER, bool NT, bool PAIR>
 __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmGroup grp, RowMap rm, int tiles_m, int tiles_n, float* partial, unsigned* arrivals, int nsplit, int kt_per_split, int turn, int wide_store, int region) {
     constexpr int TM = 32 * MI, TN = 32 * NJ;
     constexpr int X_TILE = TM * MID_K, W_TILE = TN * MID_K;  // halves per ring slot
@@ -156,11 +161,15 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
         }
     }
     const int64_t wstep = (WL == W_KN) ? (int64_t)MID_K * g.ldw : (WL == W_NK ? MID_K : 1024);
-    const int first = n0 / MID_TURN_COLS * turn % ktiles;
+    const int slice = PAIR ? ktiles >> 1 : ktiles, start = n0 / MID_TURN_COLS * turn % ktiles;
+    const bool other = PAIR && start >= slice;  // the second slice of the pair comes first
+    const int first = start - (other ? slice : 0);
     // the tile index is clamped to the last one: the loop body is branch-free, the extra loads refill slots nobody reads
     auto at = [&](int kt) {
-        const int t = (kt < ktiles ? kt : ktiles - 1) + first;
-        return (int64_t)(t < ktiles ? t : t - ktiles);
+        const int c = kt < ktiles ? kt : ktiles - 1;
+        const bool second = PAIR && c >= slice;
+        const int t = c - (second ? slice : 0) + first;
+        return (int64_t)((second != other ? slice : 0) + (t < slice ? t : t - slice));
     };
     auto x_tile = [&](int kt) { return reinterpret_cast<const char*>(X + at(kt) * MID_K); };
     auto w_tile = [&](int kt) { return reinterpret_cast<const char*>(W + at(kt) * wstep); };
@@ -182,6 +191,15 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
     for (int i = 0; i < MI; ++i)
 #pragma unroll
         for (int j = 0; j < NJ; ++j) acc[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+
+    // the second slice of a pair has sums of its own, all in registers
+    float4_t more[PAIR ? MI : 1][PAIR ? NJ : 1];
+    if constexpr (PAIR) {
+#pragma unroll
+        for (int i = 0; i < MI; ++i)
+#pragma unroll
+            for (int j = 0; j < NJ; ++j) more[i][j] = float4_t{0.f, 0.f, 0.f, 0.f};
+    }
 
     // LDS addresses of this lane's fragments inside a slot, per k-step (row groups 16 apart travel as instruction offsets)
     unsigned xaddr[2], waddr[2], wfrag[NJ];
@@ -228,13 +246,13 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
     constexpr int NMFMA = MI * NJ;
     constexpr int DS_SPAN = NMFMA * 3 / 4;
     // One phase = the MFMAs of one k-step with the LDS reads of the next and NL loads of later k-tiles between them
-    auto phase = [&](auto loads, auto kstep, half8_t (&ma)[MI], half8_t (&mb)[NJ], half8_t (&ra)[MI], half8_t (&rb)[NJ], unsigned rx, unsigned rw, auto&& load) {
+    auto phase = [&](float4_t (&sum)[MI][NJ], auto loads, auto kstep, half8_t (&ma)[MI], half8_t (&mb)[NJ], half8_t (&ra)[MI], half8_t (&rb)[NJ], unsigned rx, unsigned rw, auto&& load) {
         constexpr int NL = decltype(loads)::value;
         constexpr int KS = decltype(kstep)::value;
         static_for<NMFMA>([&](auto mc) {
             constexpr int m = decltype(mc)::value;
             constexpr int i = m / NJ, j = m % NJ;
-            mfma16_acc(acc[i][j], mb[j], ma[i]);
+            mfma16_acc(sum[i][j], mb[j], ma[i]);
             static_for<NL>([&](auto lc) {
                 constexpr int l = decltype(lc)::value;
                 if constexpr (l * NMFMA / NL == m) load(l);
@@ -280,34 +298,43 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
             slot = next;
             next = next == S - 1 ? 0 : next + 1;
         };
-        for (;;) {
-            {   // even k-tile: the second X tile of the last pair, then a pair of W tiles, into the slots of k-tiles kt - 1 and kt
-                const char* xg = x_tile(kt - 1 + S);
-                half_t* const xs = smem + prev * X_TILE;
-                phase(std::integral_constant<int, MI>{}, Step0{}, a0, b0, a1, b1, x_at(slot), w_at(slot), [&](int l) { issue_x(l, xg, xs); });
-                publish(std::integral_constant<int, EVEN>{});
-                const char* wg0 = w_tile(kt - 1 + S);
-                const char* wg1 = w_tile(kt + S);
-                half_t* const ws0 = wring + prev * W_TILE;
-                half_t* const ws1 = wring + slot * W_TILE;
-                phase(std::integral_constant<int, 2 * NJ>{}, Step1{}, a1, b1, a0, b0, x_at(next), w_at(next),
-                      [&](int l) { l < NJ ? issue_w(l, wg0, ws0) : issue_w(l - NJ, wg1, ws1); });
-                arrive(Step0{}, a0, b0);
+        // (two loops, one after the other, for a pair: one loop over both would move the accumulators from registers to registers)
+        auto run = [&](float4_t (&sum)[MI][NJ], int end) {
+            for (;;) {
+                {   // even k-tile: the second X tile of the last pair, then a pair of W tiles, into the slots of k-tiles kt - 1 and kt
+                    const char* xg = x_tile(kt - 1 + S);
+                    half_t* const xs = smem + prev * X_TILE;
+                    phase(sum, std::integral_constant<int, MI>{}, Step0{}, a0, b0, a1, b1, x_at(slot), w_at(slot), [&](int l) { issue_x(l, xg, xs); });
+                    publish(std::integral_constant<int, EVEN>{});
+                    const char* wg0 = w_tile(kt - 1 + S);
+                    const char* wg1 = w_tile(kt + S);
+                    half_t* const ws0 = wring + prev * W_TILE;
+                    half_t* const ws1 = wring + slot * W_TILE;
+                    phase(sum, std::integral_constant<int, 2 * NJ>{}, Step1{}, a1, b1, a0, b0, x_at(next), w_at(next),
+                          [&](int l) { l < NJ ? issue_w(l, wg0, ws0) : issue_w(l - NJ, wg1, ws1); });
+                    arrive(Step0{}, a0, b0);
+                }
+                if (++kt >= end) break;
+                advance();
+                {   // odd k-tile: the first X tile of the pair
+                    phase(sum, std::integral_constant<int, 0>{}, Step0{}, a0, b0, a1, b1, x_at(slot), w_at(slot), [](int) {});
+                    publish(std::integral_constant<int, ODD>{});
+                    const char* xg = x_tile(kt - 1 + S);
+                    half_t* const xs = smem + prev * X_TILE;
+                    phase(sum, std::integral_constant<int, MI>{}, Step1{}, a1, b1, a0, b0, x_at(next), w_at(next), [&](int l) { issue_x(l, xg, xs); });
+                    arrive(Step0{}, a0, b0);
+                }
+                if (++kt >= end) break;
+                advance();
             }
-            if (++kt >= ktiles) break;
+        };
+        run(acc, slice);
+        if constexpr (PAIR) {
             advance();
-            {   // odd k-tile: the first X tile of the pair
-                phase(std::integral_constant<int, 0>{}, Step0{}, a0, b0, a1, b1, x_at(slot), w_at(slot), [](int) {});
-                publish(std::integral_constant<int, ODD>{});
-                const char* xg = x_tile(kt - 1 + S);
-                half_t* const xs = smem + prev * X_TILE;
-                phase(std::integral_constant<int, MI>{}, Step1{}, a1, b1, a0, b0, x_at(next), w_at(next), [&](int l) { issue_x(l, xg, xs); });
-                arrive(Step0{}, a0, b0);
-            }
-            if (++kt >= ktiles) break;
-            advance();
+            run(more, ktiles);
         }
     } else {
+        static_assert(!PAIR, "pairs of slices: only where loads go out in pairs");
         // The loads of k-tiles kt + XS and kt + WS go out once tile kt is done with: NOW of them under its second k-step and the others under
         // the first k-step of the next.
         constexpr int SMAX = XS > WS ? XS : WS, SMIN = XS < WS ? XS : WS;
@@ -333,7 +360,7 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
             const char* wg0 = w_tile(kt - 1 + WS);
             half_t* const xs0 = smem + xprev * X_TILE;
             half_t* const ws0 = wring + wprev * W_TILE;
-            phase(std::integral_constant<int, NLOAD - NOW>{}, Step0{}, a0, b0, a1, b1, x_at(xslot), w_at(wslot), [&](int l) { issue_one(l + NOW, xg0, wg0, xs0, ws0); });
+            phase(acc, std::integral_constant<int, NLOAD - NOW>{}, Step0{}, a0, b0, a1, b1, x_at(xslot), w_at(wslot), [&](int l) { issue_one(l + NOW, xg0, wg0, xs0, ws0); });
             publish(std::integral_constant<int, (SMIN - 2) * NLOAD + NDEEP>{});
             const char* xg = x_tile(kt + XS);
             const char* wg = w_tile(kt + WS);
@@ -343,7 +370,7 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
             wprev = wslot;
             xslot = xslot == XS - 1 ? 0 : xslot + 1;
             wslot = wslot == WS - 1 ? 0 : wslot + 1;
-            phase(std::integral_constant<int, NOW>{}, Step1{}, a1, b1, a0, b0, x_at(xslot), w_at(wslot), [&](int l) { issue_one(l, xg, wg, xs, ws); });
+            phase(acc, std::integral_constant<int, NOW>{}, Step1{}, a1, b1, a0, b0, x_at(xslot), w_at(wslot), [&](int l) { issue_one(l, xg, wg, xs, ws); });
             arrive(Step0{}, a0, b0);
         } while (++kt < ktiles);
     }
@@ -353,14 +380,20 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
 #pragma unroll
     for (int i = 0; i < MI; ++i)
 #pragma unroll
-        for (int j = 0; j < NJ; ++j) asm volatile("" : "+a"(acc[i][j]));
+        for (int j = 0; j < NJ; ++j) {
+            asm volatile("" : "+a"(acc[i][j]));
+            if constexpr (PAIR) {
+                asm volatile("" : "+a"(more[i][j]));
+                acc[i][j] += more[i][j];
+            }
+        }
 
     // ---- epilogue: acc[i][j][r] = Y[m0 + wm*16*MI + i*16 + l16][n0 + wn*16*NJ + j*16 + 4*lk + r] ---------------------------
     // ---- K-slices: the slice of a tile that arrives last takes the others' fp32 sums from the stream's workspace (lane-contiguous),
-    // adds all of them in slice order and goes on to the epilogue.  Nobody waits for a workgroup that may not be running: the wait
-    // below is for slices that have already arrived and are storing, microseconds.  It is bounded (a second or so) for a caller who
-    // breaks the rule that one launch runs at a time on a workspace (a captured graph replayed on two streams at once): wrong sums
-    // then, but the launch ends.  The counters are back at zero when the launch ends.
+    // adds all of them in slice order (four as two pairs, as workgroups that take a pair each do) and goes on to the epilogue.  Nobody waits
+    // for a workgroup that may not be running: the wait below is for slices that have already arrived and are storing, microseconds.  It is
+    // bounded (a second or so) for a caller who breaks the rule that one launch runs at a time on a workspace (a captured graph replayed on
+    // two streams at once): wrong sums then, but the launch ends.  The counters are back at zero when the launch ends.
     if (nsplit > 1) {
         constexpr int SLICE = MI * NJ * MID_THREADS * 16;  // bytes
         // Small tiles: every slice stores its sums, then counts itself in (one trip to the counter).  Large ones: a slice first learns
@@ -435,6 +468,9 @@ __global__ __launch_bounds__(MID_THREADS, 1) void gemm_f16_mid(GemmArgs g, GemmG
 #pragma unroll
                             for (int r = 0; r < 4; ++r) v[r] = sp < nsplit ? w[r] : v[r];
                         }
+                        const float4_t pairs = (p[0][f] + p[1][f]) + (p[2][f] + p[3][f]);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) v[r] = nsplit == 4 ? pairs[r] : v[r];
                         acc[(f0 + f) / NJ][(f0 + f) % NJ] = v;
                     }
             }
@@ -531,7 +567,7 @@ constexpr int mid_order(int wl, int mi, int nj) {
     return mi == 1 && nj == 4 && wl != W_KN ? MID_BURST : mid_depth(mi, nj) > 3 || nj == 4 ? MID_PAIRS : MID_SPREAD;
 }
 
-template <int WL, int MI, int NJ, int ORDER, bool NT>
+template <int WL, int MI, int NJ, int ORDER, bool NT, bool PAIR = false>
 static void launch_mid_order(const GemmArgs& g, const GemmGroup& grp, const RowMap& rm, const MidLaunch& l) {
     constexpr int XS = mid_xs(MI, NJ), WS = mid_ws(MI, NJ);
     const int tiles_m = (g.M + 32 * MI - 1) / (32 * MI), tiles_n = g.N / (32 * NJ) * grp.count;
@@ -543,7 +579,7 @@ static void launch_mid_order(const GemmArgs& g, const GemmGroup& grp, const RowM
     for (int i = 0; i < grp.count; ++i)
         if (!aligned16(grp.Y[i]) || (g.epi.kind == LG_EPI_BIAS_HEADS || g.epi.kind == LG_EPI_BIAS_HEADS_ROWS ? (g.epi.d % 8 != 0) : (grp.ldy[i] % 8 != 0))) wide = 0;
     // set once per instantiation; the initialisation of a function-local static is thread-safe
-    static const hipError_t attr_rc = hipFuncSetAttribute((const void*)gemm_f16_mid<WL, MI, NJ, XS, WS, ORDER, NT>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
+    static const hipError_t attr_rc = hipFuncSetAttribute((const void*)gemm_f16_mid<WL, MI, NJ, XS, WS, ORDER, NT, PAIR>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)smem);
     (void)attr_rc;
     // Tiles of 160 to 224 rows are placed where they make more than one round (2560 rows x 12288 x 16384 822 -> 788 us, 5120 x 4096 x 4096 152 ->
     // 142); in one round it gains nothing (1280 x 8192 x 2048 41 -> 41.5), and smaller tiles lose by it.
@@ -559,12 +595,14 @@ static void launch_mid_order(const GemmArgs& g, const GemmGroup& grp, const RowM
         }
         if (region) region |= P << 8;
     }
-    hipLaunchKernelGGL((gemm_f16_mid<WL, MI, NJ, XS, WS, ORDER, NT>), dim3((unsigned)blocks), dim3(MID_THREADS), smem, l.stream, g, grp, rm, tiles_m, tiles_n,
+    hipLaunchKernelGGL((gemm_f16_mid<WL, MI, NJ, XS, WS, ORDER, NT, PAIR>), dim3((unsigned)blocks), dim3(MID_THREADS), smem, l.stream, g, grp, rm, tiles_m, tiles_n,
                        l.si.ws, l.si.arrivals, l.nsplit, l.kt_per_split, l.turn, wide, region);
 }
 
 template <int WL, int MI, int NJ, bool NT>
 static void launch_mid_tile(const GemmArgs& g, const GemmGroup& grp, const RowMap& rm, const MidLaunch& l) {
+    if constexpr (WL != W_KN && MI == MID_PAIR_MI && NJ == MID_PAIR_NJ)
+        if (l.pairs) return launch_mid_order<WL, MI, NJ, MID_PAIRS, NT, true>(g, grp, rm, l);
     if constexpr (WL == W_KN && MI == 4 && NJ == 6 && !NT)
         if (g.M >= kSequentialRows) return launch_mid_order<WL, MI, NJ, MID_BURST, NT>(g, grp, rm, l);
     launch_mid_order<WL, MI, NJ, mid_order(WL, MI, NJ), NT>(g, grp, rm, l);
