@@ -1,6 +1,6 @@
 // attention_aux.hip -- the reference-shaped helper kernels around the attention GEMMs:
 // Q/K/V bias + head transpose, scale+mask+softmax (in place), transpose back.
-// All are pure HBM streaming; 16-byte accesses, one wave64 per softmax row.
+// All are pure HBM streaming; 16-byte accesses.
 #include "common.hpp"
 
 namespace lg {
@@ -114,33 +114,76 @@ static int launch_transpose(T* dst, const T* src, int batch, int seq, int head_n
 
 // ---- softmax (attention_kernels.cu:395-680) -----------------------------------------------------------
 //   t = qk*scalar + (1 - mask)*(-10000);  p = exp(t - max t);  out = p / (sum p + 1e-6)
-// One wave64 per row, the row held in registers as NC vectors of 16 bytes per lane, at any alignment (global memory takes such loads
-// and stores as whole ones; only the last vector of a row that is not whole goes element by element).  Bound by memory: 2 x 48 x 333
-// rows of 333 halves 22 us, 44 in one workgroup and three passes per row, which rows longer than 512 vectors still take.
-template <typename T, int NC>
+// LPR lanes per row, the row held in registers as NC vectors of 16 bytes per lane, at any alignment (global memory takes such loads and
+// stores as whole ones; a last vector that is not whole is read as one too, with elements before it).  What a row costs besides its
+// elements -- its place in the mask, two butterflies, a reciprocal -- is a few hundred vector instructions for a wave however many rows it
+// holds, and short rows are bound by it: so a wave has as many rows as it has room for, two vectors a lane from 33 vectors on.  One row a
+// wave before, us, fp16: 8 x 48 heads, 128 tokens 18.3 -> 6.1, 4 x 16, 200 7.3 -> 4.6, 2 x 48, 333 19.4 -> 13.6, 512 20.6 -> 18.0; fp32
+// 8 x 48, 128 15.2 -> 8.3, 4 x 16, 200 6.6 -> 5.1, 2 x 48, 333 20.4 -> 18.8, longer ones level (memory).  Rows longer than 512 vectors take a workgroup
+// and three passes each.
+// the vector without its first `bytes` bytes (a multiple of the element's size); what comes after its last ones is anything
+template <int SIZE, typename V>
+__device__ __forceinline__ V vec_from(V v, int bytes) {
+    typedef unsigned uint4_t __attribute__((ext_vector_type(4)));
+    const uint4_t u = __builtin_bit_cast(uint4_t, v);
+    const bool by8 = bytes & 8, by4 = bytes & 4;
+    const unsigned a0 = by8 ? u[2] : u[0], a1 = by8 ? u[3] : u[1];
+    unsigned b0 = by4 ? a1 : a0, b1 = by4 ? u[2] : a1, b2 = by4 ? u[3] : u[2], b3 = u[3];
+    if (SIZE == 2) {
+        const unsigned bits = (bytes & 2) * 8;
+        b0 = __builtin_amdgcn_alignbit(b1, b0, bits);
+        b1 = __builtin_amdgcn_alignbit(b2, b1, bits);
+        b2 = __builtin_amdgcn_alignbit(b3, b2, bits);
+        b3 = __builtin_amdgcn_alignbit(0, b3, bits);
+    }
+    return __builtin_bit_cast(V, uint4_t{b0, b1, b2, b3});
+}
+
+template <typename T, int NC, int LPR>
 __global__ __launch_bounds__(256) void softmax_wave_kernel(T* buf, const T* __restrict__ mask, int seq, int head_num,
                                                            int64_t rows, float scalar) {
     constexpr int VN = Vec16<T>::N;
+    typedef T aligned_t __attribute__((ext_vector_type(VN)));
     typedef T vec_t __attribute__((ext_vector_type(VN), aligned(sizeof(T))));
-    const int lane = threadIdx.x & 63;
-    const int64_t row = (int64_t)blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+    const int lane = threadIdx.x % LPR;
+    const int64_t row = (int64_t)blockIdx.x * (256 / LPR) + threadIdx.x / LPR;
     if (row >= rows) return;
-    const int64_t b = row / ((int64_t)head_num * seq);
-    const int sq = (int)(row % seq);
+    int64_t b;
+    int sq;
+    if (rows <= 0x7fffffff) {
+        const unsigned head = (unsigned)row / (unsigned)seq;
+        b = head / (unsigned)head_num;
+        sq = (int)((unsigned)row - head * (unsigned)seq);
+    } else {
+        b = row / ((int64_t)head_num * seq);
+        sq = (int)(row % seq);
+    }
     T* p = buf + row * seq;
     const T* mrow = mask + (b * seq + sq) * (int64_t)seq;
+    // in a row that is no whole number of vectors, whether the lanes' vectors c are all inside
+    auto inside = [&](int c) { return seq % VN == 0 || (c + 1) * LPR * VN <= seq; };
     float t[NC][VN];
     float mx = -1e20f;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-        const int i = (lane + c * 64) * VN;  // this lane's first element of the vector
+        const int i = (lane + c * LPR) * VN;  // this lane's first element of the vector
 #pragma unroll
         for (int j = 0; j < VN; ++j) t[c][j] = -1e20f;
-        if (i + VN <= seq) {
-            const vec_t a = *reinterpret_cast<const vec_t*>(p + i), m = *reinterpret_cast<const vec_t*>(mrow + i);
+        if (inside(c)) {
+            if (i < seq) {
+                const vec_t a = *reinterpret_cast<const vec_t*>(p + i), m = *reinterpret_cast<const vec_t*>(mrow + i);
 #pragma unroll
-            for (int j = 0; j < VN; ++j) t[c][j] = (float)a[j] * scalar + (1.0f - (float)m[j]) * -10000.0f;
-        } else if (i < seq) {
+                for (int j = 0; j < VN; ++j) t[c][j] = (float)a[j] * scalar + (1.0f - (float)m[j]) * -10000.0f;
+            }
+        } else if (seq >= VN) {
+            // the last vector, which is not whole, comes with elements before it, and the lanes beyond read the same one
+            const int at = min(i, seq - VN), skip = (i - at) * (int)sizeof(T);
+            const aligned_t a = vec_from<sizeof(T)>((aligned_t)*reinterpret_cast<const vec_t*>(p + at), skip);
+            const aligned_t m = vec_from<sizeof(T)>((aligned_t)*reinterpret_cast<const vec_t*>(mrow + at), skip);
+#pragma unroll
+            for (int j = 0; j < VN; ++j)
+                if (i + j < seq) t[c][j] = (float)a[j] * scalar + (1.0f - (float)m[j]) * -10000.0f;
+        } else {
 #pragma unroll
             for (int j = 0; j < VN; ++j)
                 if (i + j < seq) t[c][j] = ldf(p + i + j) * scalar + (1.0f - ldf(mrow + i + j)) * -10000.0f;
@@ -148,24 +191,29 @@ __global__ __launch_bounds__(256) void softmax_wave_kernel(T* buf, const T* __re
 #pragma unroll
         for (int j = 0; j < VN; ++j) mx = fmaxf(mx, t[c][j]);
     }
-    mx = wave_max(mx);
+    mx = lanes_max<LPR>(mx);
     float sum = 0.f;
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-        const int i = (lane + c * 64) * VN;
-        if (i < seq) {
+        const int i = (lane + c * LPR) * VN;
 #pragma unroll
-            for (int j = 0; j < VN; ++j) {
-                t[c][j] = __expf(t[c][j] - mx);
-                if (i + j < seq) sum += t[c][j];
+        for (int j = 0; j < VN; ++j) t[c][j] = __expf(t[c][j] - mx);
+        if (inside(c)) {
+            if (i < seq) {
+#pragma unroll
+                for (int j = 0; j < VN; ++j) sum += t[c][j];
             }
+        } else {
+#pragma unroll
+            for (int j = 0; j < VN; ++j)
+                if (i + j < seq) sum += t[c][j];
         }
     }
-    sum = wave_sum(sum);
+    sum = lanes_sum<LPR>(sum);
     const float inv = 1.0f / (sum + 1e-6f);
 #pragma unroll
     for (int c = 0; c < NC; ++c) {
-        const int i = (lane + c * 64) * VN;
+        const int i = (lane + c * LPR) * VN;
         if (i + VN <= seq) {
             vec_t o;
 #pragma unroll
@@ -210,16 +258,19 @@ static int launch_softmax(T* buf, const T* mask, int batch, int seq, int head_nu
     constexpr int VN = Vec16<T>::N;
     const int nvec = (seq + VN - 1) / VN;
     if (nvec <= 64 * 8) {
-        const int nc = (nvec + 63) / 64;
-        const int64_t grid = (rows + 3) / 4;
+        const int lanes = nvec <= 8 ? 8 : nvec <= 16 ? 16 : nvec <= 64 ? 32 : 64;
+        const int64_t grid = (rows + 256 / lanes - 1) / (256 / lanes);
         if (grid > 0x7fffffff) { set_error("attn_softmax: too many rows"); return LG_ERR_INVALID; }
-#define LG_SM_LAUNCH(NCC)                                                                                          \
-    hipLaunchKernelGGL((softmax_wave_kernel<T, NCC>), dim3((unsigned)grid), dim3(256), 0, stream, buf, mask, seq,   \
+#define LG_SM_LAUNCH(NCC, LANES)                                                                                          \
+    hipLaunchKernelGGL((softmax_wave_kernel<T, NCC, LANES>), dim3((unsigned)grid), dim3(256), 0, stream, buf, mask, seq,   \
                        head_num, rows, scalar)
-        if (nc <= 1) LG_SM_LAUNCH(1);
-        else if (nc <= 2) LG_SM_LAUNCH(2);
-        else if (nc <= 4) LG_SM_LAUNCH(4);
-        else LG_SM_LAUNCH(8);
+        if (nvec <= 8) LG_SM_LAUNCH(1, 8);
+        else if (nvec <= 16) LG_SM_LAUNCH(1, 16);
+        else if (nvec <= 32) LG_SM_LAUNCH(1, 32);
+        else if (nvec <= 64) LG_SM_LAUNCH(2, 32);
+        else if (nvec <= 128) LG_SM_LAUNCH(2, 64);
+        else if (nvec <= 256) LG_SM_LAUNCH(4, 64);
+        else LG_SM_LAUNCH(8, 64);
 #undef LG_SM_LAUNCH
     } else {
         if (rows > 0x7fffffff) { set_error("attn_softmax: too many rows"); return LG_ERR_INVALID; }

@@ -70,9 +70,9 @@ __device__ __forceinline__ float lane_step(float v, Op op) {
 // all steps from G / 2 down to 1: every lane of G adjacent ones gets the result over them
 template <int G, class Op>
 __device__ __forceinline__ float lanes_reduce(float v, Op op) {
-    static_assert(G == 4 || G == 8 || G == 16 || G == 64, "groups in use");
+    static_assert(G == 4 || G == 8 || G == 16 || G == 32 || G == 64, "groups in use");
     if constexpr (G == 64) v = lane_step<32, false>(v, op);
-    if constexpr (G == 64) v = lane_step<16, false>(v, op);
+    if constexpr (G >= 32) v = lane_step<16, false>(v, op);
     if constexpr (G >= 16) v = lane_step<8, false>(v, op);
     if constexpr (G >= 8) v = lane_step<4, (G >= 16)>(v, op);
     v = lane_step<2, false>(v, op);
@@ -83,9 +83,11 @@ __device__ __forceinline__ float lanes_sum(float v) {
     return lanes_reduce<G>(v, [](float a, float b) { return a + b; });
 }
 __device__ __forceinline__ float wave_sum(float v) { return lanes_sum<kWave>(v); }
-__device__ __forceinline__ float wave_max(float v) {
-    return lanes_reduce<kWave>(v, [](float a, float b) { return fmaxf(a, b); });
+template <int G>
+__device__ __forceinline__ float lanes_max(float v) {
+    return lanes_reduce<G>(v, [](float a, float b) { return fmaxf(a, b); });
 }
+__device__ __forceinline__ float wave_max(float v) { return lanes_max<kWave>(v); }
 
 // Block-wide sum for up to 1024 threads (16 waves); every thread gets the result.
 // `scratch` must hold 16 floats; two back-to-back calls may reuse it (barrier at entry).
